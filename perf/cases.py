@@ -17,6 +17,11 @@ operator), ``st27`` (27-point stencil), ``band`` (banded, dense enough for
 the tile path), ``rmat`` (power law).  ``prepare`` makes operands on the GPU.
 A random structure is drawn once per case and relabelled by the seed (rows and
 columns permuted, so that the sizes of C stay), and the values are the seed's.
+
+The handles work on one torch stream, on which the results are allocated too,
+as a program with several handles needs: torch hands a dropped result's memory
+out again at once to work of the stream it belongs to, and kernels of another
+stream may still be reading or writing there.
 """
 from __future__ import annotations
 
@@ -28,6 +33,14 @@ import torch
 import tilespgemm_amd as tsg
 
 DEV = "cuda:0"
+_stream = None
+
+
+def _work_stream():
+    global _stream
+    if _stream is None:
+        _stream = torch.cuda.Stream()
+    return _stream
 
 
 def listed():
@@ -265,13 +278,16 @@ def prepare(case, seed):
     if op == "served":
         state["server"] = tsg.Server(0, workers=3, max_batch=64)
         return state
+    stream = _work_stream()
+    stream.wait_stream(torch.cuda.current_stream())
     mode = tsg.FP_SEPARATE if case.get("separate") else tsg.FP_FUSED
-    h = state["handle"] = tsg.Handle(0, fp_mode=mode)
-    if op == "values":
-        ic, nnz = h.symbolic(*pairs[0])
-        state["ic"] = ic
-        state["jc"] = torch.empty(nnz, dtype=torch.int32, device=DEV)
-        state["c"] = torch.empty(nnz, dtype=torch.float64, device=DEV)
+    with torch.cuda.stream(stream):
+        h = state["handle"] = tsg.Handle(0, fp_mode=mode)
+        if op == "values":
+            ic, nnz = h.symbolic(*pairs[0])
+            state["ic"] = ic
+            state["jc"] = torch.empty(nnz, dtype=torch.int32, device=DEV)
+            state["c"] = torch.empty(nnz, dtype=torch.float64, device=DEV)
     return state
 
 
@@ -287,7 +303,11 @@ def run(state):
         server = state["server"]
         tickets = [server.submit(A, B) for A, B in pairs]
         return [list(server.fetch_device(t)[:3]) for t in tickets]
-    h = state["handle"]
+    with torch.cuda.stream(_work_stream()):
+        return _run_handle(op, state["handle"], pairs, state)
+
+
+def _run_handle(op, h, pairs, state):
     if op == "batch":
         arr, ic, per, _, tot = h.batch_symbolic(pairs)
         jc = torch.empty(max(tot, 1), dtype=torch.int32, device=DEV)
