@@ -1,5 +1,5 @@
-// Flat product expansion, LDS hash tables, ordered accumulation and
-// group-wide sorts shared by the row path and the tile path (gfx950, wave64).
+// Flat product expansion, LDS hash tables and ordered accumulation shared by
+// the row path and the tile path (gfx950, wave64).
 #pragma once
 
 #include "tsg_device.h"
@@ -243,128 +243,3 @@ __device__ __forceinline__ void ordered_accumulate(bool act, int slot, double a,
         wave_lds_fence();
     }
 }
-
-// Bitonic sort of n (power of two) keys with values, by the G lanes of a
-// group (G <= 64, so wave-synchronous) or by a whole block (GROUP_IS_BLOCK).
-template <int G>
-__device__ __forceinline__ void bitonic_sort_group(int *keys, double *vals, int n) {
-    const int l = __lane_id() & (G - 1);
-    for (int kk = 2; kk <= n; kk <<= 1) {
-        for (int j = kk >> 1; j > 0; j >>= 1) {
-            for (int i = l; i < n; i += G) {
-                int ixj = i ^ j;
-                if (ixj > i) {
-                    int ki = keys[i], kx = keys[ixj];
-                    bool asc = (i & kk) == 0;
-                    if ((ki > kx) == asc) {
-                        keys[i] = kx;
-                        keys[ixj] = ki;
-                        double t = vals[i];
-                        vals[i] = vals[ixj];
-                        vals[ixj] = t;
-                    }
-                }
-            }
-            wave_lds_fence();
-        }
-    }
-}
-
-// Stable LSD radix sort of n keys (with values) by the G lanes of a group:
-// 8-bit digits of (key - kmin) over `bits` bits; src/dst ping-pong buffers of
-// n entries each; hist is a 256-entry LDS array owned by the group.  Each
-// chunk of G entries is split by digit with ballots (lanes with equal digits
-// keep their order), so the sort is stable.  Returns true when the sorted
-// data ends in dst.
-template <int G>
-__device__ __forceinline__ bool radix_sort_group(int *skeys, double *svals, int *dkeys,
-                                                 double *dvals, int n, int kmin, int bits,
-                                                 unsigned *hist) {
-    const int l = __lane_id() & (G - 1);
-    const int gb = __lane_id() & ~(G - 1);
-    const unsigned long long gm = G == 64 ? ~0ull : ((1ull << G) - 1);
-    const unsigned long long below = (1ull << l) - 1;
-    bool in_dst = false;
-    for (int shift = 0; shift < bits; shift += 8) {
-        int *ik = in_dst ? dkeys : skeys;
-        double *iv = in_dst ? dvals : svals;
-        int *ok = in_dst ? skeys : dkeys;
-        double *ov = in_dst ? svals : dvals;
-        for (int i = l; i < 256; i += G) hist[i] = 0u;
-        wave_lds_fence();
-        // histogram: one add per digit group of a chunk
-        for (int c0 = 0; c0 < n; c0 += G) {
-            const bool act = c0 + l < n;
-            const unsigned d = act ? ((unsigned)(ik[c0 + l] - kmin) >> shift) & 255u : 0u;
-            unsigned long long m = (__ballot(act) >> gb) & gm;
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const unsigned long long bb = (__ballot((d >> b) & 1u) >> gb) & gm;
-                m &= ((d >> b) & 1u) ? bb : ~bb;
-            }
-            if (act && (m & below) == 0) hist[d] += (unsigned)__popcll(m);
-            wave_lds_fence();
-        }
-        // exclusive scan of the 256 counts: 256/G consecutive bins per lane,
-        // then one group scan of the lanes' sums
-        {
-            constexpr int PER = 256 / G;
-            int cnt[PER];
-            int sum = 0;
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                cnt[q] = (int)hist[l * PER + q];
-                sum += cnt[q];
-            }
-            int run = group_incl_scan<G>(sum) - sum;
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                hist[l * PER + q] = (unsigned)run;
-                run += cnt[q];
-            }
-        }
-        wave_lds_fence();
-        // stable scatter
-        for (int c0 = 0; c0 < n; c0 += G) {
-            const bool act = c0 + l < n;
-            const int key = act ? ik[c0 + l] : 0;
-            const double val = act ? iv[c0 + l] : 0.0;
-            const unsigned d = act ? ((unsigned)(key - kmin) >> shift) & 255u : 0u;
-            unsigned long long m = (__ballot(act) >> gb) & gm;
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const unsigned long long bb = (__ballot((d >> b) & 1u) >> gb) & gm;
-                m &= ((d >> b) & 1u) ? bb : ~bb;
-            }
-            const int rank = __popcll(m & below);
-            const unsigned base = act ? hist[d] : 0u;
-            wave_lds_fence();
-            if (act) {
-                ok[base + rank] = key;
-                ov[base + rank] = val;
-                if ((m >> l) == 1ull) hist[d] = base + (unsigned)__popcll(m);   // last of its digit
-            }
-            wave_lds_fence();
-        }
-        in_dst = !in_dst;
-    }
-    return in_dst;
-}
-
-__device__ __forceinline__ void bitonic_sort_keys_group64(int *keys, int n) {
-    const int l = __lane_id();
-    for (int kk = 2; kk <= n; kk <<= 1) {
-        for (int j = kk >> 1; j > 0; j >>= 1) {
-            for (int i = l; i < n; i += 64) {
-                int ixj = i ^ j;
-                if (ixj > i) {
-                    int ki = keys[i], kx = keys[ixj];
-                    bool asc = (i & kk) == 0;
-                    if ((ki > kx) == asc) { keys[i] = kx; keys[ixj] = ki; }
-                }
-            }
-            wave_lds_fence();
-        }
-    }
-}
-

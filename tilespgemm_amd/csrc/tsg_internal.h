@@ -114,8 +114,8 @@ struct StageTimer {
 
 // ------------------------------------------------------------ row path
 // Tuning parameters of the row path (tsg_set_row_bins): rows with at most
-// bin1 / bin2 / bin3 intermediate products go to the 16-, 32- and 64-lane
-// hash kernels, the rest to the big-row path.
+// bin1 products take 16 lanes each, up to bin2 and bin3 a wave each, the rest
+// go to the big-row path.
 struct RowTuning {
     int bin1 = 64, bin2 = 256, bin3 = 1024;
     int64_t item_sort_min = int64_t(1) << 18;  // big-row items column-ordered from this many
@@ -144,13 +144,6 @@ struct RowPlan {
     // bins: small rows (by products) and big rows
     int *bin_rows = nullptr;         // [m] rows grouped by bin
     int *bin_start = nullptr;        // [nbins+1] device
-    int2 *span = nullptr;            // [m] column span (lo, hi) of each small row
-    uint8_t *narrow3 = nullptr;      // [m] class of each row of the 1024-product bin:
-                                     // 1 narrow, 2/3 span <= 2048 words with > / <= 512
-                                     // outputs, 0 wider
-    int *rows3 = nullptr;            // that bin's class-1 rows first, class-0 rows last
-    int *rows3r = nullptr;           // its class-2 rows first, class-3 rows last
-    int n3cls[4] = {0, 0, 0, 0};     // (host) rows per class
     int bin_start_h[16] = {0};       // host copy (after symbolic)
     int nbins = 0;
     // big-row structures

@@ -10,10 +10,12 @@
 //     order (thmkl_dcsrmultcsr.c:61-72), so results are bitwise equal to the
 //     CPU reference.  Products are expanded flat, a wave at a time in A-row
 //     order ("t-major"); lanes of one batch that hit the same accumulator slot
-//     are serialized in lane order by tag rounds (LDS atomicMin on a small
-//     bucket table), so the parallel sum equals the sequential one.
-//   * Small rows (<= SMALL_PROD products): one lane group per row, LDS hash
-//     table, output sorted by an in-LDS bitonic sort.
+//     take turns in product order (one B row after the other, or tag rounds:
+//     LDS atomicMin on a small bucket table), so the parallel sum equals the
+//     sequential one.
+//   * Small rows (<= SMALL_PROD products): one lane group per row with all its
+//     products in registers (tsg_flat.h); an output's place is its column's
+//     rank in a two-level bitmap, so C comes out sorted with no hash or sort.
 //   * Big rows: the symbolic phase cuts each row's column span into bands of
 //     65536 columns, marks the row's columns of a band in an LDS bitmap and
 //     records the count of every 1024-column sub-block (and, when memory
@@ -29,6 +31,7 @@
 #include <cmath>
 #include "tsg_device.h"
 #include "tsg_expand.h"
+#include "tsg_flat.h"
 
 #include <algorithm>
 #include <map>
@@ -37,9 +40,13 @@
 namespace {
 
 constexpr int SMALL_PROD = 1024;       // rows up to this many products: small path
-constexpr int NBINS = 5;               // 0: empty, 1..3: small, 4: big
-constexpr int BIN_BIG = 4;
-constexpr int bin_limit[NBINS] = {0, 64, 256, SMALL_PROD, 0x7fffffff};
+constexpr int MID_PROD = 512;          // of these, up to this many: 8 registers a lane
+constexpr int FLAT_ENT = 64;           // A entries of a small row kept in LDS; rows with
+                                       // more (1024 kept: 17 KB instead of 5.5) have a bin
+constexpr int NBINS = 7;               // 0: empty, 1..4: small, 5: small of many entries, 6: big
+constexpr int BIN_MANY = 5;
+constexpr int BIN_BIG = 6;
+constexpr int bin_limit[NBINS] = {0, 64, 256, MID_PROD, SMALL_PROD, SMALL_PROD, 0x7fffffff};
 
 constexpr int SUB_SHIFT = 10;          // sub-block = 1024 columns
 constexpr int BAND_SHIFT = 6;          // symbolic band = 64 sub-blocks (65536 columns)
@@ -61,40 +68,37 @@ constexpr int RANK_U = 8;
 // ER batch rows of <= 1024 products 62.0 -> 57.2 ms, 27-point 64^3 3.05 ->
 // 2.93 ms.
 constexpr int SMALL_U = 8;
-// Rows of the 64-lane bin whose column span fits 1024 bitmap words and whose
-// outputs number at most 512 (meshes and stencils) run in the rank kernel's
-// 1024-word variant: 10 KB of LDS per row instead of 25 KB.
-constexpr int NARROW_WORDS = 1024;
-constexpr int NARROW_OUT = NARROW_WORDS / 2;
 constexpr int BIG_SYM_U = 4;
 constexpr int ITEM_U = 4;
 
 struct BinStarts { int s[NBINS + 1]; };
 
-// Row bins by intermediate products: (0, l1] -> 16-lane groups with 128 hash
-// slots, (l1, l2] -> 32 lanes and 512 slots, (l2, l3] -> 64 lanes and 2048
-// slots, above l3 -> the big-row path.  Each small kernel is exact for any
-// row up to bin_limit[b] products (hash load <= 1/2), so any limits with
-// l1 <= 64, l2 <= 256, l3 <= 1024 (checked on the host) are valid; they are
-// tuning parameters (tsg_set_row_bins).
+// Row bins by intermediate products: (0, l1] -> 16 lanes a row, (l1, l2],
+// (l2, MID_PROD] and (MID_PROD, l3] -> a wave a row with 4, 8 and 16 products
+// a lane (those with more than FLAT_ENT A entries in a bin of their own),
+// above l3 -> the big-row path.  Each small kernel is exact for any row up to
+// bin_limit[b] products, so any limits with l1 <= 64, l2 <= 256, l3 <= 1024
+// (checked on the host) are valid; they are tuning parameters
+// (tsg_set_row_bins).
 struct BinLimits { int l1, l2, l3; };
 
-__device__ __forceinline__ int bin_of(int64_t prod, BinLimits lim) {
+__device__ __forceinline__ int bin_of(int64_t prod, int entries, BinLimits lim) {
     if (prod == 0) return 0;
     if (prod <= lim.l1) return 1;
+    if (prod > lim.l3) return BIN_BIG;
+    if (entries > FLAT_ENT) return BIN_MANY;
     if (prod <= lim.l2) return 2;
-    if (prod <= lim.l3) return 3;
-    return BIN_BIG;
+    return prod <= MID_PROD ? 3 : 4;
 }
 
 // ------------------------------------------------------------------ binning
-__global__ void k_bin_count(int m, const int64_t *__restrict__ rowprod, BinLimits lim,
-                            int *__restrict__ cnt) {
+__global__ void k_bin_count(int m, const int64_t *__restrict__ rowprod,
+                            const int *__restrict__ ia, BinLimits lim, int *__restrict__ cnt) {
     __shared__ int s_cnt[NBINS];
     if (threadIdx.x < NBINS) s_cnt[threadIdx.x] = 0;
     __syncthreads();
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m) atomicAdd(&s_cnt[bin_of(rowprod[i], lim)], 1);
+    if (i < m) atomicAdd(&s_cnt[bin_of(rowprod[i], ia[i + 1] - ia[i], lim)], 1);
     __syncthreads();
     if (threadIdx.x < NBINS && s_cnt[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], s_cnt[threadIdx.x]);
 }
@@ -103,6 +107,7 @@ __global__ void k_bin_count(int m, const int64_t *__restrict__ rowprod, BinLimit
 // gives each lane its slot among the wave's rows of that bin; per block, one
 // LDS atomic per wave and bin; per grid, one global atomic per block and bin.
 __global__ void __launch_bounds__(256) k_bin_scatter(int m, const int64_t *__restrict__ rowprod,
+                                                     const int *__restrict__ ia,
                                                      BinLimits lim, BinStarts st,
                                                      int *__restrict__ fill,
                                                      int *__restrict__ bin_rows,
@@ -112,7 +117,7 @@ __global__ void __launch_bounds__(256) k_bin_scatter(int m, const int64_t *__res
     __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const int b = i < m ? bin_of(rowprod[i], lim) : -1;
+    const int b = i < m ? bin_of(rowprod[i], ia[i + 1] - ia[i], lim) : -1;
     if (b == 0 || b == BIN_BIG) rownnz[i] = 0;
     const uint64_t below = (uint64_t(1) << lane) - 1;
     int pos = 0;
@@ -130,43 +135,6 @@ __global__ void __launch_bounds__(256) k_bin_scatter(int m, const int64_t *__res
         s_base[threadIdx.x] = atomicAdd(&fill[threadIdx.x], s_cnt[threadIdx.x]);
     __syncthreads();
     if (b > 0) bin_rows[st.s[b] + s_base[b] + pos] = i;
-}
-
-// Rows of the <= 1024-product bin split by the class the symbolic phase gave
-// them (see k_small_symbolic): class-1 rows to the front of out, class-0
-// rows to its back, class-2 rows to the front of out2, class-3 rows to its
-// back (any order inside each part, as rows are independent); count[c]
-// (zero on entry) ends as class c's size.
-__global__ void __launch_bounds__(256) k_split_bin3(int n, const int *__restrict__ rows,
-                                                    const uint8_t *__restrict__ cls_of,
-                                                    int *__restrict__ out, int *__restrict__ out2,
-                                                    int *__restrict__ count) {
-    __shared__ int s_cnt[4], s_base[4];
-    if (threadIdx.x < 4) s_cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const int row = i < n ? rows[i] : -1;
-    const int cls = i < n ? (int)cls_of[row] : -1;
-    const uint64_t below = (uint64_t(1) << lane) - 1;
-    int pos = 0;
-    for (int q = 0; q < 4; q++) {
-        const uint64_t mask = __ballot(cls == q);
-        if (!mask) continue;
-        const int leader = __ffsll((unsigned long long)mask) - 1;
-        int wbase = 0;
-        if (lane == leader) wbase = atomicAdd(&s_cnt[q], __popcll(mask));
-        wbase = __shfl(wbase, leader);
-        if (cls == q) pos = wbase + __popcll(mask & below);
-    }
-    __syncthreads();
-    if (threadIdx.x < 4 && s_cnt[threadIdx.x])
-        s_base[threadIdx.x] = atomicAdd(&count[threadIdx.x], s_cnt[threadIdx.x]);
-    __syncthreads();
-    if (cls == 1) out[s_base[1] + pos] = row;
-    else if (cls == 0) out[n - 1 - (s_base[0] + pos)] = row;
-    else if (cls == 2) out2[s_base[2] + pos] = row;
-    else if (cls == 3) out2[n - 1 - (s_base[3] + pos)] = row;
 }
 
 // Column span [lo, hi] of a row's products, from the first and last column
@@ -197,19 +165,14 @@ __device__ __forceinline__ void row_span(int pa, int pe, const int *__restrict__
 // ------------------------------------------------------ small rows: symbolic
 // Output count of each small row (rownnz), G lanes per row: a bitmap over
 // the row's column span when it fits SLOTS words, else an LDS hash of SLOTS
-// keys.  With narrow (the <= 1024-product bin), each row's numeric class: 1
-// when its span fits NARROW_WORDS words and its outputs NARROW_OUT, 3 when
-// its span fits SLOTS words and its outputs NARROW_OUT, 2 when its span fits
-// SLOTS words, 0 otherwise.
+// keys.
 template <int G, int SLOTS>
 __global__ void __launch_bounds__(256) k_small_symbolic(int nrows, const int *__restrict__ rows,
                                                         const int *__restrict__ ia,
                                                         const int *__restrict__ ja,
                                                         const int *__restrict__ ib,
                                                         const int *__restrict__ jb,
-                                                        int64_t *__restrict__ rownnz,
-                                                        int2 *__restrict__ span,
-                                                        uint8_t *__restrict__ narrow) {
+                                                        int64_t *__restrict__ rownnz) {
     constexpr int RPB = 256 / G;
     __shared__ __align__(16) int s_keys[RPB * SLOTS];
     __shared__ int s_mark[256];
@@ -223,7 +186,6 @@ __global__ void __launch_bounds__(256) k_small_symbolic(int nrows, const int *__
     const int row = rows[r];
     int lo, hi;
     row_span<G>(ia[row], ia[row + 1], ja, ib, jb, lo, hi);
-    if (l == 0) span[row] = make_int2(lo, hi);
     const int nw = hi >= lo ? ((hi - lo) >> 5) + 1 : 0;
     if (nw <= SLOTS) {
         // the row's columns fit a bitmap over its span in the table's space:
@@ -248,11 +210,7 @@ __global__ void __launch_bounds__(256) k_small_symbolic(int nrows, const int *__
             cnt += __popc(wv.x) + __popc(wv.y) + __popc(wv.z) + __popc(wv.w);
         }
         cnt = group_sum<G>(cnt);
-        if (l == 0) {
-            rownnz[row] = cnt;
-            if (narrow)
-                narrow[row] = cnt <= NARROW_OUT ? (nw <= NARROW_WORDS ? 1 : 3) : 2;
-        }
+        if (l == 0) rownnz[row] = cnt;
         return;
     }
     for (int i = l; i < SLOTS; i += G) keys[i] = -1;
@@ -268,349 +226,125 @@ __global__ void __launch_bounds__(256) k_small_symbolic(int nrows, const int *__
                                       }
                                   });
     created_cnt = group_sum<G>(created_cnt);
-    if (l == 0) {
-        rownnz[row] = created_cnt;
-        if (narrow) narrow[row] = 0;
-    }
+    if (l == 0) rownnz[row] = created_cnt;
 }
 
 // ------------------------------------------------------- small rows: numeric
-// RPB rows per block of RPB*G threads; LDS per row: SLOTS keys and values,
-// then the tags of the ordered accumulation, reused as the 256-entry radix
-// histogram once accumulation is over (rows of <= 64 products never need
-// the radix sort: at most 64 outputs go to the bitonic sort).
-template <int G, int SLOTS>
-constexpr int small_tag_words() {
-    return SLOTS > 128 ? (4 * G > 256 ? 4 * G : 256) : 4 * G;
-}
-template <int G, int SLOTS>
-constexpr size_t small_numeric_row_bytes() {
-    return (size_t)SLOTS * 12 + (size_t)small_tag_words<G, SLOTS>() * 4;
-}
-template <int G, int SLOTS, bool FUSED, int RPB>
-__global__ void __launch_bounds__(RPB * G) k_small_numeric(int nrows, const int *__restrict__ rows,
-                                                       const int *__restrict__ ia,
-                                                       const int *__restrict__ ja,
-                                                       const double *__restrict__ a,
-                                                       const int *__restrict__ ib,
-                                                       const int *__restrict__ jb,
-                                                       const double *__restrict__ b,
-                                                       const int64_t *__restrict__ ic,
-                                                       int *__restrict__ jc,
-                                                       double *__restrict__ c, int b_strict,
-                                                       const int2 *__restrict__ span) {
-    constexpr int NT = 4 * G;
-    constexpr int TW = small_tag_words<G, SLOTS>();
-    extern __shared__ __align__(16) unsigned char smem[];
-    double *s_vals = reinterpret_cast<double *>(smem);
-    int *s_keys = reinterpret_cast<int *>(s_vals + RPB * SLOTS);
-    unsigned *s_tags = reinterpret_cast<unsigned *>(s_keys + RPB * SLOTS);
-    const int grp = threadIdx.x / G;
+// A batch whose products come from at most this many B rows is accumulated
+// one B row after the other; past that, tag rounds take fewer steps.
+constexpr int FLAT_SEGS = 12;
+
+// One row of at most G * NB products, G lanes a row (tsg_flat.h), its entries
+// in S.  The columns and B values of every product are gathered once into
+// registers, the columns ranked, C's columns written, and the values summed
+// in LDS in product order, ACC outputs at a time: a batch of G products takes
+// one step when they come from one B row (distinct columns) or when a check
+// finds their outputs distinct, one step per B row when those are few, else
+// tag rounds.
+template <bool FUSED, int G, int U, int NB, int E, int LW, int ACC>
+__device__ __forceinline__ void flat_numeric_row(FlatSmem<G * U, E, LW, ACC> &S,
+                                                 unsigned *tags, int total, int64_t o,
+                                                 int64_t nrow, const int *__restrict__ jb,
+                                                 const double *__restrict__ b,
+                                                 int *__restrict__ jc, double *__restrict__ c,
+                                                 int b_strict) {
+    constexpr int NT = ACC / 4;                    // a byte per output of a pass
     const int l = threadIdx.x & (G - 1);
-    int *keys = s_keys + grp * SLOTS;
-    double *vals = s_vals + grp * SLOTS;
-    unsigned *tags = s_tags + grp * TW;
-    unsigned *hist = tags;      // after the accumulation
-    const int r = blockIdx.x * RPB + grp;
-    __shared__ int s_mark[RPB * G];
-    for (int i = l; i < NT; i += G) tags[i] = 0xffffffffu;
-    s_mark[threadIdx.x] = -1;
-    wave_lds_fence();
-    if (r >= nrows) return;
-    const int row = rows[r];
+    // few products share an output
+    const bool sparse = nrow * 4 >= (int64_t)total * 3;
+    const FlatHeads<G, U> heads(S.starts);
+    int col[NB], rank[NB];
+    double bv[NB];
     {
-        // the row's column span, from the symbolic phase
-        const int2 sp = span[row];
-        const int lo = sp.x, hi = sp.y;
-        const int nw = hi >= lo ? ((hi - lo) >> 5) + 1 : 0;
-        if (nw <= SLOTS) {
-            // Rank path: the row's span fits a bitmap in the table's space.
-            // Mark the columns, prefix-count the words, then accumulate every
-            // product at its column's rank (outputs come out sorted: no hash,
-            // compaction or sort).  Key space: SLOTS bitmap words; value space:
-            // the words' prefix counts (first half, as ints) and the outputs
-            // (second half, <= SLOTS/2 of them).
-            // The bitmap loops take four words per lane (16-byte LDS accesses;
-            // SLOTS is a multiple of 4, so the rounded-up word count fits).
-            unsigned *bmp = reinterpret_cast<unsigned *>(keys);
-            uint4 *bmp4 = reinterpret_cast<uint4 *>(keys);
-            int *pfx = reinterpret_cast<int *>(vals);
-            int4 *pfx4 = reinterpret_cast<int4 *>(vals);
-            double *acc = vals + SLOTS / 2;
-            const int64_t o = ic[row];
-            const int nnz = (int)(ic[row + 1] - o);
-            const int nw4 = (nw + 3) >> 2;
-            for (int i = l; i < nw4; i += G) bmp4[i] = make_uint4(0u, 0u, 0u, 0u);
-            wave_lds_fence();
-            for_products<G, SMALL_U, false, false>(
-                ia[row], ia[row + 1], 0, G, ja, nullptr, ib, jb, nullptr, BlockPtrs(), 0, 0,
-                s_mark + grp * G, [&](bool act, int col, double, double, bool) {
-                    if (act) {
-                        const int cc = col - lo;
-                        lds_set_bit(&bmp[cc >> 5], 1u << (cc & 31));
-                    }
-                });
-            wave_lds_fence();
-            int carry = 0;
-            for (int q0 = 0; q0 < nw4; q0 += G) {
-                const int q = q0 + l;
-                const uint4 wv = q < nw4 ? bmp4[q] : make_uint4(0u, 0u, 0u, 0u);
-                const int p0 = __popc(wv.x), p1 = __popc(wv.y), p2 = __popc(wv.z);
-                const int pc = p0 + p1 + p2 + __popc(wv.w);
-                const int incl = group_incl_scan<G>(pc);
-                if (q < nw4) {
-                    const int b0 = carry + incl - pc;
-                    pfx4[q] = make_int4(b0, b0 + p0, b0 + p0 + p1, b0 + p0 + p1 + p2);
-                }
-                carry += group_last<G>(incl);
-            }
-            for (int i = l; i < nnz; i += G) acc[i] = 0.0;
-            wave_lds_fence();
-            for_products<G, SMALL_U, false, true>(
-                ia[row], ia[row + 1], 0, G, ja, a, ib, jb, b, BlockPtrs(), 0, 0,
-                s_mark + grp * G, [&](bool act, int col, double av, double bv, bool single) {
-                    int rank = 0;
-                    if (act) {
-                        const int cc = col - lo;
-                        const int w = cc >> 5;
-                        rank = pfx[w] + __popc(bmp[w] & ((1u << (cc & 31)) - 1u));
-                    }
-                    ordered_accumulate<FUSED, NT>(act && rank < nnz, rank, av, bv, acc, tags,
-                                                  (unsigned)l, single && b_strict);
-                });
-            wave_lds_fence();
-            for (int i = l; i < nnz; i += G) c[o + i] = acc[i];
-            for (int q = l; q < nw4; q += G) {
-                const uint4 wv = bmp4[q];
-                const int4 pv = pfx4[q];
-                const unsigned ws[4] = {wv.x, wv.y, wv.z, wv.w};
-                const int ps[4] = {pv.x, pv.y, pv.z, pv.w};
+        int e[NB];
+        int before = -1;               // entries that start before the batch, less one
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    unsigned word = ws[j];
-                    int pos = ps[j];
-                    const int cb = lo + ((4 * q + j) << 5);
-                    while (word) {
-                        const int bit = __ffs(word) - 1;
-                        word &= word - 1;
-                        if (pos < nnz) jc[o + pos] = cb + bit;
-                        pos++;
-                    }
-                }
-            }
-            return;
+        for (int u = 0; u < NB; u++) {
+            const unsigned long long m = heads(u);
+            e[u] = S.off[heads.at(m, before)] + min(u * G + l, total - 1);
+            before += __popcll(m);
+            col[u] = jb[e[u]];
         }
+#pragma unroll
+        for (int u = 0; u < NB; u++) bv[u] = b[e[u]];
     }
-    for (int i = l; i < SLOTS; i += G) { keys[i] = -1; vals[i] = 0.0; }
+    const int found = flat_ranks<G, NB, true>(S, col, rank, !sparse);
+    // the symbolic phase counted the same outputs
+    const int nnz = group_uniform<G>((int)min((int64_t)found, nrow));
+#pragma unroll
+    for (int u = 0; u < NB; u++) S.cols[rank[u]] = col[u];
     wave_lds_fence();
-    for_products<G, SMALL_U, false, true>(ia[row], ia[row + 1], 0, G, ja, a, ib, jb, b,
-                                          BlockPtrs(), 0, 0, s_mark + grp * G,
-                                          [&](bool act, int col, double av, double bv, bool single) {
-                                     int slot = 0;
-                                     if (act) {
-                                         bool created;
-                                         slot = hash_insert<SLOTS>(keys, col, created);
-                                     }
-                                     wave_lds_fence();
-                                     ordered_accumulate<FUSED, NT>(act, slot, av, bv, vals, tags,
-                                                                   (unsigned)l, single && b_strict);
-                                 });
-    // compact the occupied slots to the front, in slot order: chunks of G
-    // slots are visited in ascending order and every entry moves to a lower
-    // or equal position, so no entry is overwritten before it is read
-    const int gb = __lane_id() & ~(G - 1);
-    const unsigned long long gm = G == 64 ? ~0ull : ((1ull << G) - 1);
-    int nocc = 0;
-    for (int c0 = 0; c0 < SLOTS; c0 += G) {
-        const int k = keys[c0 + l];
-        const double v = vals[c0 + l];
-        const bool occ = k != -1;
-        const unsigned long long bal = (__ballot(occ) >> gb) & gm;
-        const int before = __popcll(bal & ((1ull << l) - 1));
+    for (int i = l; i < nnz; i += G) jc[o + i] = S.cols[i];
+    uint8_t *own = reinterpret_cast<uint8_t *>(tags);
+    for (int r0 = 0; r0 < nnz; r0 += ACC) {
+        const int nout = min(ACC, nnz - r0);
         wave_lds_fence();
-        if (occ) {
-            keys[nocc + before] = k;
-            vals[nocc + before] = v;
-        }
-        nocc += __popcll(bal);
+        for (int i = l; i < nout; i += G) S.acc[i] = 0.0;
         wave_lds_fence();
-    }
-    const int64_t o = ic[row];
-    const int nnz = (int)(ic[row + 1] - o);
-    if (nocc <= 64) {
-        int n2 = 1;
-        while (n2 < nocc) n2 <<= 1;
-        for (int i = nocc + l; i < n2; i += G) keys[i] = 0x7fffffff;
-        wave_lds_fence();
-        bitonic_sort_group<G>(keys, vals, n2);
-        for (int i = l; i < nnz; i += G) {
-            jc[o + i] = keys[i];
-            c[o + i] = vals[i];
-        }
-        return;
-    }
-    // radix sort on keys relative to the row's smallest column; the back
-    // half of the table (occupancy <= SLOTS/2) is the ping-pong buffer
-    if constexpr (SLOTS > 128) {
-        int kmin = 0x7fffffff, kmax = 0;
-        for (int i = l; i < nocc; i += G) {
-            kmin = min(kmin, keys[i]);
-            kmax = max(kmax, keys[i]);
-        }
+        int before = 0;                // entries that start before the batch
 #pragma unroll
-        for (int d = G / 2; d > 0; d >>= 1) {
-            kmin = min(kmin, __shfl_xor(kmin, d, G));
-            kmax = max(kmax, __shfl_xor(kmax, d, G));
-        }
-        const int span = kmax - kmin;
-        const int nw = (span >> 5) + 1;              // bitmap words over [kmin, kmax]
-        if (nw <= SLOTS) {
-            // rank by bitmap: the free back halves of the table hold one bit per
-            // column of the row's span (the value half, SLOTS words) and the
-            // outputs before every pair of words (the key half); an entry's
-            // position is its pair's prefix plus the bits below it
-            unsigned *bmp = reinterpret_cast<unsigned *>(vals + SLOTS / 2);
-            int *pfx = keys + SLOTS / 2;
-            for (int i = l; i < nw; i += G) bmp[i] = 0u;
-            wave_lds_fence();
-            for (int i = l; i < nocc; i += G) {
-                const int kk = keys[i] - kmin;
-                atomicOr(&bmp[kk >> 5], 1u << (kk & 31));
+        for (int u = 0; u < NB; u++) {
+            // the batch's B rows: the product's index among them (from 1),
+            // their number, the entry of the first
+            const unsigned long long hm = heads(u);
+            const unsigned long long m = hm | 1ull;
+            const int seg = heads.at(m, 0);
+            const int nseg = __popcll(m);
+            const int first = before - (int)(~hm & 1ull);
+            before += __popcll(hm);
+            const int out = rank[u] - r0;
+            const bool act = u * G + l < total && (unsigned)out < (unsigned)nout;
+            const double av = S.a[first + seg - 1];
+            bool clash = !b_strict || nseg > 1;
+            if (clash && b_strict && sparse) {
+                if (act) own[out] = (uint8_t)l;
+                wave_lds_fence();
+                clash = group_ballot<G>(act && own[out] != (uint8_t)l) != 0;
+                wave_lds_fence();
             }
-            wave_lds_fence();
-            const int npair = (nw + 1) >> 1;
-            int carry = 0;
-            for (int p0 = 0; p0 < npair; p0 += G) {
-                const int p = p0 + l;
-                int pc = 0;
-                if (p < npair) {
-                    pc = __popc(bmp[2 * p]);
-                    if (2 * p + 1 < nw) pc += __popc(bmp[2 * p + 1]);
+            if (!clash) {
+                if (act) S.acc[out] = acc_step<FUSED>(S.acc[out], av, bv[u]);
+                wave_lds_fence();
+            } else if (b_strict && nseg <= FLAT_SEGS) {
+                for (int s = 1; s <= nseg; s++) {
+                    if (act && seg == s) S.acc[out] = acc_step<FUSED>(S.acc[out], av, bv[u]);
+                    wave_lds_fence();
                 }
-                const int incl = group_incl_scan<G>(pc);
-                if (p < npair) pfx[p] = carry + incl - pc;
-                carry += group_last<G>(incl);
+            } else {
+                for (int i = l; i < NT; i += G) tags[i] = 0xffffffffu;
+                wave_lds_fence();
+                ordered_accumulate<FUSED, NT>(act, out, av, bv[u], S.acc, tags, (unsigned)l,
+                                              false);
             }
-            wave_lds_fence();
-            for (int i = l; i < nocc; i += G) {
-                const int kk = keys[i] - kmin;
-                const int w = kk >> 5;
-                int rank = pfx[w >> 1] + __popc(bmp[w] & ((1u << (kk & 31)) - 1u));
-                if (w & 1) rank += __popc(bmp[w - 1]);
-                if (rank < nnz) {
-                    jc[o + rank] = keys[i];
-                    c[o + rank] = vals[i];
-                }
-            }
-            return;
         }
-        const int bits = span > 0 ? 32 - __clz(span) : 1;
-        const bool in_dst = radix_sort_group<G>(keys, vals, keys + SLOTS / 2, vals + SLOTS / 2,
-                                                nocc, kmin, bits, hist);
-        const int *sk = in_dst ? keys + SLOTS / 2 : keys;
-        const double *sv = in_dst ? vals + SLOTS / 2 : vals;
-        for (int i = l; i < nnz; i += G) {
-            jc[o + i] = sk[i];
-            c[o + i] = sv[i];
-        }
+        for (int i = l; i < nout; i += G) c[o + r0 + i] = S.acc[i];
     }
 }
 
-// Rows of the <= 1024-product bin whose column span fits RK_WORDS bitmap
-// words and whose outputs number at most RK_OUT: the rank path alone, 64
-// lanes per row.  LDS: the span bitmap, one output count per 4 words, the
-// row's values and the accumulation tags -- 19.7 KB for (2048, 1024)
-// instead of the hash-capable kernel's 25 KB (8 rows per CU resident instead
-// of 6), 15.6 KB for (2048, 512) and 10.5 KB for the narrow rows' (1024,
-// 512).  Mark, prefix, accumulate at each column's rank, write.
-template <bool FUSED, int RK_WORDS, int RK_OUT>
-__global__ void __launch_bounds__(64) k_small_numeric_rank(
+template <bool FUSED, int G, int U, int E, int LW, int ACC, int THREADS, int MINW = 1>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(MINW)))
+k_flat_numeric(
     int nrows, const int *__restrict__ rows, const int *__restrict__ ia,
     const int *__restrict__ ja, const double *__restrict__ a, const int *__restrict__ ib,
     const int *__restrict__ jb, const double *__restrict__ b, const int64_t *__restrict__ ic,
-    int *__restrict__ jc, double *__restrict__ c, int b_strict, const int2 *__restrict__ span) {
-    constexpr int G = 64, NT = 4 * G;
-    __shared__ __align__(16) unsigned bmp[RK_WORDS];
-    __shared__ int pfx[RK_WORDS / 4];
-    __shared__ double acc[RK_OUT];
-    __shared__ unsigned tags[NT];
-    __shared__ int s_mark[G];
-    const int l = threadIdx.x;
-    for (int i = l; i < NT; i += G) tags[i] = 0xffffffffu;
-    s_mark[l] = -1;
-    wave_lds_fence();
-    if ((int)blockIdx.x >= nrows) return;
-    const int row = rows[blockIdx.x];
-    // the row's column span, from the symbolic phase, which put the row here
-    // because the span fits RK_WORDS
-    const int2 sp = span[row];
-    const int lo = sp.x, hi = sp.y;
-    const int nw = hi >= lo ? min(((hi - lo) >> 5) + 1, RK_WORDS) : 0;
-    const int nw4 = (nw + 3) >> 2;
-    uint4 *bmp4 = reinterpret_cast<uint4 *>(bmp);
+    int *__restrict__ jc, double *__restrict__ c, int b_strict) {
+    constexpr int RPB = THREADS / G;
+    __shared__ __align__(16) FlatSmem<G * U, E, LW, ACC> s_row[RPB];
+    __shared__ unsigned s_tags[RPB][ACC / 4];
+    const int grp = threadIdx.x / G;
+    FlatSmem<G * U, E, LW, ACC> &S = s_row[grp];
+    const int r = blockIdx.x * RPB + grp;
+    if (r >= nrows) return;
+    const int row = group_uniform<G>(rows[r]);
     const int64_t o = ic[row];
     const int64_t nrow = ic[row + 1] - o;
-    const int nnz = (int)(nrow < RK_OUT ? nrow : RK_OUT);
-    // columns outside [lo, lo + 32*nw) cannot occur (B rows are ascending);
-    // the unsigned test keeps every LDS index in range regardless
-    const unsigned span_cols = (unsigned)nw << 5;
-    for (int i = l; i < nw4; i += G) bmp4[i] = make_uint4(0u, 0u, 0u, 0u);
-    wave_lds_fence();
-    for_products<G, SMALL_U, false, false>(ia[row], ia[row + 1], 0, G, ja, nullptr, ib, jb,
-                                           nullptr, BlockPtrs(), 0, 0, s_mark,
-                                           [&](bool act, int col, double, double, bool) {
-                                               const int cc = col - lo;
-                                               if (act && (unsigned)cc < span_cols)
-                                                   lds_set_bit(&bmp[cc >> 5], 1u << (cc & 31));
-                                           });
-    wave_lds_fence();
-    int carry = 0;
-    for (int q0 = 0; q0 < nw4; q0 += G) {
-        const int q = q0 + l;
-        const uint4 wv = q < nw4 ? bmp4[q] : make_uint4(0u, 0u, 0u, 0u);
-        const int pc = __popc(wv.x) + __popc(wv.y) + __popc(wv.z) + __popc(wv.w);
-        const int incl = group_incl_scan<G>(pc);
-        if (q < nw4) pfx[q] = carry + incl - pc;
-        carry += group_last<G>(incl);
-    }
-    for (int i = l; i < nnz; i += G) acc[i] = 0.0;
-    wave_lds_fence();
-    for_products<G, SMALL_U, false, true>(
-        ia[row], ia[row + 1], 0, G, ja, a, ib, jb, b, BlockPtrs(), 0, 0, s_mark,
-        [&](bool act, int col, double av, double bv, bool single) {
-            int rank = 0;
-            const int cc = col - lo;
-            const int w = cc >> 5;
-            const bool in = act && (unsigned)cc < span_cols;
-            if (in) {
-                const uint4 wv = bmp4[w >> 2];
-                const int j = w & 3;
-                rank = pfx[w >> 2] + (j > 0 ? __popc(wv.x) : 0) + (j > 1 ? __popc(wv.y) : 0) +
-                       (j > 2 ? __popc(wv.z) : 0);
-                const unsigned cur = j == 0 ? wv.x : j == 1 ? wv.y : j == 2 ? wv.z : wv.w;
-                rank += __popc(cur & ((1u << (cc & 31)) - 1u));
-            }
-            ordered_accumulate<FUSED, NT>(in && rank < nnz, rank, av, bv, acc, tags,
-                                          (unsigned)l, single && b_strict);
-        });
-    wave_lds_fence();
-    for (int i = l; i < nnz; i += G) c[o + i] = acc[i];
-    for (int q = l; q < nw4; q += G) {
-        const uint4 wv = bmp4[q];
-        const unsigned ws[4] = {wv.x, wv.y, wv.z, wv.w};
-        int pos = pfx[q];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            unsigned word = ws[j];
-            const int cb = lo + ((4 * q + j) << 5);
-            while (word) {
-                const int bit = __ffs(word) - 1;
-                word &= word - 1;
-                if (pos < nnz) jc[o + pos] = cb + bit;
-                pos++;
-            }
-        }
-    }
+    const int total = flat_entries<G>(S, ia[row], ia[row + 1], ja, a, ib);
+    if (total <= 0) return;
+    if (G == 64 && total <= G * U / 4 * 3)
+        flat_numeric_row<FUSED, G, U, U / 4 * 3>(S, s_tags[grp], total, o, nrow, jb, b, jc, c,
+                                                 b_strict);
+    else
+        flat_numeric_row<FUSED, G, U, U>(S, s_tags[grp], total, o, nrow, jb, b, jc, c, b_strict);
 }
 
 // -------------------------------------------------------- big rows: span
@@ -1477,7 +1211,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     const int m = A.rows, n = A.cols, k = B.cols;
     TSG_CHECK(tune.bin1 >= 0 && tune.bin1 <= bin_limit[1] && tune.bin1 <= tune.bin2 &&
                   tune.bin2 <= bin_limit[2] && tune.bin2 <= tune.bin3 &&
-                  tune.bin3 <= bin_limit[3],
+                  tune.bin3 <= bin_limit[4],
               TSG_ERR_INVALID, "row bins out of range");
     const BinLimits lim{tune.bin1, tune.bin2, tune.bin3};
     p = RowPlan();
@@ -1487,15 +1221,15 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     p.rowprod = ws.alloc_n<int64_t>((size_t)m + 1);
     p.rownnz = ws.alloc_n<int64_t>((size_t)m + 1);
     p.bin_rows = ws.alloc_n<int>((size_t)m + 1);
-    int *d_cnt = ws.alloc_n<int>(2 * NBINS + 4);
+    int *d_cnt = ws.alloc_n<int>(2 * NBINS);
     int64_t *scan_tmp = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)m + 1));
 
     tm.begin("row.products+bins");
     csr_row_products(m, A.ptr, A.idx, A.nnz, B.ptr, p.rowprod, ws, s);
-    TSG_HIP_TRY(hipMemsetAsync(d_cnt, 0, sizeof(int) * (2 * NBINS + 4), s));
+    TSG_HIP_TRY(hipMemsetAsync(d_cnt, 0, sizeof(int) * (2 * NBINS), s));
     if (m > 0) {
-        hipLaunchKernelGGL(k_bin_count, dim3(grid_for(m, 256)), dim3(256), 0, s, m, p.rowprod, lim,
-                           d_cnt);
+        hipLaunchKernelGGL(k_bin_count, dim3(grid_for(m, 256)), dim3(256), 0, s, m, p.rowprod,
+                           A.ptr, lim, d_cnt);
         TSG_LAUNCH_CHECK();
     }
     int h_cnt[NBINS];
@@ -1507,8 +1241,8 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     for (int b = 0; b <= NBINS; b++) p.bin_start_h[b] = st.s[b];
     p.nbins = NBINS;
     if (m > 0) {
-        hipLaunchKernelGGL(k_bin_scatter, dim3(grid_for(m, 256)), dim3(256), 0, s, m, p.rowprod, lim,
-                           st, d_cnt + NBINS, p.bin_rows, p.rownnz);
+        hipLaunchKernelGGL(k_bin_scatter, dim3(grid_for(m, 256)), dim3(256), 0, s, m, p.rowprod,
+                           A.ptr, lim, st, d_cnt + NBINS, p.bin_rows, p.rownnz);
         TSG_LAUNCH_CHECK();
     }
     tm.end();
@@ -1516,49 +1250,27 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     // small rows
     tm.begin("row.small_symbolic");
     {
-        p.span = ws.alloc_n<int2>((size_t)m);
-        const int *rows1 = p.bin_rows + st.s[1];
-        int n1 = st.s[2] - st.s[1];
-        if (n1 > 0) {
-            hipLaunchKernelGGL((k_small_symbolic<16, 128>), dim3(grid_for(n1, 16)), dim3(256), 0,
-                               s, n1, rows1, A.ptr, A.idx, B.ptr, B.idx, p.rownnz, p.span, nullptr);
+        auto launch = [&](auto kern, int rpb, int b0, int b1) {
+            const int nr = st.s[b1 + 1] - st.s[b0];
+            if (nr <= 0) return;
+            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(256), 0, s, nr,
+                               p.bin_rows + st.s[b0], A.ptr, A.idx, B.ptr, B.idx, p.rownnz);
             TSG_LAUNCH_CHECK();
-        }
-        const int *rows2 = p.bin_rows + st.s[2];
-        int n2 = st.s[3] - st.s[2];
-        if (n2 > 0) {
-            hipLaunchKernelGGL((k_small_symbolic<32, 512>), dim3(grid_for(n2, 8)), dim3(256), 0,
-                               s, n2, rows2, A.ptr, A.idx, B.ptr, B.idx, p.rownnz, p.span, nullptr);
-            TSG_LAUNCH_CHECK();
-        }
-        const int *rows3 = p.bin_rows + st.s[3];
-        int n3 = st.s[4] - st.s[3];
-        if (n3 > 0) {
-            p.narrow3 = ws.alloc_n<uint8_t>((size_t)m);
-            hipLaunchKernelGGL((k_small_symbolic<64, 2048>), dim3(grid_for(n3, 4)), dim3(256), 0,
-                               s, n3, rows3, A.ptr, A.idx, B.ptr, B.idx, p.rownnz, p.span, p.narrow3);
-            TSG_LAUNCH_CHECK();
-            // each numeric variant launches over its own rows; the class
-            // sizes come back with the phase's last host round trip
-            p.rows3 = ws.alloc_n<int>((size_t)n3);
-            p.rows3r = ws.alloc_n<int>((size_t)n3);
-            hipLaunchKernelGGL(k_split_bin3, dim3(grid_for(n3, 256)), dim3(256), 0, s, n3, rows3,
-                               p.narrow3, p.rows3, p.rows3r, d_cnt + 2 * NBINS);
-            TSG_LAUNCH_CHECK();
-            TSG_HIP_TRY(hipMemcpyAsync(p.n3cls, d_cnt + 2 * NBINS, 4 * sizeof(int),
-                                       hipMemcpyDeviceToHost, s));
-        }
+        };
+        launch(k_small_symbolic<16, 128>, 16, 1, 1);
+        launch(k_small_symbolic<32, 512>, 8, 2, 2);
+        launch(k_small_symbolic<64, 2048>, 4, 3, BIN_MANY);
     }
     tm.end();
 
     // big rows
-    p.nbig = st.s[5] - st.s[4];
+    p.nbig = st.s[BIN_BIG + 1] - st.s[BIN_BIG];
     p.sub_shift = SUB_SHIFT;
     int64_t *band_off = nullptr, *band_base = nullptr, *row_loff = nullptr;
     unsigned long long *row_cur = nullptr;
     unsigned *d_overflow = nullptr;
     if (p.nbig > 0) {
-        const int *rowsb = p.bin_rows + st.s[4];
+        const int *rowsb = p.bin_rows + st.s[BIN_BIG];
         tm.begin("row.big_symbolic");
         // column span of every big row, in sub-blocks, span offsets and the
         // band units over the spans
@@ -1710,7 +1422,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     int64_t h_tot[2] = {0, 0};
     if (p.nbig > 0) {
         tm.begin("row.items");
-        const int *rowsb = p.bin_rows + st.s[4];
+        const int *rowsb = p.bin_rows + st.s[BIN_BIG];
         p.item_cnt = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         int64_t *tmp2 = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)p.nbig + 1));
         // Narrow (8-sub-block) windows when the spans are wide enough that
@@ -1798,43 +1510,19 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
     const int *st = p.bin_start_h;
     tm.begin("row.small_numeric");
     {
-        // rows of <= 64 and <= 256 products: 16 and 2 rows per block of the
-        // hash-capable kernel; rows of <= 1024 products by the class the
-        // symbolic phase gave them: the rank-only kernel's 1024- and 2048-word
-        // variants, the hash-capable kernel for wider spans (1 row per block)
-        auto launch = [&](auto kern, int rpb, int g, size_t per_row, const int *rows, int nr) {
+        auto launch = [&](auto kern, int rpb, int threads, int bin) {
+            const int nr = st[bin + 1] - st[bin];
             if (nr <= 0) return;
-            const size_t sm = per_row * rpb;
-            set_smem(kern, sm);
-            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(rpb * g), sm, s, nr, rows,
-                               A.ptr, A.idx, A.val, B.ptr, B.idx, B.val, d_ic, d_jc, d_c,
-                               (int)p.b_strict, p.span);
+            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
+                               bins + st[bin], A.ptr, A.idx, A.val, B.ptr, B.idx, B.val, d_ic,
+                               d_jc, d_c, (int)p.b_strict);
             TSG_LAUNCH_CHECK();
         };
-        launch(k_small_numeric<16, 128, FUSED, 16>, 16, 16, small_numeric_row_bytes<16, 128>(),
-               bins + st[1], st[2] - st[1]);
-        launch(k_small_numeric<32, 512, FUSED, 2>, 2, 32, small_numeric_row_bytes<32, 512>(),
-               bins + st[2], st[3] - st[2]);
-        const int n3 = st[4] - st[3];
-        if (n3 > 0) {
-            // classes from the symbolic phase: [1 | ... | 0] in rows3,
-            // [2 | ... | 3] in rows3r
-            const int n_hash = p.n3cls[0], n_narrow = p.n3cls[1], n_rank = p.n3cls[2],
-                      n_rank512 = p.n3cls[3];
-            auto launch_rank = [&](auto kern, const int *rows, int nr) {
-                if (nr <= 0) return;
-                hipLaunchKernelGGL(kern, dim3((unsigned)nr), dim3(64), 0, s, nr, rows, A.ptr,
-                                   A.idx, A.val, B.ptr, B.idx, B.val, d_ic, d_jc, d_c,
-                                   (int)p.b_strict, p.span);
-                TSG_LAUNCH_CHECK();
-            };
-            launch_rank(k_small_numeric_rank<FUSED, NARROW_WORDS, NARROW_OUT>, p.rows3, n_narrow);
-            launch_rank(k_small_numeric_rank<FUSED, 2048, 1024>, p.rows3r, n_rank);
-            launch_rank(k_small_numeric_rank<FUSED, 2048, NARROW_OUT>, p.rows3r + (n3 - n_rank512),
-                        n_rank512);
-            launch(k_small_numeric<64, 2048, FUSED, 1>, 1, 64, small_numeric_row_bytes<64, 2048>(),
-                   p.rows3 + (n3 - n_hash), n_hash);
-        }
+        launch(k_flat_numeric<FUSED, 16, 4, 64, 64, 64, 256>, 16, 256, 1);
+        launch(k_flat_numeric<FUSED, 64, 4, 64, 512, 256, 64>, 1, 64, 2);
+        launch(k_flat_numeric<FUSED, 64, 8, 64, 512, 512, 64>, 1, 64, 3);
+        launch(k_flat_numeric<FUSED, 64, 16, 64, 512, 512, 64>, 1, 64, 4);
+        launch(k_flat_numeric<FUSED, 64, 16, 1024, 512, 512, 64>, 1, 64, 5);
     }
     tm.end();
     if (p.nitems > 0 && p.use_rank) {
