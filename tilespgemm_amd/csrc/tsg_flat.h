@@ -162,6 +162,28 @@ __device__ __forceinline__ int flat_ranks(FlatSmem<P, E, LW, ACC> &S, const int 
     }
     lo = group_uniform<G>(group_min_i32<G>(lo));
     hi = group_uniform<G>(group_max_i32<G>(hi));
+    if constexpr (!RANKS) {
+        // counted alone, columns of a span that fits need one level of bits
+        if (hi - lo < LW * 64) {
+            unsigned *bits = reinterpret_cast<unsigned *>(S.l1);
+            uint4 *bits4 = reinterpret_cast<uint4 *>(S.l1);
+            const int n4 = ((hi - lo) >> 7) + 1;
+            for (int i = l; i < n4; i += G) bits4[i] = make_uint4(0u, 0u, 0u, 0u);
+            wave_lds_fence();
+#pragma unroll
+            for (int u = 0; u < NB; u++) {
+                const int cc = col[u] - lo;
+                lds_set_bit(&bits[cc >> 5], 1u << (cc & 31));
+            }
+            wave_lds_fence();
+            int n = 0;
+            for (int i = l; i < n4; i += G) {
+                const uint4 v = bits4[i];
+                n += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);
+            }
+            return group_sum<G>(n);
+        }
+    }
     // one window of columns from lo; part: it may leave some out
     auto window = [&](int done, auto part_t) {
         constexpr bool part = decltype(part_t)::value;

@@ -62,12 +62,6 @@ static_assert(ITEM_CAP >= (1 << SUB_SHIFT), "an item must hold a full sub-block"
 constexpr int ITEM_TAGS = 256;
 constexpr int ITEM_WAVES = 1;          // waves per block (one item per wave)
 constexpr int RANK_U = 8;
-// Product batches in flight per lane in the small-row kernels: their LDS
-// tables already cap residency, so registers for more loads in flight are
-// free up to 8 (48 VGPRs; 16 would cut residency by registers).  2 -> 8:
-// ER batch rows of <= 1024 products 62.0 -> 57.2 ms, 27-point 64^3 3.05 ->
-// 2.93 ms.
-constexpr int SMALL_U = 8;
 constexpr int BIG_SYM_U = 4;
 constexpr int ITEM_U = 4;
 
@@ -137,96 +131,50 @@ __global__ void __launch_bounds__(256) k_bin_scatter(int m, const int64_t *__res
     if (b > 0) bin_rows[st.s[b] + s_base[b] + pos] = i;
 }
 
-// Column span [lo, hi] of a row's products, from the first and last column
-// of each B row its A entries name (lo > hi for a row without products); G
-// lanes of a group.
-template <int G>
-__device__ __forceinline__ void row_span(int pa, int pe, const int *__restrict__ ja,
-                                         const int *__restrict__ ib,
-                                         const int *__restrict__ jb, int &lo, int &hi) {
-    const int l = __lane_id() & (G - 1);
-    lo = 0x7fffffff;
-    hi = -1;
-    for (int p = pa + l; p < pe; p += G) {
-        const int t = ja[p];
-        const int b0 = ib[t], b1 = ib[t + 1];
-        if (b0 < b1) {
-            lo = min(lo, jb[b0]);
-            hi = max(hi, jb[b1 - 1]);
-        }
-    }
+// ------------------------------------------------------ small rows: symbolic
+// Output count of each row of at most G * U products (rownnz), G lanes a row:
+// the columns gathered into registers and counted by the bitmaps of
+// tsg_flat.h.  Bound: random B rows by memory (ER batch, rows of 513..1024
+// products: 2.7 ms, 14 GB of column lines), stencils by issue.  Against a
+// separate pass for the row's span and a flat expansion in rounds into one
+// bitmap or hash: ER batch of 512 9.3 -> 5.6 ms, 27-point 64^3 0.46 -> 0.24 ms,
+// rectangular ER 75 -> 58 us, R-MAT 2^18 0.39 -> 0.09 ms.  6 waves per SIMD at
+// 16 products a lane: 3.2 ms (ER) and 258 us (stencil) unforced, 2.8 and 225 at
+// 5, 2.7 and 213 at 6, 3.4 and 212 at 7 (spills).
+template <int G, int U, int NB, int E, int LW>
+__device__ __forceinline__ int flat_count_row(FlatSmem<G * U, E, LW, 1> &S, int total,
+                                              const int *__restrict__ jb) {
+    const int l = threadIdx.x & (G - 1);
+    const FlatHeads<G, U> heads(S.starts);
+    int col[NB], rank[NB];
+    int before = -1;                   // entries that start before the batch, less one
 #pragma unroll
-    for (int d = G / 2; d > 0; d >>= 1) {
-        lo = min(lo, __shfl_xor(lo, d, G));
-        hi = max(hi, __shfl_xor(hi, d, G));
+    for (int u = 0; u < NB; u++) {
+        const unsigned long long m = heads(u);
+        col[u] = jb[S.off[heads.at(m, before)] + min(u * G + l, total - 1)];
+        before += __popcll(m);
     }
+    return flat_ranks<G, NB, false>(S, col, rank, true);
 }
 
-// ------------------------------------------------------ small rows: symbolic
-// Output count of each small row (rownnz), G lanes per row: a bitmap over
-// the row's column span when it fits SLOTS words, else an LDS hash of SLOTS
-// keys.
-template <int G, int SLOTS>
-__global__ void __launch_bounds__(256) k_small_symbolic(int nrows, const int *__restrict__ rows,
-                                                        const int *__restrict__ ia,
-                                                        const int *__restrict__ ja,
-                                                        const int *__restrict__ ib,
-                                                        const int *__restrict__ jb,
-                                                        int64_t *__restrict__ rownnz) {
-    constexpr int RPB = 256 / G;
-    __shared__ __align__(16) int s_keys[RPB * SLOTS];
-    __shared__ int s_mark[256];
+template <int G, int U, int E, int LW, int THREADS, int MINW = 1>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(MINW)))
+k_flat_symbolic(int nrows, const int *__restrict__ rows, const int *__restrict__ ia,
+                const int *__restrict__ ja, const int *__restrict__ ib,
+                const int *__restrict__ jb, int64_t *__restrict__ rownnz) {
+    constexpr int RPB = THREADS / G;
+    __shared__ __align__(16) FlatSmem<G * U, E, LW, 1> s_row[RPB];
     const int grp = threadIdx.x / G;
-    const int l = threadIdx.x & (G - 1);
-    int *keys = s_keys + grp * SLOTS;
+    FlatSmem<G * U, E, LW, 1> &S = s_row[grp];
     const int r = blockIdx.x * RPB + grp;
-    s_mark[threadIdx.x] = -1;
-    wave_lds_fence();
     if (r >= nrows) return;
-    const int row = rows[r];
-    int lo, hi;
-    row_span<G>(ia[row], ia[row + 1], ja, ib, jb, lo, hi);
-    const int nw = hi >= lo ? ((hi - lo) >> 5) + 1 : 0;
-    if (nw <= SLOTS) {
-        // the row's columns fit a bitmap over its span in the table's space:
-        // mark them and count the bits (no hashing)
-        unsigned *bmp = reinterpret_cast<unsigned *>(keys);
-        uint4 *bmp4 = reinterpret_cast<uint4 *>(keys);
-        const int nw4 = (nw + 3) >> 2;
-        for (int i = l; i < nw4; i += G) bmp4[i] = make_uint4(0u, 0u, 0u, 0u);
-        wave_lds_fence();
-        for_products<G, SMALL_U, false, false>(ia[row], ia[row + 1], 0, G, ja, nullptr, ib, jb,
-                                               nullptr, BlockPtrs(), 0, 0, s_mark + grp * G,
-                                               [&](bool act, int col, double, double, bool) {
-                                                   if (act) {
-                                                       const int cc = col - lo;
-                                                       lds_set_bit(&bmp[cc >> 5], 1u << (cc & 31));
-                                                   }
-                                               });
-        wave_lds_fence();
-        int cnt = 0;
-        for (int i = l; i < nw4; i += G) {
-            const uint4 wv = bmp4[i];
-            cnt += __popc(wv.x) + __popc(wv.y) + __popc(wv.z) + __popc(wv.w);
-        }
-        cnt = group_sum<G>(cnt);
-        if (l == 0) rownnz[row] = cnt;
-        return;
-    }
-    for (int i = l; i < SLOTS; i += G) keys[i] = -1;
-    wave_lds_fence();
-    int created_cnt = 0;
-    for_products<G, SMALL_U, false, false>(ia[row], ia[row + 1], 0, G, ja, nullptr, ib, jb,
-                                           nullptr, BlockPtrs(), 0, 0, s_mark + grp * G,
-                                           [&](bool act, int col, double, double, bool) {
-                                      if (act) {
-                                          bool created;
-                                          hash_insert<SLOTS>(keys, col, created);
-                                          created_cnt += created;
-                                      }
-                                  });
-    created_cnt = group_sum<G>(created_cnt);
-    if (l == 0) rownnz[row] = created_cnt;
+    const int row = group_uniform<G>(rows[r]);
+    const int total = flat_entries<G>(S, ia[row], ia[row + 1], ja, (const double *)nullptr, ib);
+    int n = 0;
+    if (total > 0)
+        n = G == 64 && total <= G * U / 4 * 3 ? flat_count_row<G, U, U / 4 * 3>(S, total, jb)
+                                              : flat_count_row<G, U, U>(S, total, jb);
+    if ((threadIdx.x & (G - 1)) == 0) rownnz[row] = n;
 }
 
 // ------------------------------------------------------- small rows: numeric
@@ -1250,16 +1198,18 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     // small rows
     tm.begin("row.small_symbolic");
     {
-        auto launch = [&](auto kern, int rpb, int b0, int b1) {
-            const int nr = st.s[b1 + 1] - st.s[b0];
+        auto launch = [&](auto kern, int rpb, int threads, int bin) {
+            const int nr = st.s[bin + 1] - st.s[bin];
             if (nr <= 0) return;
-            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(256), 0, s, nr,
-                               p.bin_rows + st.s[b0], A.ptr, A.idx, B.ptr, B.idx, p.rownnz);
+            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
+                               p.bin_rows + st.s[bin], A.ptr, A.idx, B.ptr, B.idx, p.rownnz);
             TSG_LAUNCH_CHECK();
         };
-        launch(k_small_symbolic<16, 128>, 16, 1, 1);
-        launch(k_small_symbolic<32, 512>, 8, 2, 2);
-        launch(k_small_symbolic<64, 2048>, 4, 3, BIN_MANY);
+        launch(k_flat_symbolic<16, 4, 64, 64, 256>, 16, 256, 1);
+        launch(k_flat_symbolic<64, 4, 64, 512, 64>, 1, 64, 2);
+        launch(k_flat_symbolic<64, 8, 64, 512, 64>, 1, 64, 3);
+        launch(k_flat_symbolic<64, 16, 64, 512, 64, 6>, 1, 64, 4);
+        launch(k_flat_symbolic<64, 16, 1024, 512, 64>, 1, 64, BIN_MANY);
     }
     tm.end();
 
@@ -1522,7 +1472,7 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
         launch(k_flat_numeric<FUSED, 64, 4, 64, 512, 256, 64>, 1, 64, 2);
         launch(k_flat_numeric<FUSED, 64, 8, 64, 512, 512, 64>, 1, 64, 3);
         launch(k_flat_numeric<FUSED, 64, 16, 64, 512, 512, 64>, 1, 64, 4);
-        launch(k_flat_numeric<FUSED, 64, 16, 1024, 512, 512, 64>, 1, 64, 5);
+        launch(k_flat_numeric<FUSED, 64, 16, 1024, 512, 512, 64>, 1, 64, BIN_MANY);
     }
     tm.end();
     if (p.nitems > 0 && p.use_rank) {
