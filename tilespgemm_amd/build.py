@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libtsg.so")
 CLI = os.path.join(HERE, "tsg_spgemm")
-SOURCES = ["tsg_util.hip", "tsg_row.hip", "tsg_tile.hip", "tsg_batch.hip", "tsg_server.hip",
+SOURCES = ["tsg_util.hip", "tsg_front.hip", "tsg_row.hip", "tsg_tile.hip", "tsg_batch.hip", "tsg_server.hip",
            "tsg_api.hip", "tsg_io.hip"]
 ARCH = os.environ.get("TSG_OFFLOAD_ARCH", "gfx950")
 

@@ -37,6 +37,53 @@ void scratch_setup(int device) {
     g_scratch_ptr[device] = ptr;
 }
 
+// Host boxes of a device's handles, from one page-locked slab per device
+// (page-locking takes ~0.1 ms, most of a handle's creation): made for the
+// first handle, freed with the last.  A handle past the slab's has its own.
+struct BoxSlab {
+    static constexpr int N = 64;
+    HostBox *base = nullptr;
+    uint64_t used = 0;           // a bit per box
+};
+std::mutex g_box_mu;
+BoxSlab g_box[MAX_DEVICES];
+
+HostBox *box_get(int device) {
+    std::lock_guard<std::mutex> lk(g_box_mu);
+    void *ptr = nullptr;
+    if (device >= 0 && device < MAX_DEVICES) {
+        BoxSlab &b = g_box[device];
+        if (!b.base) {
+            TSG_HIP_TRY(hipHostMalloc(&ptr, sizeof(HostBox) * BoxSlab::N, hipHostMallocDefault));
+            b.base = static_cast<HostBox *>(ptr);
+        }
+        for (int i = 0; i < BoxSlab::N; i++) {
+            if ((b.used >> i) & 1u) continue;
+            b.used |= uint64_t(1) << i;
+            return b.base + i;
+        }
+    }
+    TSG_HIP_TRY(hipHostMalloc(&ptr, sizeof(HostBox), hipHostMallocDefault));
+    return static_cast<HostBox *>(ptr);
+}
+
+void box_put(int device, HostBox *box) {
+    if (!box) return;
+    std::lock_guard<std::mutex> lk(g_box_mu);
+    if (device >= 0 && device < MAX_DEVICES) {
+        BoxSlab &b = g_box[device];
+        if (b.base && box >= b.base && box < b.base + BoxSlab::N) {
+            b.used &= ~(uint64_t(1) << (box - b.base));
+            if (!b.used) {
+                (void)hipHostFree(b.base);
+                b.base = nullptr;
+            }
+            return;
+        }
+    }
+    (void)hipHostFree(box);
+}
+
 std::mutex g_err_mu;
 std::string g_err;
 
@@ -134,15 +181,23 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
             tile_count_early(A, earlyA, ws, h->stream);
             if (!b_is_a) tile_count_early(B, earlyB, ws, h->stream);
         };
-    const int vf =
-        validate_csr_pair(A, B, ws, h->stream, want_sample ? sample : nullptr, early);
+    // with the tile path not forced, the row path's products and bins too
+    RowFront front;
+    const Arena::Mark before = ws.mark();
+    tm.begin("front");
+    const int vf = front_pass(A, B, ws, h->stream, h->box, want_sample ? sample : nullptr,
+                              h->method == TSG_METHOD_TILE ? nullptr : &front, &tune, early);
+    tm.end();
     TSG_CHECK((vf & 0x303) == 0, TSG_ERR_INVALID,
               std::string("invalid CSR input: ") + ((vf & 0x3) ? "A" : "B") +
                   ((vf & 0x101) ? " has bad row pointers" : " has a column out of range"));
     int method = choose_method(h, A, (vf & 0x404) == 0, want_sample ? sample : nullptr, ws);
     method_used = method;
     if (method == TSG_METHOD_TILE) {
+        // (with the tile path forced, its tile counts are kept)
+        const Arena::Mark mk = h->method == TSG_METHOD_TILE ? ws.mark() : before;
         try {
+            ws.rewind(mk);
             tile_symbolic(tile, A, B, b_is_a, d_ic, nnz_c, ws, h->stream, tm, h->cus, &earlyA,
                           &earlyB);
         } catch (const TsgError &e) {
@@ -156,6 +211,10 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
             tile.valid = false;
             method = TSG_METHOD_ROW;
             method_used = method;
+            // the tile path's structures give way, and the row path's are
+            // made again over them
+            ws.rewind(before);
+            (void)front_pass(A, B, ws, h->stream, h->box, nullptr, &front, &tune);
         }
     }
     if (method == TSG_METHOD_ROW) {
@@ -176,9 +235,9 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
             csr_sort_rows(n, k, d_ib, d_jb, nnz_b, b_idx, b_perm, ws, aux, h->stream);
             Bs.idx = b_idx;
             // duplicates remain after sorting: strict only if none
-            b_strict = (validate_csr_pair(Bs, Bs, aux, h->stream) & 0x4) == 0;
+            b_strict = (front_pass(Bs, Bs, aux, h->stream, h->box) & 0x4) == 0;
         }
-        row_symbolic(row, A, Bs, d_ic, nnz_c, ws, h->stream, tm, h->cus, tune);
+        row_symbolic(row, A, Bs, d_ic, nnz_c, front, h->box, ws, h->stream, tm, tune);
         row.b_strict = b_strict;
         row.b_canon = b_idx != nullptr;
         row.b_idx = b_idx;
@@ -235,7 +294,14 @@ int tsg_create(tsg_handle_t *handle, int device) {
         TSG_HIP_TRY(hipStreamCreate(&h->own_stream));
         h->stream = h->own_stream;
         h->tm.stream = h->stream;
-        scratch_setup(device);
+        try {
+            h->box = box_get(device);
+            scratch_setup(device);
+        } catch (...) {
+            box_put(device, h->box);
+            (void)hipStreamDestroy(h->own_stream);
+            throw;
+        }
         *handle = h.release();
     });
 }
@@ -250,6 +316,7 @@ int tsg_destroy(tsg_handle_t h) {
         h->bws.release();
         h->aux.release();
         if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
+        box_put(h->device, h->box);
     }
     delete h;
     return TSG_OK;
@@ -497,7 +564,7 @@ int tsg_intermediate_products(tsg_handle_t h, int m, int n, const int *d_ia, con
         DeviceGuard dg(h->device);
         h->aux.reset();
         CsrIn A{m, n, d_ia, d_ja, nullptr, nnz_a};
-        const int vf = validate_csr_pair(A, A, h->aux, h->stream);
+        const int vf = front_pass(A, A, h->aux, h->stream, h->box);
         TSG_CHECK((vf & 0x3) == 0, TSG_ERR_INVALID,
                   std::string("invalid CSR input: A") +
                       ((vf & 0x1) ? " has bad row pointers" : " has a column out of range"));

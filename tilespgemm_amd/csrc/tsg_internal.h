@@ -58,6 +58,10 @@ public:
     // what is held is dropped first.
     void attach(void *base, size_t bytes, const char *what);
     size_t used() const;
+    // What is allocated after a mark is given back by rewinding to it.
+    struct Mark { size_t cur, used; };
+    Mark mark() const;
+    void rewind(Mark m);
 
 private:
     struct Block { char *base; size_t size; size_t used; };
@@ -72,8 +76,10 @@ private:
 // Exclusive scan of n int64 counts in place into out[0..n] (out[n] = total).
 // in and out may alias.  tmp must hold scan_tmp_elems(n) int64.
 size_t scan_tmp_elems(size_t n);
+// With total set, the grand total is written there too (device memory, or
+// host memory the device can write).
 void exclusive_scan_i64(const int64_t *in, int64_t *out, size_t n, int64_t *tmp,
-                        hipStream_t s);
+                        hipStream_t s, int64_t *total = nullptr);
 // The int32 scan sums in int64; with total set, the exact int64 grand total
 // is written there too (the caller checks it against INT32_MAX).
 void exclusive_scan_i32(const int32_t *in, int32_t *out, size_t n, int64_t *tmp,
@@ -112,7 +118,57 @@ struct StageTimer {
     ~StageTimer();
 };
 
+// ---------------------------------------------------------- host results
+// Host memory of a handle that kernels write their small results into: they
+// are there once the stream is synchronized, with no copy in between.
+constexpr int ROW_BINS = 7;
+struct alignas(256) HostBox {
+    unsigned flags[2];
+    int bins[ROW_BINS];
+    unsigned long long sample[2];
+    int64_t v[8];
+};
+// Up to 8 int64 values of device memory into box->v.
+struct PublishList { const int64_t *p[8]; };
+void publish_i64(const PublishList &src, int n, HostBox *box, hipStream_t s);
+
 // ------------------------------------------------------------ row path
+// Row bins by intermediate products: (0, l1] -> 16 lanes a row, (l1, l2],
+// (l2, ROW_MID_PROD] and (ROW_MID_PROD, l3] -> a wave a row with 4, 8 and 16
+// products a lane (those with more than ROW_FLAT_ENT A entries in a bin of
+// their own), above l3 -> the big-row path.  Each small kernel is exact for
+// any row up to its register count, so any limits with l1 <= 64, l2 <= 256,
+// l3 <= 1024 (checked on the host) are valid; they are tuning parameters
+// (tsg_set_row_bins).
+constexpr int ROW_MID_PROD = 512;
+constexpr int ROW_FLAT_ENT = 64;
+constexpr int ROW_BIN_MANY = 5;
+constexpr int ROW_BIN_BIG = 6;
+struct RowBinLimits { int l1, l2, l3; };
+
+__host__ __device__ inline int row_bin_of(int64_t prod, int entries, RowBinLimits lim) {
+    if (prod == 0) return 0;
+    if (prod <= lim.l1) return 1;
+    if (prod > lim.l3) return ROW_BIN_BIG;
+    if (entries > ROW_FLAT_ENT) return ROW_BIN_MANY;
+    if (prod <= lim.l2) return 2;
+    return prod <= ROW_MID_PROD ? 3 : 4;
+}
+
+// The row path's share of the first pass over the operands: products per row
+// and the rows of each bin.  Bins 2k + 1 and 2k + 2 share a list, one from its
+// front, the other from its back.
+struct RowFront {
+    int64_t *rowprod = nullptr;      // [m]
+    int64_t *rownnz = nullptr;       // [m+1] zero for rows of bin 0 and big rows
+    int *list[3] = {nullptr, nullptr, nullptr};
+    int nlist = 0;                   // ints of each list
+    int count[ROW_BINS] = {0};       // (host) rows per bin
+    const int *rows(int bin) const {
+        return list[(bin - 1) >> 1] + ((bin & 1) ? 0 : nlist - count[bin]);
+    }
+};
+
 // Tuning parameters of the row path (tsg_set_row_bins): rows with at most
 // bin1 products take 16 lanes each, up to bin2 and bin3 a wave each, the rest
 // go to the big-row path.
@@ -138,14 +194,7 @@ struct RowPlan {
     bool valid = false;
     bool b_strict = false;           // B rows strictly ascending (no duplicates)
     int m = 0, n = 0, k = 0;
-    // per-row products and output counts
-    int64_t *rowprod = nullptr;      // [m]
-    int64_t *rownnz = nullptr;       // [m+1] (scratch for the scan)
-    // bins: small rows (by products) and big rows
-    int *bin_rows = nullptr;         // [m] rows grouped by bin
-    int *bin_start = nullptr;        // [nbins+1] device
-    int bin_start_h[16] = {0};       // host copy (after symbolic)
-    int nbins = 0;
+    RowFront front;                  // products per row, rows per bin
     // big-row structures
     int nbig = 0;
     int sub_shift = 0;               // log2 sub-block width (columns)
@@ -186,8 +235,8 @@ struct RowPlan {
 };
 
 void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic,
-                  int64_t *nnz_c, Arena &ws, hipStream_t s, StageTimer &tm, int cus,
-                  const RowTuning &tune = RowTuning());
+                  int64_t *nnz_c, const RowFront &front, HostBox *box, Arena &ws, hipStream_t s,
+                  StageTimer &tm, const RowTuning &tune);
 void row_numeric(RowPlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_ic,
                  int *d_jc, double *d_c, int fused, Arena &ws, hipStream_t s,
                  StageTimer &tm, int cus);
@@ -301,6 +350,7 @@ struct tsg_handle_s {
     Arena ws;       // plan of the last symbolic phase
     Arena bws;      // batch layout (outlives the plan's reset)
     Arena aux;      // scratch of utility calls (transpose, product counts)
+    HostBox *box = nullptr;   // pinned; results of the phases' kernels
     RowPlan row;
     TilePlan tile;
     BatchState batch;
@@ -317,18 +367,18 @@ void batch_numeric(tsg_handle_t h, int count, const tsg_product_t *prods, const 
 void batch_rebase(tsg_handle_t h, const int64_t *d_ic, int64_t *d_out);
 
 // CSR utilities
-// Validation of A and B on the device, one host round trip (flags: A in
-// bits 0-7, B in bits 8-15; 1 bad row pointers, 2 column out of range, 4 not
-// strictly ascending).  With density_sample, A's tile-density sample
-// (tile_sample_launch) runs beside the checks and its {tiles, entries} come
-// back in the same round trip; before_sync enqueues more work (and read-
-// backs) ahead of that round trip.
-int validate_csr_pair(const CsrIn &A, const CsrIn &B, Arena &ws, hipStream_t s,
-                      unsigned long long *density_sample = nullptr,
-                      const std::function<void()> &before_sync = {});
-// entries per non-empty 16x16 tile of X (tsg_tile.hip; a sample decides when
-// clear of the threshold)
-void tile_sample_launch(const CsrIn &X, unsigned long long *sums, hipStream_t s);
+// First pass over the operands (tsg_front.hip): checks of A and B on the
+// device, one host round trip (flags: A in bits 0-7, B in bits 8-15; 1 bad row
+// pointers, 2 column out of range, 4 not strictly ascending).  With
+// density_sample, the {tiles, entries} of a sample of A's tile rows; with rows
+// (and tune), the row path's products and bins.  before_sync enqueues more
+// work (and read-backs) ahead of the round trip.
+int front_pass(const CsrIn &A, const CsrIn &B, Arena &ws, hipStream_t s, HostBox *box,
+               unsigned long long *density_sample = nullptr, RowFront *rows = nullptr,
+               const RowTuning *tune = nullptr, const std::function<void()> &before_sync = {});
+// entries per non-empty 16x16 tile of X (tsg_tile.hip; a sample of every
+// tile_sample_step-th tile row decides when clear of the threshold)
+int tile_sample_step(int blkm);
 double tile_density(const CsrIn &X, double threshold, Arena &ws, hipStream_t s,
                     const unsigned long long *sample = nullptr);
 void csr_transpose(int m, int n, const int *ia, const int *ja, const double *a,

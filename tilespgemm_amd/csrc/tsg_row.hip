@@ -40,13 +40,6 @@
 namespace {
 
 constexpr int SMALL_PROD = 1024;       // rows up to this many products: small path
-constexpr int MID_PROD = 512;          // of these, up to this many: 8 registers a lane
-constexpr int FLAT_ENT = 64;           // A entries of a small row kept in LDS; rows with
-                                       // more (1024 kept: 17 KB instead of 5.5) have a bin
-constexpr int NBINS = 7;               // 0: empty, 1..4: small, 5: small of many entries, 6: big
-constexpr int BIN_MANY = 5;
-constexpr int BIN_BIG = 6;
-constexpr int bin_limit[NBINS] = {0, 64, 256, MID_PROD, SMALL_PROD, SMALL_PROD, 0x7fffffff};
 
 constexpr int SUB_SHIFT = 10;          // sub-block = 1024 columns
 constexpr int BAND_SHIFT = 6;          // symbolic band = 64 sub-blocks (65536 columns)
@@ -64,72 +57,6 @@ constexpr int ITEM_WAVES = 1;          // waves per block (one item per wave)
 constexpr int RANK_U = 8;
 constexpr int BIG_SYM_U = 4;
 constexpr int ITEM_U = 4;
-
-struct BinStarts { int s[NBINS + 1]; };
-
-// Row bins by intermediate products: (0, l1] -> 16 lanes a row, (l1, l2],
-// (l2, MID_PROD] and (MID_PROD, l3] -> a wave a row with 4, 8 and 16 products
-// a lane (those with more than FLAT_ENT A entries in a bin of their own),
-// above l3 -> the big-row path.  Each small kernel is exact for any row up to
-// bin_limit[b] products, so any limits with l1 <= 64, l2 <= 256, l3 <= 1024
-// (checked on the host) are valid; they are tuning parameters
-// (tsg_set_row_bins).
-struct BinLimits { int l1, l2, l3; };
-
-__device__ __forceinline__ int bin_of(int64_t prod, int entries, BinLimits lim) {
-    if (prod == 0) return 0;
-    if (prod <= lim.l1) return 1;
-    if (prod > lim.l3) return BIN_BIG;
-    if (entries > FLAT_ENT) return BIN_MANY;
-    if (prod <= lim.l2) return 2;
-    return prod <= MID_PROD ? 3 : 4;
-}
-
-// ------------------------------------------------------------------ binning
-__global__ void k_bin_count(int m, const int64_t *__restrict__ rowprod,
-                            const int *__restrict__ ia, BinLimits lim, int *__restrict__ cnt) {
-    __shared__ int s_cnt[NBINS];
-    if (threadIdx.x < NBINS) s_cnt[threadIdx.x] = 0;
-    __syncthreads();
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m) atomicAdd(&s_cnt[bin_of(rowprod[i], ia[i + 1] - ia[i], lim)], 1);
-    __syncthreads();
-    if (threadIdx.x < NBINS && s_cnt[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], s_cnt[threadIdx.x]);
-}
-
-// Rows go to their bin's list in any order: per wave, one ballot per bin
-// gives each lane its slot among the wave's rows of that bin; per block, one
-// LDS atomic per wave and bin; per grid, one global atomic per block and bin.
-__global__ void __launch_bounds__(256) k_bin_scatter(int m, const int64_t *__restrict__ rowprod,
-                                                     const int *__restrict__ ia,
-                                                     BinLimits lim, BinStarts st,
-                                                     int *__restrict__ fill,
-                                                     int *__restrict__ bin_rows,
-                                                     int64_t *__restrict__ rownnz) {
-    __shared__ int s_cnt[NBINS], s_base[NBINS];
-    if (threadIdx.x < NBINS) s_cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const int b = i < m ? bin_of(rowprod[i], ia[i + 1] - ia[i], lim) : -1;
-    if (b == 0 || b == BIN_BIG) rownnz[i] = 0;
-    const uint64_t below = (uint64_t(1) << lane) - 1;
-    int pos = 0;
-    for (int q = 1; q < NBINS; q++) {
-        const uint64_t mask = __ballot(b == q);
-        if (!mask) continue;
-        const int leader = __ffsll((unsigned long long)mask) - 1;
-        int wbase = 0;
-        if (lane == leader) wbase = atomicAdd(&s_cnt[q], __popcll(mask));
-        wbase = __shfl(wbase, leader);
-        if (b == q) pos = wbase + __popcll(mask & below);
-    }
-    __syncthreads();
-    if (threadIdx.x > 0 && threadIdx.x < NBINS && s_cnt[threadIdx.x])
-        s_base[threadIdx.x] = atomicAdd(&fill[threadIdx.x], s_cnt[threadIdx.x]);
-    __syncthreads();
-    if (b > 0) bin_rows[st.s[b] + s_base[b] + pos] = i;
-}
 
 // ------------------------------------------------------ small rows: symbolic
 // Output count of each row of at most G * U products (rownnz), G lanes a row:
@@ -399,7 +326,7 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
     const int64_t *__restrict__ sb_off, uint16_t *__restrict__ subcnt,
     int64_t *__restrict__ rownnz, const int64_t *__restrict__ band_off,
     int64_t *__restrict__ band_base, unsigned long long *__restrict__ row_cur,
-    const int64_t *__restrict__ row_off, unsigned *__restrict__ overflow,
+    const int64_t *__restrict__ row_off, int64_t *__restrict__ overflow,
     unsigned *__restrict__ subocc, unsigned *__restrict__ words_out) {
     constexpr int NW = BAND_T / 64;
     constexpr int TW = BAND_WORDS / BAND_T;        // words per thread, half a sub-block
@@ -496,7 +423,7 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
             if (threadIdx.x == 0) {
                 long long base = (long long)ticket;
                 if (base + padded > row_off[r + 1]) {
-                    atomicOr(overflow, 1u);
+                    *overflow = 1;
                     base = -1;
                 }
                 band_base[band_off[r] + u] = base;
@@ -1155,72 +1082,45 @@ void set_smem(K kernel, size_t bytes) {
 
 // =================================================================== host
 void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int64_t *nnz_c,
-                  Arena &ws, hipStream_t s, StageTimer &tm, int /*cus*/, const RowTuning &tune) {
+                  const RowFront &front, HostBox *box, Arena &ws, hipStream_t s, StageTimer &tm,
+                  const RowTuning &tune) {
     const int m = A.rows, n = A.cols, k = B.cols;
-    TSG_CHECK(tune.bin1 >= 0 && tune.bin1 <= bin_limit[1] && tune.bin1 <= tune.bin2 &&
-                  tune.bin2 <= bin_limit[2] && tune.bin2 <= tune.bin3 &&
-                  tune.bin3 <= bin_limit[4],
+    TSG_CHECK(tune.bin1 >= 0 && tune.bin1 <= 64 && tune.bin1 <= tune.bin2 && tune.bin2 <= 256 &&
+                  tune.bin2 <= tune.bin3 && tune.bin3 <= SMALL_PROD,
               TSG_ERR_INVALID, "row bins out of range");
-    const BinLimits lim{tune.bin1, tune.bin2, tune.bin3};
     p = RowPlan();
     p.m = m;
     p.n = n;
     p.k = k;
-    p.rowprod = ws.alloc_n<int64_t>((size_t)m + 1);
-    p.rownnz = ws.alloc_n<int64_t>((size_t)m + 1);
-    p.bin_rows = ws.alloc_n<int>((size_t)m + 1);
-    int *d_cnt = ws.alloc_n<int>(2 * NBINS);
+    p.front = front;
     int64_t *scan_tmp = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)m + 1));
-
-    tm.begin("row.products+bins");
-    csr_row_products(m, A.ptr, A.idx, A.nnz, B.ptr, p.rowprod, ws, s);
-    TSG_HIP_TRY(hipMemsetAsync(d_cnt, 0, sizeof(int) * (2 * NBINS), s));
-    if (m > 0) {
-        hipLaunchKernelGGL(k_bin_count, dim3(grid_for(m, 256)), dim3(256), 0, s, m, p.rowprod,
-                           A.ptr, lim, d_cnt);
-        TSG_LAUNCH_CHECK();
-    }
-    int h_cnt[NBINS];
-    TSG_HIP_TRY(hipMemcpyAsync(h_cnt, d_cnt, sizeof(h_cnt), hipMemcpyDeviceToHost, s));
-    TSG_HIP_TRY(hipStreamSynchronize(s));
-    BinStarts st;
-    st.s[0] = 0;
-    for (int b = 0; b < NBINS; b++) st.s[b + 1] = st.s[b] + (b == 0 ? 0 : h_cnt[b]);
-    for (int b = 0; b <= NBINS; b++) p.bin_start_h[b] = st.s[b];
-    p.nbins = NBINS;
-    if (m > 0) {
-        hipLaunchKernelGGL(k_bin_scatter, dim3(grid_for(m, 256)), dim3(256), 0, s, m, p.rowprod,
-                           A.ptr, lim, st, d_cnt + NBINS, p.bin_rows, p.rownnz);
-        TSG_LAUNCH_CHECK();
-    }
-    tm.end();
 
     // small rows
     tm.begin("row.small_symbolic");
     {
         auto launch = [&](auto kern, int rpb, int threads, int bin) {
-            const int nr = st.s[bin + 1] - st.s[bin];
+            const int nr = front.count[bin];
             if (nr <= 0) return;
             hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
-                               p.bin_rows + st.s[bin], A.ptr, A.idx, B.ptr, B.idx, p.rownnz);
+                               front.rows(bin), A.ptr, A.idx, B.ptr, B.idx, front.rownnz);
             TSG_LAUNCH_CHECK();
         };
         launch(k_flat_symbolic<16, 4, 64, 64, 256>, 16, 256, 1);
         launch(k_flat_symbolic<64, 4, 64, 512, 64>, 1, 64, 2);
         launch(k_flat_symbolic<64, 8, 64, 512, 64>, 1, 64, 3);
         launch(k_flat_symbolic<64, 16, 64, 512, 64, 6>, 1, 64, 4);
-        launch(k_flat_symbolic<64, 16, 1024, 512, 64>, 1, 64, BIN_MANY);
+        launch(k_flat_symbolic<64, 16, 1024, 512, 64>, 1, 64, ROW_BIN_MANY);
     }
     tm.end();
 
     // big rows
-    p.nbig = st.s[BIN_BIG + 1] - st.s[BIN_BIG];
+    p.nbig = front.count[ROW_BIN_BIG];
     p.sub_shift = SUB_SHIFT;
     int64_t *band_off = nullptr, *band_base = nullptr, *row_loff = nullptr;
     unsigned long long *row_cur = nullptr;
-    unsigned *d_overflow = nullptr;
+    int64_t *d_overflow = nullptr;
     if (p.nbig > 0) {
-        const int *rowsb = p.bin_rows + st.s[BIN_BIG];
+        const int *rowsb = front.rows(ROW_BIN_BIG);
         tm.begin("row.big_symbolic");
         // column span of every big row, in sub-blocks, span offsets and the
         // band units over the spans
@@ -1232,7 +1132,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         int64_t *a_prod = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         row_loff = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         hipLaunchKernelGGL(k_big_span, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0, s,
-                           p.nbig, rowsb, A.ptr, A.idx, B.ptr, B.idx, p.rowprod, p.span_sb0,
+                           p.nbig, rowsb, A.ptr, A.idx, B.ptr, B.idx, front.rowprod, p.span_sb0,
                            p.sb_off, a_ent, a_prod, row_loff);
         TSG_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_band_count, dim3(grid_for((size_t)p.nbig, 256)), dim3(256), 0, s,
@@ -1243,18 +1143,12 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         exclusive_scan_i64(a_ent, a_ent, (size_t)p.nbig, tmp_sb, s);
         exclusive_scan_i64(a_prod, a_prod, (size_t)p.nbig, tmp_sb, s);
         exclusive_scan_i64(row_loff, row_loff, (size_t)p.nbig, tmp_sb, s);
-        int64_t tot2[5] = {0, 0, 0, 0, 0};
-        TSG_HIP_TRY(hipMemcpyAsync(&tot2[0], p.sb_off + p.nbig, sizeof(int64_t),
-                                   hipMemcpyDeviceToHost, s));
-        TSG_HIP_TRY(hipMemcpyAsync(&tot2[1], band_off + p.nbig, sizeof(int64_t),
-                                   hipMemcpyDeviceToHost, s));
-        TSG_HIP_TRY(hipMemcpyAsync(&tot2[2], a_ent + p.nbig, sizeof(int64_t),
-                                   hipMemcpyDeviceToHost, s));
-        TSG_HIP_TRY(hipMemcpyAsync(&tot2[3], a_prod + p.nbig, sizeof(int64_t),
-                                   hipMemcpyDeviceToHost, s));
-        TSG_HIP_TRY(hipMemcpyAsync(&tot2[4], row_loff + p.nbig, sizeof(int64_t),
-                                   hipMemcpyDeviceToHost, s));
+        publish_i64({{p.sb_off + p.nbig, band_off + p.nbig, a_ent + p.nbig, a_prod + p.nbig,
+                      row_loff + p.nbig}},
+                    5, box, s);
         TSG_HIP_TRY(hipStreamSynchronize(s));
+        int64_t tot2[5];
+        std::copy(box->v, box->v + 5, tot2);
         const int64_t nsb_total = tot2[0], nunits = tot2[1];
         p.nsb_total = nsb_total;
         p.subcnt = ws.alloc_n<uint16_t>((size_t)nsb_total + 1);
@@ -1277,10 +1171,10 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         if (p.use_rank) {
             band_base = ws.alloc_n<int64_t>((size_t)nunits + 1);
             row_cur = ws.alloc_n<unsigned long long>((size_t)p.nbig + 1);
-            d_overflow = ws.alloc_n<unsigned>(1);
+            d_overflow = ws.alloc_n<int64_t>(1);
             TSG_HIP_TRY(hipMemcpyAsync(row_cur, row_loff, sizeof(int64_t) * (size_t)p.nbig,
                                        hipMemcpyDeviceToDevice, s));
-            TSG_HIP_TRY(hipMemsetAsync(d_overflow, 0, sizeof(unsigned), s));
+            TSG_HIP_TRY(hipMemsetAsync(d_overflow, 0, sizeof(int64_t), s));
         }
         // B as {column, value} records for the rank kernel's gathers
         p.bpk = p.use_rank ? ws.alloc_n<int4>((size_t)B.nnz + 1) : nullptr;
@@ -1358,7 +1252,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         hipLaunchKernelGGL(k_big_symbolic,
                            dim3((unsigned)std::min<int64_t>(nunits, int64_t(1) << 30)),
                            dim3(BAND_T), 0, s, nunits, units, rowsb, k, A.ptr, A.idx, B.ptr,
-                           B.idx, block_ptrs(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, p.rownnz,
+                           B.idx, block_ptrs(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, front.rownnz,
                            band_off, band_base, row_cur, row_loff, d_overflow, p.subocc,
                            p.bandwords);
         TSG_LAUNCH_CHECK();
@@ -1366,13 +1260,13 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     }
 
     tm.begin("row.scan");
-    exclusive_scan_i64(p.rownnz, d_ic, (size_t)m, scan_tmp, s);
+    exclusive_scan_i64(front.rownnz, d_ic, (size_t)m, scan_tmp, s, &box->v[7]);
     tm.end();
 
     int64_t h_tot[2] = {0, 0};
     if (p.nbig > 0) {
         tm.begin("row.items");
-        const int *rowsb = p.bin_rows + st.s[BIN_BIG];
+        const int *rowsb = front.rows(ROW_BIN_BIG);
         p.item_cnt = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         int64_t *tmp2 = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)p.nbig + 1));
         // Narrow (8-sub-block) windows when the spans are wide enough that
@@ -1392,14 +1286,11 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         else
             items_kernel(k_items<false, 16>, p.item_cnt, nullptr, nullptr);
         exclusive_scan_i64(p.item_cnt, p.item_cnt, (size_t)p.nbig, tmp2, s);
-        unsigned h_overflow = 0;
-        TSG_HIP_TRY(hipMemcpyAsync(&h_tot[1], p.item_cnt + p.nbig, sizeof(int64_t),
-                                   hipMemcpyDeviceToHost, s));
-        TSG_HIP_TRY(hipMemcpyAsync(&h_tot[0], d_ic + m, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        if (d_overflow)
-            TSG_HIP_TRY(hipMemcpyAsync(&h_overflow, d_overflow, sizeof(h_overflow),
-                                       hipMemcpyDeviceToHost, s));
+        publish_i64({{p.item_cnt + p.nbig, d_overflow}}, d_overflow ? 2 : 1, box, s);
         TSG_HIP_TRY(hipStreamSynchronize(s));
+        h_tot[0] = box->v[7];
+        h_tot[1] = box->v[0];
+        const int64_t h_overflow = d_overflow ? box->v[1] : 0;
         // the lists are sized by a bound on the outputs, so this holds unless
         // the symbolic phase itself went wrong
         TSG_CHECK(h_overflow == 0, TSG_ERR_OVERFLOW, "big-row word lists exceed their bound");
@@ -1436,18 +1327,16 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
             TSG_LAUNCH_CHECK();
             p.items = items_s;
             if (p.use_rank) {
-                int64_t h_cls[2] = {0, 0};
-                TSG_HIP_TRY(hipMemcpyAsync(h_cls, d_small, sizeof(h_cls), hipMemcpyDeviceToHost,
-                                           s));
+                publish_i64({{d_small, d_small + 1}}, 2, box, s);
                 TSG_HIP_TRY(hipStreamSynchronize(s));
-                p.nitems_small = h_cls[0];
-                p.nitems_mid = h_cls[0] + h_cls[1];
+                p.nitems_small = box->v[0];
+                p.nitems_mid = box->v[0] + box->v[1];
             }
         }
         tm.end();
     } else {
-        TSG_HIP_TRY(hipMemcpyAsync(&h_tot[0], d_ic + m, sizeof(int64_t), hipMemcpyDeviceToHost, s));
         TSG_HIP_TRY(hipStreamSynchronize(s));
+        h_tot[0] = box->v[7];
     }
     *nnz_c = h_tot[0];
     p.valid = true;
@@ -1456,15 +1345,14 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
 template <bool FUSED>
 static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_ic,
                           int *d_jc, double *d_c, hipStream_t s, StageTimer &tm) {
-    const int *bins = p.bin_rows;
-    const int *st = p.bin_start_h;
+    const RowFront &front = p.front;
     tm.begin("row.small_numeric");
     {
         auto launch = [&](auto kern, int rpb, int threads, int bin) {
-            const int nr = st[bin + 1] - st[bin];
+            const int nr = front.count[bin];
             if (nr <= 0) return;
             hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
-                               bins + st[bin], A.ptr, A.idx, A.val, B.ptr, B.idx, B.val, d_ic,
+                               front.rows(bin), A.ptr, A.idx, A.val, B.ptr, B.idx, B.val, d_ic,
                                d_jc, d_c, (int)p.b_strict);
             TSG_LAUNCH_CHECK();
         };
@@ -1472,7 +1360,7 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
         launch(k_flat_numeric<FUSED, 64, 4, 64, 512, 256, 64>, 1, 64, 2);
         launch(k_flat_numeric<FUSED, 64, 8, 64, 512, 512, 64>, 1, 64, 3);
         launch(k_flat_numeric<FUSED, 64, 16, 64, 512, 512, 64>, 1, 64, 4);
-        launch(k_flat_numeric<FUSED, 64, 16, 1024, 512, 512, 64>, 1, 64, BIN_MANY);
+        launch(k_flat_numeric<FUSED, 64, 16, 1024, 512, 512, 64>, 1, 64, ROW_BIN_MANY);
     }
     tm.end();
     if (p.nitems > 0 && p.use_rank) {

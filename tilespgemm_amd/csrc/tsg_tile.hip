@@ -33,6 +33,7 @@
 #include "tsg_internal.h"
 #include "tsg_device.h"
 #include "tsg_expand.h"
+#include "tsg_sample.h"
 
 #include <algorithm>
 #include <climits>
@@ -119,53 +120,6 @@ __global__ void __launch_bounds__(256) k_tile_convert(
 // the bitmap window covers 65536 tile columns per pass.
 constexpr int TC_WAVES = 4;
 constexpr int TC_WORDS = 2048;
-constexpr int TC_U = 4;
-
-// Row pointers are clamped to [0, nnz] and columns to [0, ncols): every
-// access stays in bounds (and the tile-column loop bounded) whatever the
-// entries hold.  A bit already set is not set again (power-law rows repeat a
-// few tile columns, whose words would serialise the LDS atomics); TC_U
-// entries per lane and pass have their loads issued together.
-template <int NT>
-struct TileCols {
-    int p1, cmax;
-    const int *ja;
-    __device__ void load(int p, int (&J)[TC_U]) const {
-#pragma unroll
-        for (int q = 0; q < TC_U; q++) {
-            const int pq = p + q * NT;
-            J[q] = pq < p1 ? min(max(ja[pq], 0), cmax) >> 4 : -1;
-        }
-    }
-    // tile-column range of the entries [p0 + t, p1) taken by thread t
-    __device__ void range(int p0, int t, int &lo, int &hi) const {
-        lo = INT_MAX;
-        hi = -1;
-        for (int p = p0 + t; p < p1; p += NT * TC_U) {
-            int J[TC_U];
-            load(p, J);
-#pragma unroll
-            for (int q = 0; q < TC_U; q++)
-                if (J[q] >= 0) {
-                    lo = min(lo, J[q]);
-                    hi = max(hi, J[q]);
-                }
-        }
-    }
-    __device__ void mark(int p0, int t, int w0, int w1, unsigned *bits) const {
-        for (int p = p0 + t; p < p1; p += NT * TC_U) {
-            int J[TC_U];
-            load(p, J);
-#pragma unroll
-            for (int q = 0; q < TC_U; q++)
-                if (J[q] >= w0 && J[q] < w1) {
-                    const unsigned bit = 1u << ((J[q] - w0) & 31);
-                    unsigned *word = &bits[(J[q] - w0) >> 5];
-                    if (!(*word & bit)) atomicOr(word, bit);
-                }
-        }
-    }
-};
 
 __global__ void __launch_bounds__(64 * TC_WAVES) k_tile_count(int m, int ncols, int64_t nnz,
                                                               int blkm,
@@ -199,57 +153,14 @@ __global__ void __launch_bounds__(64 * TC_WAVES) k_tile_count(int m, int ncols, 
     if (l == 0) tcount[I] = count;
 }
 
-// AUTO's density sample: tile rows 0, step, 2*step, ... (the grid has one
-// block per sampled row, so every block's row is < blkm), one 256-thread
-// block each sharing a bitmap of 262144 tile columns per pass -- a
-// power-law matrix puts most of its entries in its first tile rows, and one
-// wave per row left the sample waiting on those.  The tile and entry counts
-// are added to sums[0] and sums[1].  Indices are clamped as above, so the
-// sample can run beside the input's validation instead of after it.
-constexpr int TS_WORDS = 8192;
-
+// The density count of tile rows 0, step, 2*step, ... (the grid has one block
+// per row taken, so every block's row is < blkm).
 __global__ void __launch_bounds__(256) k_tile_sample(int m, int ncols, int64_t nnz, int step,
                                                      const int *__restrict__ ia,
                                                      const int *__restrict__ ja,
                                                      unsigned long long *__restrict__ sums) {
     __shared__ unsigned bits[TS_WORDS];
-    __shared__ int s_lo[4], s_hi[4];
-    __shared__ int s_cnt[4];
-    const int I = blockIdx.x * step;
-    const int t = threadIdx.x, l = t & 63, w = t >> 6;
-    const int p0 = (int)min((int64_t)max(ia[I * 16], 0), nnz);
-    const int p1 = (int)min((int64_t)max(ia[min(m, I * 16 + 16)], p0), nnz);
-    const TileCols<256> tc{p1, max(ncols - 1, 0), ja};
-    int lo, hi;
-    tc.range(p0, t, lo, hi);
-    lo = wave_min(lo);
-    hi = wave_max(hi);
-    if (l == 0) {
-        s_lo[w] = lo;
-        s_hi[w] = hi;
-    }
-    __syncthreads();
-    lo = min(min(s_lo[0], s_lo[1]), min(s_lo[2], s_lo[3]));
-    hi = max(max(s_hi[0], s_hi[1]), max(s_hi[2], s_hi[3]));
-    int count = 0;
-    // lo and hi are the block's: every thread takes every pass and barrier
-    for (int w0 = lo; w0 <= hi; w0 += TS_WORDS * 32) {
-        const int w1 = min(hi + 1, w0 + TS_WORDS * 32);
-        const int nwords = (w1 - w0 + 31) >> 5;
-        for (int i = t; i < nwords; i += 256) bits[i] = 0u;
-        __syncthreads();
-        tc.mark(p0, t, w0, w1, bits);
-        __syncthreads();
-        for (int i = t; i < nwords; i += 256) count += __popc(bits[i]);
-        __syncthreads();
-    }
-    count = wave_sum(count);
-    if (l == 0) s_cnt[w] = count;
-    __syncthreads();
-    if (t == 0) {
-        atomicAdd(&sums[0], (unsigned long long)(s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3]));
-        atomicAdd(&sums[1], (unsigned long long)(p1 - p0));
-    }
+    tile_sample_row(blockIdx.x * step, m, ncols, nnz, ia, ja, sums, bits);
 }
 
 __global__ void k_perm_scatter(int64_t nnz, const int *__restrict__ perm,
@@ -1281,10 +1192,9 @@ void tile_numeric(TilePlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_
 // Entries per non-empty 16x16 tile of X, used to choose between the tile
 // path and the row path.  A deterministic sample of <= 1024 tile rows
 // decides unless it lands near the threshold, where every tile row is
-// counted.  tile_sample_launch enqueues the sample's count (sums = {tiles,
-// entries}, zeroed by the caller) so that it can share a host round trip
-// with other work; tile_density takes its result, or counts itself.
-static int tile_sample_step(int blkm) { return blkm > 1024 ? (blkm + 1023) / 1024 : 1; }
+// counted.  The sample comes with the input checks (front_pass), or is taken
+// here.
+int tile_sample_step(int blkm) { return blkm > 1024 ? (blkm + 1023) / 1024 : 1; }
 
 static void tile_count_launch(const CsrIn &X, int step, unsigned long long *sums,
                               hipStream_t s) {
@@ -1295,12 +1205,6 @@ static void tile_count_launch(const CsrIn &X, int step, unsigned long long *sums
     hipLaunchKernelGGL(k_tile_sample, dim3((unsigned)nrows), dim3(256), 0, s, X.rows, X.cols,
                        X.nnz, step, X.ptr, X.idx, sums);
     TSG_LAUNCH_CHECK();
-}
-
-void tile_sample_launch(const CsrIn &X, unsigned long long *sums, hipStream_t s) {
-    const int blkm = (X.rows + 15) / 16;
-    if (blkm == 0 || X.nnz == 0) return;
-    tile_count_launch(X, tile_sample_step(blkm), sums, s);
 }
 
 double tile_density(const CsrIn &X, double threshold, Arena &ws, hipStream_t s,

@@ -37,6 +37,16 @@ void Arena::reset() {
     cur_ = 0;
 }
 
+Arena::Mark Arena::mark() const {
+    return Mark{cur_, cur_ < blocks_.size() ? blocks_[cur_].used : 0};
+}
+
+void Arena::rewind(Mark m) {
+    for (size_t i = m.cur + 1; i < blocks_.size(); i++) blocks_[i].used = 0;
+    if (m.cur < blocks_.size()) blocks_[m.cur].used = m.used;
+    cur_ = m.cur;
+}
+
 void *Arena::alloc(size_t bytes) {
     bytes = (bytes + 255) & ~size_t(255);
     while (cur_ < blocks_.size()) {
@@ -69,13 +79,15 @@ void *Arena::alloc(size_t bytes) {
 }
 
 // ================================================================= scans
-// Three-phase exclusive scan: per-block totals, recursive scan of the totals,
-// per-block rescan with the block's offset.  1024 elements per 256-thread
-// block (4 per thread).
+// Exclusive scan: per-block totals, then a rescan of each block with its
+// offset, which up to SCAN_FLAT blocks add up themselves from the totals (a
+// launch less); past that the totals are scanned first, recursively.  1024
+// elements per 256-thread block (4 per thread).
 namespace {
 constexpr int SCAN_T = 256;
 constexpr int SCAN_PER = 4;
 constexpr int SCAN_BLK = SCAN_T * SCAN_PER;
+constexpr size_t SCAN_FLAT = 2048;
 
 template <class T>
 __device__ __forceinline__ long long block_excl_scan(long long x, long long *total) {
@@ -121,7 +133,14 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_apply(const T *in, T *out, size
     }
     long long tot;
     long long ex = block_excl_scan<T>(s, &tot);
-    long long run = ex + (has_offs ? offs[blockIdx.x] : 0);
+    long long before = 0;              // of earlier blocks: 1 scanned, 2 totals
+    if (has_offs == 1) before = offs[blockIdx.x];
+    if (has_offs == 2) {
+        long long part = 0;
+        for (unsigned i = threadIdx.x; i < blockIdx.x; i += SCAN_T) part += offs[i];
+        (void)block_excl_scan<T>(part, &before);
+    }
+    long long run = ex + before;
 #pragma unroll
     for (int i = 0; i < SCAN_PER; i++) {
         if (base + i < n) out[base + i] = (T)run;
@@ -155,9 +174,10 @@ void scan_rec(const T *in, T *out, size_t n, long long *tmp, hipStream_t s,
     long long *rest = tmp + nb + 1;
     hipLaunchKernelGGL(k_scan_reduce<T>, dim3((unsigned)nb), dim3(SCAN_T), 0, s, in, n, sums);
     TSG_LAUNCH_CHECK();
-    scan_rec<long long>(sums, sums, nb, rest, s);
+    const bool flat = nb <= SCAN_FLAT;
+    if (!flat) scan_rec<long long>(sums, sums, nb, rest, s);
     hipLaunchKernelGGL(k_scan_apply<T>, dim3((unsigned)nb), dim3(SCAN_T), 0, s, in, out, n,
-                       (const long long *)sums, 1, total);
+                       (const long long *)sums, flat ? 2 : 1, total);
     TSG_LAUNCH_CHECK();
 }
 }  // namespace
@@ -175,8 +195,21 @@ size_t scan_tmp_elems(size_t n) {
 // The apply pass reads in[] before any block writes out[] only within its own
 // block range, so in == out is safe: every block reads its elements before
 // writing them, and out[n] lies outside every block's input range.
-void exclusive_scan_i64(const int64_t *in, int64_t *out, size_t n, int64_t *tmp, hipStream_t s) {
-    scan_rec<long long>((const long long *)in, (long long *)out, n, (long long *)tmp, s);
+void exclusive_scan_i64(const int64_t *in, int64_t *out, size_t n, int64_t *tmp, hipStream_t s,
+                        int64_t *total) {
+    scan_rec<long long>((const long long *)in, (long long *)out, n, (long long *)tmp, s,
+                        (long long *)total);
+}
+
+__global__ void __launch_bounds__(64) k_publish(PublishList src, int n,
+                                                int64_t *__restrict__ out) {
+    const int t = threadIdx.x;
+    if (t < n) out[t] = *src.p[t];
+}
+
+void publish_i64(const PublishList &src, int n, HostBox *box, hipStream_t s) {
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, src, n, box->v);
+    TSG_LAUNCH_CHECK();
 }
 
 void exclusive_scan_i32(const int32_t *in, int32_t *out, size_t n, int64_t *tmp, hipStream_t s,
@@ -221,100 +254,10 @@ void StageTimer::finalize() {
 
 StageTimer::~StageTimer() { clear(); }
 
-// ======================================================= validation
-// flags: bit 0 bad row pointers, bit 1 column out of range, bit 2 a row not
-// strictly ascending (unsorted or duplicate columns).  Reads stay inside
-// [0, nnz) whatever the row pointers hold.
 // The kernels below run between kernels that stream gigabytes, so their
 // operands are cold in every cache: each keeps its chain of dependent loads
 // to two or three (no searches, no per-row loops), which is what sets their
 // duration.
-
-// Threads check row pointers t < m and entries t < nnz (grid-stride).  Rows
-// are sorted and duplicate-free iff every descent ja[p-1] >= ja[p] (p > 0)
-// sits at the first entry of a non-empty row, i.e. iff the number of all
-// descents equals the number of descents at row starts: out[1] counts the
-// former, out[2] the latter (summed per block, one atomic per block and
-// counter).  Every access stays inside ia[0..m] and ja[0..nnz) whatever the
-// contents.
-__global__ void __launch_bounds__(256) k_validate(int m, int n, const int *__restrict__ ia,
-                                                  const int *__restrict__ ja, int64_t nnz,
-                                                  int *__restrict__ out) {
-    __shared__ int s_cnt[2][4];
-    int f = 0;
-    int at_start = 0, descent = 0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t lim = nnz > m ? nnz : m;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < lim; t += stride) {
-        if (t < m) {
-            const int64_t lo = ia[t], hi = ia[t + 1];
-            if (lo > hi || lo < 0 || hi > nnz) f |= 1;
-            if (t == 0 && lo != 0) f |= 1;
-            if (t == m - 1 && hi != nnz) f |= 1;
-            if (lo > 0 && lo < hi && hi <= nnz) at_start += ja[lo - 1] >= ja[lo];
-        }
-        if (t < nnz) {
-            const int c = ja[t];
-            if (c < 0 || c >= n) f |= 2;
-            if (t > 0) descent += ja[t - 1] >= c;
-        }
-    }
-    descent = wave_sum(descent);
-    at_start = wave_sum(at_start);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        s_cnt[0][w] = descent;
-        s_cnt[1][w] = at_start;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int d = s_cnt[0][0] + s_cnt[0][1] + s_cnt[0][2] + s_cnt[0][3];
-        const int st = s_cnt[1][0] + s_cnt[1][1] + s_cnt[1][2] + s_cnt[1][3];
-        if (d) atomicAdd(&out[1], d);
-        if (st) atomicAdd(&out[2], st);
-    }
-    if (f) atomicOr(&out[0], f);
-}
-
-int validate_csr_pair(const CsrIn &A, const CsrIn &B, Arena &ws, hipStream_t s,
-                      unsigned long long *density_sample,
-                      const std::function<void()> &before_sync) {
-    // six flag/count ints, then the two sums of the density sample
-    unsigned long long *buf = ws.alloc_n<unsigned long long>(5);
-    int *d = reinterpret_cast<int *>(buf);
-    TSG_HIP_TRY(hipMemsetAsync(buf, 0, 5 * sizeof(unsigned long long), s));
-    if (density_sample) tile_sample_launch(A, buf + 3, s);
-    // a fixed grid (grid-stride inside): few per-block atomics on the counters
-    auto threads = [](const CsrIn &X) {
-        return std::min(std::max((size_t)X.rows, (size_t)X.nnz), (size_t)256 * 2048);
-    };
-    if (A.rows > 0) {
-        hipLaunchKernelGGL(k_validate, dim3(grid_for(threads(A), 256)), dim3(256), 0, s, A.rows,
-                           A.cols, A.ptr, A.idx, A.nnz, d);
-        TSG_LAUNCH_CHECK();
-    }
-    if (B.rows > 0 && (B.ptr != A.ptr || B.idx != A.idx || B.cols != A.cols)) {
-        hipLaunchKernelGGL(k_validate, dim3(grid_for(threads(B), 256)), dim3(256), 0, s, B.rows,
-                           B.cols, B.ptr, B.idx, B.nnz, d + 3);
-        TSG_LAUNCH_CHECK();
-    }
-    if (before_sync) before_sync();
-    unsigned long long hb[5] = {0, 0, 0, 0, 0};
-    TSG_HIP_TRY(hipMemcpyAsync(hb, buf, sizeof(hb), hipMemcpyDeviceToHost, s));
-    TSG_HIP_TRY(hipStreamSynchronize(s));
-    int h[6];
-    std::memcpy(h, hb, sizeof(h));
-    if (density_sample) {
-        density_sample[0] = hb[3];
-        density_sample[1] = hb[4];
-    }
-    int fa = h[0], fb = h[3];
-    if (h[1] != h[2]) fa |= 4;
-    if (h[4] != h[5]) fb |= 4;
-    if (A.rows == 0 && A.nnz != 0) fa |= 1;
-    if (B.rows == 0 && B.nnz != 0) fb |= 1;
-    return fa | (fb << 8);
-}
 
 // ======================================================= row products
 // rowprod[i] = sum over A's entries a_ik in row i of |row k of B|
