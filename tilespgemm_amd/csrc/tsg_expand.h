@@ -31,57 +31,90 @@ __device__ __forceinline__ int brange_lo(const BlockPtrs &bp, const int *__restr
     return lo;
 }
 
-// Products of one group of G A entries: lane l's A entry contributes the B
-// positions [lo, lo + cnt) with value a.  Batches of G products are handed to
-// f in product order (see for_products); bofs/bstep select every bstep-th
-// batch starting at bofs.  s_mark: the group's G ints of LDS, all -1 on entry
-// and on return.
+// A batch of 64 products seen by the functions below: act marks the lanes
+// that hold a product; seg is the lane's A entry among the batch's (from 1)
+// and nseg their number (uniform); products of one A entry are one B row's:
+// distinct columns whenever B's rows are duplicate-free.
+struct Batch {
+    bool act;
+    int col;
+    double a, b;
+    int seg, nseg;
+};
+
+// Products of one group of 64 A entries: lane l's A entry contributes the B
+// positions [lo, lo + cnt) with value a.  Batches of 64 products are handed
+// to f in product order (see for_products); bofs/bstep select every bstep-th
+// batch starting at bofs.
+//
+// A product finds its A entry by counting: the entries with products move to
+// the front lanes (a permutation, once per group), a bit is set in LDS (heads:
+// 64 ints, any content) where each one's products start, and product q
+// belongs to entry (bits at or below q) - 1.  A batch's 64 bits are a scalar,
+// so the count is two instructions, against a running maximum over marks
+// written per batch (an LDS round trip and six steps): R-MAT 2^18, items of
+// more than 512 outputs, 1.19 -> 0.96 ms; R-MAT 2^20 with 8 draws a row, 21.6
+// -> 20.7 ms, and its symbolic bands 14.1 -> 13.2 ms.
 // PACKED: B's entries are also given as 16-byte {column, -, value} records
 // (bpk), so a product's column and value come from one load and, for a short
 // range, one cache line.
-template <int G, int U, bool VALUES, bool PACKED = false, class F>
+template <int U, int BSTEP, bool VALUES, bool PACKED = false, class F>
 __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
                                              const int *__restrict__ jb,
-                                             const double *__restrict__ bval, int *s_mark,
-                                             F &&f, int bofs = 0, int bstep = 1,
+                                             const double *__restrict__ bval, int *heads, F &&f,
+                                             int bofs = 0,
                                              const int4 *__restrict__ bpk = nullptr) {
-    static_assert(G >= 16, "segment lookup scans 16, 32 or 64 lanes");
-    const int l = __lane_id() & (G - 1);
-    const int gbase = __lane_id() & ~(G - 1);
-    const unsigned long long gmask = G == 64 ? ~0ull : ((1ull << G) - 1);
-    const int incl = group_incl_scan<G>(cnt);
-    const int total = group_last<G>(incl);
+    static_assert(2 * U * BSTEP <= 64, "a round's start bits are a word a lane");
+    const int l = __lane_id();
+    const int incl = wave_incl_scan(cnt);
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    if (total <= 0) return;
     const int start = incl - cnt;
-    // position in B of product q of source lane s: off_s + q
-    const int off = lo - start;
-    for (int base = bofs * G; base < total; base += G * U * bstep) {
-        int e[U], sl[U];
+    const unsigned long long some = __ballot(cnt > 0);
+    int off;                           // of the l-th entry with products
+    double av = 0.0;
+    {
+        const unsigned long long below = (1ull << l) - 1;
+        const int to = 4 * (cnt > 0 ? __popcll(some & below)
+                                    : __popcll(some) + __popcll(~some & below));
+        off = __builtin_amdgcn_ds_permute(to, lo - start);
+        if (VALUES)
+            av = __hiloint2double(__builtin_amdgcn_ds_permute(to, __double2hiint(a)),
+                                  __builtin_amdgcn_ds_permute(to, __double2loint(a)));
+    }
+    for (int base = 0; base < total; base += 64 * U * BSTEP) {
+        wave_lds_fence();
+        if (l < 2 * U * BSTEP) heads[l] = 0;
+        wave_lds_fence();
+        const int at = start - base;
+        if (cnt > 0 && at >= 0 && at < 64 * U * BSTEP)
+            atomicOr(reinterpret_cast<unsigned *>(heads) + (at >> 5), 1u << (at & 31));
+        wave_lds_fence();
+        const int hv = l < 2 * U * BSTEP ? heads[l] : 0;
+        // entries that start before the batch, less one
+        int before = __popcll(__ballot(cnt > 0 && at < 0)) - 1;
+        int e[U], sl[U], seg[U], nseg[U];
         bool act[U];
-        double as[U];
-        // batches of this chunk holding products: the rest are skipped
-        // (uniform over the group; with G == 64, over the wave)
-        const int nb = (total - base + G * bstep - 1) / (G * bstep);
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            act[u] = false;
-            as[u] = 0.0;
-            e[u] = 0;
-            sl[u] = 0;
-            if (u < nb) {
-                const int qb = base + u * G * bstep;
-                const int q = qb + l;
+        for (int v = 0; v < U * BSTEP; v++) {
+            const unsigned long long m =
+                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane(hv, 2 * v + 1) << 32) |
+                (unsigned)__builtin_amdgcn_readlane(hv, 2 * v);
+            const int u = v / BSTEP;
+            if (BSTEP == 1 || v % BSTEP == bofs) {
+                const int q = base + 64 * v + l;
+                // bits at or below the lane: those of m >> 1 below it, bit 0
+                const unsigned long long m1 = m >> 1;
+                sl[u] = (int)__builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m1 >> 32),
+                    __builtin_amdgcn_mbcnt_lo((unsigned)m1, (unsigned)(before + (int)(m & 1))));
+                const int first = before + (int)(m & 1);
+                seg[u] = sl[u] - first + 1;
+                nseg[u] = __popcll(m | 1ull);
                 act[u] = q < total;
-                wave_lds_fence();
-                if (cnt > 0 && start < qb + G && incl > qb)
-                    s_mark[start > qb ? start - qb : 0] = l;
-                wave_lds_fence();
-                const int v = s_mark[l];
-                s_mark[l] = -1;
-                const int s = dpp_incl_max<G>(v);
-                as[u] = VALUES ? __shfl(a, s, G) : 0.0;
-                e[u] = __shfl(off, s, G) + q;
-                sl[u] = s;
+                e[u] = __shfl(off, sl[u], 64) + q;
             }
+            before += __popcll(m);
         }
         int col[U];
         double bv[U];
@@ -98,45 +131,31 @@ __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            if (base + u * G * bstep < total) {
-                const int s0 = group_first<G>(sl[u]);
-                const unsigned long long diff = __ballot(act[u] && sl[u] != s0);
-                const bool single = ((diff >> gbase) & gmask) == 0;
-                f(act[u], col[u], as[u], bv[u], single);
+            if (base + 64 * (u * BSTEP + bofs) < total) {
+                const double as = VALUES ? __shfl(av, sl[u], 64) : 0.0;
+                f(Batch{act[u], col[u], as, bv[u], seg[u], nseg[u]});
             }
         }
     }
 }
 
-// Visits the products of the A entries [pa, pe) of one row in A-row order,
-// G lanes at a time, optionally restricted to B columns [c0, c1).  The
-// A entries are taken in groups of G starting at pa + gofs, stride gstride.
-// f(active, col, a, b, single) is called once per batch by every lane of the
-// group; batches are issued in product order and lane order inside a batch is
-// product order.  U batches are gathered before the first is handed to f, so
-// each lane keeps U independent loads in flight.  single is true when all
-// active lanes of the batch come from the same A entry (one B row: distinct
-// columns whenever B's rows are duplicate-free).
-// Batch striding (bofs, bstep): only batches bofs, bofs + bstep, ... of
-// every group are visited, so several waves can share one group's products
-// (used where the order of products does not matter).
-// s_mark: the group's G ints of LDS, all -1 on entry and on return.  A
-// batch finds the A entry of each of its products there: every non-empty
-// segment (the products of one A entry) that overlaps the batch's window of
-// G products writes its lane at its first position in the window, and a
-// running maximum over the window gives each position its segment.
-template <int G, int U, bool RANGED, bool VALUES, class F>
-__device__ __forceinline__ void for_products(int pa, int pe, int gofs, int gstride,
-                                             const int *__restrict__ ja,
+// Visits the products of the A entries [pa, pe) of one row in A-row order, a
+// wave's 64 entries at a time, optionally restricted to B columns [c0, c1).
+// f(batch) is called once per batch by every lane; batches are issued in
+// product order and lane order inside a batch is product order.  U batches
+// are gathered before the first is handed to f, so each lane keeps U
+// independent loads in flight.  Batch striding (bofs, BSTEP): only batches
+// bofs, bofs + BSTEP, ... of every group are visited, so several waves can
+// share one group's products (used where the order of products does not
+// matter).  heads: 64 ints of LDS.
+template <int U, int BSTEP, bool RANGED, bool VALUES, class F>
+__device__ __forceinline__ void for_products(int pa, int pe, const int *__restrict__ ja,
                                              const double *__restrict__ aval,
                                              const int *__restrict__ ib,
                                              const int *__restrict__ jb,
-                                             const double *__restrict__ bval,
-                                             BlockPtrs bp, int c0, int c1, int *s_mark,
-                                             F &&f, int bofs = 0,
-                                             int bstep = 1) {
-    static_assert(G >= 16, "segment lookup scans 16, 32 or 64 lanes");
-    const int l = __lane_id() & (G - 1);
+                                             const double *__restrict__ bval, BlockPtrs bp,
+                                             int c0, int c1, int *heads, F &&f, int bofs = 0) {
+    const int l = __lane_id();
     // Software pipeline over groups of A entries: the A entry (t, a) of group
     // g+2 and the B range of group g+1 are loaded while group g's products
     // are processed.
@@ -162,20 +181,19 @@ __device__ __forceinline__ void for_products(int pa, int pe, int gofs, int gstri
             }
         }
     };
-    int g = pa + gofs;
     int t0, t1;
     double a0, a1;
-    load_t(g, t0, a0);
-    load_t(g + gstride, t1, a1);
+    load_t(pa, t0, a0);
+    load_t(pa + 64, t1, a1);
     int lo, hi;
     load_range(t0, lo, hi);
-    for (; g < pe; g += gstride) {
+    for (int g = pa; g < pe; g += 64) {
         const double a = a0;
         int lo_n, hi_n, t2;
         double a2;
         load_range(t1, lo_n, hi_n);                 // next group's B ranges
-        load_t(g + 2 * gstride, t2, a2);            // group after next
-        expand_group<G, U, VALUES>(lo, hi - lo, a, jb, bval, s_mark, f, bofs, bstep);
+        load_t(g + 128, t2, a2);                    // group after next
+        expand_group<U, BSTEP, VALUES>(lo, max(hi - lo, 0), a, jb, bval, heads, f, bofs);
         lo = lo_n;
         hi = hi_n;
         t1 = t2;

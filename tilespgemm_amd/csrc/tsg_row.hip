@@ -332,11 +332,10 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
     constexpr int TW = BAND_WORDS / BAND_T;        // words per thread, half a sub-block
     static_assert(TW == 16 && 2 * TW == (1 << (SUB_SHIFT - 5)), "a sub-block is two threads' words");
     __shared__ __align__(16) unsigned bits[BAND_WORDS];
-    __shared__ int s_mark[NW][64];
+    __shared__ int s_heads[NW][64];
     __shared__ int s_wsum[NW];
     __shared__ long long s_base;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    s_mark[wave][lane] = -1;
     for (int64_t ui = blockIdx.x; ui < nunits; ui += gridDim.x) {
         const int2 un = units[ui];
         const int r = un.x, u = un.y;
@@ -347,17 +346,18 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
         const int c0 = sb0 << SUB_SHIFT;
         const int c1 = (int)min((int64_t)k, (int64_t)(sb0 + nsb) << SUB_SHIFT);
         const int words = (c1 - c0 + 31) >> 5;
-        for (int i = threadIdx.x; i < words; i += BAND_T) bits[i] = 0u;
+        for (int i = threadIdx.x; 4 * i < words; i += BAND_T)
+            reinterpret_cast<uint4 *>(bits)[i] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
-        for_products<64, BIG_SYM_U, true, false>(
-            ia[row], ia[row + 1], 0, 64, ja, nullptr, ib, jb, nullptr, bp, c0, c1, s_mark[wave],
-            [&](bool act, int col, double, double, bool) {
-                if (act) {
-                    const int cc = col - c0;
+        for_products<BIG_SYM_U, NW, true, false>(
+            ia[row], ia[row + 1], ja, nullptr, ib, jb, nullptr, bp, c0, c1, s_heads[wave],
+            [&](const Batch &t) {
+                if (t.act) {
+                    const int cc = t.col - c0;
                     lds_set_bit(&bits[cc >> 5], 1u << (cc & 31));
                 }
             },
-            wave, NW);
+            wave);
         __syncthreads();
         // thread t takes words [TW t, TW t + TW) (words past the band's end
         // are stale); threads 2s and 2s + 1 hold sub-block s
@@ -525,6 +525,16 @@ __global__ void __launch_bounds__(256) k_bptr(int n, const int *__restrict__ ib,
 }
 
 // ------------------------------------------------------------- item plan
+constexpr int SMALL_ITEM = 256;
+constexpr int MID_ITEM = 512;
+// Sparse stretches go into wide items of up to this many outputs.  R-MAT 2^20
+// with 8 draws a row, both sparse kernels: 31.7 ms without wide items (its
+// 30M items of <= 256 outputs hold 45 each, and each costs its A entries, two
+// block pointers an entry and its tables), 20.2 up to 256, 19.2 up to 384,
+// 19.3 up to 512; R-MAT 2^18 with 4: 1.27, 1.01, 0.98, 0.96; ER batch of 512:
+// 6.0, 5.9, 5.1, 4.3.
+constexpr int WIDE_CAP = 512;
+static_assert(WIDE_CAP <= MID_ITEM, "wide items run in the sparse kernels");
 
 // Split of each big row into items: the row's span is cut into windows of
 // WSB sub-blocks (at most ITEM_WBITS columns); inside a window, runs of
@@ -543,8 +553,11 @@ __global__ void __launch_bounds__(256) k_bptr(int n, const int *__restrict__ ib,
 // band's windows inside one pass of 64 windows, so the item's place in its
 // band's list is its count of non-empty words before it less that of the
 // band's first window.
+// Wide items: an aligned run of 2, 4 or 8 windows of one band whose outputs
+// number at most wide_cap becomes one item (the longest such run).
 template <bool FILL, int WSB>
 __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__ rows, int k,
+                                               int wide_cap,
                                                const int *__restrict__ span_sb0,
                                                const int64_t *__restrict__ sb_off,
                                                const uint16_t *__restrict__ subcnt,
@@ -581,7 +594,7 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
             os[q] = FILL && words && q < len ? __popc(subocc[sb_off[r] + j0 + q]) : 0;
             nzt += os[q];
         }
-        int nit = 0, tot = 0;
+        int nit = 0, tot = 0, firstq = WSB, lastq = -1;
         {
             int start = -1, cnt = 0;
 #pragma unroll
@@ -596,9 +609,34 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                     cnt += cs[q];
                 }
                 tot += cs[q];
+                if (cs[q] != 0) {
+                    firstq = min(firstq, q);
+                    lastq = q;
+                }
             }
             if (start >= 0 && cnt > 0) nit++;
         }
+        // the run of windows this one is in: its length, outputs, first and
+        // last sub-block with outputs
+        int run = 1, run_tot = tot;
+        int sb_first = lastq >= 0 ? j0 + firstq : 0x7fffffff;
+        int sb_last = lastq >= 0 ? j0 + lastq : -1;
+        {
+            int g_tot = tot, g_first = sb_first, g_last = sb_last;
+#pragma unroll
+            for (int g = 2; g <= WPB; g <<= 1) {
+                g_tot += __shfl_xor(g_tot, g >> 1, 64);
+                g_first = min(g_first, __shfl_xor(g_first, g >> 1, 64));
+                g_last = max(g_last, __shfl_xor(g_last, g >> 1, 64));
+                if (g_tot <= wide_cap) {
+                    run = g;
+                    run_tot = g_tot;
+                    sb_first = g_first;
+                    sb_last = g_last;
+                }
+            }
+        }
+        if (run > 1) nit = (l & (run - 1)) == 0 && run_tot > 0 ? 1 : 0;
         const int it_incl = wave_incl_scan(nit);
         const int out_incl = wave_incl_scan(tot);
         // non-empty words of this pass before this window, and before the
@@ -612,9 +650,17 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
             // this window's first non-empty word in the band word lists
             const int64_t wb =
                 words ? band_base[band_off[r] + win / WPB] + (nz_excl - band_nz) : 0;
+            if (run > 1) {
+                items[w] = ItemRec{make_int4(row, (first + sb_first) << SUB_SHIFT,
+                                             min(k, (first + sb_last + 1) << SUB_SHIFT),
+                                             words ? (int)(sb_off[r] + sb_first) : r),
+                                   out, wb};
+                item_n[w] = run_tot;
+            }
             int start = -1, cnt = 0, nzrun = 0, nzs = 0;
 #pragma unroll
             for (int q = 0; q < WSB; q++) {
+                if (run > 1) break;
                 if (start >= 0 && cnt + cs[q] > ITEM_CAP) {
                     items[w] = ItemRec{make_int4(row, (cbase + start) << SUB_SHIFT,
                                                  min(k, (cbase + q) << SUB_SHIFT),
@@ -635,7 +681,7 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                 }
                 nzrun += os[q];
             }
-            if (start >= 0 && cnt > 0) {
+            if (run == 1 && start >= 0 && cnt > 0) {
                 items[w] = ItemRec{make_int4(row, (cbase + start) << SUB_SHIFT,
                                              min(k, (cbase + len) << SUB_SHIFT),
                                              words ? (int)(sb_off[r] + j0 + start) : r),
@@ -660,25 +706,14 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
 // kernel whose value array holds just that class's items, so smaller items
 // take less LDS and more of them are resident.  block_small[b] and
 // block_mid[b] count block b's items of the first two classes.
-constexpr int SMALL_ITEM = 256;
-constexpr int MID_ITEM = 512;
-// The small-item kernel is bound by how many items are resident: with its
-// 5.3 KB of LDS a wave, registers set the limit, so it runs 4 product
-// batches in flight per lane at 6 waves per SIMD (<= 80 VGPRs) instead of 8
-// at 4.  Big numeric on R-MAT 2^20 A*A^T: 149.7 ms at (8, 4); 142.5 at
-// (6, 5); 136.4 at (4, 6); 139.7 at (3, 7) and 138.9 at (2, 8), both with
-// a few registers spilled.
-constexpr int SMALL_RANK_U = 4;
-constexpr int SMALL_MINW = 6;
-// the middle class: 7.3 KB of LDS a wave allows 21 waves per CU, so 5 per
-// SIMD, with 6 batches in flight (<= 96 VGPRs).  (The last class stays at 8
-// batches: its LDS caps it at 14 waves per CU, and 10 or 12 batches in the
-// registers that leaves gave 133.3 and 135.1 ms against 134.2.)  R-MAT 2^20 A*A^T: items
-// of > 256 outputs 96.8 ms in one class, 77.3 + 16.9 ms in two.  (Cutting
-// items at 512 outputs where whole sub-blocks allow, so that fewer land in
-// the last class: 148 ms in all instead of 134, more (A entry, item) pairs.)
+// Product batches in flight per lane and waves per SIMD of the two sparse
+// item kernels.  R-MAT 2^20 (8 draws a row), <= 256 outputs: 6.0 ms at (4, 6),
+// 5.8 at (6, 5) and (4, 7), 6.2 at (8, 5); <= 512: 13.3 at (6, 5), 12.7 at
+// (6, 4), 12.9 at (8, 4), 13.0 at (4, 5).
+constexpr int SMALL_RANK_U = 6;
+constexpr int SMALL_MINW = 5;
 constexpr int MID_RANK_U = 6;
-constexpr int MID_MINW = 5;
+constexpr int MID_MINW = 4;
 
 __global__ void __launch_bounds__(256) k_item_keys(int64_t n, const ItemRec *__restrict__ items,
                                                    const int *__restrict__ item_n, int class_bit,
@@ -721,7 +756,7 @@ struct ItemSmem {
     unsigned short ids[ITEM_SLOTS];
     unsigned bits[ITEM_WORDS];
     unsigned tags[ITEM_TAGS];
-    int mark[64];                 // segment marks of the product expansion
+    int heads[64];                // start bits of the product expansion
     int nid;
 };
 
@@ -736,7 +771,6 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
     ItemSmem &S = reinterpret_cast<ItemSmem *>(smem)[threadIdx.x >> 6];
     const int l = __lane_id();
     for (int i = l; i < ITEM_TAGS; i += 64) S.tags[i] = 0xffffffffu;
-    S.mark[l] = -1;
     const int64_t wave_id = (int64_t)blockIdx.x * ITEM_WAVES + (threadIdx.x >> 6);
     const int64_t nwaves = (int64_t)gridDim.x * ITEM_WAVES;
     for (int64_t it = wave_id; it < nitems; it += nwaves) {
@@ -747,25 +781,24 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
         for (int i = l; i < nwords; i += 64) S.bits[i] = 0u;
         if (l == 0) S.nid = 0;
         wave_lds_fence();
-        for_products<64, ITEM_U, true, true>(
-            ia[row], ia[row + 1], 0, 64, ja, a, ib, jb, b, bp, c0, c1, S.mark,
-            [&](bool act, int col, double av, double bv, bool single) {
+        for_products<ITEM_U, 1, true, true>(
+            ia[row], ia[row + 1], ja, a, ib, jb, b, bp, c0, c1, S.heads, [&](const Batch &t) {
                 int slot = -1;
-                if (act) {
+                if (t.act) {
                     bool created;
-                    slot = hash_insert<ITEM_SLOTS>(S.keys, col, created);
+                    slot = hash_insert<ITEM_SLOTS>(S.keys, t.col, created);
                     if (created) {
                         const int id = atomicAdd(&S.nid, 1);
                         S.ids[slot] = (unsigned short)id;
                         S.vals[id] = 0.0;
-                        const int cc = col - c0;
+                        const int cc = t.col - c0;
                         atomicOr(&S.bits[cc >> 5], 1u << (cc & 31));
                     }
                 }
                 wave_lds_fence();
                 const int id = slot >= 0 ? (int)S.ids[slot] : -1;
-                ordered_accumulate<FUSED, ITEM_TAGS>(act, id, av, bv, S.vals, S.tags,
-                                                     (unsigned)l, single && b_strict);
+                ordered_accumulate<FUSED, ITEM_TAGS>(t.act, id, t.a, t.b, S.vals, S.tags,
+                                                     (unsigned)l, t.nseg == 1 && b_strict);
             });
         wave_lds_fence();
         // emit in column order: bitmap words -> ranks -> hash lookups
@@ -799,12 +832,12 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
 // in a dense rank-ordered array that is written out coalesced.
 // WORDS: bitmap words of the widest item (256 or 512: items of 8192 or
 // 16384 columns).
-template <int WORDS, int CAP = ITEM_CAP>
+template <int WORDS>
 struct RankSmem {
     uint2 words[WORDS];           // {bitmap word, outputs before it}
-    double vals[CAP];
+    double vals[ITEM_CAP];
     unsigned tags[ITEM_TAGS];     // bucketed by rank
-    int mark[64];                 // segment marks of the product expansion
+    int heads[64];                // start bits of the product expansion
 };
 
 // Rank table of one item, in two parts so that other loads can be issued
@@ -844,8 +877,8 @@ __device__ __forceinline__ void item_words(const unsigned *__restrict__ list, un
     }
 }
 
-template <int WORDS, int CAP, int WCH = WORDS / 64>
-__device__ __forceinline__ int item_rank_build(RankSmem<WORDS, CAP> &S, unsigned (&wv)[WCH], int c0,
+template <int WORDS, int WCH = WORDS / 64>
+__device__ __forceinline__ int item_rank_build(RankSmem<WORDS> &S, unsigned (&wv)[WCH], int c0,
                                                int c1, int64_t o, int *__restrict__ jc) {
     const int l = __lane_id();
     const int nwords = (c1 - c0 + 31) >> 5;
@@ -884,8 +917,8 @@ __device__ __forceinline__ int item_rank_build(RankSmem<WORDS, CAP> &S, unsigned
 }
 
 // Writes an item's cnt values to C at offset o, straight from LDS.
-template <int WORDS, int CAP>
-__device__ __forceinline__ void item_store_values(RankSmem<WORDS, CAP> &S, int cnt, int64_t o,
+template <int WORDS>
+__device__ __forceinline__ void item_store_values(RankSmem<WORDS> &S, int cnt, int64_t o,
                                                   double *__restrict__ c) {
     const int l = __lane_id();
     wave_lds_fence();
@@ -895,38 +928,39 @@ __device__ __forceinline__ void item_store_values(RankSmem<WORDS, CAP> &S, int c
 
 // Accumulates one batch of products into the item's rank-ordered values:
 // a batch from one A entry (distinct columns when B's rows are strictly
-// ascending) adds directly, any other batch by tag rounds in lane order.
-template <bool FUSED, int WORDS, int CAP>
-__device__ __forceinline__ void item_accumulate(RankSmem<WORDS, CAP> &S, int c0, bool act, int col,
-                                                double av, double bv, bool single, int b_strict) {
+// ascending) adds directly, one from a few A entries one entry after the
+// other, any other by tag rounds in lane order.
+template <bool FUSED, int WORDS>
+__device__ __forceinline__ void item_accumulate(RankSmem<WORDS> &S, int c0, const Batch &t,
+                                                int b_strict) {
     int rank = -1;
-    if (act) {
-        const int cc = col - c0;
+    if (t.act) {
+        const int cc = t.col - c0;
         const uint2 wd = S.words[cc >> 5];
         rank = (int)wd.y + __popc(wd.x & ((1u << (cc & 31)) - 1u));
     }
-    if (single && b_strict) {
-        if (rank >= 0) S.vals[rank] = acc_step<FUSED>(S.vals[rank], av, bv);
-        wave_lds_fence();
+    if (b_strict && t.nseg <= FLAT_SEGS) {
+        for (int s = 1; s <= t.nseg; s++) {
+            if (rank >= 0 && t.seg == s) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
+            wave_lds_fence();
+        }
         return;
     }
-    ordered_accumulate<FUSED, ITEM_TAGS>(rank >= 0, rank, av, bv, S.vals, S.tags,
+    ordered_accumulate<FUSED, ITEM_TAGS>(rank >= 0, rank, t.a, t.b, S.vals, S.tags,
                                          (unsigned)__lane_id(), false);
 }
 
-template <bool FUSED, int WORDS, int CAP = ITEM_CAP, int U = RANK_U, int MINW = 1>
-__global__ void __launch_bounds__(64 * ITEM_WAVES) __attribute__((amdgpu_waves_per_eu(MINW)))
-k_big_numeric_rank(
+template <bool FUSED, int WORDS>
+__global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric_rank(
     int64_t nitems, const ItemRec *__restrict__ items, const unsigned *__restrict__ wlist,
     const unsigned *__restrict__ subocc, const int *__restrict__ ia, const int *__restrict__ ja,
     const double *__restrict__ a, const int *__restrict__ jb, const double *__restrict__ b,
     const int4 *__restrict__ bpk, BlockPtrs bp, int *__restrict__ jc, double *__restrict__ c,
     int b_strict) {
     extern __shared__ __align__(16) unsigned char smem[];
-    RankSmem<WORDS, CAP> &S = reinterpret_cast<RankSmem<WORDS, CAP> *>(smem)[threadIdx.x >> 6];
+    RankSmem<WORDS> &S = reinterpret_cast<RankSmem<WORDS> *>(smem)[threadIdx.x >> 6];
     const int l = __lane_id();
     for (int i = l; i < ITEM_TAGS; i += 64) S.tags[i] = 0xffffffffu;
-    S.mark[l] = -1;
     const int64_t wave_id = (int64_t)blockIdx.x * ITEM_WAVES + (threadIdx.x >> 6);
     const int64_t nwaves = (int64_t)gridDim.x * ITEM_WAVES;
     // the next item's descriptor is loaded when an item starts, and its
@@ -1004,9 +1038,9 @@ k_big_numeric_rank(
         item_words(ilist, iocc, pre, c0, c1, wv);
         int lo, hi;
         load_range(t0, lo, hi);
-        const int cnt = item_rank_build<WORDS, CAP>(S, wv, c0, c1, o, jc);
-        auto f = [&](bool act, int col, double av, double bv, bool single) {
-            item_accumulate<FUSED, WORDS, CAP>(S, c0, act, col, av, bv, single, b_strict);
+        const int cnt = item_rank_build<WORDS>(S, wv, c0, c1, o, jc);
+        auto f = [&](const Batch &t) {
+            item_accumulate<FUSED, WORDS>(S, c0, t, b_strict);
         };
         for (int g = ipa; g < ipe; g += 64) {
             const double ag = a0;
@@ -1014,7 +1048,8 @@ k_big_numeric_rank(
             double a2;
             load_range(t1, lo_n, hi_n);
             load_t(g + 128, t2, a2);
-            expand_group<64, U, true, true>(lo, hi - lo, ag, jb, b, S.mark, f, 0, 1, bpk);
+            expand_group<RANK_U, 1, true, true>(lo, max(hi - lo, 0), ag, jb, b, S.heads, f, 0,
+                                                bpk);
             lo = lo_n;
             hi = hi_n;
             t1 = t2;
@@ -1023,6 +1058,143 @@ k_big_numeric_rank(
         }
         if (next < nitems) locate(next);
         item_store_values(S, cnt, o, c);
+    }
+}
+
+// Items of at most CAP outputs, however wide up to a band: the rank of a
+// column goes through the item's sub-blocks (mask of non-empty words, words
+// before it) to its word (bits, outputs before it), so table and work follow
+// the outputs and not the columns.  The outputs' columns are noted by the
+// products (as offsets in the item) instead of expanded from the words.
+//
+// The dense tables it replaces for these items cost ~500 vector instructions
+// an item whatever its products (the issue rate bound them: 25 of 29 ms of
+// R-MAT 2^20 with 8 draws a row); now 5.8 ms, with the 257..512-output items
+// 37.7 -> 18.5 ms.  Larger items keep the dense table: one lookup a product,
+// and they run at the memory's rate (4.65 TB/s).
+template <int CAP>
+struct SparseSmem {
+    uint2 words[CAP];             // {bits, outputs before}
+    double vals[CAP];
+    uint2 sub[1 << BAND_SHIFT];   // {mask of non-empty words, words before}
+    uint16_t cols[CAP];
+    unsigned tags[CAP / 4];       // a byte per output, or tag buckets
+    int heads[64];
+};
+
+template <bool FUSED, int CAP, int U, int MINW>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MINW)))
+k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
+                     const unsigned *__restrict__ wlist, const unsigned *__restrict__ subocc,
+                     const int *__restrict__ ia, const int *__restrict__ ja,
+                     const double *__restrict__ a, const int *__restrict__ jb,
+                     const int4 *__restrict__ bpk, BlockPtrs bp, int *__restrict__ jc,
+                     double *__restrict__ c, int b_strict) {
+    __shared__ __align__(16) SparseSmem<CAP> S;
+    constexpr int NT = CAP / 4;
+    const int l = threadIdx.x;
+    uint8_t *own = reinterpret_cast<uint8_t *>(S.tags);
+    for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const int4 item = items[it].d;
+        const int64_t o = items[it].off;
+        const unsigned *list = wlist + items[it].wpos;
+        const int c0 = item.y, c1 = item.z;
+        const int pa = ia[item.x], pe = ia[item.x + 1];
+        const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 1 << BAND_SHIFT);
+        const unsigned occ = l < nsb ? subocc[(int64_t)item.w + l] : 0u;
+        auto load_t = [&](int g, int &t, double &av) {
+            const int p = g + l;
+            t = -1;
+            av = 0.0;
+            if (p < pe) {
+                t = ja[p];
+                av = a[p];
+            }
+        };
+        auto load_range = [&](int t, int &lo, int &hi) {
+            lo = 0;
+            hi = 0;
+            if (t >= 0) {
+                lo = brange_lo(bp, jb, t, c0);
+                hi = brange_lo(bp, jb, t, c1);
+            }
+        };
+        int t0, lo, hi;
+        double a0;
+        load_t(pa, t0, a0);
+        const int pc = __popc(occ);
+        const int incl = wave_incl_scan(pc);
+        // every non-empty word has an output
+        const int nw = min(__builtin_amdgcn_readlane(incl, 63), CAP);
+        unsigned wv[CAP / 64];
+#pragma unroll
+        for (int j = 0; j < CAP / 64; j++)
+            wv[j] = j * 64 + l < nw ? __builtin_nontemporal_load(list + j * 64 + l) : 0u;
+        load_range(t0, lo, hi);
+        S.sub[l] = make_uint2(occ, (unsigned)(incl - pc));
+        int cnt = 0;
+#pragma unroll
+        for (int j = 0; j < CAP / 64; j++) {
+            if (j * 64 < nw) {
+                const int p = __popc(wv[j]);
+                const int in = wave_incl_scan(p);
+                if (j * 64 + l < nw)
+                    S.words[j * 64 + l] = make_uint2(wv[j], (unsigned)(cnt + in - p));
+                cnt += __builtin_amdgcn_readlane(in, 63);
+            }
+        }
+        cnt = min(cnt, CAP);
+        for (int i = l; i < cnt; i += 64) S.vals[i] = 0.0;
+        wave_lds_fence();
+        auto f = [&](const Batch &t) {
+            int rank = -1;
+            if (t.act) {
+                const int cc = t.col - c0;
+                const uint2 sb = S.sub[(cc >> SUB_SHIFT) & ((1 << BAND_SHIFT) - 1)];
+                const int w = (int)sb.y + (int)__popc(sb.x & ((1u << ((cc >> 5) & 31)) - 1u));
+                const uint2 wd = S.words[min(w, CAP - 1)];
+                rank = min((int)wd.y + (int)__popc(wd.x & ((1u << (cc & 31)) - 1u)), CAP - 1);
+                S.cols[rank] = (uint16_t)cc;
+            }
+            bool clash = t.nseg > 1 || !b_strict;
+            if (b_strict && t.nseg > 2) {
+                if (t.act) own[rank] = (uint8_t)l;
+                wave_lds_fence();
+                clash = __ballot(t.act && own[rank] != (uint8_t)l) != 0;
+                wave_lds_fence();
+            }
+            if (!clash) {
+                if (t.act) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
+                wave_lds_fence();
+            } else if (b_strict && t.nseg <= FLAT_SEGS) {
+                for (int s = 1; s <= t.nseg; s++) {
+                    if (t.act && t.seg == s) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
+                    wave_lds_fence();
+                }
+            } else {
+                for (int i = l; i < NT; i += 64) S.tags[i] = 0xffffffffu;
+                wave_lds_fence();
+                ordered_accumulate<FUSED, NT>(t.act, rank, t.a, t.b, S.vals, S.tags, (unsigned)l,
+                                              false);
+            }
+        };
+        for (int g = pa; g < pe; g += 64) {
+            int t1, lo_n, hi_n;
+            double a1;
+            load_t(g + 64, t1, a1);
+            load_range(t1, lo_n, hi_n);
+            expand_group<U, 1, true, true>(lo, max(hi - lo, 0), a0, jb, nullptr, S.heads, f, 0,
+                                           bpk);
+            lo = lo_n;
+            hi = hi_n;
+            a0 = a1;
+        }
+        wave_lds_fence();
+        for (int i = l; i < cnt; i += 64) {
+            __builtin_nontemporal_store(c0 + (int)S.cols[i], jc + o + i);
+            __builtin_nontemporal_store(S.vals[i], c + o + i);
+        }
+        wave_lds_fence();
     }
 }
 
@@ -1275,9 +1447,12 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         // windows otherwise (fewer items, fewer (A entry, item) pairs).
         const bool narrow = p.column_order;
         p.narrow_items = narrow;
+        // sparse stretches in wide items, for the kernel whose work and LDS
+        // follow the outputs, not the columns (rank mode, by size class)
+        const int wide_cap = narrow && p.use_rank ? WIDE_CAP : 0;
         auto items_kernel = [&](auto kern, int64_t *cnt, ItemRec *it, int *itn) {
             hipLaunchKernelGGL(kern, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0, s,
-                               p.nbig, rowsb, k, p.span_sb0, p.sb_off, p.subcnt, d_ic, cnt, it,
+                               p.nbig, rowsb, k, wide_cap, p.span_sb0, p.sb_off, p.subcnt, d_ic, cnt, it,
                                itn, p.subocc, band_off, band_base);
             TSG_LAUNCH_CHECK();
         };
@@ -1382,20 +1557,22 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
         // the size classes (sorted in this order) in kernels with value
         // arrays of their size
         const int64_t ns = p.nitems_small, nm = std::max(p.nitems_mid, ns);
+        auto launch_sparse = [&](auto kern, int64_t i0, int64_t i1) {
+            if (i1 <= i0) return;
+            hipLaunchKernelGGL(kern, dim3(item_grid(i1 - i0)), dim3(64), 0, s, i1 - i0,
+                               p.items + i0, p.bandwords, p.subocc, A.ptr, A.idx, A.val, B.idx,
+                               p.bpk, block_ptrs(p, B.ptr), d_jc, d_c, (int)p.b_strict);
+            TSG_LAUNCH_CHECK();
+        };
+        launch_sparse(k_big_numeric_sparse<FUSED, SMALL_ITEM, SMALL_RANK_U, SMALL_MINW>, 0, ns);
+        launch_sparse(k_big_numeric_sparse<FUSED, MID_ITEM, MID_RANK_U, MID_MINW>, ns, nm);
+        // the rest: items of more outputs in column order, all in rows' order
         if (p.narrow_items) {
             constexpr int W = ITEM_WORDS / 2;
-            launch_rank(k_big_numeric_rank<FUSED, W, SMALL_ITEM, SMALL_RANK_U, SMALL_MINW>,
-                        sizeof(RankSmem<W, SMALL_ITEM>) * ITEM_WAVES, 0, ns);
-            launch_rank(k_big_numeric_rank<FUSED, W, MID_ITEM, MID_RANK_U, MID_MINW>,
-                        sizeof(RankSmem<W, MID_ITEM>) * ITEM_WAVES, ns, nm);
             launch_rank(k_big_numeric_rank<FUSED, W>, sizeof(RankSmem<W>) * ITEM_WAVES, nm,
                         p.nitems);
         } else {
             constexpr int W = ITEM_WORDS;
-            launch_rank(k_big_numeric_rank<FUSED, W, SMALL_ITEM, SMALL_RANK_U, SMALL_MINW>,
-                        sizeof(RankSmem<W, SMALL_ITEM>) * ITEM_WAVES, 0, ns);
-            launch_rank(k_big_numeric_rank<FUSED, W, MID_ITEM, MID_RANK_U, MID_MINW>,
-                        sizeof(RankSmem<W, MID_ITEM>) * ITEM_WAVES, ns, nm);
             launch_rank(k_big_numeric_rank<FUSED, W>, sizeof(RankSmem<W>) * ITEM_WAVES, nm,
                         p.nitems);
         }
