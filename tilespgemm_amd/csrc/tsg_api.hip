@@ -178,8 +178,8 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
     std::function<void()> early;
     if (h->method == TSG_METHOD_TILE)
         early = [&] {
-            tile_count_early(A, earlyA, ws, h->stream);
-            if (!b_is_a) tile_count_early(B, earlyB, ws, h->stream);
+            tile_count_early(A, earlyA, &h->box->v[0], ws, h->stream);
+            if (!b_is_a) tile_count_early(B, earlyB, &h->box->v[1], ws, h->stream);
         };
     // with the tile path not forced, the row path's products and bins too
     RowFront front;
@@ -188,6 +188,8 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
     const int vf = front_pass(A, B, ws, h->stream, h->box, want_sample ? sample : nullptr,
                               h->method == TSG_METHOD_TILE ? nullptr : &front, &tune, early);
     tm.end();
+    if (earlyA.tile_ptr) earlyA.nt = (int)h->box->v[0];
+    if (earlyB.tile_ptr) earlyB.nt = (int)h->box->v[1];
     TSG_CHECK((vf & 0x303) == 0, TSG_ERR_INVALID,
               std::string("invalid CSR input: ") + ((vf & 0x3) ? "A" : "B") +
                   ((vf & 0x101) ? " has bad row pointers" : " has a column out of range"));
@@ -198,7 +200,7 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
         const Arena::Mark mk = h->method == TSG_METHOD_TILE ? ws.mark() : before;
         try {
             ws.rewind(mk);
-            tile_symbolic(tile, A, B, b_is_a, d_ic, nnz_c, ws, h->stream, tm, h->cus, &earlyA,
+            tile_symbolic(tile, A, B, b_is_a, d_ic, nnz_c, h->box, ws, h->stream, tm, &earlyA,
                           &earlyB);
         } catch (const TsgError &e) {
             // AUTO's choice falls back to the row path when the tile path's
@@ -258,7 +260,7 @@ void numeric_from(tsg_handle_t h, int method_used, RowPlan &row, TilePlan &tile,
     const int fused = h->fp_mode == TSG_FP_FUSED;
     if (method_used == TSG_METHOD_TILE) {
         TSG_CHECK(tile.valid, TSG_ERR_STATE, "numeric phase without a symbolic phase");
-        tile_numeric(tile, A, B, d_ic, d_jc, d_c, fused, ws, h->stream, tm, h->cus);
+        tile_numeric(tile, A, B, d_ic, d_jc, d_c, fused, h->stream, tm);
     } else {
         TSG_CHECK(row.valid, TSG_ERR_STATE, "numeric phase without a symbolic phase");
         CsrIn Bs = B;

@@ -311,14 +311,14 @@ struct EarlyTileCount {
     int *tile_ptr = nullptr;     // [blkm+1] device
     int nt = -1;                 // host, after the round trip
 };
-void tile_count_early(const CsrIn &X, EarlyTileCount &e, Arena &ws, hipStream_t s);
+void tile_count_early(const CsrIn &X, EarlyTileCount &e, int64_t *total, Arena &ws,
+                      hipStream_t s);
 void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a,
-                   int64_t *d_ic, int64_t *nnz_c, Arena &ws, hipStream_t s,
-                   StageTimer &tm, int cus, const EarlyTileCount *earlyA = nullptr,
+                   int64_t *d_ic, int64_t *nnz_c, HostBox *box, Arena &ws, hipStream_t s,
+                   StageTimer &tm, const EarlyTileCount *earlyA = nullptr,
                    const EarlyTileCount *earlyB = nullptr);
 void tile_numeric(TilePlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_ic,
-                  int *d_jc, double *d_c, int fused, Arena &ws, hipStream_t s,
-                  StageTimer &tm, int cus);
+                  int *d_jc, double *d_c, int fused, hipStream_t s, StageTimer &tm);
 
 // ------------------------------------------------------------ batches
 // A batch laid out as one block-diagonal product (tsg_batch.hip).

@@ -54,13 +54,17 @@ __device__ __forceinline__ int wave_min(int x) { return group_min<64>(x); }
 
 // ---------------------------------------------------------------- convert
 // One 16-lane group per tile row; lane r handles CSR row 16*I + r.  A
-// block's 16 tile rows hold one contiguous range of ja: when it has at most
+// block's tile rows hold one contiguous range of ja: when it has at most
 // CV_STAGE entries it is staged in LDS first (coalesced loads), and the rows
-// are walked there instead of with a dependent global load per entry (the
-// 27-point stencil's 6,912 entries per block fit).
-constexpr int CV_STAGE = 8192;
+// are walked there instead of with a dependent global load per entry.  Bound
+// by that walk's latency, so a block takes few tile rows: more blocks walk at
+// once, and each holds more entries per row before its stage is full.  Rows
+// of 33 entries, 65537 of them: 41 us at 16 tile rows and 8192 entries (which
+// 8448 do not fit), 34 at 16 and 12288, 35 at 8 and 8192, 31 at 4 and 4096.
+constexpr int CV_STAGE = 4096;
+constexpr int CV_TR = 4;
 
-__global__ void __launch_bounds__(256) k_tile_convert(
+__global__ void __launch_bounds__(16 * CV_TR) k_tile_convert(
     int m, int blkm, const int *__restrict__ ia, const int *__restrict__ ja,
     const int *__restrict__ tile_ptr, int *__restrict__ tile_col, int *__restrict__ tile_off,
     uint16_t *__restrict__ mask, uint8_t *__restrict__ rowptr, uint8_t *__restrict__ idx,
@@ -490,7 +494,7 @@ __device__ __forceinline__ int tile_units_in(int64_t nnz, int q) {
 // Units per bin: summed over each wave first (one LDS atomic per wave and
 // bin; a thread's own atomics on the three counters had serialised).
 __global__ void __launch_bounds__(256) k_tbin_count(int n, const int64_t *__restrict__ off,
-                                                    int *__restrict__ cnt) {
+                                                    int64_t *__restrict__ cnt) {
     __shared__ int s_cnt[TBINS];
     if (threadIdx.x < TBINS) s_cnt[threadIdx.x] = 0;
     __syncthreads();
@@ -502,7 +506,9 @@ __global__ void __launch_bounds__(256) k_tbin_count(int n, const int64_t *__rest
         if (__lane_id() == 0 && u) atomicAdd(&s_cnt[q], u);
     }
     __syncthreads();
-    if (threadIdx.x < TBINS && s_cnt[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], s_cnt[threadIdx.x]);
+    if (threadIdx.x < TBINS && s_cnt[threadIdx.x])
+        atomicAdd(reinterpret_cast<unsigned long long *>(cnt + threadIdx.x),
+                  (unsigned long long)s_cnt[threadIdx.x]);
 }
 
 // A unit's record carries its tile's pairs (first one, count), so the
@@ -517,8 +523,8 @@ __global__ void __launch_bounds__(256) k_tbin_count(int n, const int64_t *__rest
 __global__ void __launch_bounds__(256) k_tbin_scatter(int n, const int64_t *__restrict__ off,
                                                       const int64_t *__restrict__ tpair,
                                                       const int64_t *__restrict__ tslot,
-                                                      const int *__restrict__ cnt,
-                                                      int *__restrict__ fill,
+                                                      const int64_t *__restrict__ cnt,
+                                                      int64_t *__restrict__ fill,
                                                       int4 *__restrict__ units) {
     __shared__ int s_cnt[TBINS], s_base[TBINS];
     if (threadIdx.x < TBINS) s_cnt[threadIdx.x] = 0;
@@ -541,8 +547,10 @@ __global__ void __launch_bounds__(256) k_tbin_scatter(int n, const int64_t *__re
     __syncthreads();
     if (threadIdx.x < TBINS && s_cnt[threadIdx.x]) {
         int start = 0;
-        for (int i = 0; i < (int)threadIdx.x; i++) start += cnt[i];
-        s_base[threadIdx.x] = start + atomicAdd(&fill[threadIdx.x], s_cnt[threadIdx.x]);
+        for (int i = 0; i < (int)threadIdx.x; i++) start += (int)cnt[i];
+        s_base[threadIdx.x] =
+            start + (int)atomicAdd(reinterpret_cast<unsigned long long *>(fill + threadIdx.x),
+                                   (unsigned long long)s_cnt[threadIdx.x]);
     }
     __syncthreads();
     const int full = (int)(nz >> 6);
@@ -569,7 +577,7 @@ __global__ void __launch_bounds__(256) k_sym_csc(int blk, const int *__restrict_
                                                  const int *__restrict__ tile_col,
                                                  int *__restrict__ csc_row,
                                                  int *__restrict__ csc_tile,
-                                                 unsigned *__restrict__ asym) {
+                                                 int64_t *__restrict__ asym) {
     const int J = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;
     const int l = threadIdx.x & 15;
     bool missing = false;
@@ -587,7 +595,7 @@ __global__ void __launch_bounds__(256) k_sym_csc(int blk, const int *__restrict_
     // one plain store per wave that found a tile without its partner (an
     // asymmetric pattern has millions: atomics on one word would queue)
     const unsigned long long bad = __ballot(missing);
-    if (bad && __lane_id() == __ffsll(bad) - 1) *asym = 1u;
+    if (bad && __lane_id() == __ffsll(bad) - 1) *asym = 1;
 }
 
 // Column layout of 16x16 tiles (B only), the transposed sub-tiles of
@@ -865,7 +873,8 @@ __global__ void __launch_bounds__(256) k_step3_out(int nunits, const int4 *__res
 }
 
 // tile counts per tile row, scanned into tile_ptr
-void tile_count_scan(const CsrIn &X, int blkm, int *tile_ptr, Arena &ws, hipStream_t s) {
+void tile_count_scan(const CsrIn &X, int blkm, int *tile_ptr, Arena &ws, hipStream_t s,
+                     int64_t *total) {
     int *tcount = ws.alloc_n<int>((size_t)blkm + 1);
     int64_t *tmp = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)blkm + 1));
     if (blkm > 0) {
@@ -873,12 +882,12 @@ void tile_count_scan(const CsrIn &X, int blkm, int *tile_ptr, Arena &ws, hipStre
                            s, X.rows, X.cols, X.nnz, blkm, X.ptr, X.idx, tcount);
         TSG_LAUNCH_CHECK();
     }
-    exclusive_scan_i32(tcount, tile_ptr, (size_t)blkm, tmp, s);
+    exclusive_scan_i32(tcount, tile_ptr, (size_t)blkm, tmp, s, total);
 }
 
 // early: the tile count already taken (tile_count_early), else counted here
 // with a host round trip of its own
-void convert(TileMat &T, const CsrIn &X, bool fill_values, Arena &ws, hipStream_t s,
+void convert(TileMat &T, const CsrIn &X, HostBox *box, Arena &ws, hipStream_t s,
              const EarlyTileCount *early) {
     T.rows = X.rows;
     T.cols = X.cols;
@@ -891,10 +900,9 @@ void convert(TileMat &T, const CsrIn &X, bool fill_values, Arena &ws, hipStream_
         nt = early->nt;
     } else {
         T.tile_ptr = ws.alloc_n<int>((size_t)T.blkm + 1);
-        tile_count_scan(X, T.blkm, T.tile_ptr, ws, s);
-        TSG_HIP_TRY(
-            hipMemcpyAsync(&nt, T.tile_ptr + T.blkm, sizeof(int), hipMemcpyDeviceToHost, s));
+        tile_count_scan(X, T.blkm, T.tile_ptr, ws, s, &box->v[0]);
         TSG_HIP_TRY(hipStreamSynchronize(s));
+        nt = (int)box->v[0];
     }
     T.numblk = nt;
     T.tile_col = ws.alloc_n<int>((size_t)nt + 1);
@@ -907,26 +915,20 @@ void convert(TileMat &T, const CsrIn &X, bool fill_values, Arena &ws, hipStream_
     if (nt == 0) {
         TSG_HIP_TRY(hipMemsetAsync(T.tile_off, 0, sizeof(int), s));
     } else {
-        hipLaunchKernelGGL(k_tile_convert, dim3(grid_for((size_t)T.blkm * 16, 256)), dim3(256),
-                           0, s, X.rows, T.blkm, X.ptr, X.idx, T.tile_ptr, T.tile_col,
+        hipLaunchKernelGGL(k_tile_convert, dim3(grid_for((size_t)T.blkm, CV_TR)),
+                           dim3(16 * CV_TR), 0, s, X.rows, T.blkm, X.ptr, X.idx, T.tile_ptr, T.tile_col,
                            T.tile_off, T.mask, T.rowptr, T.idx, T.perm);
-        TSG_LAUNCH_CHECK();
-    }
-    if (fill_values && X.val && X.nnz > 0) {
-        hipLaunchKernelGGL(k_perm_scatter, dim3(grid_for((size_t)X.nnz, 256)), dim3(256), 0, s,
-                           X.nnz, T.perm, X.val, T.val);
         TSG_LAUNCH_CHECK();
     }
 }
 
 }  // namespace
 
-void tile_count_early(const CsrIn &X, EarlyTileCount &e, Arena &ws, hipStream_t s) {
+void tile_count_early(const CsrIn &X, EarlyTileCount &e, int64_t *total, Arena &ws,
+                      hipStream_t s) {
     const int blkm = (X.rows + 15) / 16;
     e.tile_ptr = ws.alloc_n<int>((size_t)blkm + 1);
-    tile_count_scan(X, blkm, e.tile_ptr, ws, s);
-    TSG_HIP_TRY(
-        hipMemcpyAsync(&e.nt, e.tile_ptr + blkm, sizeof(int), hipMemcpyDeviceToHost, s));
+    tile_count_scan(X, blkm, e.tile_ptr, ws, s, total);
 }
 
 void check_tile_count(int64_t n_c_tiles) {
@@ -936,19 +938,18 @@ void check_tile_count(int64_t n_c_tiles) {
 }
 
 void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int64_t *d_ic,
-                   int64_t *nnz_c, Arena &ws, hipStream_t s, StageTimer &tm, int cus,
+                   int64_t *nnz_c, HostBox *box, Arena &ws, hipStream_t s, StageTimer &tm,
                    const EarlyTileCount *earlyA, const EarlyTileCount *earlyB) {
-    (void)cus;
     p = TilePlan();
     p.b_is_a = b_is_a;
     const int m = A.rows;
     tm.begin("tile.convert");
-    convert(p.A, A, false, ws, s, earlyA);
+    convert(p.A, A, box, ws, s, earlyA);
     if (b_is_a) {
         // B shares A's structure (its column-major values are its own, below)
         p.B = p.A;
     } else {
-        convert(p.B, B, false, ws, s, earlyB);
+        convert(p.B, B, box, ws, s, earlyB);
     }
     // tile-CSC index of B: transpose of its tile pattern.  For C = A*A the
     // pattern is first taken as symmetric (its transpose is itself, with the
@@ -958,15 +959,16 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
     TB.csc_row = ws.alloc_n<int>((size_t)TB.numblk + 1);
     TB.csc_tile = ws.alloc_n<int>((size_t)TB.numblk + 1);
     const bool try_sym = b_is_a && TB.blkm == TB.blkn && TB.numblk > 0;
-    unsigned *d_asym = nullptr;
+    // the asymmetry flag, and the unit counters of the numeric kernels' bins
+    int64_t *d_asym = ws.alloc_n<int64_t>(1 + 2 * TBINS);
+    int64_t *bcnt = d_asym + 1;
+    TSG_HIP_TRY(hipMemsetAsync(d_asym, 0, sizeof(int64_t) * (1 + 2 * TBINS), s));
     auto transpose = [&] {
         TB.csc_ptr = ws.alloc_n<int>((size_t)TB.blkn + 1);
         csr_transpose(TB.blkm, TB.blkn, TB.tile_ptr, TB.tile_col, nullptr, TB.numblk,
                       TB.csc_ptr, TB.csc_row, nullptr, ws, s, TB.csc_tile);
     };
     if (try_sym) {
-        d_asym = ws.alloc_n<unsigned>(1);
-        TSG_HIP_TRY(hipMemsetAsync(d_asym, 0, sizeof(unsigned), s));
         TB.csc_ptr = TB.tile_ptr;
         hipLaunchKernelGGL(k_sym_csc, dim3(grid_for((size_t)TB.blkm * 16, 256)), dim3(256), 0, s,
                            TB.blkm, TB.tile_ptr, TB.tile_col, TB.csc_row, TB.csc_tile, d_asym);
@@ -1022,13 +1024,9 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
         TSG_LAUNCH_CHECK();
     }
     exclusive_scan_i64(pslot, pslot, (size_t)blkm, tmp, s);
-    int64_t nC64 = 0, nslots = 0;
-    unsigned h_asym = 0;
-    TSG_HIP_TRY(hipMemcpyAsync(&nC64, d_nC, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    TSG_HIP_TRY(hipMemcpyAsync(&nslots, pslot + blkm, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    if (d_asym)
-        TSG_HIP_TRY(hipMemcpyAsync(&h_asym, d_asym, sizeof(unsigned), hipMemcpyDeviceToHost, s));
+    publish_i64({{d_nC, pslot + blkm, d_asym}}, 3, box, s);
     TSG_HIP_TRY(hipStreamSynchronize(s));
+    const int64_t nC64 = box->v[0], nslots = box->v[1], h_asym = box->v[2];
     if (h_asym) transpose();
     if (b_is_a) {
         p.A.csc_ptr = TB.csc_ptr;
@@ -1064,7 +1062,6 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
         p.pairs = ws.alloc_n<int2>((size_t)nslots + 1);
     }
     p.rownnz = ws.alloc_n<int64_t>((size_t)m + 1);
-    TSG_HIP_TRY(hipMemsetAsync(p.rownnz, 0, sizeof(int64_t) * ((size_t)m + 1), s));
     if (blkm > 0) {
         hipLaunchKernelGGL(k_step2, dim3(grid_for(blkm, S2_WAVES)), dim3(64 * S2_WAVES), 0, s, m,
                            blkm, p.A.tile_ptr, p.A.tile_col, p.A.mask, TB.csc_ptr, TB.csc_row,
@@ -1079,8 +1076,6 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
     int64_t *tmpm = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)m + 1));
     exclusive_scan_i64(p.rownnz, d_ic, (size_t)m, tmpm, s);
     // C tiles by output count for the numeric kernels
-    int *bcnt = ws.alloc_n<int>(2 * TBINS);
-    TSG_HIP_TRY(hipMemsetAsync(bcnt, 0, 2 * TBINS * sizeof(int), s));
     if (nC > 0) {
         hipLaunchKernelGGL(k_tbin_count, dim3(grid_for((size_t)nC, 256)), dim3(256), 0, s, nC,
                            p.offC, bcnt);
@@ -1088,14 +1083,11 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
     }
     tm.end();
     // nnz(C), the matched-pair total and the bin counts in one round trip
-    int64_t h64[2] = {0, 0};
-    int hb[TBINS] = {0, 0, 0};
-    TSG_HIP_TRY(hipMemcpyAsync(&h64[0], d_ic + m, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    if (!direct_pairs)
-        TSG_HIP_TRY(hipMemcpyAsync(&h64[1], p.tpair + nC, sizeof(int64_t), hipMemcpyDeviceToHost,
-                                   s));
-    TSG_HIP_TRY(hipMemcpyAsync(hb, bcnt, sizeof(hb), hipMemcpyDeviceToHost, s));
+    static_assert(TBINS == 3, "the bins' counts are published one by one");
+    publish_i64({{d_ic + m, p.tpair + nC, bcnt, bcnt + 1, bcnt + 2}}, 5, box, s);
     TSG_HIP_TRY(hipStreamSynchronize(s));
+    const int64_t h64[2] = {box->v[0], direct_pairs ? 0 : box->v[1]};
+    const int hb[TBINS] = {(int)box->v[2], (int)box->v[3], (int)box->v[4]};
     // the numeric phase's work units, sized by the counts just read
     int nunits = 0;
     for (int b = 0; b < TBINS; b++) nunits += hb[b];
@@ -1154,9 +1146,7 @@ static void tile_numeric_t(TilePlan &p, const double *valB, const int64_t *d_ic,
 }
 
 void tile_numeric(TilePlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_ic, int *d_jc,
-                  double *d_c, int fused, Arena &ws, hipStream_t s, StageTimer &tm, int cus) {
-    (void)ws;
-    (void)cus;
+                  double *d_c, int fused, hipStream_t s, StageTimer &tm) {
     TSG_CHECK(p.valid && p.A.rows == A.rows && p.A.cols == A.cols && p.B.cols == B.cols,
               TSG_ERR_STATE, "tile numeric phase without a matching symbolic phase");
     tm.begin("tile.values");
