@@ -44,8 +44,7 @@ struct Batch {
 
 // Products of one group of 64 A entries: lane l's A entry contributes the B
 // positions [lo, lo + cnt) with value a.  Batches of 64 products are handed
-// to f in product order (see for_products); bofs/bstep select every bstep-th
-// batch starting at bofs.
+// to f in product order (see for_products).
 //
 // A product finds its A entry by counting: the entries with products move to
 // the front lanes (a permutation, once per group), a bit is set in LDS (heads:
@@ -54,17 +53,16 @@ struct Batch {
 // so the count is two instructions, against a running maximum over marks
 // written per batch (an LDS round trip and six steps): R-MAT 2^18, items of
 // more than 512 outputs, 1.19 -> 0.96 ms; R-MAT 2^20 with 8 draws a row, 21.6
-// -> 20.7 ms, and its symbolic bands 14.1 -> 13.2 ms.
+// -> 20.7 ms, and its symbolic bands 14.1 -> 13.3 ms.
 // PACKED: B's entries are also given as 16-byte {column, -, value} records
 // (bpk), so a product's column and value come from one load and, for a short
 // range, one cache line.
-template <int U, int BSTEP, bool VALUES, bool PACKED = false, class F>
+template <int U, bool VALUES, bool PACKED = false, class F>
 __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
                                              const int *__restrict__ jb,
                                              const double *__restrict__ bval, int *heads, F &&f,
-                                             int bofs = 0,
                                              const int4 *__restrict__ bpk = nullptr) {
-    static_assert(2 * U * BSTEP <= 64, "a round's start bits are a word a lane");
+    static_assert(2 * U <= 64, "a round's start bits are a word a lane");
     const int l = __lane_id();
     const int incl = wave_incl_scan(cnt);
     const int total = __builtin_amdgcn_readlane(incl, 63);
@@ -82,38 +80,34 @@ __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
             av = __hiloint2double(__builtin_amdgcn_ds_permute(to, __double2hiint(a)),
                                   __builtin_amdgcn_ds_permute(to, __double2loint(a)));
     }
-    for (int base = 0; base < total; base += 64 * U * BSTEP) {
+    for (int base = 0; base < total; base += 64 * U) {
         wave_lds_fence();
-        if (l < 2 * U * BSTEP) heads[l] = 0;
+        if (l < 2 * U) heads[l] = 0;
         wave_lds_fence();
         const int at = start - base;
-        if (cnt > 0 && at >= 0 && at < 64 * U * BSTEP)
+        if (cnt > 0 && at >= 0 && at < 64 * U)
             atomicOr(reinterpret_cast<unsigned *>(heads) + (at >> 5), 1u << (at & 31));
         wave_lds_fence();
-        const int hv = l < 2 * U * BSTEP ? heads[l] : 0;
+        const int hv = l < 2 * U ? heads[l] : 0;
         // entries that start before the batch, less one
         int before = __popcll(__ballot(cnt > 0 && at < 0)) - 1;
         int e[U], sl[U], seg[U], nseg[U];
         bool act[U];
 #pragma unroll
-        for (int v = 0; v < U * BSTEP; v++) {
+        for (int u = 0; u < U; u++) {
             const unsigned long long m =
-                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane(hv, 2 * v + 1) << 32) |
-                (unsigned)__builtin_amdgcn_readlane(hv, 2 * v);
-            const int u = v / BSTEP;
-            if (BSTEP == 1 || v % BSTEP == bofs) {
-                const int q = base + 64 * v + l;
-                // bits at or below the lane: those of m >> 1 below it, bit 0
-                const unsigned long long m1 = m >> 1;
-                sl[u] = (int)__builtin_amdgcn_mbcnt_hi(
-                    (unsigned)(m1 >> 32),
-                    __builtin_amdgcn_mbcnt_lo((unsigned)m1, (unsigned)(before + (int)(m & 1))));
-                const int first = before + (int)(m & 1);
-                seg[u] = sl[u] - first + 1;
-                nseg[u] = __popcll(m | 1ull);
-                act[u] = q < total;
-                e[u] = __shfl(off, sl[u], 64) + q;
-            }
+                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane(hv, 2 * u + 1) << 32) |
+                (unsigned)__builtin_amdgcn_readlane(hv, 2 * u);
+            const int q = base + 64 * u + l;
+            // bits at or below the lane: those of m >> 1 below it, bit 0
+            const unsigned long long m1 = m >> 1;
+            const int first = before + (int)(m & 1);
+            sl[u] = (int)__builtin_amdgcn_mbcnt_hi(
+                (unsigned)(m1 >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m1, (unsigned)first));
+            seg[u] = sl[u] - first + 1;
+            nseg[u] = __popcll(m | 1ull);
+            act[u] = q < total;
+            e[u] = __shfl(off, sl[u], 64) + q;
             before += __popcll(m);
         }
         int col[U];
@@ -131,7 +125,7 @@ __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            if (base + 64 * (u * BSTEP + bofs) < total) {
+            if (base + 64 * u < total) {
                 const double as = VALUES ? __shfl(av, sl[u], 64) : 0.0;
                 f(Batch{act[u], col[u], as, bv[u], seg[u], nseg[u]});
             }
@@ -144,23 +138,25 @@ __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
 // f(batch) is called once per batch by every lane; batches are issued in
 // product order and lane order inside a batch is product order.  U batches
 // are gathered before the first is handed to f, so each lane keeps U
-// independent loads in flight.  Batch striding (bofs, BSTEP): only batches
-// bofs, bofs + BSTEP, ... of every group are visited, so several waves can
-// share one group's products (used where the order of products does not
-// matter).  heads: 64 ints of LDS.
-template <int U, int BSTEP, bool RANGED, bool VALUES, class F>
+// independent loads in flight.  With PARTS > 1 only the A entries part,
+// part + PARTS, ... are visited, so several waves can share a row where the
+// order of products does not matter (entries, not batches of one group: what
+// a group costs before its first product is then spent once, and alternate
+// entries, because a row's first ones may name the longest B rows).  heads:
+// 64 ints of LDS.
+template <int U, int PARTS, bool RANGED, bool VALUES, class F>
 __device__ __forceinline__ void for_products(int pa, int pe, const int *__restrict__ ja,
                                              const double *__restrict__ aval,
                                              const int *__restrict__ ib,
                                              const int *__restrict__ jb,
                                              const double *__restrict__ bval, BlockPtrs bp,
-                                             int c0, int c1, int *heads, F &&f, int bofs = 0) {
+                                             int c0, int c1, int *heads, F &&f, int part = 0) {
     const int l = __lane_id();
     // Software pipeline over groups of A entries: the A entry (t, a) of group
     // g+2 and the B range of group g+1 are loaded while group g's products
     // are processed.
     auto load_t = [&](int g, int &t, double &a) {
-        const int p = g + l;
+        const int p = g + PARTS * l + part;
         t = -1;
         a = 0.0;
         if (g < pe && p < pe) {
@@ -184,16 +180,16 @@ __device__ __forceinline__ void for_products(int pa, int pe, const int *__restri
     int t0, t1;
     double a0, a1;
     load_t(pa, t0, a0);
-    load_t(pa + 64, t1, a1);
+    load_t(pa + 64 * PARTS, t1, a1);
     int lo, hi;
     load_range(t0, lo, hi);
-    for (int g = pa; g < pe; g += 64) {
+    for (int g = pa; g < pe; g += 64 * PARTS) {
         const double a = a0;
         int lo_n, hi_n, t2;
         double a2;
         load_range(t1, lo_n, hi_n);                 // next group's B ranges
-        load_t(g + 128, t2, a2);                    // group after next
-        expand_group<U, BSTEP, VALUES>(lo, max(hi - lo, 0), a, jb, bval, heads, f, bofs);
+        load_t(g + 128 * PARTS, t2, a2);            // group after next
+        expand_group<U, VALUES>(lo, max(hi - lo, 0), a, jb, bval, heads, f);
         lo = lo_n;
         hi = hi_n;
         t1 = t2;

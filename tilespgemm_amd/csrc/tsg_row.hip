@@ -55,7 +55,7 @@ static_assert(ITEM_CAP >= (1 << SUB_SHIFT), "an item must hold a full sub-block"
 constexpr int ITEM_TAGS = 256;
 constexpr int ITEM_WAVES = 1;          // waves per block (one item per wave)
 constexpr int RANK_U = 8;
-constexpr int BIG_SYM_U = 4;
+constexpr int BIG_SYM_U = 8;
 constexpr int ITEM_U = 4;
 
 // ------------------------------------------------------ small rows: symbolic
@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(256) k_gather_units(int64_t n, const int *__re
 
 // One block per band unit: LDS bitmap over the band, the row's products in
 // the band (B rows restricted through the block pointers) marked by the 2
-// waves taking every other batch of 64 products; then the band's sub-block
+// waves, each taking every other A entry; then the band's sub-block
 // output counts, its share of the row's output count (rownnz of big rows is
 // zero on entry) and, when words is given, the band's bitmap in sparse form:
 // per sub-block a mask of its non-empty words (subocc), and the non-empty
@@ -317,6 +317,11 @@ __global__ void __launch_bounds__(256) k_gather_units(int64_t n, const int *__re
 // cursor for all bands had them queue on a single address; the cursor's
 // result is first needed after the staging).  A band whose list would pass
 // its row's region writes none and sets *overflow, which the host checks.
+// Bound by vector instructions, most of them per group of 64 A entries and not
+// per product, so the waves share a row by entries (sharing each group's
+// batches repeated that work in both: R-MAT 2^20 with 8 draws a row 13.3 ms,
+// now 11.8; 2^18 with 4, times its transpose, 0.64 -> 0.47), 8 batches in
+// flight (4: 12.0 and 0.54 ms; 2: 12.9 and 0.70).
 // 8 waves per SIMD, as with no word lists (the kernel waits on its gathers;
 // its arguments alone would take the scalar registers past that).
 __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))) k_big_symbolic(
@@ -1048,8 +1053,7 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric_rank(
             double a2;
             load_range(t1, lo_n, hi_n);
             load_t(g + 128, t2, a2);
-            expand_group<RANK_U, 1, true, true>(lo, max(hi - lo, 0), ag, jb, b, S.heads, f, 0,
-                                                bpk);
+            expand_group<RANK_U, true, true>(lo, max(hi - lo, 0), ag, jb, b, S.heads, f, bpk);
             lo = lo_n;
             hi = hi_n;
             t1 = t2;
@@ -1183,8 +1187,7 @@ k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
             double a1;
             load_t(g + 64, t1, a1);
             load_range(t1, lo_n, hi_n);
-            expand_group<U, 1, true, true>(lo, max(hi - lo, 0), a0, jb, nullptr, S.heads, f, 0,
-                                           bpk);
+            expand_group<U, true, true>(lo, max(hi - lo, 0), a0, jb, nullptr, S.heads, f, bpk);
             lo = lo_n;
             hi = hi_n;
             a0 = a1;
