@@ -134,8 +134,8 @@ int tsg_get_tuning(tsg_handle_t handle, double *tile_density, int *bin1, int *bi
  * 16384 columns, the symbolic band units and the numeric items are run in
  * order of their first column (a radix sort in the symbolic phase), so the
  * units in flight together read B entries of one narrow column band and
- * find them in L2; the B block pointers are then laid out block-major and
- * the items cut to 8192 columns.  Below that the sort costs more than it
+ * find them in L2; B is then cut by a run directory and the items cut to
+ * 8192 columns.  Below that the sort costs more than it
  * saves.  Default 2^18 (R-MAT n=2^20 A*A^T: 24M windows; n=2^18 with 4
  * draws per row: 523K, 6.48 -> 6.10 ms in column order; n=2^16: 108K,
  * even; n=2^14: 1.68 -> 1.89 ms).  0 always sorts.  Changes speed only. */
@@ -152,10 +152,12 @@ int tsg_set_item_order(tsg_handle_t handle, int64_t min_items);
  * dense bitmaps would.  Negative (the default): min(48 GiB, 40% of free
  * device memory). */
 int tsg_set_bitmap_budget(tsg_handle_t handle, int64_t bytes);
-/* Memory for the B block-pointer table of the big-row path (no counterpart
- * in the reference): one position per B row and 1024-column block while the
- * table takes at most this many bytes, else blocks of 2048, 4096, ...
- * columns (up to 2^30) with a binary search inside a block.  0: no table,
+/* Memory for the B block-pointer table of the big-row path, or B's run
+ * directory where the work runs in column order (no counterpart in the
+ * reference): one position per B row and 1024-column block (the directory:
+ * 24 bytes per 32 B rows and block, and 56 per entry) while that takes at
+ * most this many bytes, else blocks of 2048, 4096, ... columns (up to 2^30;
+ * the directory up to 65536) with a binary search inside a block.  0: none,
  * every range is searched inside its B row.  Negative (the default): 6 GiB,
  * and no table when building it would cost more than 8 entries per lookup
  * it serves (a few big rows against many B rows, as in batches of small

@@ -4,16 +4,13 @@
 
 #include "tsg_device.h"
 
-// ------------------------------------------------- flat product expansion
+// ------------------------------------------------- ranges of B's rows
 // B block pointers: entry (row t, block b) = first position of B row t with
-// column >= b << bs, at p[t*tstride + b*bstride].  Row-major (tstride =
-// blocks+1, bstride = 1) keeps a row's entries together; block-major
-// (tstride = 1, bstride = rows of B) keeps a block's entries for all rows
-// together, which suits work that runs in column order: it looks up a few
-// blocks at a time, whose entries stay in L2.
+// column >= b << bs, at p[t*tstride + b] (a row's entries together).  B's row
+// pointers are a table of one block.
 struct BlockPtrs {
     const int *p = nullptr;
-    int64_t tstride = 0, bstride = 0;
+    int64_t tstride = 0;
     int bs = 0;
 };
 
@@ -22,15 +19,130 @@ struct BlockPtrs {
 __device__ __forceinline__ int brange_lo(const BlockPtrs &bp, const int *__restrict__ jb, int t,
                                          int c) {
     const int b = c >> bp.bs;
-    const int64_t e = (int64_t)t * bp.tstride + (int64_t)b * bp.bstride;
+    const int64_t e = (int64_t)t * bp.tstride + b;
     int lo = bp.p[e];
     if (c & ((1 << bp.bs) - 1)) {
-        int hi = bp.p[e + bp.bstride];
+        int hi = bp.p[e + 1];
         lo = lower_bound_i32(jb, lo, hi, c);
     }
     return lo;
 }
 
+// How B's rows are cut to an item: by the run directory where it is there,
+// else by block pointers.
+struct BRows {
+    BlockPtrs bp;
+    RunDir dir;
+};
+
+// B rows' positions with columns in [c0, c1), in two steps so that loads can
+// be issued ahead: ahead(t), then range(t, that, lo, hi); t < 0: none.  DIR: by
+// the run directory; [c0, c1) then holds all the work's columns in an aligned
+// power of two of sub-blocks, so its runs are those of the smallest block that
+// holds it.
+template <bool DIR>
+struct ItemRange {
+    const BRows *b;
+    const int *jb;
+    const uint2 *cells;
+    int c0, c1;
+    __device__ __forceinline__ ItemRange(const BRows &b_, const int *jb_, int c0_, int c1_)
+        : b(&b_), jb(jb_), c0(c0_), c1(c1_) {
+        if (DIR) {
+            const unsigned x = (unsigned)(c0 ^ (c1 - 1)) >> b->dir.shift;
+            const int v = x ? 32 - __clz(x) : 0;
+            cells = b->dir.cells + run_dir_block(b->dir.nblk, b->dir.shift, v, c0) * b->dir.ngrp;
+        }
+    }
+    __device__ __forceinline__ uint2 ahead(int t) const {
+        return DIR && t >= 0 ? cells[t >> 5] : make_uint2(0u, 0u);
+    }
+    __device__ __forceinline__ void range(int t, uint2 w, int &lo, int &hi) const {
+        lo = 0;
+        hi = 0;
+        if (DIR) {
+            const unsigned bit = 1u << (t & 31);
+            if (w.x & bit) {
+                const int2 r = b->dir.runs[w.y + __popc(w.x & (bit - 1))];
+                lo = r.x;
+                hi = r.y;
+                if (b->dir.coarse) {       // a block may hold more than the item
+                    lo = lower_bound_i32(jb, lo, hi, c0);
+                    hi = lower_bound_i32(jb, lo, hi, c1);
+                }
+            }
+        } else if (t >= 0) {
+            lo = brange_lo(b->bp, jb, t, c0);
+            hi = brange_lo(b->bp, jb, t, c1);
+        }
+    }
+};
+
+// B's whole rows.
+struct RowRange {
+    const int *ib;
+    __device__ __forceinline__ uint2 ahead(int) const { return make_uint2(0u, 0u); }
+    __device__ __forceinline__ void range(int t, uint2, int &lo, int &hi) const {
+        lo = t >= 0 ? ib[t] : 0;
+        hi = t >= 0 ? ib[t + 1] : 0;
+    }
+};
+
+// A row's entries [pa, pe) in groups of 64, loaded ahead of their use: while
+// a group's products are processed, the next group's B ranges and values, the
+// cells of the group after that and the A columns of the third are loading.
+// load() and cells() start it, first() gives group 0's ranges (each uses what
+// the one before has loaded, so other work goes between them).  With PARTS > 1
+// only the entries part, part + PARTS, ... are visited.
+template <bool VALUES, int PARTS>
+struct EntryPipe {
+    const int *ja;
+    const double *aval;
+    int pa, pe, part;
+    int t1, t2;
+    uint2 w1;
+    int lo, hi, lo1, hi1;          // the group's ranges, and the next one's
+    double a, a1;
+    __device__ __forceinline__ int col(int g) const {
+        const int p = g + PARTS * __lane_id() + part;
+        return g < pe && p < pe ? ja[p] : -1;
+    }
+    __device__ __forceinline__ double val(int g) const {
+        const int p = g + PARTS * __lane_id() + part;
+        return VALUES && g < pe && p < pe ? aval[p] : 0.0;
+    }
+    __device__ __forceinline__ void load(int pa_, int pe_) {
+        pa = pa_;
+        pe = pe_;
+        t1 = col(pa);
+        t2 = col(pa + 64 * PARTS);
+    }
+    template <class R>
+    __device__ __forceinline__ void cells(const R &rows) {
+        w1 = rows.ahead(t1);
+    }
+    // the next group's ranges, and what lies behind them; g: the group at hand
+    template <class R>
+    __device__ __forceinline__ void ahead(int g, const R &rows) {
+        rows.range(t1, w1, lo1, hi1);
+        a1 = val(g + 64 * PARTS);
+        t1 = t2;
+        w1 = rows.ahead(t2);
+        t2 = col(g + 3 * 64 * PARTS);
+    }
+    __device__ __forceinline__ void take() {
+        lo = lo1;
+        hi = hi1;
+        a = a1;
+    }
+    template <class R>
+    __device__ __forceinline__ void first(const R &rows) {
+        ahead(pa - 64 * PARTS, rows);
+        take();
+    }
+};
+
+// ------------------------------------------------- flat product expansion
 // A batch of 64 products seen by the functions below: act marks the lanes
 // that hold a product; seg is the lane's A entry among the batch's (from 1)
 // and nseg their number (uniform); products of one A entry are one B row's:
@@ -48,7 +160,7 @@ struct Batch {
 //
 // A product finds its A entry by counting: the entries with products move to
 // the front lanes (a permutation, once per group), a bit is set in LDS (heads:
-// 64 ints, any content) where each one's products start, and product q
+// 2 U ints, any content) where each one's products start, and product q
 // belongs to entry (bits at or below q) - 1.  A batch's 64 bits are a scalar,
 // so the count is two instructions, against a running maximum over marks
 // written per batch (an LDS round trip and six steps): R-MAT 2^18, items of
@@ -134,67 +246,33 @@ __device__ __forceinline__ void expand_group(int lo, int cnt, double a,
 }
 
 // Visits the products of the A entries [pa, pe) of one row in A-row order, a
-// wave's 64 entries at a time, optionally restricted to B columns [c0, c1).
-// f(batch) is called once per batch by every lane; batches are issued in
-// product order and lane order inside a batch is product order.  U batches
-// are gathered before the first is handed to f, so each lane keeps U
-// independent loads in flight.  With PARTS > 1 only the A entries part,
-// part + PARTS, ... are visited, so several waves can share a row where the
-// order of products does not matter (entries, not batches of one group: what
-// a group costs before its first product is then spent once, and alternate
-// entries, because a row's first ones may name the longest B rows).  heads:
-// 64 ints of LDS.
-template <int U, int PARTS, bool RANGED, bool VALUES, class F>
+// wave's 64 entries at a time, each entry's B positions given by rows (an
+// ItemRange or RowRange).  f(batch) is called once per batch by every lane;
+// batches are issued in product order and lane order inside a batch is product
+// order.  U batches are gathered before the first is handed to f, so each lane
+// keeps U independent loads in flight.  With PARTS > 1 only the A entries
+// part, part + PARTS, ... are visited, so several waves can share a row where
+// the order of products does not matter (entries, not batches of one group:
+// what a group costs before its first product is then spent once, and
+// alternate entries, because a row's first ones may name the longest B rows).
+// heads: 2 U ints of LDS.
+template <int U, int PARTS, bool VALUES, class R, class F>
 __device__ __forceinline__ void for_products(int pa, int pe, const int *__restrict__ ja,
-                                             const double *__restrict__ aval,
-                                             const int *__restrict__ ib,
+                                             const double *__restrict__ aval, const R &rows,
                                              const int *__restrict__ jb,
-                                             const double *__restrict__ bval, BlockPtrs bp,
-                                             int c0, int c1, int *heads, F &&f, int part = 0) {
-    const int l = __lane_id();
-    // Software pipeline over groups of A entries: the A entry (t, a) of group
-    // g+2 and the B range of group g+1 are loaded while group g's products
-    // are processed.
-    auto load_t = [&](int g, int &t, double &a) {
-        const int p = g + PARTS * l + part;
-        t = -1;
-        a = 0.0;
-        if (g < pe && p < pe) {
-            t = ja[p];
-            if (VALUES) a = aval[p];
-        }
-    };
-    auto load_range = [&](int t, int &lo, int &hi) {
-        lo = 0;
-        hi = 0;
-        if (t >= 0) {
-            if (RANGED) {
-                lo = brange_lo(bp, jb, t, c0);
-                hi = brange_lo(bp, jb, t, c1);
-            } else {
-                lo = ib[t];
-                hi = ib[t + 1];
-            }
-        }
-    };
-    int t0, t1;
-    double a0, a1;
-    load_t(pa, t0, a0);
-    load_t(pa + 64 * PARTS, t1, a1);
-    int lo, hi;
-    load_range(t0, lo, hi);
+                                             const double *__restrict__ bval, int *heads, F &&f,
+                                             int part = 0) {
+    EntryPipe<VALUES, PARTS> pipe;
+    pipe.ja = ja;
+    pipe.aval = aval;
+    pipe.part = part;
+    pipe.load(pa, pe);
+    pipe.cells(rows);
+    pipe.first(rows);
     for (int g = pa; g < pe; g += 64 * PARTS) {
-        const double a = a0;
-        int lo_n, hi_n, t2;
-        double a2;
-        load_range(t1, lo_n, hi_n);                 // next group's B ranges
-        load_t(g + 128 * PARTS, t2, a2);            // group after next
-        expand_group<U, VALUES>(lo, max(hi - lo, 0), a, jb, bval, heads, f);
-        lo = lo_n;
-        hi = hi_n;
-        t1 = t2;
-        a0 = a1;
-        a1 = a2;
+        pipe.ahead(g, rows);
+        expand_group<U, VALUES>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, jb, bval, heads, f);
+        pipe.take();
     }
 }
 
@@ -247,10 +325,16 @@ __device__ __forceinline__ void ordered_accumulate(bool act, int slot, double a,
     while (__ballot(pending)) {
         if (pending) atomicMin(&tags[bucket], me);
         wave_lds_fence();
-        bool win = pending && tags[bucket] == me;
+        // both reads in one wait: the value is used by the bucket's winner
+        unsigned first = 0u;
+        double v = 0.0;
+        if (pending) {
+            first = tags[bucket];
+            v = vals[slot];
+        }
         wave_lds_fence();
-        if (win) {
-            vals[slot] = acc_step<FUSED>(vals[slot], a, b);
+        if (pending && first == me) {
+            vals[slot] = acc_step<FUSED>(v, a, b);
             tags[bucket] = 0xffffffffu;
             pending = false;
         }

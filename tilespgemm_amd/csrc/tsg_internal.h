@@ -176,7 +176,7 @@ struct RowTuning {
     int bin1 = 64, bin2 = 256, bin3 = 1024;
     int64_t item_sort_min = int64_t(1) << 18;  // big-row items column-ordered from this many
     int64_t bitmap_budget = -1;  // bytes of big-row bitmaps (sparse form) kept; < 0: min(48 GiB, 40% of free)
-    int64_t bptr_budget = -1;    // bytes of the B block-pointer table; < 0: 6 GiB
+    int64_t bptr_budget = -1;    // bytes of B's block pointers or run directory; < 0: 6 GiB
 };
 
 // One big-row item: d = {row, first column, end column, first sub-block in
@@ -190,6 +190,31 @@ struct ItemRec {
 };
 static_assert(sizeof(ItemRec) == 32, "item records are 32 bytes");
 
+// Run directory of B, for work in column order.  The columns are cut in
+// blocks of 1 << shift, of 2 << shift and so on, up to a band: level v's
+// blocks are 1 << (shift + v) columns wide.  A run is a B row's entries in one
+// block; block b of level v has a cell for every 32 B rows: which of them have
+// a run there, and the number of runs of earlier cells, so row t's run is
+// found in runs[] ({first, end} positions in B) by counting bits.  An item's
+// rows then cost a lookup in one block's cells (256 KB for 2^20 rows, which
+// stay in L2) and, for rows with a run only, one in its runs; block pointers
+// cost two reads from 4 MB each.  Level v's blocks are cells[blocks before v +
+// b], blocks before v = 2 nblk - (2 nblk >> v).
+struct RunDir {
+    const uint2 *cells = nullptr;
+    const int2 *runs = nullptr;
+    int ngrp = 0;                  // cells a block
+    int nblk = 0;                  // blocks of level 0 (whole bands)
+    int shift = 0;
+    int coarse = 0;                // blocks of level 0 may be wider than items
+};
+
+__host__ __device__ __forceinline__ int64_t run_dir_block(int nblk, int shift, int v, int c) {
+    return 2ll * nblk - (2ll * nblk >> v) + (c >> (shift + v));
+}
+
+constexpr int ITEM_CLASSES = 3;       // size classes of the row path's items
+
 struct RowPlan {
     bool valid = false;
     bool b_strict = false;           // B rows strictly ascending (no duplicates)
@@ -202,16 +227,17 @@ struct RowPlan {
     int64_t *sb_off = nullptr;       // [nbig+1] span offsets (sub-blocks)
     int64_t nsb_total = 0;
     uint16_t *subcnt = nullptr;      // [nsb_total] outputs per span sub-block
-    // B block-pointer table for big-row items
+    // B's rows cut to big-row bands and items: by the run directory (column
+    // order) or the block-pointer table; with neither, B's row pointers serve
+    // as a table of one block
+    RunDir dir;
     int blk_shift = 0;               // log2 block width (columns)
     int nblk = 0;                    // blocks per B row (+1 stored)
-    int *bptr = nullptr;             // [(nblk+1) * n]: block-major with column_order
-    bool bptr_rowptr = false;        // no table: B's row pointers serve as one block
+    int *bptr = nullptr;             // [(nblk+1) * n]
     bool column_order = false;       // big-row bands and items run in column order
     // items
     int64_t nitems = 0;
-    int64_t nitems_small = 0;        // items of <= 256 outputs, first in items (column order)
-    int64_t nitems_mid = 0;          // end of the items of <= 512 outputs, next
+    int64_t class_end[ITEM_CLASSES] = {};   // ends of the items' size classes (column order)
     int64_t *item_cnt = nullptr;     // [nbig+1] items per big row -> offsets
     ItemRec *items = nullptr;        // by c0 (column order) or by row
     bool narrow_items = false;       // items of <= 8192 columns (else <= 16384)

@@ -23,9 +23,10 @@
 //     sub-block, and those words); the numeric phase splits the row into
 //     items of <= ITEM_CAP outputs and <= 16384 columns, each accumulated by
 //     one wave into a rank-ordered LDS array (rank from the stored bitmap)
-//     and written in column order.  A B block pointer table gives each B row's
-//     sub-range of a band or item without a search; bands and items run in
-//     order of their first column, so those in flight share a band of B.
+//     and written in column order.  Bands and items of wide matrices run in
+//     order of their first column, so those in flight share a band of B, and a
+//     run directory of B gives each B row's entries in a band or item; else a
+//     table of block pointers does, or a search.
 #include "tsg_internal.h"
 
 #include <cmath>
@@ -265,19 +266,29 @@ __global__ void __launch_bounds__(256) k_big_span(int nbig, const int *__restric
         nprod[r] = rowprod[row];
         // a multiple of BAND_PAD, so every band's list starts 16-byte aligned
         lbound[r] = ((min(rowprod[row], ns << (SUB_SHIFT - 5)) + BAND_PAD - 1) & -BAND_PAD) +
-                    BAND_PAD * ((ns + (1 << BAND_SHIFT) - 1) >> BAND_SHIFT);
+                    BAND_PAD * (((ns + (1 << BAND_SHIFT) - 1) >> BAND_SHIFT) + 1);
     }
 }
 
 // -------------------------------------------------------- big rows: symbolic
 // A big row's span is cut into bands of 64 sub-blocks; a band unit {r, u}
-// covers span sub-blocks [64u, 64u + 64) of big row r.  Units are run in
-// order of their first column (like the numeric items), so the units in
-// flight read B columns of one narrow band, which the L2 caches keep.
-__global__ void __launch_bounds__(256) k_band_count(int nbig, const int64_t *__restrict__ nsb,
+// covers span sub-blocks [64u - lead, 64u + 64 - lead) of big row r.  Units are
+// run in order of their first column (like the numeric items), so the units
+// in flight read B columns of one narrow band, which the L2 caches keep; bands
+// are then the matrix's (lead = the sub-blocks of the first band before the
+// span), as the run directory of B has them, else the span's (lead = 0).
+__device__ __forceinline__ int band_lead(int span_sb0) {
+    return span_sb0 & ((1 << BAND_SHIFT) - 1);
+}
+
+__global__ void __launch_bounds__(256) k_band_count(int nbig, int64_t sort_min,
+                                                    const int *__restrict__ span_sb0,
+                                                    const int64_t *__restrict__ sb_off,
                                                     int64_t *__restrict__ cnt) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nbig) cnt[r] = (nsb[r] + (1 << BAND_SHIFT) - 1) >> BAND_SHIFT;
+    if (r >= nbig) return;
+    const int lead = sb_off[nbig] / 16 >= sort_min ? band_lead(span_sb0[r]) : 0;
+    cnt[r] = (lead + sb_off[r + 1] - sb_off[r] + (1 << BAND_SHIFT) - 1) >> BAND_SHIFT;
 }
 
 __global__ void __launch_bounds__(256) k_band_fill(int nbig, const int *__restrict__ span_sb0,
@@ -289,7 +300,7 @@ __global__ void __launch_bounds__(256) k_band_fill(int nbig, const int *__restri
     const int64_t o = off[r], n = off[r + 1] - o;
     for (int u = 0; u < n; u++) {
         units[o + u] = make_int2(r, u);
-        keys[o + u] = span_sb0[r] + (u << BAND_SHIFT);
+        keys[o + u] = span_sb0[r] + (u << BAND_SHIFT);   // its band's, less than one off
     }
 }
 
@@ -301,7 +312,7 @@ __global__ void __launch_bounds__(256) k_gather_units(int64_t n, const int *__re
 }
 
 // One block per band unit: LDS bitmap over the band, the row's products in
-// the band (B rows restricted through the block pointers) marked by the 2
+// the band (B rows cut to the band by brows) marked by the 2
 // waves, each taking every other A entry; then the band's sub-block
 // output counts, its share of the row's output count (rownnz of big rows is
 // zero on entry) and, when words is given, the band's bitmap in sparse form:
@@ -324,10 +335,11 @@ __global__ void __launch_bounds__(256) k_gather_units(int64_t n, const int *__re
 // flight (4: 12.0 and 0.54 ms; 2: 12.9 and 0.70).
 // 8 waves per SIMD, as with no word lists (the kernel waits on its gathers;
 // its arguments alone would take the scalar registers past that).
+template <bool DIR>
 __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))) k_big_symbolic(
     int64_t nunits, const int2 *__restrict__ units, const int *__restrict__ rows, int k,
-    const int *__restrict__ ia, const int *__restrict__ ja, const int *__restrict__ ib,
-    const int *__restrict__ jb, BlockPtrs bp, const int *__restrict__ span_sb0,
+    int by_band, const int *__restrict__ ia, const int *__restrict__ ja,
+    const int *__restrict__ jb, BRows brows, const int *__restrict__ span_sb0,
     const int64_t *__restrict__ sb_off, uint16_t *__restrict__ subcnt,
     int64_t *__restrict__ rownnz, const int64_t *__restrict__ band_off,
     int64_t *__restrict__ band_base, unsigned long long *__restrict__ row_cur,
@@ -345,18 +357,20 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
         const int2 un = units[ui];
         const int r = un.x, u = un.y;
         const int row = rows[r];
-        const int64_t so = sb_off[r] + ((int64_t)u << BAND_SHIFT);
-        const int nsb = (int)min((int64_t)1 << BAND_SHIFT, sb_off[r + 1] - so);
-        const int sb0 = span_sb0[r] + (u << BAND_SHIFT);
+        const int lead = by_band ? band_lead(span_sb0[r]) : 0;
+        const int j0 = max((u << BAND_SHIFT) - lead, 0);
+        const int64_t so = sb_off[r] + j0;
+        const int nsb = (int)min((int64_t)((u + 1) << BAND_SHIFT) - lead - j0, sb_off[r + 1] - so);
+        const int sb0 = span_sb0[r] + j0;
         const int c0 = sb0 << SUB_SHIFT;
         const int c1 = (int)min((int64_t)k, (int64_t)(sb0 + nsb) << SUB_SHIFT);
         const int words = (c1 - c0 + 31) >> 5;
         for (int i = threadIdx.x; 4 * i < words; i += BAND_T)
             reinterpret_cast<uint4 *>(bits)[i] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
-        for_products<BIG_SYM_U, NW, true, false>(
-            ia[row], ia[row + 1], ja, nullptr, ib, jb, nullptr, bp, c0, c1, s_heads[wave],
-            [&](const Batch &t) {
+        for_products<BIG_SYM_U, NW, false>(
+            ia[row], ia[row + 1], ja, nullptr, ItemRange<DIR>(brows, jb, c0, c1), jb, nullptr,
+            s_heads[wave], [&](const Batch &t) {
                 if (t.act) {
                     const int cc = t.col - c0;
                     lds_set_bit(&bits[cc >> 5], 1u << (cc & 31));
@@ -467,83 +481,190 @@ __global__ void __launch_bounds__(256) k_bptr_rows(int n, const int *__restrict_
     }
 }
 
-// Block-major table: bptr[b*n + t] = first position of B row t with column
-// >= b << bs.  A block of 4 waves takes 64 B rows; for each range of 64 blocks
-// the waves fill an LDS tile [block][row], a lane per block searching inside
-// its row, then write it out as 64 consecutive rows per block (256-byte runs).
-// The 64 rows' columns are one contiguous range of jb: when it holds at most
-// BPT_STAGE entries (R-MAT 2^20's B averages ~940 per 64 rows) it is staged
-// in LDS once and every search runs there; otherwise the searches read jb.
-// The searches wait on their loads, so residency mattered with global
-// searches (a 128-block tile took 6.2 ms instead of 4.5 ms for R-MAT 2^20's
-// 16,385 x 2^20 table, a 32-block one 7.1 ms), and still does with staged
-// ones: blocks of 128 or 256 rows (512- or 1024-byte runs) took 6.6 and
-// 8.4 ms instead of 4.5.
-constexpr int BPT_ROWS = 64, BPT_BLK = 64, BPT_STAGE = 2048;
+// Run directory (RunDir), built in three passes: the cells' bits, the scan of
+// their counts, the runs.
+//
+// Bits: a block takes DIR_ROWS B rows and ranges of DIR_BLK blocks of level 0,
+// marks them in LDS and folds each level's pairs of blocks into the next's.
+// The bits go out cell-major, DIR_ROWS / 32 consecutive cells a block.  Bound
+// by the busiest block, that of the longest rows: 1.2 ms with 512 rows and
+// threads a block (R-MAT 2^20), 0.6 with 256 and 1024.
+constexpr int DIR_ROWS = 256, DIR_GRP = DIR_ROWS / 32, DIR_BLK = 512;
 
-__device__ __forceinline__ int lds_lower_bound(const int *a, int lo, int hi, int key) {
-    while (lo < hi) {
+// row (of nr from the first) of the entry at position e: rp ascending
+__device__ __forceinline__ int dir_row_of(const int *rp, int nr, int e) {
+    int lo = 0, hi = nr;               // rp[lo] <= e < rp[hi]
+    while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (a[mid] < key) lo = mid + 1;
+        if (rp[mid] <= e) lo = mid;
         else hi = mid;
     }
     return lo;
 }
 
-__global__ void __launch_bounds__(256) k_bptr(int n, const int *__restrict__ ib,
-                                              const int *__restrict__ jb, int nblk, int bs,
-                                              int *__restrict__ bptr) {
-    __shared__ int tile[BPT_BLK][BPT_ROWS + 1];
-    __shared__ int s_col[BPT_STAGE];
-    __shared__ int s_rp[BPT_ROWS + 1];
-    const int t0 = blockIdx.x * BPT_ROWS;
-    const int nr = min(BPT_ROWS, n - t0);
+__global__ void __launch_bounds__(1024) k_dir_bits(int n, const int *__restrict__ ib,
+                                                  const int *__restrict__ jb, int ngrp, int nblk,
+                                                  int shift, int levels,
+                                                  unsigned *__restrict__ bits) {
+    __shared__ int s_rp[DIR_ROWS + 1];
+    __shared__ unsigned s_bits[2 * DIR_BLK * DIR_GRP];
+    const int t0 = blockIdx.x * DIR_ROWS, g0 = blockIdx.x * DIR_GRP;
+    const int nr = min(DIR_ROWS, n - t0), ng = min(DIR_GRP, ngrp - g0);
     for (int i = threadIdx.x; i <= nr; i += blockDim.x) s_rp[i] = ib[t0 + i];
     __syncthreads();
-    const int e0 = s_rp[0];
-    const bool staged = s_rp[nr] - e0 <= BPT_STAGE;
-    if (staged)
-        for (int i = threadIdx.x; i < s_rp[nr] - e0; i += blockDim.x) s_col[i] = jb[e0 + i];
+    for (int b0 = 0; b0 < nblk; b0 += DIR_BLK) {
+        for (int i = threadIdx.x; i < DIR_BLK * DIR_GRP; i += blockDim.x) s_bits[i] = 0u;
+        __syncthreads();
+        for (int e = s_rp[0] + threadIdx.x; e < s_rp[nr]; e += blockDim.x) {
+            const int b = (jb[e] >> shift) - b0;
+            if (b >= 0 && b < DIR_BLK) {
+                const int r = dir_row_of(s_rp, nr, e);
+                lds_set_bit(&s_bits[b * DIR_GRP + (r >> 5)], 1u << (r & 31));
+            }
+        }
+        __syncthreads();
+        unsigned *lev = s_bits;
+        int cnt = min(DIR_BLK, nblk - b0);          // a multiple of 1 << (levels - 1)
+        for (int v = 0; v < levels; v++, cnt >>= 1) {
+            unsigned *out = bits + run_dir_block(nblk, 0, v, b0) * ngrp + g0;
+            for (int i = threadIdx.x; i < cnt * DIR_GRP; i += blockDim.x)
+                if (i % DIR_GRP < ng) out[(int64_t)(i / DIR_GRP) * ngrp + i % DIR_GRP] = lev[i];
+            unsigned *up = lev + cnt * DIR_GRP;
+            for (int i = threadIdx.x; i < (cnt >> 1) * DIR_GRP; i += blockDim.x) {
+                const int a = (i / DIR_GRP) * 2 * DIR_GRP + i % DIR_GRP;
+                up[i] = lev[a] | lev[a + DIR_GRP];
+            }
+            lev = up;
+            __syncthreads();
+        }
+    }
+}
+
+// Scan of the cells' counts: chunks of DIR_CHUNK cells, a total each (then
+// scanned), and the cells {bits, runs before}.
+constexpr int DIR_CHUNK = 8192;
+
+__global__ void __launch_bounds__(256) k_dir_sums(int64_t ncells, const unsigned *__restrict__ bits,
+                                                  int64_t *__restrict__ sums) {
+    __shared__ int s_sum[4];
+    int64_t i = (int64_t)blockIdx.x * DIR_CHUNK + threadIdx.x * 4;
+    int c = 0;
+#pragma unroll
+    for (int q = 0; q < DIR_CHUNK / 1024; q++, i += 1024) {
+        // (the array is whole chunks)
+        const uint4 v = *reinterpret_cast<const uint4 *>(bits + i);
+        c += i < ncells ? __popc(v.x) : 0;
+        c += i + 1 < ncells ? __popc(v.y) : 0;
+        c += i + 2 < ncells ? __popc(v.z) : 0;
+        c += i + 3 < ncells ? __popc(v.w) : 0;
+    }
+    c = wave_sum(c);
+    if (__lane_id() == 0) s_sum[threadIdx.x >> 6] = c;
     __syncthreads();
-    for (int b0 = 0; b0 <= nblk; b0 += BPT_BLK) {
-        // (row, block) pairs, a thread each: a row's blocks in consecutive lanes
-        for (int i = threadIdx.x; i < nr * BPT_BLK; i += blockDim.x) {
-            const int r = i / BPT_BLK, bb = i % BPT_BLK;
-            const int b = b0 + bb;
-            if (b > nblk) continue;
-            const int lo = s_rp[r], hi = s_rp[r + 1];
-            int pos = hi;
-            if (b < nblk)
-                pos = staged ? e0 + lds_lower_bound(s_col, lo - e0, hi - e0, b << bs)
-                             : lower_bound_i32(jb, lo, hi, b << bs);
-            tile[bb][r] = pos;
+    if (threadIdx.x == 0) sums[blockIdx.x] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+}
+
+__global__ void __launch_bounds__(256) k_dir_cells(int64_t ncells,
+                                                   const unsigned *__restrict__ bits,
+                                                   const int64_t *__restrict__ sums,
+                                                   uint2 *__restrict__ cells) {
+    __shared__ int s_sum[4];
+    const int w = threadIdx.x >> 6;
+    int before = (int)sums[blockIdx.x];
+    for (int q = 0; q < DIR_CHUNK / 1024; q++) {
+        const int64_t i = (int64_t)blockIdx.x * DIR_CHUNK + q * 1024 + threadIdx.x * 4;
+        uint4 v = *reinterpret_cast<const uint4 *>(bits + i);
+        if (i >= ncells) v.x = 0;
+        if (i + 1 >= ncells) v.y = 0;
+        if (i + 2 >= ncells) v.z = 0;
+        if (i + 3 >= ncells) v.w = 0;
+        const int a = __popc(v.x), b = a + __popc(v.y), c = b + __popc(v.z), d = c + __popc(v.w);
+        const int incl = wave_incl_scan(d);
+        if (__lane_id() == 63) s_sum[w] = incl;
+        __syncthreads();
+        int at = before + incl - d;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (k < w) at += s_sum[k];
+            before += s_sum[k];
         }
         __syncthreads();
-        // a block's rows in consecutive lanes: runs of 4 * BPT_ROWS bytes
-        for (int i = threadIdx.x; i < BPT_BLK * BPT_ROWS; i += blockDim.x) {
-            const int bb = i / BPT_ROWS, r = i % BPT_ROWS;
-            const int b = b0 + bb;
-            if (b <= nblk && r < nr) bptr[(size_t)b * n + t0 + r] = tile[bb][r];
+        uint4 *out = reinterpret_cast<uint4 *>(cells + i);
+        out[0] = make_uint4(v.x, (unsigned)at, v.y, (unsigned)(at + a));
+        out[1] = make_uint4(v.z, (unsigned)(at + b), v.w, (unsigned)(at + c));
+    }
+}
+
+// Runs: a thread per entry, which at each level stores its run's first
+// position if it is the first and the end if it is the last.  Bound by the
+// latency of a cell's read and the store behind it, so the levels' reads are
+// issued together; blocks take entries, not rows, which hub rows make uneven
+// (R-MAT 2^20
+// with 8 draws a row: blocks of 512 rows 6.6 ms, of 64 rows 3.2, of entries
+// 0.6).
+constexpr int RUN_ENT = 512;
+
+__global__ void __launch_bounds__(256) k_dir_runs(int n, int nnz, const int *__restrict__ ib,
+                                                  const int *__restrict__ jb, int ngrp, int nblk,
+                                                  int shift, int levels,
+                                                  const uint2 *__restrict__ cells,
+                                                  int2 *__restrict__ runs) {
+    __shared__ int s_r[2];
+    const int e0 = blockIdx.x * RUN_ENT, e1 = min(e0 + RUN_ENT, nnz);
+    if (threadIdx.x < 2) {
+        // row of the block's first and last entry: the last t with ib[t] <= e
+        const int e = threadIdx.x ? e1 - 1 : e0;
+        s_r[threadIdx.x] = lower_bound_i32(ib, 0, n, e + 1) - 1;
+    }
+    __syncthreads();
+    for (int e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
+        const int r = lower_bound_i32(ib, s_r[0], s_r[1] + 1, e + 1) - 1;
+        const int c = jb[e];
+        // level-0 blocks of the entry and of its neighbours (-1: none)
+        const int b = c >> shift;
+        const int pb = e > ib[r] ? jb[e - 1] >> shift : -1;
+        const int nb = e + 1 < ib[r + 1] ? jb[e + 1] >> shift : -1;
+        const uint2 *mine = cells + (r >> 5);
+        const unsigned below = (1u << (r & 31)) - 1u;
+        bool first[BAND_SHIFT + 1], last[BAND_SHIFT + 1];
+        uint2 w[BAND_SHIFT + 1];
+#pragma unroll
+        for (int v = 0; v <= BAND_SHIFT; v++) {
+            first[v] = v < levels && (pb < 0 || (pb >> v) != (b >> v));
+            last[v] = v < levels && (nb < 0 || (nb >> v) != (b >> v));
+            w[v] = first[v] || last[v] ? mine[run_dir_block(nblk, shift, v, c) * ngrp]
+                                       : make_uint2(0u, 0u);
         }
-        __syncthreads();
+#pragma unroll
+        for (int v = 0; v <= BAND_SHIFT; v++) {
+            int2 *run = runs + w[v].y + __popc(w[v].x & below);
+            if (first[v] && last[v])
+                *run = make_int2(e, e + 1);
+            else if (first[v])
+                run->x = e;
+            else if (last[v])
+                run->y = e + 1;
+        }
     }
 }
 
 // ------------------------------------------------------------- item plan
-constexpr int SMALL_ITEM = 256;
-constexpr int MID_ITEM = 512;
+constexpr int ITEM_BOUND[ITEM_CLASSES] = {256, 512, ITEM_CAP};
+constexpr int SPARSE_CLASSES = 2;
 // Sparse stretches go into wide items of up to this many outputs.  R-MAT 2^20
 // with 8 draws a row, both sparse kernels: 31.7 ms without wide items (its
 // 30M items of <= 256 outputs hold 45 each, and each costs its A entries, two
-// block pointers an entry and its tables), 20.2 up to 256, 19.2 up to 384,
+// lookups an entry and its tables), 20.2 up to 256, 19.2 up to 384,
 // 19.3 up to 512; R-MAT 2^18 with 4: 1.27, 1.01, 0.98, 0.96; ER batch of 512:
 // 6.0, 5.9, 5.1, 4.3.
 constexpr int WIDE_CAP = 512;
-static_assert(WIDE_CAP <= MID_ITEM, "wide items run in the sparse kernels");
+static_assert(WIDE_CAP <= ITEM_BOUND[SPARSE_CLASSES - 1], "wide items run in the sparse kernels");
 
 // Split of each big row into items: the row's span is cut into windows of
 // WSB sub-blocks (at most ITEM_WBITS columns); inside a window, runs of
-// sub-blocks with at most ITEM_CAP outputs, leading empty sub-blocks skipped.
+// sub-blocks with at most ITEM_CAP outputs, empty sub-blocks at their ends left
+// out; with by_band aligned runs of 8, 4, 2 or 1 sub-blocks, which the run
+// directory of B has blocks for.
 // One wave per big row, one lane per window (64 windows per pass): a lane
 // loads its window's counts at once and splits them in registers, and wave
 // scans place the items and their outputs.  FILL=false counts items per
@@ -562,7 +683,7 @@ static_assert(WIDE_CAP <= MID_ITEM, "wide items run in the sparse kernels");
 // number at most wide_cap becomes one item (the longest such run).
 template <bool FILL, int WSB>
 __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__ rows, int k,
-                                               int wide_cap,
+                                               int by_band, int wide_cap,
                                                const int *__restrict__ span_sb0,
                                                const int64_t *__restrict__ sb_off,
                                                const uint16_t *__restrict__ subcnt,
@@ -583,43 +704,72 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
     const int row = rows[r];
     const uint16_t *sc = subcnt + sb_off[r];
     const int nsb = (int)(sb_off[r + 1] - sb_off[r]);
+    // windows are cut from the first band's start with by_band
+    const int lead = by_band ? band_lead(span_sb0[r]) : 0;
     const int first = span_sb0[r];
-    const int nwin = (nsb + WSB - 1) / WSB;
+    const int nwin = (lead + nsb + WSB - 1) / WSB;
     int64_t wbase = FILL ? item_cnt[r] : 0;
     int64_t obase = FILL ? ic[row] : 0;
     for (int w0 = 0; w0 < nwin; w0 += 64) {
         const int win = w0 + l;
-        const int j0 = win * WSB;
+        const int j0 = win * WSB - lead;
         const int len = win < nwin ? min(WSB, nsb - j0) : 0;
         int cs[WSB], os[WSB];
         int nzt = 0;
 #pragma unroll
         for (int q = 0; q < WSB; q++) {
-            cs[q] = q < len ? (int)sc[j0 + q] : 0;
-            os[q] = FILL && words && q < len ? __popc(subocc[sb_off[r] + j0 + q]) : 0;
+            const bool in = q < len && j0 + q >= 0;
+            cs[q] = in ? (int)sc[j0 + q] : 0;
+            os[q] = FILL && words && in ? __popc(subocc[sb_off[r] + j0 + q]) : 0;
             nzt += os[q];
         }
         int nit = 0, tot = 0, firstq = WSB, lastq = -1;
-        {
-            int start = -1, cnt = 0;
+#pragma unroll
+        for (int q = 0; q < WSB; q++) {
+            tot += cs[q];
+            if (cs[q] != 0) {
+                firstq = min(firstq, q);
+                lastq = q;
+            }
+        }
+        // ends[q]: an item ends with sub-block q
+        bool ends[WSB];
+        if (by_band) {
+            // halves, quarters, ... until a part has at most ITEM_CAP outputs
+            int part[WSB];
 #pragma unroll
             for (int q = 0; q < WSB; q++) {
-                if (start >= 0 && cnt + cs[q] > ITEM_CAP) {
-                    nit++;
-                    start = -1;
-                    cnt = 0;
-                }
-                if (cs[q] != 0 || start >= 0) {
-                    if (start < 0) start = q;
-                    cnt += cs[q];
-                }
-                tot += cs[q];
-                if (cs[q] != 0) {
-                    firstq = min(firstq, q);
-                    lastq = q;
+                part[q] = cs[q];
+                ends[q] = true;
+            }
+#pragma unroll
+            for (int z = 2; z <= WSB; z <<= 1) {
+#pragma unroll
+                for (int q = 0; q < WSB; q += z) {
+                    // both halves are whole (their sums fit) and so is the sum
+                    part[q] += part[q + z / 2];
+                    ends[q + z / 2 - 1] = part[q] > ITEM_CAP;
                 }
             }
-            if (start >= 0 && cnt > 0) nit++;
+        } else {
+            int cnt = 0;
+#pragma unroll
+            for (int q = 0; q < WSB; q++) {
+                cnt += cs[q];
+                ends[q] = q + 1 == WSB || cnt + cs[q + 1 < WSB ? q + 1 : q] > ITEM_CAP;
+                if (ends[q]) cnt = 0;
+            }
+        }
+        {
+            int cnt = 0;
+#pragma unroll
+            for (int q = 0; q < WSB; q++) {
+                cnt += cs[q];
+                if (ends[q]) {
+                    nit += cnt > 0;
+                    cnt = 0;
+                }
+            }
         }
         // the run of windows this one is in: its length, outputs, first and
         // last sub-block with outputs
@@ -662,13 +812,23 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                                    out, wb};
                 item_n[w] = run_tot;
             }
-            int start = -1, cnt = 0, nzrun = 0, nzs = 0;
+            // an item's columns: from its first sub-block with outputs to its last
+            int start = -1, stop = 0, cnt = 0, nzrun = 0, nzs = 0;
 #pragma unroll
             for (int q = 0; q < WSB; q++) {
                 if (run > 1) break;
-                if (start >= 0 && cnt + cs[q] > ITEM_CAP) {
+                if (cs[q] != 0) {
+                    if (start < 0) {
+                        start = q;
+                        nzs = nzrun;
+                    }
+                    stop = q + 1;
+                    cnt += cs[q];
+                }
+                nzrun += os[q];
+                if (ends[q] && cnt > 0) {
                     items[w] = ItemRec{make_int4(row, (cbase + start) << SUB_SHIFT,
-                                                 min(k, (cbase + q) << SUB_SHIFT),
+                                                 min(k, (cbase + stop) << SUB_SHIFT),
                                                  words ? (int)(sb_off[r] + j0 + start) : r),
                                        out, wb + nzs};
                     item_n[w] = cnt;
@@ -677,21 +837,6 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                     start = -1;
                     cnt = 0;
                 }
-                if (cs[q] != 0 || start >= 0) {
-                    if (start < 0) {
-                        start = q;
-                        nzs = nzrun;
-                    }
-                    cnt += cs[q];
-                }
-                nzrun += os[q];
-            }
-            if (run == 1 && start >= 0 && cnt > 0) {
-                items[w] = ItemRec{make_int4(row, (cbase + start) << SUB_SHIFT,
-                                             min(k, (cbase + len) << SUB_SHIFT),
-                                             words ? (int)(sb_off[r] + j0 + start) : r),
-                                   out, wb + nzs};
-                item_n[w] = cnt;
             }
         }
         wbase += group_last<64>(it_incl);
@@ -705,42 +850,54 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
 // items in this order, so the items in flight at any time gather B entries
 // of one narrow column band, which the L2 caches keep, instead of bands
 // spread over all of B.
-// Items sort by size class -- at most SMALL_ITEM outputs, at most MID_ITEM,
-// more -- then by first column: key = class << class_bit | first sub-block
-// (class_bit < 0: no classes).  The numeric phase runs each class in a
-// kernel whose value array holds just that class's items, so smaller items
-// take less LDS and more of them are resident.  block_small[b] and
-// block_mid[b] count block b's items of the first two classes.
-// Product batches in flight per lane and waves per SIMD of the two sparse
-// item kernels.  R-MAT 2^20 (8 draws a row), <= 256 outputs: 6.0 ms at (4, 6),
-// 5.8 at (6, 5) and (4, 7), 6.2 at (8, 5); <= 512: 13.3 at (6, 5), 12.7 at
-// (6, 4), 12.9 at (8, 4), 13.0 at (4, 5).
-constexpr int SMALL_RANK_U = 6;
-constexpr int SMALL_MINW = 5;
-constexpr int MID_RANK_U = 6;
-constexpr int MID_MINW = 4;
-
+// Items sort by size class (ITEM_BOUND), then by first column, after those of
+// rows of LONG_ROW entries or more: an item is one wave's work, so a class ends
+// no sooner than its longest item, which had better start first (R-MAT 2^18
+// times its transpose, items of <= 512 outputs 0.69 -> 0.56 ms).
+// key = class << class_bit + 1 | 1 << class_bit | first sub-block (a long
+// row's without the 1; class_bit < 0: the sub-block only).  The numeric phase
+// runs each class in a kernel whose tables hold just that class's items: the
+// waves an LDS holds set its speed.  R-MAT 2^20 with 8 draws a row: <= 256
+// outputs 5.8 -> 4.2 ms (4 batches in flight, 8 waves per SIMD; 6 batches: 4.7),
+// <= 512 12.8 -> 11.8 (at 4 waves).  Finer classes gained nothing there (384:
+// 4.2 + 7.5 ms; 768: 7.8 + 7.9 against 15.9) and cost R-MAT 2^18 a tail each.
+// class_cnt counts the items of each class but the last.
 __global__ void __launch_bounds__(256) k_item_keys(int64_t n, const ItemRec *__restrict__ items,
-                                                   const int *__restrict__ item_n, int class_bit,
+                                                   const int *__restrict__ item_n,
+                                                   const int *__restrict__ ia, int class_bit,
                                                    int *__restrict__ keys,
-                                                   int *__restrict__ block_small,
-                                                   int *__restrict__ block_mid) {
-    __shared__ int s_cnt[2][4];
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int cls = 0;
-    if (i < n && class_bit >= 0) cls = item_n[i] <= SMALL_ITEM ? 0 : item_n[i] <= MID_ITEM ? 1 : 2;
-    if (i < n) keys[i] = (cls << max(class_bit, 0)) | (items[i].d.y >> SUB_SHIFT);
-    const unsigned long long b0 = __ballot(i < n && class_bit >= 0 && cls == 0);
-    const unsigned long long b1 = __ballot(i < n && class_bit >= 0 && cls == 1);
-    if (__lane_id() == 0) {
-        s_cnt[0][threadIdx.x >> 6] = __popcll(b0);
-        s_cnt[1][threadIdx.x >> 6] = __popcll(b1);
-    }
+                                                   unsigned long long *__restrict__ class_cnt) {
+    constexpr int PER = 16, LONG_ROW = 1024;
+    __shared__ int s_cnt[ITEM_CLASSES - 1];
+    if (threadIdx.x < ITEM_CLASSES - 1) s_cnt[threadIdx.x] = 0;
     __syncthreads();
-    if (threadIdx.x < 2)
-        (threadIdx.x ? block_mid : block_small)[blockIdx.x] =
-            s_cnt[threadIdx.x][0] + s_cnt[threadIdx.x][1] + s_cnt[threadIdx.x][2] +
-            s_cnt[threadIdx.x][3];
+    int cnt[ITEM_CLASSES - 1] = {};
+    for (int q = 0; q < PER; q++) {
+        const int64_t i = ((int64_t)blockIdx.x * PER + q) * 256 + threadIdx.x;
+        int cls = ITEM_CLASSES - 1;
+        if (i < n) {
+            if (class_bit >= 0) {
+                const int outputs = item_n[i];
+#pragma unroll
+                for (int c = ITEM_CLASSES - 2; c >= 0; c--)
+                    if (outputs <= ITEM_BOUND[c]) cls = c;
+            }
+            const int4 d = items[i].d;
+            int key = d.y >> SUB_SHIFT;
+            if (class_bit >= 0) {
+                const bool other = ia[d.x + 1] - ia[d.x] < LONG_ROW;
+                key |= (2 * cls + (other ? 1 : 0)) << class_bit;
+            }
+            keys[i] = key;
+        }
+#pragma unroll
+        for (int c = 0; c < ITEM_CLASSES - 1; c++) cnt[c] += __popcll(__ballot(cls == c));
+    }
+    if (__lane_id() == 0)
+        for (int c = 0; c < ITEM_CLASSES - 1; c++) atomicAdd(&s_cnt[c], cnt[c]);
+    __syncthreads();
+    if (threadIdx.x < ITEM_CLASSES - 1 && s_cnt[threadIdx.x])
+        atomicAdd(class_cnt + threadIdx.x, (unsigned long long)s_cnt[threadIdx.x]);
 }
 
 __global__ void __launch_bounds__(256) k_gather_items(int64_t n, const int *__restrict__ order,
@@ -765,12 +922,11 @@ struct ItemSmem {
     int nid;
 };
 
-template <bool FUSED>
+template <bool FUSED, bool DIR>
 __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
     int64_t nitems, const ItemRec *__restrict__ items,
     const int *__restrict__ ia, const int *__restrict__ ja, const double *__restrict__ a,
-    const int *__restrict__ ib, const int *__restrict__ jb, const double *__restrict__ b,
-    BlockPtrs bp, int *__restrict__ jc,
+    const int *__restrict__ jb, const double *__restrict__ b, BRows brows, int *__restrict__ jc,
     double *__restrict__ c, int b_strict) {
     extern __shared__ __align__(16) unsigned char smem[];
     ItemSmem &S = reinterpret_cast<ItemSmem *>(smem)[threadIdx.x >> 6];
@@ -786,8 +942,9 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
         for (int i = l; i < nwords; i += 64) S.bits[i] = 0u;
         if (l == 0) S.nid = 0;
         wave_lds_fence();
-        for_products<ITEM_U, 1, true, true>(
-            ia[row], ia[row + 1], ja, a, ib, jb, b, bp, c0, c1, S.heads, [&](const Batch &t) {
+        for_products<ITEM_U, 1, true>(
+            ia[row], ia[row + 1], ja, a, ItemRange<DIR>(brows, jb, c0, c1), jb, b, S.heads,
+            [&](const Batch &t) {
                 int slot = -1;
                 if (t.act) {
                     bool created;
@@ -829,20 +986,29 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
     }
 }
 
+constexpr int RANK_SEGS = 8;           // entries of a batch added one after the other
+constexpr int RANK_TAGS = 128;         // tag buckets of the rank-indexed kernel
+
 // Rank-indexed variant: the symbolic phase stored every big row's column
 // bitmap (in sparse form: per sub-block a mask of its non-empty words, and
 // those words), so an item's outputs are known before its products are
-// visited.  The rank of column j inside the item is prefix[w] + popc(bits[w]
-// below j) -- one LDS read of a {bits, prefix} pair -- and values accumulate
+// visited.  The rank of column j inside the item is pre[w] + popc(bits[w]
+// below j), and values accumulate
 // in a dense rank-ordered array that is written out coalesced.
 // WORDS: bitmap words of the widest item (256 or 512: items of 8192 or
 // 16384 columns).
+// 10048 bytes at 8192 columns: 16 waves a CU.  Their number sets the kernel's
+// speed, the latency of a group's loads and LDS turns its bound: R-MAT 2^20
+// with 8 draws a row, 26.8 ms at 10 waves, 22.5 at 12, 18.6 at 14 (pairs of
+// words and prefixes, 256 tags), 16.5 now, with both reads of a tag round in
+// one wait.
 template <int WORDS>
 struct RankSmem {
-    uint2 words[WORDS];           // {bitmap word, outputs before it}
     double vals[ITEM_CAP];
-    unsigned tags[ITEM_TAGS];     // bucketed by rank
-    int heads[64];                // start bits of the product expansion
+    uint2 bits[WORDS / 2];        // 64 columns each
+    uint16_t pre[WORDS / 2];      // outputs before them
+    unsigned tags[RANK_TAGS];     // bucketed by rank
+    int heads[2 * RANK_U];        // start bits of the product expansion
 };
 
 // Rank table of one item, in two parts so that other loads can be issued
@@ -883,8 +1049,8 @@ __device__ __forceinline__ void item_words(const unsigned *__restrict__ list, un
 }
 
 template <int WORDS, int WCH = WORDS / 64>
-__device__ __forceinline__ int item_rank_build(RankSmem<WORDS> &S, unsigned (&wv)[WCH], int c0,
-                                               int c1, int64_t o, int *__restrict__ jc) {
+__device__ __forceinline__ int item_rank_build(RankSmem<WORDS> &S, unsigned (&wv)[WCH],
+                                               int c0, int c1, int64_t o, int *__restrict__ jc) {
     const int l = __lane_id();
     const int nwords = (c1 - c0 + 31) >> 5;
     // the 64-word chunks are scanned independently
@@ -903,7 +1069,10 @@ __device__ __forceinline__ int item_rank_build(RankSmem<WORDS> &S, unsigned (&wv
     for (int j = 0; j < WCH; j++) {
         const int w = j * 64 + l;
         const int base = cnt + incl[j] - __popc(wv[j]);
-        if (w < nwords) S.words[w] = make_uint2(wv[j], (unsigned)base);
+        if (w < nwords) {
+            reinterpret_cast<unsigned *>(S.bits)[w] = wv[j];
+            if (!(w & 1)) S.pre[w >> 1] = (uint16_t)base;
+        }
         unsigned word = wv[j];
         int pos = base;
         while (word) {
@@ -941,126 +1110,61 @@ __device__ __forceinline__ void item_accumulate(RankSmem<WORDS> &S, int c0, cons
     int rank = -1;
     if (t.act) {
         const int cc = t.col - c0;
-        const uint2 wd = S.words[cc >> 5];
-        rank = (int)wd.y + __popc(wd.x & ((1u << (cc & 31)) - 1u));
+        const uint2 wd = S.bits[cc >> 6];
+        const unsigned below = (1u << (cc & 31)) - 1u;
+        rank = (int)S.pre[cc >> 6] + __popc(wd.x & (cc & 32 ? ~0u : below)) +
+               __popc(wd.y & (cc & 32 ? below : 0u));
     }
-    if (b_strict && t.nseg <= FLAT_SEGS) {
+    if (b_strict && t.nseg <= RANK_SEGS) {
         for (int s = 1; s <= t.nseg; s++) {
             if (rank >= 0 && t.seg == s) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
             wave_lds_fence();
         }
         return;
     }
-    ordered_accumulate<FUSED, ITEM_TAGS>(rank >= 0, rank, t.a, t.b, S.vals, S.tags,
+    ordered_accumulate<FUSED, RANK_TAGS>(rank >= 0, rank, t.a, t.b, S.vals, S.tags,
                                          (unsigned)__lane_id(), false);
 }
 
-template <bool FUSED, int WORDS>
-__global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric_rank(
+template <bool FUSED, int WORDS, bool DIR>
+__global__ void __launch_bounds__(64) k_big_numeric_rank(
     int64_t nitems, const ItemRec *__restrict__ items, const unsigned *__restrict__ wlist,
     const unsigned *__restrict__ subocc, const int *__restrict__ ia, const int *__restrict__ ja,
-    const double *__restrict__ a, const int *__restrict__ jb, const double *__restrict__ b,
-    const int4 *__restrict__ bpk, BlockPtrs bp, int *__restrict__ jc, double *__restrict__ c,
-    int b_strict) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    RankSmem<WORDS> &S = reinterpret_cast<RankSmem<WORDS> *>(smem)[threadIdx.x >> 6];
-    const int l = __lane_id();
-    for (int i = l; i < ITEM_TAGS; i += 64) S.tags[i] = 0xffffffffu;
-    const int64_t wave_id = (int64_t)blockIdx.x * ITEM_WAVES + (threadIdx.x >> 6);
-    const int64_t nwaves = (int64_t)gridDim.x * ITEM_WAVES;
-    // the next item's descriptor is loaded when an item starts, and its
-    // sub-block masks, word-list position and A row bounds while the item's
-    // outputs are stored, so an item's first product loads need no chain of
-    // dependent loads.  Those and the item's output offset go into one
-    // register, a lane each (lanes 0..15 the masks, 16 and 17 the position,
-    // 18 and 19 the row bounds, 20 and 21 the offset: one load instruction,
-    // and they reach scalar registers at the item's start -- the small-item
-    // kernel has no vector registers to spare).
-    int4 item = make_int4(0, 0, 0, 0);
-    unsigned nx = 0u;
-    auto locate = [&](int64_t at) {
+    const double *__restrict__ a, const int *__restrict__ jb, const int4 *__restrict__ bpk, BRows brows,
+    int *__restrict__ jc, double *__restrict__ c, int b_strict) {
+    __shared__ RankSmem<WORDS> S;
+    const int l = threadIdx.x;
+    for (int i = l; i < RANK_TAGS; i += 64) S.tags[i] = 0xffffffffu;
+    for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const int4 item = items[it].d;
+        const int64_t o = items[it].off;
+        const unsigned *list = wlist + items[it].wpos;
+        const int c0 = item.y, c1 = item.z;
+        // the rank table is built after the first groups' A entries and cells
+        // are issued, so the word loads and that chain of loads overlap
+        const ItemRange<DIR> range(brows, jb, c0, c1);
+        EntryPipe<true, 1> pipe;
+        pipe.ja = ja;
+        pipe.aval = a;
+        pipe.part = 0;
+        pipe.load(ia[item.x], ia[item.x + 1]);
         // item.w: the item's first sub-block in subocc
-        const int nsb = (item.z - item.y + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT;
-        const unsigned *src = nullptr;
-        if (l < min(nsb, 2 * (WORDS / 64)))
-            src = subocc + ((int64_t)item.w + l);
-        else if (l == 16 || l == 17)
-            src = reinterpret_cast<const unsigned *>(&items[at].wpos) + (l - 16);
-        else if (l == 18 || l == 19)
-            src = reinterpret_cast<const unsigned *>(ia + item.x) + (l - 18);
-        else if (l == 20 || l == 21)
-            src = reinterpret_cast<const unsigned *>(&items[at].off) + (l - 20);
-        nx = src ? *src : 0u;
-    };
-    // (streaming loads of the item descriptors and A entries, read once per
-    // item, were measured slower: 158 -> 166 ms on R-MAT 2^20 A*A^T)
-    if (wave_id < nitems) {
-        item = items[wave_id].d;
-        locate(wave_id);
-    }
-    for (int64_t it = wave_id; it < nitems; it += nwaves) {
-        const int c0 = __builtin_amdgcn_readfirstlane(item.y);
-        const int c1 = __builtin_amdgcn_readfirstlane(item.z);
-        const unsigned iocc = l < 16 ? nx : 0u;
-        const int ipa = __builtin_amdgcn_readlane((int)nx, 18);
-        const int ipe = __builtin_amdgcn_readlane((int)nx, 19);
-        const int64_t iwpos =
-            (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)nx, 17) << 32) |
-                      (uint32_t)__builtin_amdgcn_readlane((int)nx, 16));
-        const unsigned *ilist = wlist + iwpos;
-        const int64_t o =
-            (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)nx, 21) << 32) |
-                      (uint32_t)__builtin_amdgcn_readlane((int)nx, 20));
-        const int64_t next = it + nwaves;
-        if (next < nitems) item = items[next].d;
-        // the product pipeline of for_products, with the rank table built
-        // after the first groups' A entries and B ranges are issued, so the
-        // word loads and that chain of dependent loads overlap
-        auto load_t = [&](int g, int &t, double &av) {
-            const int p = g + l;
-            t = -1;
-            av = 0.0;
-            if (g < ipe && p < ipe) {
-                t = ja[p];
-                av = a[p];
-            }
-        };
-        auto load_range = [&](int t, int &lo, int &hi) {
-            lo = 0;
-            hi = 0;
-            if (t >= 0) {
-                lo = brange_lo(bp, jb, t, c0);
-                hi = brange_lo(bp, jb, t, c1);
-            }
-        };
-        int t0, t1;
-        double a0, a1;
-        load_t(ipa, t0, a0);
-        load_t(ipa + 64, t1, a1);
-        const int pc = __popc(iocc);
+        const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 2 * (WORDS / 64));
+        const unsigned occ = l < nsb ? subocc[(int64_t)item.w + l] : 0u;
+        pipe.cells(range);
+        const int pc = __popc(occ);
         const int pre = dpp_incl_scan<16>(pc) - pc;
         unsigned wv[WORDS / 64];
-        item_words(ilist, iocc, pre, c0, c1, wv);
-        int lo, hi;
-        load_range(t0, lo, hi);
-        const int cnt = item_rank_build<WORDS>(S, wv, c0, c1, o, jc);
-        auto f = [&](const Batch &t) {
-            item_accumulate<FUSED, WORDS>(S, c0, t, b_strict);
-        };
-        for (int g = ipa; g < ipe; g += 64) {
-            const double ag = a0;
-            int lo_n, hi_n, t2;
-            double a2;
-            load_range(t1, lo_n, hi_n);
-            load_t(g + 128, t2, a2);
-            expand_group<RANK_U, true, true>(lo, max(hi - lo, 0), ag, jb, b, S.heads, f, bpk);
-            lo = lo_n;
-            hi = hi_n;
-            t1 = t2;
-            a0 = a1;
-            a1 = a2;
+        item_words(list, occ, pre, c0, c1, wv);
+        pipe.first(range);
+        const int cnt = item_rank_build(S, wv, c0, c1, o, jc);
+        auto f = [&](const Batch &t) { item_accumulate<FUSED>(S, c0, t, b_strict); };
+        for (int g = pipe.pa; g < pipe.pe; g += 64) {
+            pipe.ahead(g, range);
+            expand_group<RANK_U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, jb,
+                                             nullptr, S.heads, f, bpk);
+            pipe.take();
         }
-        if (next < nitems) locate(next);
         item_store_values(S, cnt, o, c);
     }
 }
@@ -1073,28 +1177,30 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric_rank(
 //
 // The dense tables it replaces for these items cost ~500 vector instructions
 // an item whatever its products (the issue rate bound them: 25 of 29 ms of
-// R-MAT 2^20 with 8 draws a row); now 5.8 ms, with the 257..512-output items
-// 37.7 -> 18.5 ms.  Larger items keep the dense table: one lookup a product,
-// and they run at the memory's rate (4.65 TB/s).
-template <int CAP>
+// R-MAT 2^20 with 8 draws a row); with the sparse tables those and the items of
+// 257..512 outputs went from 37.7 to 18.5 ms, and to 16.0 with the run directory
+// and tables of half the size.  Bound by latency, so by the waves an LDS holds.
+// Larger items keep the dense table: one lookup a product.
+template <int CAP, int U>
 struct SparseSmem {
-    uint2 words[CAP];             // {bits, outputs before}
     double vals[CAP];
+    unsigned words[CAP];          // the item's words
+    uint16_t pre[CAP];            // outputs before them
     uint2 sub[1 << BAND_SHIFT];   // {mask of non-empty words, words before}
     uint16_t cols[CAP];
     unsigned tags[CAP / 4];       // a byte per output, or tag buckets
-    int heads[64];
+    int heads[2 * U];
 };
 
-template <bool FUSED, int CAP, int U, int MINW>
+template <bool FUSED, int CAP, int U, int MINW, bool DIR>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MINW)))
 k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
                      const unsigned *__restrict__ wlist, const unsigned *__restrict__ subocc,
                      const int *__restrict__ ia, const int *__restrict__ ja,
                      const double *__restrict__ a, const int *__restrict__ jb,
-                     const int4 *__restrict__ bpk, BlockPtrs bp, int *__restrict__ jc,
+                     const int4 *__restrict__ bpk, BRows brows, int *__restrict__ jc,
                      double *__restrict__ c, int b_strict) {
-    __shared__ __align__(16) SparseSmem<CAP> S;
+    __shared__ __align__(16) SparseSmem<CAP, U> S;
     constexpr int NT = CAP / 4;
     const int l = threadIdx.x;
     uint8_t *own = reinterpret_cast<uint8_t *>(S.tags);
@@ -1103,29 +1209,15 @@ k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
         const int64_t o = items[it].off;
         const unsigned *list = wlist + items[it].wpos;
         const int c0 = item.y, c1 = item.z;
-        const int pa = ia[item.x], pe = ia[item.x + 1];
+        const ItemRange<DIR> range(brows, jb, c0, c1);
+        EntryPipe<true, 1> pipe;
+        pipe.ja = ja;
+        pipe.aval = a;
+        pipe.part = 0;
+        pipe.load(ia[item.x], ia[item.x + 1]);
         const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 1 << BAND_SHIFT);
         const unsigned occ = l < nsb ? subocc[(int64_t)item.w + l] : 0u;
-        auto load_t = [&](int g, int &t, double &av) {
-            const int p = g + l;
-            t = -1;
-            av = 0.0;
-            if (p < pe) {
-                t = ja[p];
-                av = a[p];
-            }
-        };
-        auto load_range = [&](int t, int &lo, int &hi) {
-            lo = 0;
-            hi = 0;
-            if (t >= 0) {
-                lo = brange_lo(bp, jb, t, c0);
-                hi = brange_lo(bp, jb, t, c1);
-            }
-        };
-        int t0, lo, hi;
-        double a0;
-        load_t(pa, t0, a0);
+        pipe.cells(range);
         const int pc = __popc(occ);
         const int incl = wave_incl_scan(pc);
         // every non-empty word has an output
@@ -1134,7 +1226,7 @@ k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
 #pragma unroll
         for (int j = 0; j < CAP / 64; j++)
             wv[j] = j * 64 + l < nw ? __builtin_nontemporal_load(list + j * 64 + l) : 0u;
-        load_range(t0, lo, hi);
+        pipe.first(range);
         S.sub[l] = make_uint2(occ, (unsigned)(incl - pc));
         int cnt = 0;
 #pragma unroll
@@ -1142,8 +1234,10 @@ k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
             if (j * 64 < nw) {
                 const int p = __popc(wv[j]);
                 const int in = wave_incl_scan(p);
-                if (j * 64 + l < nw)
-                    S.words[j * 64 + l] = make_uint2(wv[j], (unsigned)(cnt + in - p));
+                if (j * 64 + l < nw) {
+                    S.words[j * 64 + l] = wv[j];
+                    S.pre[j * 64 + l] = (uint16_t)(cnt + in - p);
+                }
                 cnt += __builtin_amdgcn_readlane(in, 63);
             }
         }
@@ -1155,9 +1249,10 @@ k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
             if (t.act) {
                 const int cc = t.col - c0;
                 const uint2 sb = S.sub[(cc >> SUB_SHIFT) & ((1 << BAND_SHIFT) - 1)];
-                const int w = (int)sb.y + (int)__popc(sb.x & ((1u << ((cc >> 5) & 31)) - 1u));
-                const uint2 wd = S.words[min(w, CAP - 1)];
-                rank = min((int)wd.y + (int)__popc(wd.x & ((1u << (cc & 31)) - 1u)), CAP - 1);
+                const int w = min(
+                    (int)sb.y + (int)__popc(sb.x & ((1u << ((cc >> 5) & 31)) - 1u)), CAP - 1);
+                rank = min((int)S.pre[w] + (int)__popc(S.words[w] & ((1u << (cc & 31)) - 1u)),
+                           CAP - 1);
                 S.cols[rank] = (uint16_t)cc;
             }
             bool clash = t.nseg > 1 || !b_strict;
@@ -1182,15 +1277,11 @@ k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
                                               false);
             }
         };
-        for (int g = pa; g < pe; g += 64) {
-            int t1, lo_n, hi_n;
-            double a1;
-            load_t(g + 64, t1, a1);
-            load_range(t1, lo_n, hi_n);
-            expand_group<U, true, true>(lo, max(hi - lo, 0), a0, jb, nullptr, S.heads, f, bpk);
-            lo = lo_n;
-            hi = hi_n;
-            a0 = a1;
+        for (int g = pipe.pa; g < pipe.pe; g += 64) {
+            pipe.ahead(g, range);
+            expand_group<U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, jb, nullptr,
+                                        S.heads, f, bpk);
+            pipe.take();
         }
         wave_lds_fence();
         for (int i = l; i < cnt; i += 64) {
@@ -1212,24 +1303,15 @@ __global__ void __launch_bounds__(256) k_pack_b(int64_t nnz, const int *__restri
     bpk[q] = make_int4(jb[q], 0, __double2loint(v), __double2hiint(v));
 }
 
-// The plan's block pointers in the layout they were built in; without a
-// table, B's row pointers b_ptr (of the call at hand) as a one-block table.
-static BlockPtrs block_ptrs(const RowPlan &p, const int *b_ptr) {
-    BlockPtrs bp;
-    bp.p = p.bptr;
-    bp.bs = p.blk_shift;
-    if (p.bptr_rowptr) {
-        bp.p = b_ptr;
-        bp.tstride = 1;
-        bp.bstride = 1;
-    } else if (p.column_order) {
-        bp.tstride = 1;
-        bp.bstride = p.n;
-    } else {
-        bp.tstride = p.nblk + 1;
-        bp.bstride = 1;
-    }
-    return bp;
+// The plan's run directory or block pointers; without either, B's row pointers
+// b_ptr (of the call at hand) as a one-block table.
+static BRows b_rows(const RowPlan &p, const int *b_ptr) {
+    BRows r;
+    r.dir = p.dir;
+    r.bp.p = p.bptr ? p.bptr : b_ptr;
+    r.bp.tstride = p.bptr ? p.nblk + 1 : 1;
+    r.bp.bs = p.bptr ? p.blk_shift : 30;
+    return r;
 }
 
 // One block per item (the hardware dispatcher hands the next item to
@@ -1310,10 +1392,10 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
                            p.nbig, rowsb, A.ptr, A.idx, B.ptr, B.idx, front.rowprod, p.span_sb0,
                            p.sb_off, a_ent, a_prod, row_loff);
         TSG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_band_count, dim3(grid_for((size_t)p.nbig, 256)), dim3(256), 0, s,
-                           p.nbig, p.sb_off, band_off);
-        TSG_LAUNCH_CHECK();
         exclusive_scan_i64(p.sb_off, p.sb_off, (size_t)p.nbig, tmp_sb, s);
+        hipLaunchKernelGGL(k_band_count, dim3(grid_for((size_t)p.nbig, 256)), dim3(256), 0, s,
+                           p.nbig, tune.item_sort_min, p.span_sb0, p.sb_off, band_off);
+        TSG_LAUNCH_CHECK();
         exclusive_scan_i64(band_off, band_off, (size_t)p.nbig, tmp_sb, s);
         exclusive_scan_i64(a_ent, a_ent, (size_t)p.nbig, tmp_sb, s);
         exclusive_scan_i64(a_prod, a_prod, (size_t)p.nbig, tmp_sb, s);
@@ -1355,14 +1437,19 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         p.bpk = p.use_rank ? ws.alloc_n<int4>((size_t)B.nnz + 1) : nullptr;
         // Spans this wide (at least item_sort_min windows of 16 sub-blocks)
         // make enough bands and items for them to run in column order, which
-        // a radix sort arranges; the block pointers are then laid out block
-        // major and the items are 8 sub-blocks wide.
+        // a radix sort arranges; B is then cut by its run directory and the
+        // items are at most 8 sub-blocks wide, or sparse.
         p.column_order = nsb_total / 16 >= tune.item_sort_min;
         tm.end();
 
-        // B block pointers at the sub-block width (item and band boundaries
-        // then need no search) while the table stays <= 6 GiB, coarser beyond.
-        // No table at all when building it would cost more than the searches
+        // Column order: the run directory of B (R-MAT 2^20 with 8 draws a row:
+        // 1.4 ms to build and 1.5 GB; the block pointers it replaces 3.3 ms
+        // and 4.3 GB, and the numeric phase waited for them half its time, on
+        // 390M of its 800M L2 misses in items of more than 512 outputs).  Rows'
+        // order: B block pointers at the sub-block width (item and band
+        // boundaries then need no search).  Either with finest blocks of 1024
+        // columns while it stays <= 6 GiB, coarser beyond (a directory that
+        // does not fit at all: a search).  Neither when building it would cost more than the searches
         // it saves -- more than 8 max(1, log2(L / 16)) entries per (A entry,
         // window of 16 sub-blocks) pair of the big rows, with the pairs
         // estimated from their A entries and average span and L, the mean
@@ -1380,27 +1467,67 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
             (double)n * (double)((((size_t)k + (1u << SUB_SHIFT) - 1) >> SUB_SHIFT) + 1);
         const double pairs = (double)tot2[2] * ((double)nsb_total / (16.0 * p.nbig) + 1.0);
         const double brow = tot2[2] > 0 ? (double)tot2[3] / (double)tot2[2] : 1.0;
-        p.bptr_rowptr = k <= (1 << 30) &&
+        const bool rowptr = k <= (1 << 30) &&
                         (tune.bptr_budget == 0 ||
                          (tune.bptr_budget < 0 &&
                           fine_entries > 8.0 * pairs * std::max(1.0, std::log2(brow / 16.0))));
-        int bs = SUB_SHIFT;
-        while (bs < 30) {
-            size_t nblk = ((size_t)k + (1u << bs) - 1) >> bs;
-            if ((size_t)n * (nblk + 1) * sizeof(int) <= bptr_cap) break;
-            bs++;
+        p.dir = RunDir();
+        p.bptr = nullptr;
+        bool table = !rowptr && n > 0;
+        if (table && p.column_order) {
+            // finest blocks of 1 << shift columns, coarser until cells (12
+            // bytes each with the bits they are built from) and runs fit
+            const int ngrp = (n + 31) / 32;
+            const int nband = (int)(((size_t)k + (1u << (SUB_SHIFT + BAND_SHIFT)) - 1) >>
+                                    (SUB_SHIFT + BAND_SHIFT));
+            for (int c = 0; c <= BAND_SHIFT && !p.dir.cells; c++) {
+                const int levels = BAND_SHIFT + 1 - c;
+                const int64_t nblk = (int64_t)nband << (BAND_SHIFT - c);
+                const int64_t ncells = (2 * nblk - (2 * nblk >> levels)) * ngrp;
+                const int64_t chunks = (ncells + DIR_CHUNK - 1) / DIR_CHUNK;
+                const int64_t max_runs = levels * (int64_t)B.nnz;
+                const size_t bytes = (size_t)chunks * (DIR_CHUNK * 12 + 8) + (size_t)max_runs * 8;
+                if (bytes > bptr_cap || max_runs >= (int64_t(1) << 31) ||
+                    nblk >= (int64_t(1) << 30) || chunks >= (int64_t(1) << 31))
+                    continue;
+                unsigned *bits = ws.alloc_n<unsigned>((size_t)chunks * DIR_CHUNK);
+                uint2 *cells = ws.alloc_n<uint2>((size_t)chunks * DIR_CHUNK);
+                int2 *runs = ws.alloc_n<int2>((size_t)max_runs + 1);
+                int64_t *sums = ws.alloc_n<int64_t>((size_t)chunks + 1);
+                int64_t *tmp = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)chunks + 1));
+                p.dir.cells = cells;
+                p.dir.runs = runs;
+                p.dir.ngrp = ngrp;
+                p.dir.nblk = (int)nblk;
+                p.dir.shift = SUB_SHIFT + c;
+                p.dir.coarse = c > 0;
+                hipLaunchKernelGGL(k_dir_bits, dim3(grid_for((size_t)n, DIR_ROWS)), dim3(1024), 0,
+                                   s, n, B.ptr, B.idx, ngrp, p.dir.nblk, p.dir.shift, levels, bits);
+                TSG_LAUNCH_CHECK();
+                hipLaunchKernelGGL(k_dir_sums, dim3((unsigned)chunks), dim3(256), 0, s, ncells,
+                                   bits, sums);
+                TSG_LAUNCH_CHECK();
+                exclusive_scan_i64(sums, sums, (size_t)chunks, tmp, s);
+                hipLaunchKernelGGL(k_dir_cells, dim3((unsigned)chunks), dim3(256), 0, s, ncells,
+                                   bits, sums, cells);
+                TSG_LAUNCH_CHECK();
+                hipLaunchKernelGGL(k_dir_runs, dim3(grid_for((size_t)B.nnz, RUN_ENT)), dim3(256), 0,
+                                   s, n, (int)B.nnz, B.ptr, B.idx, ngrp, p.dir.nblk, p.dir.shift, levels,
+                                   cells, runs);
+                TSG_LAUNCH_CHECK();
+            }
+            table = !p.dir.cells && k > (1 << 30);
         }
-        if (p.bptr_rowptr) bs = 30;
-        p.blk_shift = bs;
-        p.nblk = (int)(((size_t)k + (1u << bs) - 1) >> bs);
-        p.bptr = p.bptr_rowptr ? nullptr : ws.alloc_n<int>((size_t)n * (p.nblk + 1));
-        if (p.bptr_rowptr) {
-            // nothing to build
-        } else if (n > 0 && p.column_order) {
-            hipLaunchKernelGGL(k_bptr, dim3(grid_for((size_t)n, BPT_ROWS)), dim3(256), 0, s, n,
-                               B.ptr, B.idx, p.nblk, bs, p.bptr);
-            TSG_LAUNCH_CHECK();
-        } else if (n > 0) {
+        if (table) {
+            int bs = SUB_SHIFT;
+            while (bs < 30) {
+                size_t nblk = ((size_t)k + (1u << bs) - 1) >> bs;
+                if ((size_t)n * (nblk + 1) * sizeof(int) <= bptr_cap) break;
+                bs++;
+            }
+            p.blk_shift = bs;
+            p.nblk = (int)(((size_t)k + (1u << bs) - 1) >> bs);
+            p.bptr = ws.alloc_n<int>((size_t)n * (p.nblk + 1));
             hipLaunchKernelGGL(k_bptr_rows, dim3(grid_for((size_t)n * 64, 256)), dim3(256), 0,
                                s, n, B.ptr, B.idx, p.nblk, bs, p.bptr);
             TSG_LAUNCH_CHECK();
@@ -1424,10 +1551,11 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
             TSG_LAUNCH_CHECK();
             units = sorted;
         }
-        hipLaunchKernelGGL(k_big_symbolic,
+        auto symbolic = p.dir.cells ? k_big_symbolic<true> : k_big_symbolic<false>;
+        hipLaunchKernelGGL(symbolic,
                            dim3((unsigned)std::min<int64_t>(nunits, int64_t(1) << 30)),
-                           dim3(BAND_T), 0, s, nunits, units, rowsb, k, A.ptr, A.idx, B.ptr,
-                           B.idx, block_ptrs(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, front.rownnz,
+                           dim3(BAND_T), 0, s, nunits, units, rowsb, k, (int)p.column_order, A.ptr,
+                           A.idx, B.idx, b_rows(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, front.rownnz,
                            band_off, band_base, row_cur, row_loff, d_overflow, p.subocc,
                            p.bandwords);
         TSG_LAUNCH_CHECK();
@@ -1452,20 +1580,25 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         p.narrow_items = narrow;
         // sparse stretches in wide items, for the kernel whose work and LDS
         // follow the outputs, not the columns (rank mode, by size class)
-        const int wide_cap = narrow && p.use_rank ? WIDE_CAP : 0;
+        int wide_cap = narrow && p.use_rank ? WIDE_CAP : 0;
         auto items_kernel = [&](auto kern, int64_t *cnt, ItemRec *it, int *itn) {
             hipLaunchKernelGGL(kern, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0, s,
-                               p.nbig, rowsb, k, wide_cap, p.span_sb0, p.sb_off, p.subcnt, d_ic, cnt, it,
+                               p.nbig, rowsb, k, (int)narrow, wide_cap, p.span_sb0, p.sb_off, p.subcnt, d_ic, cnt, it,
                                itn, p.subocc, band_off, band_base);
             TSG_LAUNCH_CHECK();
         };
-        if (narrow)
-            items_kernel(k_items<false, 8>, p.item_cnt, nullptr, nullptr);
-        else
-            items_kernel(k_items<false, 16>, p.item_cnt, nullptr, nullptr);
-        exclusive_scan_i64(p.item_cnt, p.item_cnt, (size_t)p.nbig, tmp2, s);
-        publish_i64({{p.item_cnt + p.nbig, d_overflow}}, d_overflow ? 2 : 1, box, s);
-        TSG_HIP_TRY(hipStreamSynchronize(s));
+        while (true) {
+            if (narrow)
+                items_kernel(k_items<false, 8>, p.item_cnt, nullptr, nullptr);
+            else
+                items_kernel(k_items<false, 16>, p.item_cnt, nullptr, nullptr);
+            exclusive_scan_i64(p.item_cnt, p.item_cnt, (size_t)p.nbig, tmp2, s);
+            publish_i64({{p.item_cnt + p.nbig, d_overflow}}, d_overflow ? 2 : 1, box, s);
+            TSG_HIP_TRY(hipStreamSynchronize(s));
+            // more than can be sorted by class: none for the sparse kernels
+            if (wide_cap == 0 || box->v[0] < (int64_t(1) << 31)) break;
+            wide_cap = 0;
+        }
         h_tot[0] = box->v[7];
         h_tot[1] = box->v[0];
         const int64_t h_overflow = d_overflow ? box->v[1] : 0;
@@ -1479,36 +1612,32 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
             items_kernel(k_items<true, 8>, p.item_cnt, p.items, item_n);
         else
             items_kernel(k_items<true, 16>, p.item_cnt, p.items, item_n);
-        p.nitems_small = 0;
-        p.nitems_mid = 0;
-        if (p.column_order && p.nitems > 1 && p.nitems < (int64_t(1) << 31)) {
+        p.class_end[ITEM_CLASSES - 1] = p.nitems;
+        if (p.column_order && p.nitems > 0 && p.nitems < (int64_t(1) << 31)) {
             const size_t ni = (size_t)p.nitems;
             int *keys = ws.alloc_n<int>(ni);
             int *order = ws.alloc_n<int>(ni);
-            const unsigned kblocks = grid_for(ni, 256);
-            int *bsmall = ws.alloc_n<int>((size_t)kblocks + 1);
-            int *bmid = ws.alloc_n<int>((size_t)kblocks + 1);
-            int64_t *tmpk = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)kblocks + 1));
-            int64_t *d_small = ws.alloc_n<int64_t>(2);
+            unsigned long long *class_cnt = ws.alloc_n<unsigned long long>(ITEM_CLASSES);
+            TSG_HIP_TRY(hipMemsetAsync(class_cnt, 0, sizeof(int64_t) * ITEM_CLASSES, s));
             int end_bit = 1;
-            while (end_bit < 29 && (int64_t(1) << end_bit) <= ((int64_t)k >> SUB_SHIFT)) end_bit++;
+            while (end_bit < 27 && (int64_t(1) << end_bit) <= ((int64_t)k >> SUB_SHIFT)) end_bit++;
             // the size class splits the rank path's items only
-            hipLaunchKernelGGL(k_item_keys, dim3(kblocks), dim3(256), 0, s, p.nitems,
-                               p.items, item_n, p.use_rank ? end_bit : -1, keys, bsmall, bmid);
+            hipLaunchKernelGGL(k_item_keys, dim3(grid_for(ni, 256 * 16)), dim3(256), 0, s,
+                               p.nitems, p.items, item_n, A.ptr, p.use_rank ? end_bit : -1, keys,
+                               class_cnt);
             TSG_LAUNCH_CHECK();
-            exclusive_scan_i32(bsmall, bsmall, (size_t)kblocks, tmpk, s, d_small);
-            exclusive_scan_i32(bmid, bmid, (size_t)kblocks, tmpk, s, d_small + 1);
-            sort_order_i32(keys, p.nitems, p.use_rank ? end_bit + 2 : end_bit, order, ws, s);
+            sort_order_i32(keys, p.nitems, p.use_rank ? end_bit + 4 : end_bit, order, ws, s);
             ItemRec *items_s = ws.alloc_n<ItemRec>(ni + 1);
             hipLaunchKernelGGL(k_gather_items, dim3(grid_for(ni, 256)), dim3(256), 0, s,
                                p.nitems, order, p.items, items_s);
             TSG_LAUNCH_CHECK();
             p.items = items_s;
             if (p.use_rank) {
-                publish_i64({{d_small, d_small + 1}}, 2, box, s);
+                const int64_t *cc = reinterpret_cast<const int64_t *>(class_cnt);
+                publish_i64({{cc, cc + 1}}, ITEM_CLASSES - 1, box, s);
                 TSG_HIP_TRY(hipStreamSynchronize(s));
-                p.nitems_small = box->v[0];
-                p.nitems_mid = box->v[0] + box->v[1];
+                int64_t end = 0;
+                for (int c = 0; c < ITEM_CLASSES - 1; c++) p.class_end[c] = end += box->v[c];
             }
         }
         tm.end();
@@ -1548,47 +1677,38 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
                                B.nnz, B.idx, B.val, p.bpk);
             TSG_LAUNCH_CHECK();
         }
-        auto launch_rank = [&](auto kern, size_t sm, int64_t i0, int64_t i1) {
-            if (i1 <= i0) return;
-            set_smem(kern, sm);
-            const unsigned grid = item_grid(i1 - i0);
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * ITEM_WAVES), sm, s, i1 - i0,
-                               p.items + i0, p.bandwords, p.subocc, A.ptr, A.idx, A.val, B.idx, B.val, p.bpk, block_ptrs(p, B.ptr),
-                               d_jc, d_c, (int)p.b_strict);
-            TSG_LAUNCH_CHECK();
-        };
-        // the size classes (sorted in this order) in kernels with value
-        // arrays of their size
-        const int64_t ns = p.nitems_small, nm = std::max(p.nitems_mid, ns);
-        auto launch_sparse = [&](auto kern, int64_t i0, int64_t i1) {
+        auto launch = [&](auto kern, int64_t i0, int64_t i1) {
             if (i1 <= i0) return;
             hipLaunchKernelGGL(kern, dim3(item_grid(i1 - i0)), dim3(64), 0, s, i1 - i0,
                                p.items + i0, p.bandwords, p.subocc, A.ptr, A.idx, A.val, B.idx,
-                               p.bpk, block_ptrs(p, B.ptr), d_jc, d_c, (int)p.b_strict);
+                               p.bpk, b_rows(p, B.ptr), d_jc, d_c, (int)p.b_strict);
             TSG_LAUNCH_CHECK();
         };
-        launch_sparse(k_big_numeric_sparse<FUSED, SMALL_ITEM, SMALL_RANK_U, SMALL_MINW>, 0, ns);
-        launch_sparse(k_big_numeric_sparse<FUSED, MID_ITEM, MID_RANK_U, MID_MINW>, ns, nm);
-        // the rest: items of more outputs in column order, all in rows' order
-        if (p.narrow_items) {
+        // the size classes, in kernels with tables of their size; in rows'
+        // order all items are of the last
+        auto by_class = [&](auto dir) {
+            constexpr bool DIR = decltype(dir)::value;
             constexpr int W = ITEM_WORDS / 2;
-            launch_rank(k_big_numeric_rank<FUSED, W>, sizeof(RankSmem<W>) * ITEM_WAVES, nm,
-                        p.nitems);
-        } else {
-            constexpr int W = ITEM_WORDS;
-            launch_rank(k_big_numeric_rank<FUSED, W>, sizeof(RankSmem<W>) * ITEM_WAVES, nm,
-                        p.nitems);
-        }
+            const int64_t *e = p.class_end;
+            launch(k_big_numeric_sparse<FUSED, ITEM_BOUND[0], 4, 8, DIR>, 0, e[0]);
+            launch(k_big_numeric_sparse<FUSED, ITEM_BOUND[1], 6, 4, DIR>, e[0], e[1]);
+            launch(k_big_numeric_rank<FUSED, W, DIR>, e[1], e[2]);
+        };
+        if (!p.narrow_items)
+            launch(k_big_numeric_rank<FUSED, ITEM_WORDS, false>, 0, p.nitems);
+        else if (p.dir.cells)
+            by_class(std::true_type());
+        else
+            by_class(std::false_type());
         tm.end();
     } else if (p.nitems > 0) {
         tm.begin("row.big_numeric");
         constexpr size_t sm = sizeof(ItemSmem) * ITEM_WAVES;
-        auto kern = k_big_numeric<FUSED>;
+        auto kern = p.dir.cells ? k_big_numeric<FUSED, true> : k_big_numeric<FUSED, false>;
         set_smem(kern, sm);
         const unsigned grid = item_grid(p.nitems);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * ITEM_WAVES), sm, s, p.nitems, p.items,
-                           A.ptr, A.idx, A.val, B.ptr, B.idx, B.val, block_ptrs(p, B.ptr),
-                           d_jc, d_c, (int)p.b_strict);
+                           A.ptr, A.idx, A.val, B.idx, B.val, b_rows(p, B.ptr), d_jc, d_c, (int)p.b_strict);
         TSG_LAUNCH_CHECK();
         tm.end();
     }

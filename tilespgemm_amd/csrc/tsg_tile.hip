@@ -220,14 +220,13 @@ __global__ void __launch_bounds__(64 * S1_WAVES) k_step1(
         const int nwords = (w1 - w0 + 31) >> 5;
         for (int i = l; i < nwords; i += 64) bits[i] = 0u;
         wave_lds_fence();
-        for_products<4, 1, false, false>(pa, pe, tcolA, nullptr, tptrB, tcolB, nullptr,
-                                         BlockPtrs(), 0, 0, s_heads[threadIdx.x >> 6],
-                                         [&](const Batch &t) {
-                                             if (t.act && t.col >= w0 && t.col < w1) {
-                                                 const int c = t.col - w0;
-                                                 lds_set_bit(&bits[c >> 5], 1u << (c & 31));
-                                             }
-                                         });
+        for_products<4, 1, false>(pa, pe, tcolA, nullptr, RowRange{tptrB}, tcolB, nullptr,
+                                  s_heads[threadIdx.x >> 6], [&](const Batch &t) {
+                                      if (t.act && t.col >= w0 && t.col < w1) {
+                                          const int c = t.col - w0;
+                                          lds_set_bit(&bits[c >> 5], 1u << (c & 31));
+                                      }
+                                  });
         wave_lds_fence();
         for (int i0 = 0; i0 < nwords; i0 += 64) {
             const int i = i0 + l;
