@@ -237,7 +237,7 @@ struct RowPlan {
     bool column_order = false;       // big-row bands and items run in column order
     // items
     int64_t nitems = 0;
-    int64_t class_end[ITEM_CLASSES] = {};   // ends of the items' size classes (column order)
+    int64_t class_end[ITEM_CLASSES - 1] = {};   // ends of the items' classes but the last
     int64_t *item_cnt = nullptr;     // [nbig+1] items per big row -> offsets
     ItemRec *items = nullptr;        // by c0 (column order) or by row
     bool narrow_items = false;       // items of <= 8192 columns (else <= 16384)

@@ -649,8 +649,8 @@ __global__ void __launch_bounds__(256) k_dir_runs(int n, int nnz, const int *__r
 }
 
 // ------------------------------------------------------------- item plan
-constexpr int ITEM_BOUND[ITEM_CLASSES] = {256, 512, ITEM_CAP};
-constexpr int SPARSE_CLASSES = 2;
+// of the sparse classes; items of more outputs are dense
+constexpr int ITEM_BOUND[2] = {256, 512};
 // Sparse stretches go into wide items of up to this many outputs.  R-MAT 2^20
 // with 8 draws a row, both sparse kernels: 31.7 ms without wide items (its
 // 30M items of <= 256 outputs hold 45 each, and each costs its A entries, two
@@ -658,7 +658,7 @@ constexpr int SPARSE_CLASSES = 2;
 // 19.3 up to 512; R-MAT 2^18 with 4: 1.27, 1.01, 0.98, 0.96; ER batch of 512:
 // 6.0, 5.9, 5.1, 4.3.
 constexpr int WIDE_CAP = 512;
-static_assert(WIDE_CAP <= ITEM_BOUND[SPARSE_CLASSES - 1], "wide items run in the sparse kernels");
+static_assert(WIDE_CAP <= ITEM_BOUND[1], "wide items run in the sparse kernels");
 
 // Split of each big row into items: the row's span is cut into windows of
 // WSB sub-blocks (at most ITEM_WBITS columns); inside a window, runs of
@@ -856,8 +856,8 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
 // times its transpose, items of <= 512 outputs 0.69 -> 0.56 ms).
 // key = class << class_bit + 1 | 1 << class_bit | first sub-block (a long
 // row's without the 1; class_bit < 0: the sub-block only).  The numeric phase
-// runs each class in a kernel whose tables hold just that class's items: the
-// waves an LDS holds set its speed.  R-MAT 2^20 with 8 draws a row: <= 256
+// runs each class with tables that hold just that class's items: the waves an
+// LDS holds set its speed.  Class 1 is the dense one.  R-MAT 2^20 with 8 draws a row: <= 256
 // outputs 5.8 -> 4.2 ms (4 batches in flight, 8 waves per SIMD; 6 batches: 4.7),
 // <= 512 12.8 -> 11.8 (at 4 waves).  Finer classes gained nothing there (384:
 // 4.2 + 7.5 ms; 768: 7.8 + 7.9 against 15.9) and cost R-MAT 2^18 a tail each.
@@ -878,9 +878,7 @@ __global__ void __launch_bounds__(256) k_item_keys(int64_t n, const ItemRec *__r
         if (i < n) {
             if (class_bit >= 0) {
                 const int outputs = item_n[i];
-#pragma unroll
-                for (int c = ITEM_CLASSES - 2; c >= 0; c--)
-                    if (outputs <= ITEM_BOUND[c]) cls = c;
+                cls = outputs <= ITEM_BOUND[0] ? 0 : outputs > ITEM_BOUND[1] ? 1 : 2;
             }
             const int4 d = items[i].d;
             int key = d.y >> SUB_SHIFT;
@@ -1090,16 +1088,6 @@ __device__ __forceinline__ int item_rank_build(RankSmem<WORDS> &S, unsigned (&wv
     return cnt;
 }
 
-// Writes an item's cnt values to C at offset o, straight from LDS.
-template <int WORDS>
-__device__ __forceinline__ void item_store_values(RankSmem<WORDS> &S, int cnt, int64_t o,
-                                                  double *__restrict__ c) {
-    const int l = __lane_id();
-    wave_lds_fence();
-    for (int i = l; i < cnt; i += 64) __builtin_nontemporal_store(S.vals[i], c + o + i);
-    wave_lds_fence();
-}
-
 // Accumulates one batch of products into the item's rank-ordered values:
 // a batch from one A entry (distinct columns when B's rows are strictly
 // ascending) adds directly, one from a few A entries one entry after the
@@ -1126,47 +1114,55 @@ __device__ __forceinline__ void item_accumulate(RankSmem<WORDS> &S, int c0, cons
                                          (unsigned)__lane_id(), false);
 }
 
+// What the item kernels work on, but for the items.
+struct ItemArgs {
+    const unsigned *wlist, *subocc;
+    const int *ia, *ja;
+    const double *a;
+    const int *jb;
+    const int4 *bpk;
+    int *jc;
+    double *c;
+    int b_strict;
+};
+
 template <bool FUSED, int WORDS, bool DIR>
-__global__ void __launch_bounds__(64) k_big_numeric_rank(
-    int64_t nitems, const ItemRec *__restrict__ items, const unsigned *__restrict__ wlist,
-    const unsigned *__restrict__ subocc, const int *__restrict__ ia, const int *__restrict__ ja,
-    const double *__restrict__ a, const int *__restrict__ jb, const int4 *__restrict__ bpk, BRows brows,
-    int *__restrict__ jc, double *__restrict__ c, int b_strict) {
-    __shared__ RankSmem<WORDS> S;
-    const int l = threadIdx.x;
+__device__ __forceinline__ void dense_item(RankSmem<WORDS> &S, const ItemRec &rec,
+                                           const ItemArgs &T, const BRows &brows) {
+    const int l = __lane_id();
     for (int i = l; i < RANK_TAGS; i += 64) S.tags[i] = 0xffffffffu;
-    for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const int4 item = items[it].d;
-        const int64_t o = items[it].off;
-        const unsigned *list = wlist + items[it].wpos;
-        const int c0 = item.y, c1 = item.z;
-        // the rank table is built after the first groups' A entries and cells
-        // are issued, so the word loads and that chain of loads overlap
-        const ItemRange<DIR> range(brows, jb, c0, c1);
-        EntryPipe<true, 1> pipe;
-        pipe.ja = ja;
-        pipe.aval = a;
-        pipe.part = 0;
-        pipe.load(ia[item.x], ia[item.x + 1]);
-        // item.w: the item's first sub-block in subocc
-        const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 2 * (WORDS / 64));
-        const unsigned occ = l < nsb ? subocc[(int64_t)item.w + l] : 0u;
-        pipe.cells(range);
-        const int pc = __popc(occ);
-        const int pre = dpp_incl_scan<16>(pc) - pc;
-        unsigned wv[WORDS / 64];
-        item_words(list, occ, pre, c0, c1, wv);
-        pipe.first(range);
-        const int cnt = item_rank_build(S, wv, c0, c1, o, jc);
-        auto f = [&](const Batch &t) { item_accumulate<FUSED>(S, c0, t, b_strict); };
-        for (int g = pipe.pa; g < pipe.pe; g += 64) {
-            pipe.ahead(g, range);
-            expand_group<RANK_U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, jb,
-                                             nullptr, S.heads, f, bpk);
-            pipe.take();
-        }
-        item_store_values(S, cnt, o, c);
+    const int4 item = rec.d;
+    const int64_t o = rec.off;
+    const unsigned *list = T.wlist + rec.wpos;
+    const int c0 = item.y, c1 = item.z;
+    // the rank table is built after the first groups' A entries and cells are
+    // issued, so the word loads and that chain of loads overlap
+    const ItemRange<DIR> range(brows, T.jb, c0, c1);
+    EntryPipe<true, 1> pipe;
+    pipe.ja = T.ja;
+    pipe.aval = T.a;
+    pipe.part = 0;
+    pipe.load(T.ia[item.x], T.ia[item.x + 1]);
+    // item.w: the item's first sub-block in subocc
+    const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 2 * (WORDS / 64));
+    const unsigned occ = l < nsb ? T.subocc[(int64_t)item.w + l] : 0u;
+    pipe.cells(range);
+    const int pc = __popc(occ);
+    const int pre = dpp_incl_scan<16>(pc) - pc;
+    unsigned wv[WORDS / 64];
+    item_words(list, occ, pre, c0, c1, wv);
+    pipe.first(range);
+    const int cnt = item_rank_build(S, wv, c0, c1, o, T.jc);
+    auto f = [&](const Batch &t) { item_accumulate<FUSED>(S, c0, t, T.b_strict); };
+    for (int g = pipe.pa; g < pipe.pe; g += 64) {
+        pipe.ahead(g, range);
+        expand_group<RANK_U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, T.jb, nullptr,
+                                         S.heads, f, T.bpk);
+        pipe.take();
     }
+    wave_lds_fence();
+    for (int i = l; i < cnt; i += 64) __builtin_nontemporal_store(S.vals[i], T.c + o + i);
+    wave_lds_fence();
 }
 
 // Items of at most CAP outputs, however wide up to a band: the rank of a
@@ -1192,103 +1188,127 @@ struct SparseSmem {
     int heads[2 * U];
 };
 
-template <bool FUSED, int CAP, int U, int MINW, bool DIR>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MINW)))
-k_big_numeric_sparse(int64_t nitems, const ItemRec *__restrict__ items,
-                     const unsigned *__restrict__ wlist, const unsigned *__restrict__ subocc,
-                     const int *__restrict__ ia, const int *__restrict__ ja,
-                     const double *__restrict__ a, const int *__restrict__ jb,
-                     const int4 *__restrict__ bpk, BRows brows, int *__restrict__ jc,
-                     double *__restrict__ c, int b_strict) {
-    __shared__ __align__(16) SparseSmem<CAP, U> S;
+template <bool FUSED, int CAP, int U, bool DIR>
+__device__ __forceinline__ void sparse_item(SparseSmem<CAP, U> &S, const ItemRec &rec,
+                                            const ItemArgs &T, const BRows &brows) {
     constexpr int NT = CAP / 4;
-    const int l = threadIdx.x;
+    const int l = __lane_id();
     uint8_t *own = reinterpret_cast<uint8_t *>(S.tags);
+    const int4 item = rec.d;
+    const int64_t o = rec.off;
+    const unsigned *list = T.wlist + rec.wpos;
+    const int c0 = item.y, c1 = item.z;
+    const ItemRange<DIR> range(brows, T.jb, c0, c1);
+    EntryPipe<true, 1> pipe;
+    pipe.ja = T.ja;
+    pipe.aval = T.a;
+    pipe.part = 0;
+    pipe.load(T.ia[item.x], T.ia[item.x + 1]);
+    const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 1 << BAND_SHIFT);
+    const unsigned occ = l < nsb ? T.subocc[(int64_t)item.w + l] : 0u;
+    pipe.cells(range);
+    const int pc = __popc(occ);
+    const int incl = wave_incl_scan(pc);
+    // every non-empty word has an output
+    const int nw = min(__builtin_amdgcn_readlane(incl, 63), CAP);
+    unsigned wv[CAP / 64];
+#pragma unroll
+    for (int j = 0; j < CAP / 64; j++)
+        wv[j] = j * 64 + l < nw ? __builtin_nontemporal_load(list + j * 64 + l) : 0u;
+    pipe.first(range);
+    S.sub[l] = make_uint2(occ, (unsigned)(incl - pc));
+    int cnt = 0;
+#pragma unroll
+    for (int j = 0; j < CAP / 64; j++) {
+        if (j * 64 < nw) {
+            const int p = __popc(wv[j]);
+            const int in = wave_incl_scan(p);
+            if (j * 64 + l < nw) {
+                S.words[j * 64 + l] = wv[j];
+                S.pre[j * 64 + l] = (uint16_t)(cnt + in - p);
+            }
+            cnt += __builtin_amdgcn_readlane(in, 63);
+        }
+    }
+    cnt = min(cnt, CAP);
+    for (int i = l; i < cnt; i += 64) S.vals[i] = 0.0;
+    wave_lds_fence();
+    auto f = [&](const Batch &t) {
+        int rank = -1;
+        if (t.act) {
+            const int cc = t.col - c0;
+            const uint2 sb = S.sub[(cc >> SUB_SHIFT) & ((1 << BAND_SHIFT) - 1)];
+            const int w = min(
+                (int)sb.y + (int)__popc(sb.x & ((1u << ((cc >> 5) & 31)) - 1u)), CAP - 1);
+            rank = min((int)S.pre[w] + (int)__popc(S.words[w] & ((1u << (cc & 31)) - 1u)),
+                       CAP - 1);
+            S.cols[rank] = (uint16_t)cc;
+        }
+        bool clash = t.nseg > 1 || !T.b_strict;
+        if (T.b_strict && t.nseg > 2) {
+            if (t.act) own[rank] = (uint8_t)l;
+            wave_lds_fence();
+            clash = __ballot(t.act && own[rank] != (uint8_t)l) != 0;
+            wave_lds_fence();
+        }
+        if (!clash) {
+            if (t.act) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
+            wave_lds_fence();
+        } else if (T.b_strict && t.nseg <= FLAT_SEGS) {
+            for (int s = 1; s <= t.nseg; s++) {
+                if (t.act && t.seg == s) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
+                wave_lds_fence();
+            }
+        } else {
+            for (int i = l; i < NT; i += 64) S.tags[i] = 0xffffffffu;
+            wave_lds_fence();
+            ordered_accumulate<FUSED, NT>(t.act, rank, t.a, t.b, S.vals, S.tags, (unsigned)l,
+                                          false);
+        }
+    };
+    for (int g = pipe.pa; g < pipe.pe; g += 64) {
+        pipe.ahead(g, range);
+        expand_group<U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, T.jb, nullptr,
+                                    S.heads, f, T.bpk);
+        pipe.take();
+    }
+    wave_lds_fence();
+    for (int i = l; i < cnt; i += 64) {
+        __builtin_nontemporal_store(c0 + (int)S.cols[i], T.jc + o + i);
+        __builtin_nontemporal_store(S.vals[i], T.c + o + i);
+    }
+    wave_lds_fence();
+}
+
+// The items of at most 256 outputs: 32 waves a CU.
+template <bool FUSED, bool DIR>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) k_big_numeric_small(
+    int64_t nitems, const ItemRec *__restrict__ items, ItemArgs T, BRows brows) {
+    __shared__ __align__(16) SparseSmem<ITEM_BOUND[0], 4> S;
+    for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x)
+        sparse_item<FUSED, ITEM_BOUND[0], 4, DIR>(S, items[it], T, brows);
+}
+
+// The others, the first ndense in dense tables (all items in rows' order): in
+// one launch, so the other class runs beside the longest items, which a wave
+// each works on for most of a small product's time (R-MAT 2^18 with 4, times
+// its transpose: 0.91 + 0.54 ms in two launches, 1.03 in one; R-MAT 2^20 with 8
+// draws a row 27.1 ms either way).  Teams of 2 to 4 waves on an item, in turns
+// by group of A entries, took 1.2 to 2 times as long: the turns are most of a
+// group's time.
+template <bool FUSED, int WORDS, bool DIR>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_big_numeric_rank(
+    int64_t nitems, int64_t ndense, const ItemRec *__restrict__ items, ItemArgs T, BRows brows) {
+    union Smem {
+        RankSmem<WORDS> dense;
+        SparseSmem<ITEM_BOUND[1], 6> sparse;
+    };
+    __shared__ __align__(16) Smem S;
     for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const int4 item = items[it].d;
-        const int64_t o = items[it].off;
-        const unsigned *list = wlist + items[it].wpos;
-        const int c0 = item.y, c1 = item.z;
-        const ItemRange<DIR> range(brows, jb, c0, c1);
-        EntryPipe<true, 1> pipe;
-        pipe.ja = ja;
-        pipe.aval = a;
-        pipe.part = 0;
-        pipe.load(ia[item.x], ia[item.x + 1]);
-        const int nsb = min((c1 - c0 + (1 << SUB_SHIFT) - 1) >> SUB_SHIFT, 1 << BAND_SHIFT);
-        const unsigned occ = l < nsb ? subocc[(int64_t)item.w + l] : 0u;
-        pipe.cells(range);
-        const int pc = __popc(occ);
-        const int incl = wave_incl_scan(pc);
-        // every non-empty word has an output
-        const int nw = min(__builtin_amdgcn_readlane(incl, 63), CAP);
-        unsigned wv[CAP / 64];
-#pragma unroll
-        for (int j = 0; j < CAP / 64; j++)
-            wv[j] = j * 64 + l < nw ? __builtin_nontemporal_load(list + j * 64 + l) : 0u;
-        pipe.first(range);
-        S.sub[l] = make_uint2(occ, (unsigned)(incl - pc));
-        int cnt = 0;
-#pragma unroll
-        for (int j = 0; j < CAP / 64; j++) {
-            if (j * 64 < nw) {
-                const int p = __popc(wv[j]);
-                const int in = wave_incl_scan(p);
-                if (j * 64 + l < nw) {
-                    S.words[j * 64 + l] = wv[j];
-                    S.pre[j * 64 + l] = (uint16_t)(cnt + in - p);
-                }
-                cnt += __builtin_amdgcn_readlane(in, 63);
-            }
-        }
-        cnt = min(cnt, CAP);
-        for (int i = l; i < cnt; i += 64) S.vals[i] = 0.0;
-        wave_lds_fence();
-        auto f = [&](const Batch &t) {
-            int rank = -1;
-            if (t.act) {
-                const int cc = t.col - c0;
-                const uint2 sb = S.sub[(cc >> SUB_SHIFT) & ((1 << BAND_SHIFT) - 1)];
-                const int w = min(
-                    (int)sb.y + (int)__popc(sb.x & ((1u << ((cc >> 5) & 31)) - 1u)), CAP - 1);
-                rank = min((int)S.pre[w] + (int)__popc(S.words[w] & ((1u << (cc & 31)) - 1u)),
-                           CAP - 1);
-                S.cols[rank] = (uint16_t)cc;
-            }
-            bool clash = t.nseg > 1 || !b_strict;
-            if (b_strict && t.nseg > 2) {
-                if (t.act) own[rank] = (uint8_t)l;
-                wave_lds_fence();
-                clash = __ballot(t.act && own[rank] != (uint8_t)l) != 0;
-                wave_lds_fence();
-            }
-            if (!clash) {
-                if (t.act) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
-                wave_lds_fence();
-            } else if (b_strict && t.nseg <= FLAT_SEGS) {
-                for (int s = 1; s <= t.nseg; s++) {
-                    if (t.act && t.seg == s) S.vals[rank] = acc_step<FUSED>(S.vals[rank], t.a, t.b);
-                    wave_lds_fence();
-                }
-            } else {
-                for (int i = l; i < NT; i += 64) S.tags[i] = 0xffffffffu;
-                wave_lds_fence();
-                ordered_accumulate<FUSED, NT>(t.act, rank, t.a, t.b, S.vals, S.tags, (unsigned)l,
-                                              false);
-            }
-        };
-        for (int g = pipe.pa; g < pipe.pe; g += 64) {
-            pipe.ahead(g, range);
-            expand_group<U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, jb, nullptr,
-                                        S.heads, f, bpk);
-            pipe.take();
-        }
-        wave_lds_fence();
-        for (int i = l; i < cnt; i += 64) {
-            __builtin_nontemporal_store(c0 + (int)S.cols[i], jc + o + i);
-            __builtin_nontemporal_store(S.vals[i], c + o + i);
-        }
-        wave_lds_fence();
+        if (it < ndense)
+            dense_item<FUSED, WORDS, DIR>(S.dense, items[it], T, brows);
+        else
+            sparse_item<FUSED, ITEM_BOUND[1], 6, DIR>(S.sparse, items[it], T, brows);
     }
 }
 
@@ -1612,7 +1632,8 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
             items_kernel(k_items<true, 8>, p.item_cnt, p.items, item_n);
         else
             items_kernel(k_items<true, 16>, p.item_cnt, p.items, item_n);
-        p.class_end[ITEM_CLASSES - 1] = p.nitems;
+        p.class_end[0] = 0;
+        p.class_end[1] = p.nitems;
         if (p.column_order && p.nitems > 0 && p.nitems < (int64_t(1) << 31)) {
             const size_t ni = (size_t)p.nitems;
             int *keys = ws.alloc_n<int>(ni);
@@ -1677,29 +1698,25 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
                                B.nnz, B.idx, B.val, p.bpk);
             TSG_LAUNCH_CHECK();
         }
-        auto launch = [&](auto kern, int64_t i0, int64_t i1) {
-            if (i1 <= i0) return;
-            hipLaunchKernelGGL(kern, dim3(item_grid(i1 - i0)), dim3(64), 0, s, i1 - i0,
-                               p.items + i0, p.bandwords, p.subocc, A.ptr, A.idx, A.val, B.idx,
-                               p.bpk, b_rows(p, B.ptr), d_jc, d_c, (int)p.b_strict);
+        const ItemArgs T{p.bandwords, p.subocc, A.ptr, A.idx,  A.val,
+                         B.idx,       p.bpk,    d_jc,  d_c,    (int)p.b_strict};
+        const BRows brows = b_rows(p, B.ptr);
+        const int64_t ns = p.class_end[0], nd = p.class_end[1] - ns;
+        if (ns > 0) {
+            auto kern = p.dir.cells ? k_big_numeric_small<FUSED, true>
+                                    : k_big_numeric_small<FUSED, false>;
+            hipLaunchKernelGGL(kern, dim3(item_grid(ns)), dim3(64), 0, s, ns, p.items, T, brows);
             TSG_LAUNCH_CHECK();
-        };
-        // the size classes, in kernels with tables of their size; in rows'
-        // order all items are of the last
-        auto by_class = [&](auto dir) {
-            constexpr bool DIR = decltype(dir)::value;
-            constexpr int W = ITEM_WORDS / 2;
-            const int64_t *e = p.class_end;
-            launch(k_big_numeric_sparse<FUSED, ITEM_BOUND[0], 4, 8, DIR>, 0, e[0]);
-            launch(k_big_numeric_sparse<FUSED, ITEM_BOUND[1], 6, 4, DIR>, e[0], e[1]);
-            launch(k_big_numeric_rank<FUSED, W, DIR>, e[1], e[2]);
-        };
-        if (!p.narrow_items)
-            launch(k_big_numeric_rank<FUSED, ITEM_WORDS, false>, 0, p.nitems);
-        else if (p.dir.cells)
-            by_class(std::true_type());
-        else
-            by_class(std::false_type());
+        }
+        if (p.nitems > ns) {
+            constexpr int W = ITEM_WORDS;
+            auto kern = !p.narrow_items ? k_big_numeric_rank<FUSED, W, false>
+                        : p.dir.cells   ? k_big_numeric_rank<FUSED, W / 2, true>
+                                        : k_big_numeric_rank<FUSED, W / 2, false>;
+            hipLaunchKernelGGL(kern, dim3(item_grid(p.nitems - ns)), dim3(64), 0, s,
+                               p.nitems - ns, nd, p.items + ns, T, brows);
+            TSG_LAUNCH_CHECK();
+        }
         tm.end();
     } else if (p.nitems > 0) {
         tm.begin("row.big_numeric");
