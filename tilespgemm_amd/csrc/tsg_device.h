@@ -136,6 +136,22 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
+constexpr unsigned XCDS = 8;
+
+// Workgroups go to the XCDs in turn, and each XCD has an L2 of its own.  The
+// piece of work of workgroup i of n, such that an XCD takes runs of CHUNK
+// consecutive pieces (0: one run, an eighth of them): neighbours, which read
+// the same rows, then share an L2 and read them from memory once, not once per
+// XCD.
+template <unsigned CHUNK>
+__device__ __forceinline__ unsigned xcd_piece(unsigned i, unsigned n) {
+    const unsigned run = CHUNK ? CHUNK : n / XCDS;
+    const unsigned round = run * XCDS;
+    if (round == 0 || i >= n / round * round) return i;
+    const unsigned q = i / round, r = i % round;
+    return q * round + (r % XCDS) * run + r / XCDS;
+}
+
 // Exclusive lower bound of key in sorted a[lo, hi).
 __device__ __forceinline__ int lower_bound_i32(const int *a, int lo, int hi, int key) {
     while (lo < hi) {

@@ -59,6 +59,13 @@ constexpr int RANK_U = 8;
 constexpr int BIG_SYM_U = 8;
 constexpr int ITEM_U = 4;
 
+// Rows an XCD takes in a run: neighbours share B rows (stencils) or a matrix of
+// a batch.  ER batch of 512, numeric, 16 products a lane: 10.74 ms in turns,
+// 10.31 in runs of 64, 10.35 of 512, 10.70 an eighth each; 27-point 64^3 687, 671,
+// 667, 677 us.  (Items and bands, which run in column order and read one band of
+// B together, gain nothing.)
+constexpr unsigned FLAT_CHUNK = 64;
+
 // ------------------------------------------------------ small rows: symbolic
 // Output count of each row of at most G * U products (rownnz), G lanes a row:
 // the columns gathered into registers and counted by the bitmaps of
@@ -94,7 +101,7 @@ k_flat_symbolic(int nrows, const int *__restrict__ rows, const int *__restrict__
     __shared__ __align__(16) FlatSmem<G * U, E, LW, 1> s_row[RPB];
     const int grp = threadIdx.x / G;
     FlatSmem<G * U, E, LW, 1> &S = s_row[grp];
-    const int r = blockIdx.x * RPB + grp;
+    const int r = xcd_piece<FLAT_CHUNK>(blockIdx.x, gridDim.x) * RPB + grp;
     if (r >= nrows) return;
     const int row = group_uniform<G>(rows[r]);
     const int total = flat_entries<G>(S, ia[row], ia[row + 1], ja, (const double *)nullptr, ib);
@@ -209,7 +216,7 @@ k_flat_numeric(
     __shared__ unsigned s_tags[RPB][ACC / 4];
     const int grp = threadIdx.x / G;
     FlatSmem<G * U, E, LW, ACC> &S = s_row[grp];
-    const int r = blockIdx.x * RPB + grp;
+    const int r = xcd_piece<FLAT_CHUNK>(blockIdx.x, gridDim.x) * RPB + grp;
     if (r >= nrows) return;
     const int row = group_uniform<G>(rows[r]);
     const int64_t o = ic[row];
