@@ -122,9 +122,10 @@ int tsg_get_method_used(tsg_handle_t handle);
  * faster on the row path and banded or block-dense matrices, at 90 and
  * more, 1.5-4x faster on the tile path).
  * Row bins: rows with at most bin1 (<= 64), bin2 (<= 256) and bin3 (<= 1024)
- * intermediate products go to the 16-, 32- and 64-lane LDS-hash kernels,
- * longer rows to the big-row path (defaults 64, 256, 1024; bin1 <= bin2 <=
- * bin3).  tilespgemm_amd.autotune searches them for a workload. */
+ * intermediate products take 16 lanes, a wave, and a wave with more
+ * registers each, longer rows go to the big-row path (defaults 64, 256, 1024;
+ * bin1 <= bin2 <= bin3; at bin3 = 1024, rows of up to 1536 products from up to
+ * 64 entries of A still take a wave).  tilespgemm_amd.autotune searches them for a workload. */
 int tsg_set_tile_density(tsg_handle_t handle, double entries_per_tile);
 int tsg_set_row_bins(tsg_handle_t handle, int bin1, int bin2, int bin3);
 int tsg_get_tuning(tsg_handle_t handle, double *tile_density, int *bin1, int *bin2,

@@ -119,7 +119,7 @@ struct FlatHeads {
     const unsigned *starts;
     int sv = 0;
     __device__ __forceinline__ explicit FlatHeads(const unsigned *s) : starts(s) {
-        if constexpr (G == 64) sv = (int)starts[__lane_id() & (2 * U - 1)];
+        if constexpr (G == 64) sv = (int)starts[min((int)__lane_id(), 2 * U - 1)];
         static_assert(G == 64 || G == 16, "a batch is two words or half a word of start bits");
     }
     // (u past the row's batches: none)

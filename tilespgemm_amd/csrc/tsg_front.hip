@@ -41,7 +41,7 @@ struct FrontMat {
 struct FrontBins {
     const int *ib;                       // B's row pointers
     int64_t *rowprod, *rownnz;
-    int *list[3];                        // bins 1 and 2, 3 and 4, 5 and 6: front, back
+    int *list[ROW_LISTS];                // bins 1 and 2, 3 and 4, ...: front, back
     int nlist;
     FrontSlot *slots;
     RowBinLimits lim;
@@ -324,7 +324,7 @@ int front_pass(const CsrIn &A, const CsrIn &B, Arena &ws, hipStream_t s, HostBox
         rows->nlist = (int)std::min<int64_t>(A.rows, A.nnz);
         rows->rowprod = ws.alloc_n<int64_t>((size_t)A.rows + 1);
         rows->rownnz = ws.alloc_n<int64_t>((size_t)A.rows + 1);
-        for (int i = 0; i < 3; i++) {
+        for (int i = 0; i < ROW_LISTS; i++) {
             rows->list[i] = ws.alloc_n<int>((size_t)rows->nlist + 1);
             P.list[i] = rows->list[i];
         }
@@ -332,7 +332,8 @@ int front_pass(const CsrIn &A, const CsrIn &B, Arena &ws, hipStream_t s, HostBox
         P.rowprod = rows->rowprod;
         P.rownnz = rows->rownnz;
         P.nlist = rows->nlist;
-        P.lim = RowBinLimits{tune->bin1, tune->bin2, tune->bin3};
+        P.lim = RowBinLimits{tune->bin1, tune->bin2, tune->bin3,
+                             tune->bin3 == ROW_SMALL_PROD ? ROW_MED_PROD : tune->bin3};
     }
     TSG_HIP_TRY(hipMemsetAsync(zero, 0, sizeof(FrontCounters) + nslots * sizeof(FrontSlot), s));
     int nsample = 0, step = 1;

@@ -121,7 +121,7 @@ struct StageTimer {
 // ---------------------------------------------------------- host results
 // Host memory of a handle that kernels write their small results into: they
 // are there once the stream is synchronized, with no copy in between.
-constexpr int ROW_BINS = 7;
+constexpr int ROW_BINS = 8;
 struct alignas(256) HostBox {
     unsigned flags[2];
     int bins[ROW_BINS];
@@ -136,20 +136,30 @@ void publish_i64(const PublishList &src, int n, HostBox *box, hipStream_t s);
 // Row bins by intermediate products: (0, l1] -> 16 lanes a row, (l1, l2],
 // (l2, ROW_MID_PROD] and (ROW_MID_PROD, l3] -> a wave a row with 4, 8 and 16
 // products a lane (those with more than ROW_FLAT_ENT A entries in a bin of
-// their own), above l3 -> the big-row path.  Each small kernel is exact for
+// their own), (l3, l4] -> 24 a lane if at most ROW_FLAT_ENT entries, the rest
+// -> the big-row path.  l4 is ROW_MED_PROD at the full l3, else l3.  ER batch of
+// 512 (a tenth of its products in rows of 1025 to 1536): 7.2 ms in the big-row
+// path, 3.5 here, at 4 waves per SIMD (3.8 at 3); R-MAT 2^20 with 8 draws a row
+// 2.0 and 0.75.
+// Each small kernel is exact for
 // any row up to its register count, so any limits with l1 <= 64, l2 <= 256,
 // l3 <= 1024 (checked on the host) are valid; they are tuning parameters
 // (tsg_set_row_bins).
 constexpr int ROW_MID_PROD = 512;
 constexpr int ROW_FLAT_ENT = 64;
+constexpr int ROW_SMALL_PROD = 1024;   // the largest l3
+constexpr int ROW_MED_PROD = 1536;
+constexpr int ROW_LISTS = ROW_BINS / 2;
 constexpr int ROW_BIN_MANY = 5;
-constexpr int ROW_BIN_BIG = 6;
-struct RowBinLimits { int l1, l2, l3; };
+constexpr int ROW_BIN_MED = 6;
+constexpr int ROW_BIN_BIG = 7;
+struct RowBinLimits { int l1, l2, l3, l4; };
 
 __host__ __device__ inline int row_bin_of(int64_t prod, int entries, RowBinLimits lim) {
     if (prod == 0) return 0;
     if (prod <= lim.l1) return 1;
-    if (prod > lim.l3) return ROW_BIN_BIG;
+    if (prod > lim.l4) return ROW_BIN_BIG;
+    if (prod > lim.l3) return entries <= ROW_FLAT_ENT ? ROW_BIN_MED : ROW_BIN_BIG;
     if (entries > ROW_FLAT_ENT) return ROW_BIN_MANY;
     if (prod <= lim.l2) return 2;
     return prod <= ROW_MID_PROD ? 3 : 4;
@@ -161,7 +171,7 @@ __host__ __device__ inline int row_bin_of(int64_t prod, int entries, RowBinLimit
 struct RowFront {
     int64_t *rowprod = nullptr;      // [m]
     int64_t *rownnz = nullptr;       // [m+1] zero for rows of bin 0 and big rows
-    int *list[3] = {nullptr, nullptr, nullptr};
+    int *list[ROW_LISTS] = {};
     int nlist = 0;                   // ints of each list
     int count[ROW_BINS] = {0};       // (host) rows per bin
     const int *rows(int bin) const {
@@ -222,6 +232,7 @@ struct RowPlan {
     RowFront front;                  // products per row, rows per bin
     // big-row structures
     int nbig = 0;
+    int64_t big_prod = 0;            // products of the big rows
     int sub_shift = 0;               // log2 sub-block width (columns)
     int *span_sb0 = nullptr;         // [nbig] first sub-block of the row's span
     int64_t *sb_off = nullptr;       // [nbig+1] span offsets (sub-blocks)

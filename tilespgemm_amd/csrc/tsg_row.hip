@@ -13,7 +13,7 @@
 //     take turns in product order (one B row after the other, or tag rounds:
 //     LDS atomicMin on a small bucket table), so the parallel sum equals the
 //     sequential one.
-//   * Small rows (<= SMALL_PROD products): one lane group per row with all its
+//   * Small rows (<= 1024 products, or 1536): one lane group per row with all its
 //     products in registers (tsg_flat.h); an output's place is its column's
 //     rank in a two-level bitmap, so C comes out sorted with no hash or sort.
 //   * Big rows: the symbolic phase cuts each row's column span into bands of
@@ -39,8 +39,6 @@
 #include <mutex>
 
 namespace {
-
-constexpr int SMALL_PROD = 1024;       // rows up to this many products: small path
 
 constexpr int SUB_SHIFT = 10;          // sub-block = 1024 columns
 constexpr int BAND_SHIFT = 6;          // symbolic band = 64 sub-blocks (65536 columns)
@@ -1330,6 +1328,29 @@ __global__ void __launch_bounds__(256) k_pack_b(int64_t nnz, const int *__restri
     bpk[q] = make_int4(jb[q], 0, __double2loint(v), __double2hiint(v));
 }
 
+// The same for the B rows that big rows name, a wave per big row (rows named
+// more than once are written with the same records): with few big rows that is
+// less than all of B (ER batch of 512 matrices: 0.67 -> 0.08 ms).
+__global__ void __launch_bounds__(256) k_pack_rows(int nbig, const int *__restrict__ rows,
+                                                   const int *__restrict__ ia,
+                                                   const int *__restrict__ ja,
+                                                   const int *__restrict__ ib,
+                                                   const int *__restrict__ jb,
+                                                   const double *__restrict__ b,
+                                                   int4 *__restrict__ bpk) {
+    const int r = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int l = __lane_id();
+    if (r >= nbig) return;
+    const int row = rows[r];
+    for (int p = ia[row]; p < ia[row + 1]; p++) {
+        const int t = ja[p];
+        for (int q = ib[t] + l; q < ib[t + 1]; q += 64) {
+            const double v = b[q];
+            bpk[q] = make_int4(jb[q], 0, __double2loint(v), __double2hiint(v));
+        }
+    }
+}
+
 // The plan's run directory or block pointers; without either, B's row pointers
 // b_ptr (of the call at hand) as a one-block table.
 static BRows b_rows(const RowPlan &p, const int *b_ptr) {
@@ -1370,7 +1391,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
                   const RowTuning &tune) {
     const int m = A.rows, n = A.cols, k = B.cols;
     TSG_CHECK(tune.bin1 >= 0 && tune.bin1 <= 64 && tune.bin1 <= tune.bin2 && tune.bin2 <= 256 &&
-                  tune.bin2 <= tune.bin3 && tune.bin3 <= SMALL_PROD,
+                  tune.bin2 <= tune.bin3 && tune.bin3 <= ROW_SMALL_PROD,
               TSG_ERR_INVALID, "row bins out of range");
     p = RowPlan();
     p.m = m;
@@ -1394,6 +1415,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         launch(k_flat_symbolic<64, 8, 64, 512, 64>, 1, 64, 3);
         launch(k_flat_symbolic<64, 16, 64, 512, 64, 6>, 1, 64, 4);
         launch(k_flat_symbolic<64, 16, 1024, 512, 64>, 1, 64, ROW_BIN_MANY);
+        launch(k_flat_symbolic<64, 24, 64, 512, 64>, 1, 64, ROW_BIN_MED);
     }
     tm.end();
 
@@ -1435,6 +1457,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         std::copy(box->v, box->v + 5, tot2);
         const int64_t nsb_total = tot2[0], nunits = tot2[1];
         p.nsb_total = nsb_total;
+        p.big_prod = tot2[3];
         p.subcnt = ws.alloc_n<uint16_t>((size_t)nsb_total + 1);
         // keep every big row's bitmap in sparse form (masks of non-empty
         // words per sub-block, and band word lists: each row's region sized
@@ -1696,11 +1719,17 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
         launch(k_flat_numeric<FUSED, 64, 8, 64, 512, 512, 64>, 1, 64, 3);
         launch(k_flat_numeric<FUSED, 64, 16, 64, 512, 512, 64>, 1, 64, 4);
         launch(k_flat_numeric<FUSED, 64, 16, 1024, 512, 512, 64>, 1, 64, ROW_BIN_MANY);
+        launch(k_flat_numeric<FUSED, 64, 24, 64, 512, 512, 64, 4>, 1, 64, ROW_BIN_MED);
     }
     tm.end();
     if (p.nitems > 0 && p.use_rank) {
         tm.begin("row.big_numeric");
-        if (B.nnz > 0) {
+        if (p.big_prod * 4 < B.nnz) {
+            hipLaunchKernelGGL(k_pack_rows, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0,
+                               s, p.nbig, front.rows(ROW_BIN_BIG), A.ptr, A.idx, B.ptr, B.idx,
+                               B.val, p.bpk);
+            TSG_LAUNCH_CHECK();
+        } else if (B.nnz > 0) {
             hipLaunchKernelGGL(k_pack_b, dim3(grid_for((size_t)B.nnz, 256)), dim3(256), 0, s,
                                B.nnz, B.idx, B.val, p.bpk);
             TSG_LAUNCH_CHECK();
