@@ -43,7 +43,7 @@ enum {
 enum {
     TSG_METHOD_AUTO = 0,    /* tile path for tile-dense A, row path else */
     TSG_METHOD_TILE = 1,    /* 16x16 bitmask tiles (TileSpGEMM)          */
-    TSG_METHOD_ROW = 2      /* row-binned hash / bitmap accumulation     */
+    TSG_METHOD_ROW = 2      /* row-binned accumulation                  */
 };
 
 enum { TSG_FP_FUSED = 0, TSG_FP_SEPARATE = 1 };

@@ -9,12 +9,11 @@ so they can be searched on the workload at hand:
 * ``tile_density``   -- AUTO takes the tile path when A holds at least this
                         many entries per non-empty 16x16 tile;
 * ``row_bins``       -- rows with at most (b1, b2, b3) intermediate products
-                        go to the 16-, 32- and 64-lane LDS-hash kernels (hash
-                        tables of 128, 512 and 2048 slots), longer rows to the
-                        big-row bitmap path;
+                        take 16 lanes or a wave each, with their products in
+                        registers, longer rows go to the big-row bitmap path;
 * ``block_pointer_budget`` -- -1: the library decides whether the big-row
-                        path builds its B block-pointer table or searches B
-                        rows; 6 GiB: the table is built whenever it fits
+                        path builds its table or directory of B or searches B
+                        rows; 6 GiB: it is built whenever it fits
                         (a numeric phase replayed many times may prefer it).
 
 Parameters change speed only: every setting gives bitwise the same C.  The

@@ -615,7 +615,7 @@ __global__ void __launch_bounds__(256) k_dir_runs(int n, int nnz, const int *__r
                                                   const uint2 *__restrict__ cells,
                                                   int2 *__restrict__ runs) {
     __shared__ int s_r[2];
-    const int e0 = blockIdx.x * RUN_ENT, e1 = min(e0 + RUN_ENT, nnz);
+    const int e0 = blockIdx.x * RUN_ENT, e1 = e0 + min(RUN_ENT, nnz - e0);
     if (threadIdx.x < 2) {
         // row of the block's first and last entry: the last t with ib[t] <= e
         const int e = threadIdx.x ? e1 - 1 : e0;
