@@ -771,45 +771,85 @@ constexpr int STEP_U = 4;
 // their run's first positions on, two values a load.  65537 rows of 33 banded
 // entries: 167 -> 116 us (one value a load 180: 31M vector instructions instead
 // of 69M, but the loads' addresses bound it, as they do now, 85% busy).
+//
 constexpr int RUN_FILL = 4;
 // two values in one load (the arrays hold one past their last)
 struct __attribute__((packed, aligned(8))) Pair8 { double x, y; };
 
+// A's values of the unit's rows, at most RUN_A of them, come through LDS: the
+// lanes of a row read the same ones, which as loads cost as many addresses as
+// B's (116 -> 102 us).  A pair's are loaded while the one before is gone
+// through; a unit whose rows hold more reads them from memory.
+constexpr int RUN_A = 64;
+
 template <bool FUSED>
 __device__ __forceinline__ double run_products(const TileArgs &T, const PairMeta *meta, int n,
-                                               int r, int c, double acc) {
+                                               int r, int c, double acc, double *sa) {
+    // the lanes at hand are the first ones, in the order of their outputs' rows
+    const int lanes = __popcll(__ballot(true)), l = __lane_id();
+    const int r0 = __builtin_amdgcn_readfirstlane(r);
+    const int r1 = __builtin_amdgcn_readlane(r, lanes - 1);
+    // the unit's rows' values of pair j: first position, number
+    auto rows_of = [&](int j, int &first, int &num) {
+        const TileRec &A = meta[j].a;
+        first = __builtin_amdgcn_readfirstlane(A.off + A.start[r0]);
+        num = __builtin_amdgcn_readfirstlane(A.off + A.start[r1] + __popc(A.mask[r1])) - first;
+    };
+    int first, num;
+    rows_of(0, first, num);
+    double va = l < num ? T.valA[first + l] : 0.0;
     for (int j = 0; j < n; j++) {
         const unsigned ma = meta[j].a.mask[r], cm = meta[j].b.mask[c];
         const unsigned hits = ma & cm;
         const int len = __popc(hits);
         // past the highest bit of hits: the k before the first product's
         const int past = hits ? 32 - __clz(hits) : 31;
-        const double *pa = T.valA + (meta[j].a.off + meta[j].a.start[r] + __popc(ma >> past));
+        const int ai = meta[j].a.off + meta[j].a.start[r] + __popc(ma >> past);
         const double *pb = T.valB + (meta[j].b.off + meta[j].b.start[c] + __popc(cm >> past));
-        for (int i = 0; i < 16 && __ballot(i < len); i += STEP_U) {
-            Pair8 x[STEP_U / 2], y[STEP_U / 2];
+        const int afirst = first, anum = num;
+        const bool staged = anum <= min(RUN_A, lanes);
+        if (staged) {
+            wave_lds_fence();
+            if (l < anum) sa[l] = va;
+            wave_lds_fence();
+        }
+        if (j + 1 < n) {
+            rows_of(j + 1, first, num);
+            va = l < num ? T.valA[first + l] : 0.0;
+        }
+        auto go = [&](auto value) {
+            for (int i = 0; i < 16 && __ballot(i < len); i += STEP_U) {
+                Pair8 x[STEP_U / 2], y[STEP_U / 2];
 #pragma unroll
-            for (int u = 0; u < STEP_U / 2; u++) {
-                x[u] = Pair8{0.0, 0.0};
-                y[u] = Pair8{0.0, 0.0};
-                if (i + 2 * u < len) {
-                    x[u] = *reinterpret_cast<const Pair8 *>(pa + i + 2 * u);
-                    y[u] = *reinterpret_cast<const Pair8 *>(pb + i + 2 * u);
+                for (int u = 0; u < STEP_U / 2; u++) {
+                    x[u] = Pair8{0.0, 0.0};
+                    y[u] = Pair8{0.0, 0.0};
+                    if (i + 2 * u < len) {
+                        y[u] = *reinterpret_cast<const Pair8 *>(pb + i + 2 * u);
+                        x[u] = value(i + 2 * u);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < STEP_U / 2; u++) {
+                    if (i + 2 * u < len) acc = acc_step<FUSED>(acc, x[u].x, y[u].x);
+                    if (i + 2 * u + 1 < len) acc = acc_step<FUSED>(acc, x[u].y, y[u].y);
                 }
             }
-#pragma unroll
-            for (int u = 0; u < STEP_U / 2; u++) {
-                if (i + 2 * u < len) acc = acc_step<FUSED>(acc, x[u].x, y[u].x);
-                if (i + 2 * u + 1 < len) acc = acc_step<FUSED>(acc, x[u].y, y[u].y);
-            }
-        }
+        };
+        if (staged)
+            go([&](int i) {
+                const int at = ai - afirst + i;
+                return Pair8{sa[at], sa[min(at + 1, RUN_A - 1)]};
+            });
+        else
+            go([&](int i) { return *reinterpret_cast<const Pair8 *>(T.valA + ai + i); });
     }
     return acc;
 }
 
 template <bool FUSED, bool RUNS>
 __device__ __forceinline__ double walk_products(const TileArgs &T, const PairMeta *meta, int n,
-                                                int r, int c, double acc) {
+                                                int r, int c, double acc, double *sa) {
     unsigned live = 0;
     int total = 0;
     bool runs = true;
@@ -824,7 +864,7 @@ __device__ __forceinline__ double walk_products(const TileArgs &T, const PairMet
     }
     if (RUNS && __ballot(!runs) == 0 &&
         2 * __popcll(__ballot(total >= RUN_FILL * n)) >= __popcll(__ballot(true)))
-        return run_products<FUSED>(T, meta, n, r, c, acc);
+        return run_products<FUSED>(T, meta, n, r, c, acc, sa);
     ProductWalk w{meta, r, c, live};
     while (true) {
         int a[STEP_U], b[STEP_U];
@@ -867,6 +907,7 @@ __global__ void __launch_bounds__(256) k_step3_out(int nunits, const int4 *__res
     constexpr int CP = 32 / TPW;
     static_assert(CP <= 32, "a lane's live pairs are a 32-bit mask");
     __shared__ PairMeta s_meta[4][TPW][CP];
+    __shared__ double s_a[4][TPW == 1 ? RUN_A : 1];
     const int lane = __lane_id();
     const int lq = lane % G, g = lane / G;
     PairMeta *meta = s_meta[threadIdx.x >> 6][g];
@@ -917,7 +958,7 @@ __global__ void __launch_bounds__(256) k_step3_out(int nunits, const int4 *__res
             wave_lds_fence();
             if (lq < n) stage_pair(T, pc == 0 ? pr0 : T.pairs[p0 + pc + lq], meta[lq]);
             wave_lds_fence();
-            if (owner) acc = walk_products<FUSED, TPW == 1>(T, meta, n, r, c, acc);
+            if (owner) acc = walk_products<FUSED, TPW == 1>(T, meta, n, r, c, acc, s_a[threadIdx.x >> 6]);
         }
         if (owner) {
             T.jc[o] = J * 16 + c;
