@@ -764,14 +764,12 @@ struct ProductWalk {
 // lane's last product repeat the first and are not accumulated).
 constexpr int STEP_U = 4;
 
-//
 // RUNS (all lanes share the pairs): when the k of every lane's products in
 // every pair are consecutive -- a run in both tiles' values -- and most lanes
 // have at least RUN_FILL a pair, the lanes go through each pair together, from
 // their run's first positions on, two values a load.  65537 rows of 33 banded
 // entries: 167 -> 116 us (one value a load 180: 31M vector instructions instead
-// of 69M, but the loads' addresses bound it, as they do now, 85% busy).
-//
+// of 69M, but the loads' addresses bound it, as they do now).
 constexpr int RUN_FILL = 4;
 // two values in one load (the arrays hold one past their last)
 struct __attribute__((packed, aligned(8))) Pair8 { double x, y; };
