@@ -153,9 +153,9 @@ __device__ __forceinline__ unsigned xcd_piece(unsigned i, unsigned n) {
 }
 
 // Exclusive lower bound of key in sorted a[lo, hi).
-__device__ __forceinline__ int lower_bound_i32(const int *a, int lo, int hi, int key) {
+__host__ __device__ __forceinline__ int lower_bound_i32(const int *a, int lo, int hi, int key) {
     while (lo < hi) {
-        int mid = (lo + hi) >> 1;
+        const int mid = lo + ((hi - lo) >> 1);   // lo + hi may pass 2^31
         if (a[mid] < key) lo = mid + 1; else hi = mid;
     }
     return lo;

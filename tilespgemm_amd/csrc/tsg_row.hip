@@ -500,7 +500,7 @@ constexpr int DIR_ROWS = 256, DIR_GRP = DIR_ROWS / 32, DIR_BLK = 512;
 __device__ __forceinline__ int dir_row_of(const int *rp, int nr, int e) {
     int lo = 0, hi = nr;               // rp[lo] <= e < rp[hi]
     while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
+        const int mid = lo + ((hi - lo) >> 1);
         if (rp[mid] <= e) lo = mid;
         else hi = mid;
     }
