@@ -88,6 +88,17 @@ struct RowRange {
     }
 };
 
+// Position p of a lane's entry in the group of a row's entries that starts at
+// g (PARTS groups interleaved, the lane's the part-th); false past the row's
+// end pe.  Groups are asked for up to three ahead of a row's last, so positions
+// are unsigned: they pass 2^31 at the end of 2^31 - 1 entries.
+template <int PARTS>
+__host__ __device__ __forceinline__ bool entry_at(unsigned g, unsigned pe, int part, int lane,
+                                                  unsigned &p) {
+    p = g + (unsigned)(PARTS * lane + part);
+    return p < pe;
+}
+
 // A row's entries [pa, pe) in groups of 64, loaded ahead of their use: while
 // a group's products are processed, the next group's B ranges and values, the
 // cells of the group after that and the A columns of the third are loading.
@@ -98,22 +109,23 @@ template <bool VALUES, int PARTS>
 struct EntryPipe {
     const int *ja;
     const double *aval;
-    int pa, pe, part;
+    unsigned pa, pe;
+    int part;
     int t1, t2;
     uint2 w1;
     int lo, hi, lo1, hi1;          // the group's ranges, and the next one's
     double a, a1;
-    __device__ __forceinline__ int col(int g) const {
-        const int p = g + PARTS * __lane_id() + part;
-        return g < pe && p < pe ? ja[p] : -1;
+    __device__ __forceinline__ int col(unsigned g) const {
+        unsigned p;
+        return entry_at<PARTS>(g, pe, part, __lane_id(), p) ? ja[p] : -1;
     }
-    __device__ __forceinline__ double val(int g) const {
-        const int p = g + PARTS * __lane_id() + part;
-        return VALUES && g < pe && p < pe ? aval[p] : 0.0;
+    __device__ __forceinline__ double val(unsigned g) const {
+        unsigned p;
+        return VALUES && entry_at<PARTS>(g, pe, part, __lane_id(), p) ? aval[p] : 0.0;
     }
     __device__ __forceinline__ void load(int pa_, int pe_) {
-        pa = pa_;
-        pe = pe_;
+        pa = (unsigned)pa_;
+        pe = (unsigned)pe_;
         t1 = col(pa);
         t2 = col(pa + 64 * PARTS);
     }
@@ -123,7 +135,7 @@ struct EntryPipe {
     }
     // the next group's ranges, and what lies behind them; g: the group at hand
     template <class R>
-    __device__ __forceinline__ void ahead(int g, const R &rows) {
+    __device__ __forceinline__ void ahead(unsigned g, const R &rows) {
         rows.range(t1, w1, lo1, hi1);
         a1 = val(g + 64 * PARTS);
         t1 = t2;
@@ -294,7 +306,7 @@ __device__ __forceinline__ void for_products(int pa, int pe, const int *__restri
     pipe.load(pa, pe);
     pipe.cells(rows);
     pipe.first(rows);
-    for (int g = pa; g < pe; g += 64 * PARTS) {
+    for (unsigned g = pipe.pa; g < pipe.pe; g += 64 * PARTS) {
         pipe.ahead(g, rows);
         expand_group<U, VALUES>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, jb, bval, heads, f);
         pipe.take();

@@ -83,11 +83,12 @@ __device__ __forceinline__ int flat_entries(FlatSmem<P, E, LW, ACC> &S, int pa, 
     for (int i = l; i < P / 32; i += G) S.starts[i] = 0u;
     wave_lds_fence();
     int nprod = 0, nent = 0;
-    for (int g = pa; g < pe; g += G) {
-        const int p = g + l;
+    // (unsigned: g passes 2^31 at the end of 2^31 - 1 entries)
+    for (unsigned g = (unsigned)pa; g < (unsigned)pe; g += G) {
+        const unsigned p = g + (unsigned)l;
         int cnt = 0, lo = 0;
         double av = 0.0;
-        if (p < pe) {
+        if (p < (unsigned)pe) {
             const int t = ja[p];
             if (ACC > 1) av = aval[p];
             lo = ib[t];

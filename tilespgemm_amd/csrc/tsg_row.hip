@@ -250,7 +250,8 @@ __global__ void __launch_bounds__(256) k_big_span(int nbig, const int *__restric
     if (r >= nbig) return;
     const int row = rows[r];
     int lo = 0x7fffffff, hi = -1;
-    for (int p = ia[row] + l; p < ia[row + 1]; p += 64) {
+    const unsigned pe = (unsigned)ia[row + 1];
+    for (unsigned p = (unsigned)ia[row] + l; p < pe; p += 64) {
         const int t = ja[p];
         const int b0 = ib[t], b1 = ib[t + 1];
         if (b0 < b1) {
@@ -520,10 +521,10 @@ __global__ void __launch_bounds__(1024) k_dir_bits(int n, const int *__restrict_
     for (int b0 = 0; b0 < nblk; b0 += DIR_BLK) {
         for (int i = threadIdx.x; i < DIR_BLK * DIR_GRP; i += blockDim.x) s_bits[i] = 0u;
         __syncthreads();
-        for (int e = s_rp[0] + threadIdx.x; e < s_rp[nr]; e += blockDim.x) {
+        for (unsigned e = s_rp[0] + threadIdx.x; e < (unsigned)s_rp[nr]; e += blockDim.x) {
             const int b = (jb[e] >> shift) - b0;
             if (b >= 0 && b < DIR_BLK) {
-                const int r = dir_row_of(s_rp, nr, e);
+                const int r = dir_row_of(s_rp, nr, (int)e);
                 lds_set_bit(&s_bits[b * DIR_GRP + (r >> 5)], 1u << (r & 31));
             }
         }
@@ -622,7 +623,8 @@ __global__ void __launch_bounds__(256) k_dir_runs(int n, int nnz, const int *__r
         s_r[threadIdx.x] = lower_bound_i32(ib, 0, n, e + 1) - 1;
     }
     __syncthreads();
-    for (int e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
+    for (unsigned q = threadIdx.x; q < (unsigned)(e1 - e0); q += blockDim.x) {
+        const int e = e0 + (int)q;
         const int r = lower_bound_i32(ib, s_r[0], s_r[1] + 1, e + 1) - 1;
         const int c = jb[e];
         // level-0 blocks of the entry and of its neighbours (-1: none)
@@ -1159,7 +1161,7 @@ __device__ __forceinline__ void dense_item(RankSmem<WORDS> &S, const ItemRec &re
     pipe.first(range);
     const int cnt = item_rank_build(S, wv, c0, c1, o, T.jc);
     auto f = [&](const Batch &t) { item_accumulate<FUSED>(S, c0, t, T.b_strict); };
-    for (int g = pipe.pa; g < pipe.pe; g += 64) {
+    for (unsigned g = pipe.pa; g < pipe.pe; g += 64) {
         pipe.ahead(g, range);
         expand_group<RANK_U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, T.jb, nullptr,
                                          S.heads, f, T.bpk);
@@ -1271,7 +1273,7 @@ __device__ __forceinline__ void sparse_item(SparseSmem<CAP, U> &S, const ItemRec
                                           false);
         }
     };
-    for (int g = pipe.pa; g < pipe.pe; g += 64) {
+    for (unsigned g = pipe.pa; g < pipe.pe; g += 64) {
         pipe.ahead(g, range);
         expand_group<U, true, true>(pipe.lo, max(pipe.hi - pipe.lo, 0), pipe.a, T.jb, nullptr,
                                     S.heads, f, T.bpk);

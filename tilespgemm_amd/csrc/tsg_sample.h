@@ -17,18 +17,20 @@ template <int NT>
 struct TileCols {
     int p1, cmax;
     const int *ja;
-    __device__ void load(int p, int (&J)[TC_U]) const {
+    // (positions are unsigned: a pass ends past 2^31 at the end of 2^31 - 1
+    // entries)
+    __device__ void load(unsigned p, int (&J)[TC_U]) const {
 #pragma unroll
         for (int q = 0; q < TC_U; q++) {
-            const int pq = p + q * NT;
-            J[q] = pq < p1 ? min(max(ja[pq], 0), cmax) >> 4 : -1;
+            const unsigned pq = p + (unsigned)(q * NT);
+            J[q] = pq < (unsigned)p1 ? min(max(ja[pq], 0), cmax) >> 4 : -1;
         }
     }
     // tile-column range of the entries [p0 + t, p1) taken by thread t
     __device__ void range(int p0, int t, int &lo, int &hi) const {
         lo = INT_MAX;
         hi = -1;
-        for (int p = p0 + t; p < p1; p += NT * TC_U) {
+        for (unsigned p = (unsigned)p0 + t; p < (unsigned)p1; p += NT * TC_U) {
             int J[TC_U];
             load(p, J);
 #pragma unroll
@@ -40,7 +42,7 @@ struct TileCols {
         }
     }
     __device__ void mark(int p0, int t, int w0, int w1, unsigned *bits) const {
-        for (int p = p0 + t; p < p1; p += NT * TC_U) {
+        for (unsigned p = (unsigned)p0 + t; p < (unsigned)p1; p += NT * TC_U) {
             int J[TC_U];
             load(p, J);
 #pragma unroll

@@ -314,9 +314,10 @@ __global__ void k_row_pos(int m, const int *__restrict__ ia, int *__restrict__ r
     const int row = (blockIdx.x * blockDim.x + threadIdx.x) >> 3;
     const int l = threadIdx.x & 7;
     if (row >= m) return;
-    for (int p = ia[row] + l; p < ia[row + 1]; p += 8) {
+    const unsigned pe = (unsigned)ia[row + 1];
+    for (unsigned p = (unsigned)ia[row] + l; p < pe; p += 8) {
         rowidx[p] = row;
-        pos[p] = p;
+        pos[p] = (int)p;
     }
 }
 
