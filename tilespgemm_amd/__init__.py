@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 from dataclasses import dataclass
 
 import numpy as np
@@ -231,8 +232,9 @@ class Result(C.Structure):
 class Server:
     """Continuous-batching request server on one device (tsg_server_*).
 
-    submit(A, B) enqueues C = A*B on device-resident operands (keep them alive
-    until the result is released) and returns a ticket; wait(ticket) blocks
+    submit(A, B) enqueues C = A*B on device-resident operands (finished, or
+    made by torch on its default stream; keep them alive until the result is
+    released) and returns a ticket; wait(ticket) blocks
     and returns the Result; fetch(ticket) copies it to host numpy arrays and
     releases it.  The estimator and each worker use a stream of their own:
     set GPU_MAX_HW_QUEUES to at least workers + 1 plus the caller's busy
@@ -336,10 +338,36 @@ def _d2d(dst, src_ptr: int):
         raise TsgError(-5, f"hipMemcpy device->device failed ({rc})")
 
 
+# Stream of the handles made on torch's default stream, one a device (kept for
+# the process).  A stream each would order with torch's default stream but not
+# with one another, while one handle's results are another's operands and torch
+# hands a dropped result's memory to whoever asks next: it knows of the default
+# stream only.
+_default_streams: dict = {}
+_default_streams_mu = threading.Lock()
+
+
+def _default_stream(device: int) -> int:
+    """A blocking stream: it orders with the null stream, which is torch's
+    default."""
+    import torch
+    with _default_streams_mu:
+        if device not in _default_streams:
+            s = C.c_void_p()
+            with torch.cuda.device(device):
+                rc = load().hipStreamCreate(C.byref(s))
+            if rc != 0:
+                raise TsgError(-5, f"hipStreamCreate failed ({rc})")
+            _default_streams[device] = s.value
+        return _default_streams[device]
+
+
 class Handle:
     """A tsg handle on one device.  Work is issued on torch's current stream
-    of that device (or, for torch's default stream, on a blocking stream that
-    orders with it), so results order naturally with torch operations."""
+    of that device, so results order naturally with torch operations and with
+    those of other handles on that stream.  For torch's default stream it is a
+    blocking stream that orders with it, shared by all such handles of the
+    device; handles that are to run side by side take streams of their own."""
 
     def __init__(self, device: int = 0, method: int = METHOD_AUTO,
                  fp_mode: int = FP_FUSED, timing: bool = False):
@@ -351,11 +379,7 @@ class Handle:
         self._h = h
         with torch.cuda.device(device):
             self.stream = torch.cuda.current_stream()
-        # torch's default stream is the null stream; the handle's own stream is
-        # a blocking stream that orders with it.  Any other torch stream is
-        # used directly.
-        if self.stream.cuda_stream:
-            _check(load().tsg_set_stream(self._h, C.c_void_p(self.stream.cuda_stream)), self._h)
+        self.set_stream(self.stream)
         self.set_method(method)
         _check(load().tsg_set_fp_mode(self._h, fp_mode), self._h)
         if timing:
@@ -373,8 +397,10 @@ class Handle:
             pass
 
     def set_stream(self, stream):
-        """Issue work on a torch stream (None: the handle's own stream)."""
+        """Issue work on a torch stream (None: torch's default stream)."""
         ptr = stream.cuda_stream if stream is not None else 0
+        if not ptr:
+            ptr = _default_stream(self.device)
         _check(load().tsg_set_stream(self._h, C.c_void_p(ptr)), self._h)
         self.stream = stream
 
