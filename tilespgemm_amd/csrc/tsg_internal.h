@@ -223,6 +223,14 @@ __host__ __device__ __forceinline__ int64_t run_dir_block(int nblk, int shift, i
     return 2ll * nblk - (2ll * nblk >> v) + (c >> (shift + v));
 }
 
+// Sub-blocks of the big rows' columns: first column of the sb-th, k past the
+// matrix's last (2^31 itself does not fit an int).
+constexpr int SUB_SHIFT = 10;          // 1024 columns
+__host__ __device__ __forceinline__ int sub_block_start(int sb, int k) {
+    const int64_t c = (int64_t)sb << SUB_SHIFT;
+    return c < k ? (int)c : k;
+}
+
 constexpr int ITEM_CLASSES = 3;       // size classes of the row path's items
 
 struct RowPlan {

@@ -40,7 +40,6 @@
 
 namespace {
 
-constexpr int SUB_SHIFT = 10;          // sub-block = 1024 columns
 constexpr int BAND_SHIFT = 6;          // symbolic band = 64 sub-blocks (65536 columns)
 constexpr int BAND_T = 128;            // threads per band unit
 constexpr int BAND_WORDS = (1 << (BAND_SHIFT + SUB_SHIFT)) / 32;
@@ -369,7 +368,7 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
         const int nsb = (int)min((int64_t)((u + 1) << BAND_SHIFT) - lead - j0, sb_off[r + 1] - so);
         const int sb0 = span_sb0[r] + j0;
         const int c0 = sb0 << SUB_SHIFT;
-        const int c1 = (int)min((int64_t)k, (int64_t)(sb0 + nsb) << SUB_SHIFT);
+        const int c1 = sub_block_start(sb0 + nsb, k);
         const int words = (c1 - c0 + 31) >> 5;
         for (int i = threadIdx.x; 4 * i < words; i += BAND_T)
             reinterpret_cast<uint4 *>(bits)[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -814,7 +813,7 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                 words ? band_base[band_off[r] + win / WPB] + (nz_excl - band_nz) : 0;
             if (run > 1) {
                 items[w] = ItemRec{make_int4(row, (first + sb_first) << SUB_SHIFT,
-                                             min(k, (first + sb_last + 1) << SUB_SHIFT),
+                                             sub_block_start(first + sb_last + 1, k),
                                              words ? (int)(sb_off[r] + sb_first) : r),
                                    out, wb};
                 item_n[w] = run_tot;
@@ -835,7 +834,7 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                 nzrun += os[q];
                 if (ends[q] && cnt > 0) {
                     items[w] = ItemRec{make_int4(row, (cbase + start) << SUB_SHIFT,
-                                                 min(k, (cbase + stop) << SUB_SHIFT),
+                                                 sub_block_start(cbase + stop, k),
                                                  words ? (int)(sb_off[r] + j0 + start) : r),
                                        out, wb + nzs};
                     item_n[w] = cnt;
