@@ -3,8 +3,6 @@
 // row's outputs, shared by the row path's symbolic and numeric kernels.
 #pragma once
 
-#include <type_traits>
-
 #include "tsg_device.h"
 
 // One group of G lanes owns one row of at most P = G * U products, product
@@ -21,11 +19,14 @@
 //            below q) - 1: one count instead of a search or a running
 //            maximum.
 //   ranks    by a bitmap of two levels, so that its space depends on the
-//            products and hardly on the columns' span: a bit per 16 columns
-//            of a window of LW * 512 columns, numbered in order; then the
+//            products and not on the columns' span: a bit per 16 columns over
+//            a span of up to LW * 512 columns, numbered in order; then the
 //            row's own 16-column words, one per level-1 bit set, their bits
-//            and the outputs before them in one int.  A span wider than the
-//            window takes several windows.
+//            and the outputs before them in one int.  In a wider span the
+//            16-column words are first numbered in blocks of 2^s of them, as
+//            many as level 1 has bits for, and the empty blocks between them
+//            left out, which divides the span by LW * 32 / P or more; once for
+//            2^20 columns, four times for 2^31.
 //
 // LDS: the steps after the entries reuse the same space one after the other.
 // E bounds the entries with products; VALS: their values are kept too; ACC:
@@ -154,14 +155,13 @@ template <int G, int NB, bool RANKS, int P, int E, int LW, int ACC>
 __device__ __forceinline__ int flat_ranks(FlatSmem<P, E, LW, ACC> &S, const int (&col)[NB],
                                           int (&rank)[NB], bool repeats) {
     const int l = __lane_id() & (G - 1);
-    constexpr int WIN = LW << 9;                   // columns of a window
     int lo = 0x7fffffff, hi = -1;
 #pragma unroll
     for (int u = 0; u < NB; u++) {
         lo = min(lo, col[u]);
         hi = max(hi, col[u]);
     }
-    lo = group_uniform<G>(group_min_i32<G>(lo));
+    lo = group_uniform<G>(group_min_i32<G>(lo)) & ~15;   // a 16-column word's first
     hi = group_uniform<G>(group_max_i32<G>(hi));
     if constexpr (!RANKS) {
         // counted alone, columns of a span that fits need one level of bits
@@ -185,81 +185,95 @@ __device__ __forceinline__ int flat_ranks(FlatSmem<P, E, LW, ACC> &S, const int 
             return group_sum<G>(n);
         }
     }
-    // one window of columns from lo; part: it may leave some out
-    auto window = [&](int done, auto part_t) {
-        constexpr bool part = decltype(part_t)::value;
-        auto in = [&](int u) { return !part || (col[u] >= lo && col[u] - lo < WIN); };
-        auto each = [&](auto f) {
+    auto each = [&](auto f) {
 #pragma unroll
-            for (int u = 0; u < NB; u++)
-                if (in(u)) f(u, col[u] - lo);
-        };
-        auto set_all = [&](auto word, auto bit) {
-            if (repeats)
-                each([&](int u, int cc) { lds_set_bit(word(u, cc), bit(cc)); });
-            else
-                each([&](int u, int cc) { atomicOr(word(u, cc), bit(cc)); });
-        };
-        const int n1 = part ? LW : ((hi - lo) >> 9) + 1;
+        for (int u = 0; u < NB; u++) f(u);
+    };
+    auto set_all = [&](auto word, auto bit) {
+        if (repeats)
+            each([&](int u) { lds_set_bit(word(u), bit(u)); });
+        else
+            each([&](int u) { atomicOr(word(u), bit(u)); });
+    };
+    // The places at(u), at most top < 32 * LW, numbered in order by level 1's
+    // bits; between(u), then put(u, number of the place).  Returns their number.
+    auto number = [&](int top, auto at, auto between, auto put) {
+        const int n1 = (top >> 5) + 1;
         for (int i = l; i < n1; i += G) S.l1[i] = make_uint2(0u, 0u);
         wave_lds_fence();
-        set_all([&](int, int cc) { return &S.l1[cc >> 9].x; },
-                [&](int cc) { return 1u << ((cc >> 4) & 31); });
+        set_all([&](int u) { return &S.l1[at(u) >> 5].x; },
+                [&](int u) { return 1u << (at(u) & 31); });
         wave_lds_fence();
-        int n2 = 0;
+        int n = 0;
         for (int i0 = 0; i0 < n1; i0 += G) {
             const int i = i0 + l;
             const int pc = i < n1 ? __popc(S.l1[i].x) : 0;
             const int incl = group_incl_scan<G>(pc);
-            if (i < n1) S.l1[i].y = (unsigned)(n2 + incl - pc);
-            n2 += group_last<G>(incl);
+            if (i < n1) S.l1[i].y = (unsigned)(n + incl - pc);
+            n += group_last<G>(incl);
         }
         wave_lds_fence();
-        // rank holds the word's number until the column's rank replaces it
-        each([&](int u, int cc) {
-            const uint2 v = S.l1[cc >> 9];
-            rank[u] = (int)v.y + __popc(v.x & ((1u << ((cc >> 4) & 31)) - 1u));
+        each(between);
+        each([&](int u) {
+            const uint2 v = S.l1[at(u) >> 5];
+            put(u, (int)v.y + __popc(v.x & ((1u << (at(u) & 31)) - 1u)));
         });
         wave_lds_fence();
-        for (int i = l; i < n2; i += G) S.l2[i] = 0u;
-        wave_lds_fence();
-        set_all([&](int u, int) { return &S.l2[rank[u]]; },
-                [&](int cc) { return 1u << (cc & 15); });
-        wave_lds_fence();
-        if constexpr (RANKS) {
-            int n = done;
-            for (int i0 = 0; i0 < n2; i0 += G) {
-                const int i = i0 + l;
-                const unsigned v = i < n2 ? S.l2[i] : 0u;
-                const int pc = __popc(v);
-                const int incl = group_incl_scan<G>(pc);
-                if (i < n2) S.l2[i] = v | ((unsigned)(n + incl - pc) << 16);
-                n += group_last<G>(incl);
-            }
-            wave_lds_fence();
-            each([&](int u, int cc) {
-                const unsigned v = S.l2[rank[u]];
-                rank[u] = (int)(v >> 16) + __popc(v & ((1u << (cc & 15)) - 1u));
-            });
-            wave_lds_fence();
-            return n;
-        } else {
-            int n = 0;
-            for (int i = l; i < n2; i += G) n += __popc(S.l2[i]);
-            return done + group_sum<G>(n);
-        }
+        return n;
     };
-    if (hi - lo < WIN) return window(0, std::false_type());
-    int done = 0;                                  // outputs of earlier windows
-    while (true) {
-        done = window(done, std::true_type());
-        if (hi - lo < WIN) return done;
-        // the next window starts at the first column past this one
-        const int past = lo + (WIN - 1);
-        int next = hi;
-#pragma unroll
-        for (int u = 0; u < NB; u++)
-            if (col[u] > past) next = min(next, col[u]);
-        lo = group_uniform<G>(group_min_i32<G>(next));
+    // rank holds the number of the product's 16-column word until the column's
+    // rank replaces it
+    constexpr int LOG = 31 - __builtin_clz(LW * 32);
+    static_assert(LW * 32 == 1 << LOG && LW * 32 >= 4 * P, "numbering blocks shortens the span");
+    auto word = [&](int u) { return (col[u] - lo) >> 4; };
+    int top = (hi - lo) >> 4, n2;
+    if (top < LW * 32) {
+        n2 = number(top, word, [](int) {}, [&](int u, int v) { rank[u] = v; });
+    } else {
+        // 32768 rows of 900 products, both phases: 0.46 ms over 2^24 columns,
+        // 0.54 over 2^30 (0.35 within the span); a span's worth of level 1
+        // after the other took 3.5 and 30
+        each([&](int u) { rank[u] = word(u); });
+        int s;
+        do {
+            s = max(32 - __builtin_clz(top | 1) - LOG, 0);
+            n2 = number(
+                top >> s, [&](int u) { return rank[u] >> s; },
+                [&](int u) {
+                    // places are made again after the scan: kept over it they
+                    // cost the kernel a wave per SIMD (134 registers, not 108)
+                    int x = rank[u];
+                    asm volatile("" : "+v"(x));
+                    rank[u] = x;
+                },
+                [&](int u, int v) { rank[u] = (v << s) | (rank[u] & ((1 << s) - 1)); });
+            top = (n2 << s) - 1;
+        } while (s > 0);
+    }
+    for (int i = l; i < n2; i += G) S.l2[i] = 0u;
+    wave_lds_fence();
+    auto in_word = [&](int u) { return col[u] & 15; };
+    set_all([&](int u) { return &S.l2[rank[u]]; }, [&](int u) { return 1u << in_word(u); });
+    wave_lds_fence();
+    int n = 0;
+    if constexpr (RANKS) {
+        for (int i0 = 0; i0 < n2; i0 += G) {
+            const int i = i0 + l;
+            const unsigned v = i < n2 ? S.l2[i] : 0u;
+            const int pc = __popc(v);
+            const int incl = group_incl_scan<G>(pc);
+            if (i < n2) S.l2[i] = v | ((unsigned)(n + incl - pc) << 16);
+            n += group_last<G>(incl);
+        }
+        wave_lds_fence();
+        each([&](int u) {
+            const unsigned v = S.l2[rank[u]];
+            rank[u] = (int)(v >> 16) + __popc(v & ((1u << in_word(u)) - 1u));
+        });
+        wave_lds_fence();
+        return n;
+    } else {
+        for (int i = l; i < n2; i += G) n += __popc(S.l2[i]);
+        return group_sum<G>(n);
     }
 }
