@@ -494,7 +494,11 @@ __global__ void __launch_bounds__(256) k_bptr_rows(int n, const int *__restrict_
 // The bits go out cell-major, DIR_ROWS / 32 consecutive cells a block.  Bound
 // by the busiest block, that of the longest rows: 1.2 ms with 512 rows and
 // threads a block (R-MAT 2^20), 0.6 with 256 and 1024.
-constexpr int DIR_ROWS = 256, DIR_GRP = DIR_ROWS / 32, DIR_BLK = 512;
+// Up to DIR_WHOLE ranges a block goes through its rows' entries for each of
+// them.  Past that (CUT) it has one range and searches each row's entries in
+// it, so that B is read once however many columns it has (B of 1000 rows of
+// 20,000 entries over 2^28 columns, symbolic phase 857 -> 7.0 ms).
+constexpr int DIR_ROWS = 256, DIR_GRP = DIR_ROWS / 32, DIR_BLK = 512, DIR_WHOLE = 2;
 
 // row (of nr from the first) of the entry at position e: rp ascending
 __device__ __forceinline__ int dir_row_of(const int *rp, int nr, int e) {
@@ -507,23 +511,48 @@ __device__ __forceinline__ int dir_row_of(const int *rp, int nr, int e) {
     return lo;
 }
 
+template <bool CUT>
 __global__ void __launch_bounds__(1024) k_dir_bits(int n, const int *__restrict__ ib,
                                                   const int *__restrict__ jb, int ngrp, int nblk,
                                                   int shift, int levels,
                                                   unsigned *__restrict__ bits) {
     __shared__ int s_rp[DIR_ROWS + 1];
+    __shared__ int s_first[CUT ? DIR_ROWS : 1], s_wave[CUT ? DIR_ROWS / 64 : 1];
     __shared__ unsigned s_bits[2 * DIR_BLK * DIR_GRP];
-    const int t0 = blockIdx.x * DIR_ROWS, g0 = blockIdx.x * DIR_GRP;
+    const int t = threadIdx.x, t0 = blockIdx.x * DIR_ROWS, g0 = blockIdx.x * DIR_GRP;
     const int nr = min(DIR_ROWS, n - t0), ng = min(DIR_GRP, ngrp - g0);
-    for (int i = threadIdx.x; i <= nr; i += blockDim.x) s_rp[i] = ib[t0 + i];
+    if (!CUT)
+        for (int i = t; i <= nr; i += blockDim.x) s_rp[i] = ib[t0 + i];
     __syncthreads();
-    for (int b0 = 0; b0 < nblk; b0 += DIR_BLK) {
-        for (int i = threadIdx.x; i < DIR_BLK * DIR_GRP; i += blockDim.x) s_bits[i] = 0u;
+    for (int b0 = blockIdx.y * DIR_BLK; b0 < nblk; b0 += gridDim.y * DIR_BLK) {
+        if (CUT) {
+            // the rows' entries in the range, back to back: first and count
+            int lo = 0, hi = 0, incl = 0;
+            if (t < nr) {
+                const int end = ib[t0 + t + 1];
+                const int64_t past = (int64_t)(b0 + DIR_BLK) << shift;
+                lo = lower_bound_i32(jb, ib[t0 + t], end, b0 << shift);
+                hi = past <= 0x7fffffff ? lower_bound_i32(jb, lo, end, (int)past) : end;
+            }
+            if (t < DIR_ROWS) {
+                incl = wave_incl_scan(hi - lo);
+                if ((t & 63) == 63) s_wave[t >> 6] = incl;
+            }
+            __syncthreads();
+            if (t < DIR_ROWS) {
+                for (int w = 0; w < t >> 6; w++) incl += s_wave[w];
+                s_rp[t + 1] = incl;
+                s_first[t] = lo - (incl - (hi - lo));
+                if (t == 0) s_rp[0] = 0;
+            }
+        }
+        for (int i = t; i < DIR_BLK * DIR_GRP; i += blockDim.x) s_bits[i] = 0u;
         __syncthreads();
-        for (unsigned e = s_rp[0] + threadIdx.x; e < (unsigned)s_rp[nr]; e += blockDim.x) {
-            const int b = (jb[e] >> shift) - b0;
+        for (unsigned e = s_rp[0] + t; e < (unsigned)s_rp[nr]; e += blockDim.x) {
+            int r = CUT ? dir_row_of(s_rp, nr, (int)e) : 0;
+            const int b = (jb[CUT ? s_first[r] + (int)e : (int)e] >> shift) - b0;
             if (b >= 0 && b < DIR_BLK) {
-                const int r = dir_row_of(s_rp, nr, (int)e);
+                if (!CUT) r = dir_row_of(s_rp, nr, (int)e);
                 lds_set_bit(&s_bits[b * DIR_GRP + (r >> 5)], 1u << (r & 31));
             }
         }
@@ -1552,8 +1581,12 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
                 p.dir.nblk = (int)nblk;
                 p.dir.shift = SUB_SHIFT + c;
                 p.dir.coarse = c > 0;
-                hipLaunchKernelGGL(k_dir_bits, dim3(grid_for((size_t)n, DIR_ROWS)), dim3(1024), 0,
-                                   s, n, B.ptr, B.idx, ngrp, p.dir.nblk, p.dir.shift, levels, bits);
+                const unsigned ranges = grid_for((size_t)nblk, DIR_BLK, 65535);
+                const bool cut = ranges > DIR_WHOLE;
+                hipLaunchKernelGGL(cut ? k_dir_bits<true> : k_dir_bits<false>,
+                                   dim3(grid_for((size_t)n, DIR_ROWS), cut ? ranges : 1),
+                                   dim3(1024), 0, s, n, B.ptr, B.idx, ngrp, p.dir.nblk,
+                                   p.dir.shift, levels, bits);
                 TSG_LAUNCH_CHECK();
                 hipLaunchKernelGGL(k_dir_sums, dim3((unsigned)chunks), dim3(256), 0, s, ncells,
                                    bits, sums);
