@@ -240,7 +240,8 @@ struct RowPlan {
     RowFront front;                  // products per row, rows per bin
     // big-row structures
     int nbig = 0;
-    int64_t big_prod = 0;            // products of the big rows
+    int64_t big_ent = 0, big_prod = 0;   // the big rows' A entries and products
+    int64_t *ent_off = nullptr;      // [nbig+1] A entries of the big rows before each
     int sub_shift = 0;               // log2 sub-block width (columns)
     int *span_sb0 = nullptr;         // [nbig] first sub-block of the row's span
     int64_t *sb_off = nullptr;       // [nbig+1] span offsets (sub-blocks)

@@ -1358,26 +1358,61 @@ __global__ void __launch_bounds__(256) k_pack_b(int64_t nnz, const int *__restri
     bpk[q] = make_int4(jb[q], 0, __double2loint(v), __double2hiint(v));
 }
 
-// The same for the B rows that big rows name, a wave per big row (rows named
-// more than once are written with the same records): with few big rows that is
-// less than all of B (ER batch of 512 matrices: 0.67 -> 0.08 ms).
-__global__ void __launch_bounds__(256) k_pack_rows(int nbig, const int *__restrict__ rows,
+// The same for the B rows that big rows name (rows named more than once are
+// written with the same records): with few big rows that is less than all of
+// B.  A block takes PACK_ENT of the big rows' A entries, whichever rows they
+// are of (ent_off: entries of the rows before each), and blockIdx.y its share
+// of their B entries, flat, so neither a long row of A nor long B rows are one
+// wave's work (a wave per big row took 25 ms for one of 50,000 entries).
+//
+// All of B takes 4.3 ps an entry, named rows 1.2 to 2 ns an A entry as they
+// lie apart, from 5 us up: 7.4M entries of B 32 us, or 5 us with 1000 A entries,
+// 20 with 16,000, 103 with 50,000; 32.5M entries 136 us, or 62 with 50,000; ER
+// batch of 512 matrices 670 us, or 32.
+constexpr int PACK_ENT = 64, PACK_ENT_COST = 256, PACK_PROD_COST = 4;
+
+__global__ void __launch_bounds__(256) k_pack_rows(int64_t nent, int nbig,
+                                                   const int64_t *__restrict__ ent_off,
+                                                   const int *__restrict__ rows,
                                                    const int *__restrict__ ia,
                                                    const int *__restrict__ ja,
                                                    const int *__restrict__ ib,
                                                    const int *__restrict__ jb,
                                                    const double *__restrict__ b,
                                                    int4 *__restrict__ bpk) {
-    const int r = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int l = __lane_id();
-    if (r >= nbig) return;
-    const int row = rows[r];
-    for (int p = ia[row]; p < ia[row + 1]; p++) {
-        const int t = ja[p];
-        for (int q = ib[t] + l; q < ib[t + 1]; q += 64) {
-            const double v = b[q];
-            bpk[q] = make_int4(jb[q], 0, __double2loint(v), __double2hiint(v));
+    __shared__ int s_end[PACK_ENT], s_first[PACK_ENT];
+    static_assert(PACK_ENT == 64, "a lane per entry");
+    if (threadIdx.x < PACK_ENT) {
+        const int64_t e = (int64_t)blockIdx.x * PACK_ENT + threadIdx.x;
+        int lo = 0, cnt = 0;
+        if (e < nent) {
+            int r = 0, hi = nbig;              // ent_off[r] <= e < ent_off[hi]
+            while (hi - r > 1) {
+                const int mid = r + ((hi - r) >> 1);
+                if (ent_off[mid] <= e) r = mid;
+                else hi = mid;
+            }
+            const int row = rows[r], p = ia[row] + (int)(e - ent_off[r]);
+            if (p < ia[row + 1]) {
+                const int t = ja[p];
+                lo = ib[t];
+                cnt = max(ib[t + 1] - lo, 0);
+            }
         }
+        const int incl = wave_incl_scan(cnt);
+        s_end[threadIdx.x] = incl;
+        s_first[threadIdx.x] = lo - (incl - cnt);
+    }
+    __syncthreads();
+    const unsigned total = (unsigned)s_end[PACK_ENT - 1];
+    for (unsigned q = blockIdx.y * 256 + threadIdx.x; q < total; q += gridDim.y * 256) {
+        int i = 0;                             // the first entry that ends past q
+#pragma unroll
+        for (int z = PACK_ENT / 2; z > 0; z >>= 1)
+            if ((unsigned)s_end[i + z - 1] <= q) i += z;
+        const int p = s_first[i] + (int)q;
+        const double v = b[p];
+        bpk[p] = make_int4(jb[p], 0, __double2loint(v), __double2hiint(v));
     }
 }
 
@@ -1464,7 +1499,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         p.sb_off = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         band_off = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         int64_t *tmp_sb = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)p.nbig + 1));
-        int64_t *a_ent = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
+        int64_t *a_ent = p.ent_off = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         int64_t *a_prod = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         row_loff = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         hipLaunchKernelGGL(k_big_span, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0, s,
@@ -1487,6 +1522,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         std::copy(box->v, box->v + 5, tot2);
         const int64_t nsb_total = tot2[0], nunits = tot2[1];
         p.nsb_total = nsb_total;
+        p.big_ent = tot2[2];
         p.big_prod = tot2[3];
         p.subcnt = ws.alloc_n<uint16_t>((size_t)nsb_total + 1);
         // keep every big row's bitmap in sparse form (masks of non-empty
@@ -1758,9 +1794,11 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
     tm.end();
     if (p.nitems > 0 && p.use_rank) {
         tm.begin("row.big_numeric");
-        if (p.big_prod * 4 < B.nnz) {
-            hipLaunchKernelGGL(k_pack_rows, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0,
-                               s, p.nbig, front.rows(ROW_BIN_BIG), A.ptr, A.idx, B.ptr, B.idx,
+        if (p.big_ent * PACK_ENT_COST < B.nnz && p.big_prod * PACK_PROD_COST < B.nnz) {
+            const unsigned groups = grid_for((size_t)p.big_ent, PACK_ENT);
+            const unsigned share = std::min(std::max(4096u / groups, 4u), 64u);
+            hipLaunchKernelGGL(k_pack_rows, dim3(groups, share), dim3(256), 0, s, p.big_ent, p.nbig,
+                               p.ent_off, front.rows(ROW_BIN_BIG), A.ptr, A.idx, B.ptr, B.idx,
                                B.val, p.bpk);
             TSG_LAUNCH_CHECK();
         } else if (B.nnz > 0) {
