@@ -197,9 +197,9 @@ int tsg_spgemm_numeric(tsg_handle_t handle, int m, int n, int k,
  * entries.  Writes d_ic and *nnz_c; when nnz(C) <= nzmax also d_jc and d_c,
  * the same bits as tsg_spgemm_symbolic + tsg_spgemm_numeric on the handle's
  * settings (method, FP mode, tuning), else returns TSG_ERR_OVERFLOW.  A
- * product whose workspace exceeds the scratch returns TSG_ERR_INVALID
- * (m and nnz(A) too large at a glance) or TSG_ERR_ALLOC (the scratch ran
- * out), with the sizes in tsg_last_error.  The handle's own plan is left as
+ * product with 28 (m + 1) + 8 (nnz(A) + 1) past the scratch's bytes returns
+ * TSG_ERR_INVALID, one whose workspace exceeds the scratch TSG_ERR_ALLOC,
+ * with the sizes in tsg_last_error.  The handle's own plan is left as
  * it was.  Calls on one device share the scratch: they are serialised and
  * each returns after its work on the handle's stream has finished (the
  * call synchronises that stream), so calls never overlap on the device. */

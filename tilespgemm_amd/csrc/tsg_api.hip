@@ -477,13 +477,15 @@ int tsg_spgemm_noalloc(tsg_handle_t h, int m, int n, int k, const int *d_ia, con
         TSG_CHECK(d_ic && nnz_c && nzmax >= 0 && (nzmax == 0 || (d_jc && d_c)), TSG_ERR_INVALID,
                   "null output or negative nzmax");
         const size_t cap = TSG_NOALLOC_SCRATCH_BYTES;
-        // the row arrays and per-entry product counts every product needs
-        // (the rest is checked as it is carved out of the scratch)
-        const double least = 28.0 * ((double)m + 1) + 8.0 * ((double)nnz_a + 1);
-        TSG_CHECK(least <= (double)cap, TSG_ERR_INVALID,
+        // the call's limit on sizes: 28 bytes a row and 8 an entry of A.  Inside
+        // it the first pass always fits (its row arrays take 16 bytes a row, and
+        // 16 more for each that has entries); the rest is checked as it is
+        // carved out of the scratch
+        const double sized = 28.0 * ((double)m + 1) + 8.0 * ((double)nnz_a + 1);
+        TSG_CHECK(sized <= (double)cap, TSG_ERR_INVALID,
                   "tsg_spgemm_noalloc: m = " + std::to_string(m) + " and nnz(A) = " +
-                      std::to_string(nnz_a) + " need more than its " + std::to_string(cap) +
-                      "-byte scratch");
+                      std::to_string(nnz_a) + " are past its limit, 28 (m + 1) + 8 (nnz(A) + 1) <= " +
+                      std::to_string(cap) + ", the bytes of its scratch");
         TSG_CHECK(h->device >= 0 && h->device < MAX_DEVICES && g_scratch_ptr[h->device],
                   TSG_ERR_STATE, "tsg_spgemm_noalloc: no scratch set up on this device");
         DeviceGuard dg(h->device);
