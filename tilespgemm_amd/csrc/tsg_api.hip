@@ -622,6 +622,10 @@ size_t tsg_plan_array_bytes(tsg_handle_t h, int which) {
     return plan_array(h, which, &p, &b) ? b : 0;
 }
 
+int tsg_plan_dir_shift(tsg_handle_t h) {
+    return h && h->row.valid && h->row.dir.cells ? h->row.dir.shift : 0;
+}
+
 int tsg_plan_array_copy(tsg_handle_t h, int which, void *dst, size_t bytes) {
     if (!h || !dst) return TSG_ERR_INVALID;
     return guarded(h, [&] {

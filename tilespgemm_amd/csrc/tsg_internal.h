@@ -231,6 +231,10 @@ __host__ __device__ __forceinline__ int sub_block_start(int sb, int k) {
     return c < k ? (int)c : k;
 }
 
+// log2 of the finest blocks of the run directory in the handle's plan, 0
+// without one (not in the public header: the tests tell the forms apart by it).
+extern "C" int tsg_plan_dir_shift(tsg_handle_t handle);
+
 constexpr int ITEM_CLASSES = 3;       // size classes of the row path's items
 
 struct RowPlan {
