@@ -147,16 +147,6 @@ int choose_method(tsg_handle_t h, const CsrIn &A, bool sorted,
     return per_tile >= h->tile_density ? TSG_METHOD_TILE : TSG_METHOD_ROW;
 }
 
-}  // namespace
-
-int device_cu_count(int device) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) != hipSuccess) return 256;
-    return prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
-}
-
-namespace {
-
 // Symbolic phase of C = A*B on the handle's stream and settings, into the
 // given plans: validation (with AUTO's density sample), the method choice,
 // then the tile or the row path.  The plan's arrays come from ws; aux holds
@@ -232,7 +222,7 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
             b_idx = ws.alloc_n<int>((size_t)nnz_b);
             b_perm = ws.alloc_n<int>((size_t)nnz_b);
             b_val = ws.alloc_n<double>((size_t)nnz_b);
-            csr_sort_rows(n, k, d_ib, d_jb, nnz_b, b_idx, b_perm, ws, aux, h->stream);
+            csr_sort_rows(n, k, d_ib, d_jb, nnz_b, b_idx, b_perm, aux, h->stream);
             Bs.idx = b_idx;
             // duplicates remain after sorting: strict only if none
             b_strict = (front_pass(Bs, Bs, aux, h->stream, h->box) & 0x4) == 0;
@@ -248,8 +238,8 @@ void symbolic_into(tsg_handle_t h, RowPlan &row, TilePlan &tile, int &method_use
 
 // Numeric phase from plans made by symbolic_into (same structure; values
 // may differ).  Arguments are checked by the caller.
-void numeric_from(tsg_handle_t h, int method_used, RowPlan &row, TilePlan &tile, Arena &ws,
-                  StageTimer &tm, int m, int n, int k, const int *d_ia, const int *d_ja,
+void numeric_from(tsg_handle_t h, int method_used, RowPlan &row, TilePlan &tile, StageTimer &tm,
+                  int m, int n, int k, const int *d_ia, const int *d_ja,
                   const double *d_a, int64_t nnz_a, const int *d_ib, const int *d_jb,
                   const double *d_b, int64_t nnz_b, const int64_t *d_ic, int *d_jc,
                   double *d_c) {
@@ -267,7 +257,7 @@ void numeric_from(tsg_handle_t h, int method_used, RowPlan &row, TilePlan &tile,
             Bs.idx = row.b_idx;
             Bs.val = row.b_val;
         }
-        row_numeric(row, A, Bs, d_ic, d_jc, d_c, fused, ws, h->stream, tm, h->cus);
+        row_numeric(row, A, Bs, d_ic, d_jc, d_c, fused, h->stream, tm);
     }
 }
 
@@ -288,7 +278,6 @@ int tsg_create(tsg_handle_t *handle, int device) {
         std::unique_ptr<tsg_handle_s> h(new tsg_handle_s());
         h->device = device;
         DeviceGuard dg(device);
-        h->cus = device_cu_count(device);
         // A blocking stream: it orders with the null stream, which is where
         // callers that never create streams (and torch's default stream) work.
         TSG_HIP_TRY(hipStreamCreate(&h->own_stream));
@@ -459,7 +448,7 @@ int tsg_spgemm_numeric(tsg_handle_t h, int m, int n, int k, const int *d_ia, con
         TSG_CHECK(nnz_a == 0 || d_a, TSG_ERR_INVALID, "null A values");
         TSG_CHECK(nnz_b == 0 || d_b, TSG_ERR_INVALID, "null B values");
         DeviceGuard dg(h->device);
-        numeric_from(h, h->method_used, h->row, h->tile, h->ws, h->tm, m, n, k, d_ia, d_ja, d_a,
+        numeric_from(h, h->method_used, h->row, h->tile, h->tm, m, n, k, d_ia, d_ja, d_a,
                      nnz_a, d_ib, d_jb, d_b, nnz_b, d_ic, d_jc, d_c);
     });
 }
@@ -519,7 +508,7 @@ int tsg_spgemm_noalloc(tsg_handle_t h, int m, int n, int k, const int *d_ia, con
                                                  std::to_string(nz) + " exceeds nzmax = " +
                                                  std::to_string(nzmax)};
         }
-        numeric_from(h, method_used, row, tile, ws, tm, m, n, k, d_ia, d_ja, d_a, nnz_a, d_ib,
+        numeric_from(h, method_used, row, tile, tm, m, n, k, d_ia, d_ja, d_a, nnz_a, d_ib,
                      d_jb, d_b, nnz_b, d_ic, d_jc, d_c);
         TSG_HIP_TRY(hipStreamSynchronize(h->stream));
     });

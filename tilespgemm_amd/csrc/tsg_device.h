@@ -32,24 +32,6 @@ __device__ __forceinline__ int dpp_incl_scan(int x) {
 
 __device__ __forceinline__ int wave_incl_scan(int x) { return dpp_incl_scan<64>(x); }
 
-// Inclusive running maximum within aligned groups of G lanes (G = 16, 32 or
-// 64) of values >= -1; same lane rules as dpp_incl_scan.
-template <int CTRL, int ROW_MASK = 0xf>
-__device__ __forceinline__ int dpp_or_minus1(int x) {
-    return __builtin_amdgcn_update_dpp(-1, x, CTRL, ROW_MASK, 0xf, false);
-}
-template <int G>
-__device__ __forceinline__ int dpp_incl_max(int x) {
-    static_assert(G == 16 || G == 32 || G == 64, "DPP scans work on 16, 32 or 64 lanes");
-    x = max(x, dpp_or_minus1<0x111>(x));
-    x = max(x, dpp_or_minus1<0x112>(x));
-    x = max(x, dpp_or_minus1<0x114>(x));
-    x = max(x, dpp_or_minus1<0x118>(x));
-    if (G >= 32) x = max(x, dpp_or_minus1<0x142, 0xa>(x));
-    if (G >= 64) x = max(x, dpp_or_minus1<0x143, 0xc>(x));
-    return x;
-}
-
 __device__ __forceinline__ long long wave_incl_scan64(long long x) {
     const int l = __lane_id();
 #pragma unroll
@@ -74,13 +56,6 @@ __device__ __forceinline__ int group_incl_scan(int x) {
         }
         return x;
     }
-}
-
-// Value of the group's first lane (a scalar read when the group is the wave).
-template <int G>
-__device__ __forceinline__ int group_first(int x) {
-    if constexpr (G == 64) return __builtin_amdgcn_readlane(x, 0);
-    else return __shfl(x, 0, G);
 }
 
 // Value of the group's last lane (a scalar read when the group is the wave).
@@ -140,16 +115,14 @@ constexpr unsigned XCDS = 8;
 
 // Workgroups go to the XCDs in turn, and each XCD has an L2 of its own.  The
 // piece of work of workgroup i of n, such that an XCD takes runs of CHUNK
-// consecutive pieces (0: one run, an eighth of them): neighbours, which read
-// the same rows, then share an L2 and read them from memory once, not once per
-// XCD.
+// consecutive pieces: neighbours, which read the same rows, then share an L2
+// and read them from memory once, not once per XCD.
 template <unsigned CHUNK>
 __device__ __forceinline__ unsigned xcd_piece(unsigned i, unsigned n) {
-    const unsigned run = CHUNK ? CHUNK : n / XCDS;
-    const unsigned round = run * XCDS;
-    if (round == 0 || i >= n / round * round) return i;
+    constexpr unsigned round = CHUNK * XCDS;
+    if (i >= n / round * round) return i;
     const unsigned q = i / round, r = i % round;
-    return q * round + (r % XCDS) * run + r / XCDS;
+    return q * round + (r % XCDS) * CHUNK + r / XCDS;
 }
 
 // Exclusive lower bound of key in sorted a[lo, hi).

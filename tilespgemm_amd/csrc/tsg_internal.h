@@ -10,9 +10,6 @@
 
 #include "../../include/tsg.h"
 
-#define TSG_WAVE 64
-#define TSG_TILE 16
-
 // ------------------------------------------------------------ error plumbing
 struct TsgError {
     int code;
@@ -92,8 +89,6 @@ static inline unsigned grid_for(size_t work, unsigned per_block, unsigned cap = 
     if (g > cap) g = cap;
     return (unsigned)g;
 }
-
-int device_cu_count(int device);
 
 // Input description shared by both paths.
 struct CsrIn {
@@ -246,7 +241,6 @@ struct RowPlan {
     int nbig = 0;
     int64_t big_ent = 0, big_prod = 0;   // the big rows' A entries and products
     int64_t *ent_off = nullptr;      // [nbig+1] A entries of the big rows before each
-    int sub_shift = 0;               // log2 sub-block width (columns)
     int *span_sb0 = nullptr;         // [nbig] first sub-block of the row's span
     int64_t *sb_off = nullptr;       // [nbig+1] span offsets (sub-blocks)
     int64_t nsb_total = 0;
@@ -288,8 +282,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic,
                   int64_t *nnz_c, const RowFront &front, HostBox *box, Arena &ws, hipStream_t s,
                   StageTimer &tm, const RowTuning &tune);
 void row_numeric(RowPlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_ic,
-                 int *d_jc, double *d_c, int fused, Arena &ws, hipStream_t s,
-                 StageTimer &tm, int cus);
+                 int *d_jc, double *d_c, int fused, hipStream_t s, StageTimer &tm);
 
 // ------------------------------------------------------------ tile path
 // One tile's numeric-phase metadata in 64 bytes (one aligned half line), so
@@ -389,7 +382,6 @@ struct BatchState {
 // ------------------------------------------------------------ handle
 struct tsg_handle_s {
     int device = 0;
-    int cus = 256;
     hipStream_t stream = nullptr;
     hipStream_t own_stream = nullptr;
     int method = TSG_METHOD_AUTO;
@@ -437,7 +429,7 @@ void csr_transpose(int m, int n, const int *ia, const int *ja, const double *a,
 // Row-sorted copy of X's columns (stable: equal columns keep their order) and
 // the original position of every sorted entry; temporaries from tmp.
 void csr_sort_rows(int m, int n, const int *ia, const int *ja, int64_t nnz, int *sorted_ja,
-                   int *perm, Arena &keep, Arena &tmp, hipStream_t s);
+                   int *perm, Arena &tmp, hipStream_t s);
 void gather_values(int64_t n, const int *perm, const double *src, double *dst, hipStream_t s);
 void sort_order_i32(const int *keys, int64_t n, int end_bit, int *order, Arena &ws,
                     hipStream_t s);

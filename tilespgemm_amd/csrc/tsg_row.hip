@@ -1486,7 +1486,6 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
 
     // big rows
     p.nbig = front.count[ROW_BIN_BIG];
-    p.sub_shift = SUB_SHIFT;
     int64_t *band_off = nullptr, *band_base = nullptr, *row_loff = nullptr;
     unsigned long long *row_cur = nullptr;
     int64_t *d_overflow = nullptr;
@@ -1840,8 +1839,7 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
 }
 
 void row_numeric(RowPlan &p, const CsrIn &A, const CsrIn &B, const int64_t *d_ic, int *d_jc,
-                 double *d_c, int fused, Arena & /*ws*/, hipStream_t s, StageTimer &tm,
-                 int /*cus*/) {
+                 double *d_c, int fused, hipStream_t s, StageTimer &tm) {
     TSG_CHECK(p.valid && p.m == A.rows && p.n == A.cols && p.k == B.cols, TSG_ERR_STATE,
               "row numeric phase without a matching symbolic phase");
     if (fused)

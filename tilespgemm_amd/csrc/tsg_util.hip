@@ -422,7 +422,7 @@ __global__ void k_gather_vals(int64_t n, const int *__restrict__ perm,
 }
 
 void csr_sort_rows(int m, int n, const int *ia, const int *ja, int64_t nnz, int *sorted_ja,
-                   int *perm, Arena &keep, Arena &tmp, hipStream_t s) {
+                   int *perm, Arena &tmp, hipStream_t s) {
     if (nnz <= 0) return;
     int *tp = tmp.alloc_n<int>((size_t)n + 1);
     int *ti = tmp.alloc_n<int>((size_t)nnz);
@@ -434,7 +434,6 @@ void csr_sort_rows(int m, int n, const int *ia, const int *ja, int64_t nnz, int 
     hipLaunchKernelGGL(k_compose_pos, dim3(grid_for((size_t)nnz, 256)), dim3(256), 0, s, nnz,
                        pos2, pos1, perm);
     TSG_LAUNCH_CHECK();
-    (void)keep;
 }
 
 void gather_values(int64_t n, const int *perm, const double *src, double *dst, hipStream_t s) {
