@@ -1,4 +1,4 @@
-"""Run directory of B's over more than two ranges of 512 blocks, where each
+"""Run directory of B over more than one range of 512 blocks, where each
 row's entries in a range are searched: rows and columns around the ranges' and
 row groups' edges, empty rows, rows that skip ranges, against the oracle on
 columns relabelled in order -- and the time to make it, which follows B's
@@ -34,7 +34,7 @@ def _handle():
 
 
 @pytest.mark.parametrize("n", [1, 33, 255, 256, 257, 600])
-@pytest.mark.parametrize("k", [2 * RANGE, 2 * RANGE + 1, 4 * RANGE + 77, 2**26 + 5, 2**31 - 1])
+@pytest.mark.parametrize("k", [RANGE, RANGE + 1, 2 * RANGE, 2 * RANGE + 1, 4 * RANGE + 77, 2**26 + 5, 2**31 - 1])
 def test_ranges_of_blocks(n, k):
     rng = np.random.default_rng(n + k % 1000)
     edges = np.unique([c for b in range(0, min(k // RANGE, 9) + 1) for d in (-1025, -1, 0, 1, 1024)

@@ -493,12 +493,13 @@ __global__ void __launch_bounds__(256) k_bptr_rows(int n, const int *__restrict_
 // marks them in LDS and folds each level's pairs of blocks into the next's.
 // The bits go out cell-major, DIR_ROWS / 32 consecutive cells a block.  Bound
 // by the busiest block, that of the longest rows: 1.2 ms with 512 rows and
-// threads a block (R-MAT 2^20), 0.6 with 256 and 1024.
-// Up to DIR_WHOLE ranges a block goes through its rows' entries for each of
-// them.  Past that (CUT) it has one range and searches each row's entries in
-// it, so that B is read once however many columns it has (B of 1000 rows of
-// 20,000 entries over 2^28 columns, symbolic phase 857 -> 7.0 ms).
-constexpr int DIR_ROWS = 256, DIR_GRP = DIR_ROWS / 32, DIR_BLK = 512, DIR_WHOLE = 2;
+// threads a block (R-MAT 2^20, whole rows), 0.5 with 256 and 1024.
+// With one range a block goes through its rows' entries.  With more (CUT) it
+// has one of them and searches each row's entries in it, so that B is read once
+// however many columns it has (B of 1000 rows of 20,000 entries over 2^28
+// columns, symbolic phase 857 -> 7.0 ms).  R-MAT with 8 draws a row, whole and
+// CUT: 2^16 (one range) 55 and 64 us, 2^18 142 and 163, 2^20 (two) 520 and 436.
+constexpr int DIR_ROWS = 256, DIR_GRP = DIR_ROWS / 32, DIR_BLK = 512;
 
 // row (of nr from the first) of the entry at position e: rp ascending
 __device__ __forceinline__ int dir_row_of(const int *rp, int nr, int e) {
@@ -1617,7 +1618,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
                 p.dir.shift = SUB_SHIFT + c;
                 p.dir.coarse = c > 0;
                 const unsigned ranges = grid_for((size_t)nblk, DIR_BLK, 65535);
-                const bool cut = ranges > DIR_WHOLE;
+                const bool cut = ranges > 1;
                 hipLaunchKernelGGL(cut ? k_dir_bits<true> : k_dir_bits<false>,
                                    dim3(grid_for((size_t)n, DIR_ROWS), cut ? ranges : 1),
                                    dim3(1024), 0, s, n, B.ptr, B.idx, ngrp, p.dir.nblk,
