@@ -117,15 +117,17 @@ int tsg_get_method_used(tsg_handle_t handle);
  * thresholds are compile-time: main_spgemm-col.cu:26-31,
  * spgemm_nsparse_kernel.h:4-14).  They change speed, never results.
  * tile_density: TSG_METHOD_AUTO takes the tile path when A holds at least
- * this many entries per non-empty 16x16 tile (default 32: measured on
- * MI355X, 5-point and 27-point stencils, at 16-19 entries per tile, run
- * faster on the row path and banded or block-dense matrices, at 90 and
- * more, 1.5-4x faster on the tile path).
+ * this many entries per non-empty 16x16 tile (default 32).  Tile and row path
+ * on MI355X, ms a product: 27-point 48^3 (19 entries per tile) 0.98 and 0.48;
+ * 65,537 rows of bands of half-width 8 (90) 0.24 and 0.24, 16 0.30 and 0.44, 32
+ * 0.60 and 1.31; diagonal blocks of 4 (64) 0.16 and 0.09, 8 (128) 0.16 and 0.10,
+ * 16 0.19 and 0.19, 64 0.52 and 1.14.
  * Row bins: rows with at most bin1 (<= 64), bin2 (<= 256) and bin3 (<= 1024)
  * intermediate products take 16 lanes, a wave, and a wave with more
  * registers each, longer rows go to the big-row path (defaults 64, 256, 1024;
  * bin1 <= bin2 <= bin3; at bin3 = 1024, rows of up to 1536 products from up to
- * 64 entries of A still take a wave).  tilespgemm_amd.autotune searches them for a workload. */
+ * 64 entries of A still take a wave).  tilespgemm_amd.autotune searches them
+ * for a workload. */
 int tsg_set_tile_density(tsg_handle_t handle, double entries_per_tile);
 int tsg_set_row_bins(tsg_handle_t handle, int bin1, int bin2, int bin3);
 int tsg_get_tuning(tsg_handle_t handle, double *tile_density, int *bin1, int *bin2,
@@ -136,10 +138,10 @@ int tsg_get_tuning(tsg_handle_t handle, double *tile_density, int *bin1, int *bi
  * order of their first column (a radix sort in the symbolic phase), so the
  * units in flight together read B entries of one narrow column band and
  * find them in L2; B is then cut by a run directory and the items cut to
- * 8192 columns.  Below that the sort costs more than it
- * saves.  Default 2^18 (R-MAT n=2^20 A*A^T: 24M windows; n=2^18 with 4
- * draws per row: 523K, 6.48 -> 6.10 ms in column order; n=2^16: 108K,
- * even; n=2^14: 1.68 -> 1.89 ms).  0 always sorts.  Changes speed only. */
+ * 8192 columns, or wider where outputs are few.  Default 2^18.  R-MAT with 8
+ * draws per row, A*A^T, in rows' and column order: n=2^14 0.69 and 0.77 ms, 2^15
+ * 1.08 and 1.13, 2^16 1.99 and 1.80, 2^17 3.6 and 2.9 (both in rows' order by
+ * default), 2^18 8.6 and 6.3.  0 always sorts.  Changes speed only. */
 int tsg_set_item_order(tsg_handle_t handle, int64_t min_items);
 /* Memory for the big rows' column bitmaps (no counterpart in the
  * reference): the symbolic phase keeps every big row's bitmap in sparse form
@@ -162,7 +164,9 @@ int tsg_set_bitmap_budget(tsg_handle_t handle, int64_t bytes);
  * every range is searched inside its B row.  Negative (the default): 6 GiB,
  * and no table when building it would cost more than 8 entries per lookup
  * it serves (a few big rows against many B rows, as in batches of small
- * products).  Changes speed only. */
+ * products; few rows of very many entries are better off with it: one of
+ * 50,000 in a band of 2^20 rows 3.9 ms, 2.6 with a budget of 6 GiB).  Changes
+ * speed only. */
 int tsg_set_block_pointer_budget(tsg_handle_t handle, int64_t bytes);
 int tsg_get_item_order(tsg_handle_t handle, int64_t *min_items);
 /* Device workspace currently held by the handle, bytes. */
@@ -271,9 +275,10 @@ typedef struct {
     int method;                  /* TSG_METHOD_*                            */
     double tile_density;         /* tsg_set_tile_density, 0 = default       */
     int bin1, bin2, bin3;        /* tsg_set_row_bins; bin3 = 0: 64/256/512,
-                                    not the library's 64/256/1024 (mid-size
-                                    requests: rows of 513-1024 products run
-                                    faster on the big-row path)            */
+                                    not the library's 64/256/1024, which
+                                    suits requests with many rows of 513 to
+                                    1536 products better and the others as
+                                    well                                   */
 } tsg_server_config_t;
 
 typedef struct {

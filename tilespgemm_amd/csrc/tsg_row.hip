@@ -111,7 +111,9 @@ k_flat_symbolic(int nrows, const int *__restrict__ rows, const int *__restrict__
 
 // ------------------------------------------------------- small rows: numeric
 // A batch whose products come from at most this many B rows is accumulated
-// one B row after the other; past that, tag rounds take fewer steps.
+// one B row after the other; past that, tag rounds take fewer steps.  Numeric
+// phase of 65537 rows of 9 banded entries: 111 us at 4, 98 at 8, 12, 20 and 64;
+// the 27-point product, wider bands and ER the same at all of them.
 constexpr int FLAT_SEGS = 12;
 
 // One row of at most G * NB products, G lanes a row (tsg_flat.h), its entries
@@ -889,7 +891,8 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
 // Items sort by size class (ITEM_BOUND), then by first column, after those of
 // rows of LONG_ROW entries or more: an item is one wave's work, so a class ends
 // no sooner than its longest item, which had better start first (R-MAT 2^18
-// times its transpose, items of <= 512 outputs 0.69 -> 0.56 ms).
+// times its transpose, items of <= 512 outputs 0.69 -> 0.56 ms; its numeric
+// phase at LONG_ROW 256, 1024 and 4096 1.44, 1.43 and 1.49 ms, 1.57 without).
 // key = class << class_bit + 1 | 1 << class_bit | first sub-block (a long
 // row's without the 1; class_bit < 0: the sub-block only).  The numeric phase
 // runs each class with tables that hold just that class's items: the waves an
@@ -1020,7 +1023,10 @@ __global__ void __launch_bounds__(64 * ITEM_WAVES) k_big_numeric(
     }
 }
 
-constexpr int RANK_SEGS = 8;           // entries of a batch added one after the other
+// Entries of a batch added one after the other.  Numeric phase at 4, 8 and 16:
+// ER 65536 with 24 a row, all rows big, 691, 685 and 766 us; R-MAT 2^16 with 8
+// draws a row 1.39, 1.26 and 1.20 ms, 2^20 31.6, 31.7 and 32.6 ms.
+constexpr int RANK_SEGS = 8;
 constexpr int RANK_TAGS = 128;         // tag buckets of the rank-indexed kernel
 
 // Rank-indexed variant: the symbolic phase stored every big row's column
@@ -1565,14 +1571,21 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         // order: B block pointers at the sub-block width (item and band
         // boundaries then need no search).  Either with finest blocks of 1024
         // columns while it stays <= 6 GiB, coarser beyond (a directory that
-        // does not fit at all: a search).  Neither when building it would cost more than the searches
-        // it saves -- more than 8 max(1, log2(L / 16)) entries per (A entry,
+        // does not fit at all: a search).  Neither when building it would cost
+        // more than the searches it saves -- more than 8 max(1, log2(L / 16)) entries per (A entry,
         // window of 16 sub-blocks) pair of the big rows, with the pairs
         // estimated from their A entries and average span and L, the mean
         // length of the B rows they reference, from their products per A
         // entry (measured on batches: an entry costs ~5 ps to build, a search
         // ~26 ps in B rows of ~30 entries, which span one or two cache lines,
-        // and several times that in rows of hundreds, where each step misses)
+        // and several times that in rows of hundreds, where each step misses;
+        // the rule is the pointers', but holds for the directory.  Whole
+        // products with it and with searches: R-MAT with 8 draws a row 2^16
+        // 1.82 and 1.95 ms, 2^18 6.4 and 11.5, 2^20 48 and 136; rows of 500 and
+        // 5000 entries, 1000 and 64 of them, in 2^20 columns of 8 entries 2.2
+        // and 1.6, 2.4 and 1.7, and searched; it is off for few long rows, whose
+        // waves wait on each search: one of 50,000 entries 2.6 and 3.9, four of
+        // 100,000 5.6 and 7.1, and searched)
         // -- or when the budget is 0: B's row pointers then act as a one-block
         // table (block width 2^30 >= k) and every range comes from a search
         // inside its B row.

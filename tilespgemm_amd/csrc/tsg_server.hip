@@ -469,12 +469,13 @@ int tsg_server_create(tsg_server_t *server, int device, const tsg_server_config_
     s->device = device;
     s->cfg = *config;
     if (s->cfg.mem_budget == 0) s->cfg.mem_budget = size_t(64) << 30;
-    // a server's requests are many mid-size products, whose rows of 513 to
-    // 1024 products run faster on the big-row path than in the hash-capable
-    // small-row kernel (R-MAT 2^18 A*A^T with 4 draws per row 6.04 -> 5.43
-    // ms; the 512-product ER batch 67.3 -> 62.7 ms); the library default of
-    // 1024 suits single products of a million rows and more (R-MAT 2^20:
-    // 183 -> 187 ms with 512)
+    // The server's default row bins.  They were set when rows of 513 to 1024
+    // products ran faster on the big-row path than in the small-row kernels
+    // of the time; against the register-held kernels they no longer do.  64/256
+    // and 512 or 1024, three workers: ten ER requests of 32 entries a row 4.3
+    // and 3.4 ms, 19 of 20 a row 3.8 and 3.2, 22 of 8 a row 1.53 and 1.55, R-MAT
+    // 2^17 and 2^18 requests and a mix of all kinds the same within 1%; the
+    // 512-product ER batch 52.3 and 30.8 ms
     if (s->cfg.bin3 <= 0) {
         s->cfg.bin1 = 64;
         s->cfg.bin2 = 256;

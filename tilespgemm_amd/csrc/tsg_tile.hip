@@ -769,7 +769,11 @@ constexpr int STEP_U = 4;
 // have at least RUN_FILL a pair, the lanes go through each pair together, from
 // their run's first positions on, two values a load.  65537 rows of 33 banded
 // entries: 167 -> 116 us (one value a load 180: 31M vector instructions instead
-// of 69M, but the loads' addresses bound it, as they do now).
+// of 69M, but the loads' addresses bound it, as they do now).  Numeric phase
+// of 65537 rows of 9, 17, 25, 33 and 65 banded entries at RUN_FILL 1, 4, 8 and
+// without runs: 53, 58, 58, 60 us; 71, 83, 89, 89; 110, 117, 151, 154; 141, 144,
+// 160, 209; 385, 381, 406, 609.  Diagonal blocks of 64: 320, 323, 319, 646; the
+// 27-point product, which hardly has runs, 533, 520, 524, 519.
 constexpr int RUN_FILL = 4;
 // two values in one load (the arrays hold one past their last)
 struct __attribute__((packed, aligned(8))) Pair8 { double x, y; };

@@ -81,7 +81,8 @@ void *Arena::alloc(size_t bytes) {
 // ================================================================= scans
 // Exclusive scan: per-block totals, then a rescan of each block with its
 // offset, which up to SCAN_FLAT blocks add up themselves from the totals (a
-// launch less); past that the totals are scanned first, recursively.  1024
+// launch less: whole ER products of 16,000 rows 97.0 -> 94.0 us, of 2^20 840 ->
+// 826; at 512 or 8192 blocks the same); past that the totals are scanned first, recursively.  1024
 // elements per 256-thread block (4 per thread).
 namespace {
 constexpr int SCAN_T = 256;
