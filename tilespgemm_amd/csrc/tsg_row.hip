@@ -1441,6 +1441,14 @@ static unsigned item_grid(int64_t nitems) {
     return (unsigned)std::min<int64_t>((nitems + ITEM_WAVES - 1) / ITEM_WAVES, int64_t(1) << 30);
 }
 
+// A bin's rows in launches of at most 2^31 threads (one launch holds less than
+// 2^32): f(first row, rows).
+template <class F>
+void flat_launches(int64_t rows, int rpb, int threads, F &&f) {
+    const int64_t most = (int64_t(1) << 31) / threads * rpb;
+    for (int64_t r0 = 0; r0 < rows; r0 += most) f(r0, (int)std::min(rows - r0, most));
+}
+
 // Raises a kernel's dynamic LDS limit once per process (later calls, e.g.
 // inside a captured numeric phase, touch no runtime state).
 template <class K>
@@ -1476,11 +1484,11 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     tm.begin("row.small_symbolic");
     {
         auto launch = [&](auto kern, int rpb, int threads, int bin) {
-            const int nr = front.count[bin];
-            if (nr <= 0) return;
-            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
-                               front.rows(bin), A.ptr, A.idx, B.ptr, B.idx, front.rownnz);
-            TSG_LAUNCH_CHECK();
+            flat_launches(front.count[bin], rpb, threads, [&](int64_t r0, int nr) {
+                hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
+                                   front.rows(bin) + r0, A.ptr, A.idx, B.ptr, B.idx, front.rownnz);
+                TSG_LAUNCH_CHECK();
+            });
         };
         launch(k_flat_symbolic<16, 4, 64, 64, 256>, 16, 256, 1);
         launch(k_flat_symbolic<64, 4, 64, 512, 64>, 1, 64, 2);
@@ -1790,12 +1798,12 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
     tm.begin("row.small_numeric");
     {
         auto launch = [&](auto kern, int rpb, int threads, int bin) {
-            const int nr = front.count[bin];
-            if (nr <= 0) return;
-            hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
-                               front.rows(bin), A.ptr, A.idx, A.val, B.ptr, B.idx, B.val, d_ic,
-                               d_jc, d_c, (int)p.b_strict);
-            TSG_LAUNCH_CHECK();
+            flat_launches(front.count[bin], rpb, threads, [&](int64_t r0, int nr) {
+                hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
+                                   front.rows(bin) + r0, A.ptr, A.idx, A.val, B.ptr, B.idx, B.val,
+                                   d_ic, d_jc, d_c, (int)p.b_strict);
+                TSG_LAUNCH_CHECK();
+            });
         };
         launch(k_flat_numeric<FUSED, 16, 4, 64, 64, 64, 256>, 16, 256, 1);
         launch(k_flat_numeric<FUSED, 64, 4, 64, 512, 256, 64>, 1, 64, 2);
