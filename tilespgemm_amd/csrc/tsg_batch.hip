@@ -107,13 +107,14 @@ static unsigned cat_grid(int64_t nnz) { return grid_for((size_t)nnz, 256 * CAT_P
 __global__ void __launch_bounds__(256) k_local_cols(int count, const int64_t *__restrict__ off,
                                                     int64_t rows, const int64_t *__restrict__ ic,
                                                     int *__restrict__ jc) {
-    const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
     const int l = threadIdx.x & 7;
-    if (r >= rows) return;
-    const int p = find_seg(off + OFF_ROW * (int64_t)(count + 1), count, r);
-    const int sub = (int)off[OFF_BCOL * (int64_t)(count + 1) + p];
-    if (sub == 0) return;
-    for (int64_t e = ic[r] + l; e < ic[r + 1]; e += 8) jc[e] -= sub;
+    for (int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3; r < rows;
+         r += (int64_t)gridDim.x * blockDim.x >> 3) {
+        const int p = find_seg(off + OFF_ROW * (int64_t)(count + 1), count, r);
+        const int sub = (int)off[OFF_BCOL * (int64_t)(count + 1) + p];
+        if (sub == 0) continue;
+        for (int64_t e = ic[r] + l; e < ic[r + 1]; e += 8) jc[e] -= sub;
+    }
 }
 
 __global__ void k_gather_row_ptrs(int count, const int64_t *__restrict__ off,
@@ -299,7 +300,7 @@ void batch_numeric(tsg_handle_t h, int count, const tsg_product_t *prods, const 
                                 S.jb, S.b, S.nnz_b, d_ic, d_jc, d_c);
     if (rc != TSG_OK) throw TsgError{rc, h->err};
     if (S.rows > 0 && !S.local_cols) {
-        hipLaunchKernelGGL(k_local_cols, dim3(grid_for((size_t)S.rows * 8, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(k_local_cols, dim3(grid_for((size_t)S.rows, 32, MAX_GRID)), dim3(256), 0, s,
                            count, S.row_off, (int64_t)S.rows, d_ic, d_jc);
         TSG_LAUNCH_CHECK();
     }

@@ -111,6 +111,14 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// Waves of a grid of whole-wave blocks.
+__device__ __forceinline__ int64_t wave_index() {
+    return ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+}
+__device__ __forceinline__ int64_t wave_count() {
+    return (int64_t)gridDim.x * blockDim.x >> 6;
+}
+
 constexpr unsigned XCDS = 8;
 
 // Workgroups go to the XCDs in turn, and each XCD has an L2 of its own.  The

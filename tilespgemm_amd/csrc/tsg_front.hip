@@ -338,7 +338,7 @@ int front_pass(const CsrIn &A, const CsrIn &B, Arena &ws, hipStream_t s, HostBox
     TSG_HIP_TRY(hipMemsetAsync(zero, 0, sizeof(FrontCounters) + nslots * sizeof(FrontSlot), s));
     int nsample = 0, step = 1;
     if (density_sample && A.rows > 0 && A.nnz > 0) {
-        const int blkm = (A.rows + 15) / 16;
+        const int blkm = tiles_of(A.rows);
         step = tile_sample_step(blkm);
         nsample = (blkm + step - 1) / step;
     }

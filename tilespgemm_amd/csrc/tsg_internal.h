@@ -90,6 +90,24 @@ static inline unsigned grid_for(size_t work, unsigned per_block, unsigned cap = 
     return (unsigned)g;
 }
 
+// A launch holds fewer than 2^32 threads; past them the count wraps, without an
+// error.  Work that can take as many either goes through a grid of at most
+// MAX_GRID blocks of 256 threads in steps, or in launches of at most 2^31
+// threads, per items a block of the threads: f(first item, items).
+constexpr unsigned MAX_GRID = 1u << 23;
+template <class F>
+void in_launches(int64_t items, int per, int threads, F &&f) {
+    const int64_t most = (int64_t(1) << 31) / threads * per;
+    for (int64_t i = 0; i < items; i += most) f(i, (int)(items - i < most ? items - i : most));
+}
+
+// 16x16 tiles that n rows or columns take.
+__host__ __device__ __forceinline__ int tiles_of(int n) { return (n >> 4) + ((n & 15) != 0); }
+// End of the rows [16 I, 16 I + 16 t) of m (16 I < m).
+__host__ __device__ __forceinline__ int tile_rows_end(int I, int t, int m) {
+    return m - 16 * I > 16 * t ? 16 * (I + t) : m;
+}
+
 // Input description shared by both paths.
 struct CsrIn {
     int rows, cols;
@@ -185,7 +203,7 @@ struct RowTuning {
 };
 
 // One big-row item: d = {row, first column, end column, first sub-block in
-// subocc (rank mode) or big-row index}, the position of its first output in
+// subocc (rank mode)}, the position of its first output in
 // C, and of its first word in the band word lists (rank mode).  One record,
 // so that gathering the items into column order reads one line per item.
 struct ItemRec {

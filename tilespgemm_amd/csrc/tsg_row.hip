@@ -246,34 +246,34 @@ __global__ void __launch_bounds__(256) k_big_span(int nbig, const int *__restric
                                                   int64_t *__restrict__ nent,
                                                   int64_t *__restrict__ nprod,
                                                   int64_t *__restrict__ lbound) {
-    const int r = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int l = threadIdx.x & 63;
-    if (r >= nbig) return;
-    const int row = rows[r];
-    int lo = 0x7fffffff, hi = -1;
-    const unsigned pe = (unsigned)ia[row + 1];
-    for (unsigned p = (unsigned)ia[row] + l; p < pe; p += 64) {
-        const int t = ja[p];
-        const int b0 = ib[t], b1 = ib[t + 1];
-        if (b0 < b1) {
-            lo = min(lo, jb[b0] >> SUB_SHIFT);
-            hi = max(hi, jb[b1 - 1] >> SUB_SHIFT);
+    for (int64_t r = wave_index(); r < nbig; r += wave_count()) {
+        const int row = rows[r];
+        int lo = 0x7fffffff, hi = -1;
+        const unsigned pe = (unsigned)ia[row + 1];
+        for (unsigned p = (unsigned)ia[row] + l; p < pe; p += 64) {
+            const int t = ja[p];
+            const int b0 = ib[t], b1 = ib[t + 1];
+            if (b0 < b1) {
+                lo = min(lo, jb[b0] >> SUB_SHIFT);
+                hi = max(hi, jb[b1 - 1] >> SUB_SHIFT);
+            }
         }
-    }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        lo = min(lo, __shfl_xor(lo, d, 64));
-        hi = max(hi, __shfl_xor(hi, d, 64));
-    }
-    if (l == 0) {
-        const int64_t ns = hi >= lo ? (int64_t)(hi - lo + 1) : 0;
-        sb0[r] = hi >= lo ? lo : 0;
-        nsb[r] = ns;
-        nent[r] = ia[row + 1] - ia[row];
-        nprod[r] = rowprod[row];
-        // a multiple of BAND_PAD, so every band's list starts 16-byte aligned
-        lbound[r] = ((min(rowprod[row], ns << (SUB_SHIFT - 5)) + BAND_PAD - 1) & -BAND_PAD) +
-                    BAND_PAD * (((ns + (1 << BAND_SHIFT) - 1) >> BAND_SHIFT) + 1);
+        for (int d = 32; d > 0; d >>= 1) {
+            lo = min(lo, __shfl_xor(lo, d, 64));
+            hi = max(hi, __shfl_xor(hi, d, 64));
+        }
+        if (l == 0) {
+            const int64_t ns = hi >= lo ? (int64_t)(hi - lo + 1) : 0;
+            sb0[r] = hi >= lo ? lo : 0;
+            nsb[r] = ns;
+            nent[r] = ia[row + 1] - ia[row];
+            nprod[r] = rowprod[row];
+            // a multiple of BAND_PAD, so every band's list starts 16-byte aligned
+            lbound[r] = ((min(rowprod[row], ns << (SUB_SHIFT - 5)) + BAND_PAD - 1) & -BAND_PAD) +
+                        BAND_PAD * (((ns + (1 << BAND_SHIFT) - 1) >> BAND_SHIFT) + 1);
+        }
     }
 }
 
@@ -478,13 +478,13 @@ __global__ void __launch_bounds__(BAND_T) __attribute__((amdgpu_waves_per_eu(8))
 __global__ void __launch_bounds__(256) k_bptr_rows(int n, const int *__restrict__ ib,
                                                    const int *__restrict__ jb, int nblk, int bs,
                                                    int *__restrict__ bptr) {
-    const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int l = threadIdx.x & 63;
-    if (t >= n) return;
-    const int lo = ib[t], hi = ib[t + 1];
-    for (int b = l; b <= nblk; b += 64) {
-        const int pos = b == nblk ? hi : lower_bound_i32(jb, lo, hi, b << bs);
-        bptr[(size_t)t * (nblk + 1) + b] = pos;
+    for (int64_t t = wave_index(); t < n; t += wave_count()) {
+        const int lo = ib[t], hi = ib[t + 1];
+        for (int b = l; b <= nblk; b += 64) {
+            const int pos = b == nblk ? hi : lower_bound_i32(jb, lo, hi, b << bs);
+            bptr[t * (nblk + 1) + b] = pos;
+        }
     }
 }
 
@@ -707,13 +707,13 @@ static_assert(WIDE_CAP <= ITEM_BOUND[1], "wide items run in the sparse kernels")
 // loads its window's counts at once and splits them in registers, and wave
 // scans place the items and their outputs.  FILL=false counts items per
 // row; FILL=true (item_cnt = exclusive item offsets) writes each item's
-// record -- {row, c0, c1, big-row index}, its first output position -- and
-// output count, and, in rank mode (band_base given), where its first
+// record -- {row, c0, c1}, its first output position -- and output count, and,
+// in rank mode (band_base given), where its first
 // non-empty word is in the band word lists of the symbolic phase (from the
 // sub-blocks' masks of non-empty words); the record's fourth field then
 // holds the item's first sub-block's index in subcnt and subocc (< 2^31 in
-// that mode) instead of the big-row index, so the numeric phase finds the
-// item's masks with no other lookup.  Windows lie inside bands, and a
+// that mode), so the numeric phase finds the item's masks with no other
+// lookup.  Windows lie inside bands, and a
 // band's windows inside one pass of 64 windows, so the item's place in its
 // band's list is its count of non-empty words before it less that of the
 // band's first window.
@@ -846,7 +846,7 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
             if (run > 1) {
                 items[w] = ItemRec{make_int4(row, (first + sb_first) << SUB_SHIFT,
                                              sub_block_start(first + sb_last + 1, k),
-                                             words ? (int)(sb_off[r] + sb_first) : r),
+                                             words ? (int)(sb_off[r] + sb_first) : 0),
                                    out, wb};
                 item_n[w] = run_tot;
             }
@@ -867,7 +867,7 @@ __global__ void __launch_bounds__(256) k_items(int nbig, const int *__restrict__
                 if (ends[q] && cnt > 0) {
                     items[w] = ItemRec{make_int4(row, (cbase + start) << SUB_SHIFT,
                                                  sub_block_start(cbase + stop, k),
-                                                 words ? (int)(sb_off[r] + j0 + start) : r),
+                                                 words ? (int)(sb_off[r] + j0 + start) : 0),
                                        out, wb + nzs};
                     item_n[w] = cnt;
                     w++;
@@ -1438,15 +1438,7 @@ static BRows b_rows(const RowPlan &p, const int *b_ptr) {
 // whichever CU frees a slot first, so no CU idles behind a long tail); the
 // item kernels keep a grid-stride loop for item counts beyond the grid limit.
 static unsigned item_grid(int64_t nitems) {
-    return (unsigned)std::min<int64_t>((nitems + ITEM_WAVES - 1) / ITEM_WAVES, int64_t(1) << 30);
-}
-
-// A bin's rows in launches of at most 2^31 threads (one launch holds less than
-// 2^32): f(first row, rows).
-template <class F>
-void flat_launches(int64_t rows, int rpb, int threads, F &&f) {
-    const int64_t most = (int64_t(1) << 31) / threads * rpb;
-    for (int64_t r0 = 0; r0 < rows; r0 += most) f(r0, (int)std::min(rows - r0, most));
+    return grid_for((size_t)nitems, ITEM_WAVES, MAX_GRID);
 }
 
 // Raises a kernel's dynamic LDS limit once per process (later calls, e.g.
@@ -1484,7 +1476,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
     tm.begin("row.small_symbolic");
     {
         auto launch = [&](auto kern, int rpb, int threads, int bin) {
-            flat_launches(front.count[bin], rpb, threads, [&](int64_t r0, int nr) {
+            in_launches(front.count[bin], rpb, threads, [&](int64_t r0, int nr) {
                 hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
                                    front.rows(bin) + r0, A.ptr, A.idx, B.ptr, B.idx, front.rownnz);
                 TSG_LAUNCH_CHECK();
@@ -1516,7 +1508,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         int64_t *a_ent = p.ent_off = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         int64_t *a_prod = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
         row_loff = ws.alloc_n<int64_t>((size_t)p.nbig + 1);
-        hipLaunchKernelGGL(k_big_span, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(k_big_span, dim3(grid_for((size_t)p.nbig, 4, MAX_GRID)), dim3(256), 0, s,
                            p.nbig, rowsb, A.ptr, A.idx, B.ptr, B.idx, front.rowprod, p.span_sb0,
                            p.sb_off, a_ent, a_prod, row_loff);
         TSG_LAUNCH_CHECK();
@@ -1669,7 +1661,7 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
             p.blk_shift = bs;
             p.nblk = (int)(((size_t)k + (1u << bs) - 1) >> bs);
             p.bptr = ws.alloc_n<int>((size_t)n * (p.nblk + 1));
-            hipLaunchKernelGGL(k_bptr_rows, dim3(grid_for((size_t)n * 64, 256)), dim3(256), 0,
+            hipLaunchKernelGGL(k_bptr_rows, dim3(grid_for((size_t)n, 4, MAX_GRID)), dim3(256), 0,
                                s, n, B.ptr, B.idx, p.nblk, bs, p.bptr);
             TSG_LAUNCH_CHECK();
         }
@@ -1694,11 +1686,10 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         }
         auto symbolic = p.dir.cells ? k_big_symbolic<true> : k_big_symbolic<false>;
         hipLaunchKernelGGL(symbolic,
-                           dim3((unsigned)std::min<int64_t>(nunits, int64_t(1) << 30)),
-                           dim3(BAND_T), 0, s, nunits, units, rowsb, k, (int)p.column_order, A.ptr,
-                           A.idx, B.idx, b_rows(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, front.rownnz,
-                           band_off, band_base, row_cur, row_loff, d_overflow, p.subocc,
-                           p.bandwords);
+                           dim3(grid_for((size_t)nunits, 1, MAX_GRID)), dim3(BAND_T), 0, s, nunits,
+                           units, rowsb, k, (int)p.column_order, A.ptr, A.idx, B.idx,
+                           b_rows(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, front.rownnz, band_off,
+                           band_base, row_cur, row_loff, d_overflow, p.subocc, p.bandwords);
         TSG_LAUNCH_CHECK();
         tm.end();
     }
@@ -1723,10 +1714,12 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         // follow the outputs, not the columns (rank mode, by size class)
         int wide_cap = narrow && p.use_rank ? WIDE_CAP : 0;
         auto items_kernel = [&](auto kern, int64_t *cnt, ItemRec *it, int *itn) {
-            hipLaunchKernelGGL(kern, dim3(grid_for((size_t)p.nbig * 64, 256)), dim3(256), 0, s,
-                               p.nbig, rowsb, k, (int)narrow, wide_cap, p.span_sb0, p.sb_off, p.subcnt, d_ic, cnt, it,
-                               itn, p.subocc, band_off, band_base);
-            TSG_LAUNCH_CHECK();
+            in_launches(p.nbig, 4, 256, [&](int64_t r0, int nr) {
+                hipLaunchKernelGGL(kern, dim3(grid_for(nr, 4)), dim3(256), 0, s, nr, rowsb + r0, k,
+                                   (int)narrow, wide_cap, p.span_sb0 + r0, p.sb_off + r0, p.subcnt,
+                                   d_ic, cnt + r0, it, itn, p.subocc, band_off + r0, band_base);
+                TSG_LAUNCH_CHECK();
+            });
         };
         while (true) {
             if (narrow)
@@ -1798,7 +1791,7 @@ static void row_numeric_t(RowPlan &p, const CsrIn &A, const CsrIn &B, const int6
     tm.begin("row.small_numeric");
     {
         auto launch = [&](auto kern, int rpb, int threads, int bin) {
-            flat_launches(front.count[bin], rpb, threads, [&](int64_t r0, int nr) {
+            in_launches(front.count[bin], rpb, threads, [&](int64_t r0, int nr) {
                 hipLaunchKernelGGL(kern, dim3(grid_for(nr, rpb)), dim3(threads), 0, s, nr,
                                    front.rows(bin) + r0, A.ptr, A.idx, A.val, B.ptr, B.idx, B.val,
                                    d_ic, d_jc, d_c, (int)p.b_strict);

@@ -72,7 +72,7 @@ __device__ __forceinline__ void tile_sample_row(int I, int m, int ncols, int64_t
     __shared__ int s_cnt[4];
     const int t = threadIdx.x, l = t & 63, w = t >> 6;
     const int p0 = (int)min((int64_t)max(ia[I * 16], 0), nnz);
-    const int p1 = (int)min((int64_t)max(ia[min(m, I * 16 + 16)], p0), nnz);
+    const int p1 = (int)min((int64_t)max(ia[tile_rows_end(I, 1, m)], p0), nnz);
     const TileCols<256> tc{p1, max(ncols - 1, 0), ja};
     int lo, hi;
     tc.range(p0, t, lo, hi);

@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(16 * CV_TR) k_tile_convert(
     __shared__ int s_col[CV_STAGE];
     const int I0 = blockIdx.x * (blockDim.x >> 4);
     const int e0 = ia[I0 * 16];
-    const int e1 = ia[min(m, (I0 + (int)(blockDim.x >> 4)) * 16)];
+    const int e1 = ia[tile_rows_end(I0, blockDim.x >> 4, m)];
     const bool staged = e1 - e0 <= CV_STAGE;
     if (staged)
         for (int i = threadIdx.x; i < e1 - e0; i += blockDim.x) s_col[i] = ja[e0 + i];
@@ -132,29 +132,30 @@ __global__ void __launch_bounds__(64 * TC_WAVES) k_tile_count(int m, int ncols, 
                                                               int *__restrict__ tcount) {
     __shared__ unsigned s_bits[TC_WAVES][TC_WORDS];
     unsigned *bits = s_bits[threadIdx.x >> 6];
-    const int I = blockIdx.x * TC_WAVES + (threadIdx.x >> 6);
     const int l = __lane_id();
-    if (I >= blkm) return;
-    const int p0 = (int)min((int64_t)max(ia[I * 16], 0), nnz);
-    const int p1 = (int)min((int64_t)max(ia[min(m, I * 16 + 16)], p0), nnz);
-    const TileCols<64> tc{p1, max(ncols - 1, 0), ja};
-    int lo, hi;
-    tc.range(p0, l, lo, hi);
-    lo = wave_min(lo);
-    hi = wave_max(hi);
-    int count = 0;
-    for (int w0 = lo; w0 <= hi; w0 += TC_WORDS * 32) {
-        const int w1 = min(hi + 1, w0 + TC_WORDS * 32);
-        const int nwords = (w1 - w0 + 31) >> 5;
-        for (int i = l; i < nwords; i += 64) bits[i] = 0u;
-        wave_lds_fence();
-        tc.mark(p0, l, w0, w1, bits);
-        wave_lds_fence();
-        for (int i = l; i < nwords; i += 64) count += __popc(bits[i]);
-        wave_lds_fence();
+    for (int64_t w = wave_index(); w < blkm; w += wave_count()) {
+        const int I = (int)w;
+        const int p0 = (int)min((int64_t)max(ia[I * 16], 0), nnz);
+        const int p1 = (int)min((int64_t)max(ia[tile_rows_end(I, 1, m)], p0), nnz);
+        const TileCols<64> tc{p1, max(ncols - 1, 0), ja};
+        int lo, hi;
+        tc.range(p0, l, lo, hi);
+        lo = wave_min(lo);
+        hi = wave_max(hi);
+        int count = 0;
+        for (int w0 = lo; w0 <= hi; w0 += TC_WORDS * 32) {
+            const int w1 = min(hi + 1, w0 + TC_WORDS * 32);
+            const int nwords = (w1 - w0 + 31) >> 5;
+            for (int i = l; i < nwords; i += 64) bits[i] = 0u;
+            wave_lds_fence();
+            tc.mark(p0, l, w0, w1, bits);
+            wave_lds_fence();
+            for (int i = l; i < nwords; i += 64) count += __popc(bits[i]);
+            wave_lds_fence();
+        }
+        count = wave_sum(count);
+        if (l == 0) tcount[I] = count;
     }
-    count = wave_sum(count);
-    if (l == 0) tcount[I] = count;
 }
 
 // The density count of tile rows 0, step, 2*step, ... (the grid has one block
@@ -610,34 +611,35 @@ __global__ void __launch_bounds__(256) k_col_layout(int numblk, const int *__res
                                                     const uint8_t *__restrict__ rowptr,
                                                     TileRec *__restrict__ rec,
                                                     int *__restrict__ cpos) {
-    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
     const int c = threadIdx.x & 15;
-    if (t >= numblk) return;
-    const uint4 *m4 = reinterpret_cast<const uint4 *>(mask + t * 16);
-    const uint4 lo = m4[0], hi = m4[1];
-    const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    unsigned cm = 0;
+    for (int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4; t < numblk;
+         t += (int64_t)gridDim.x * blockDim.x >> 4) {
+        const uint4 *m4 = reinterpret_cast<const uint4 *>(mask + t * 16);
+        const uint4 lo = m4[0], hi = m4[1];
+        const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        unsigned cm = 0;
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
-        const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
-        cm |= ((row >> (15 - c)) & 1u) << (15 - k);
-    }
-    const int cnt = __popc(cm);
-    const int cstart = group_incl_scan<16>(cnt) - cnt;
-    const int off = tile_off[t];
-    rec[t].mask[c] = (uint16_t)cm;
-    rec[t].start[c] = (uint8_t)cstart;
-    if (c == 0) rec[t].off = off;
-    const uint4 rp = *reinterpret_cast<const uint4 *>(rowptr + t * 16);
-    int j = 0;
+        for (int k = 0; k < 16; k++) {
+            const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+            cm |= ((row >> (15 - c)) & 1u) << (15 - k);
+        }
+        const int cnt = __popc(cm);
+        const int cstart = group_incl_scan<16>(cnt) - cnt;
+        const int off = tile_off[t];
+        rec[t].mask[c] = (uint16_t)cm;
+        rec[t].start[c] = (uint8_t)cstart;
+        if (c == 0) rec[t].off = off;
+        const uint4 rp = *reinterpret_cast<const uint4 *>(rowptr + t * 16);
+        int j = 0;
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
-        const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
-        if ((row >> (15 - c)) & 1u) {
-            const int rw = (int)((k < 8 ? (k < 4 ? rp.x : rp.y) : (k < 12 ? rp.z : rp.w)) >>
-                                 ((k & 3) * 8)) & 255;
-            cpos[off + rw + __popc(row >> (16 - c))] = off + cstart + j;
-            j++;
+        for (int k = 0; k < 16; k++) {
+            const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+            if ((row >> (15 - c)) & 1u) {
+                const int rw = (int)((k < 8 ? (k < 4 ? rp.x : rp.y) : (k < 12 ? rp.z : rp.w)) >>
+                                     ((k & 3) * 8)) & 255;
+                cpos[off + rw + __popc(row >> (16 - c))] = off + cstart + j;
+                j++;
+            }
         }
     }
 }
@@ -975,8 +977,8 @@ void tile_count_scan(const CsrIn &X, int blkm, int *tile_ptr, Arena &ws, hipStre
     int *tcount = ws.alloc_n<int>((size_t)blkm + 1);
     int64_t *tmp = ws.alloc_n<int64_t>(scan_tmp_elems((size_t)blkm + 1));
     if (blkm > 0) {
-        hipLaunchKernelGGL(k_tile_count, dim3(grid_for(blkm, TC_WAVES)), dim3(64 * TC_WAVES), 0,
-                           s, X.rows, X.cols, X.nnz, blkm, X.ptr, X.idx, tcount);
+        hipLaunchKernelGGL(k_tile_count, dim3(grid_for(blkm, TC_WAVES, MAX_GRID)),
+                           dim3(64 * TC_WAVES), 0, s, X.rows, X.cols, X.nnz, blkm, X.ptr, X.idx, tcount);
         TSG_LAUNCH_CHECK();
     }
     exclusive_scan_i32(tcount, tile_ptr, (size_t)blkm, tmp, s, total);
@@ -988,8 +990,8 @@ void convert(TileMat &T, const CsrIn &X, HostBox *box, Arena &ws, hipStream_t s,
              const EarlyTileCount *early) {
     T.rows = X.rows;
     T.cols = X.cols;
-    T.blkm = (X.rows + 15) / 16;
-    T.blkn = (X.cols + 15) / 16;
+    T.blkm = tiles_of(X.rows);
+    T.blkn = tiles_of(X.cols);
     T.nnz = X.nnz;
     int nt = 0;
     if (early && early->nt >= 0) {
@@ -1023,7 +1025,7 @@ void convert(TileMat &T, const CsrIn &X, HostBox *box, Arena &ws, hipStream_t s,
 
 void tile_count_early(const CsrIn &X, EarlyTileCount &e, int64_t *total, Arena &ws,
                       hipStream_t s) {
-    const int blkm = (X.rows + 15) / 16;
+    const int blkm = tiles_of(X.rows);
     e.tile_ptr = ws.alloc_n<int>((size_t)blkm + 1);
     tile_count_scan(X, blkm, e.tile_ptr, ws, s, total);
 }
@@ -1039,6 +1041,9 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
                    const EarlyTileCount *earlyA, const EarlyTileCount *earlyB) {
     p = TilePlan();
     p.b_is_a = b_is_a;
+    // a wave per tile row in steps 1 and 2: 2^32 threads from 2^26 tile rows
+    TSG_CHECK(tiles_of(A.rows) < (1 << 26), TSG_ERR_OVERFLOW,
+              "the tile path takes fewer than 2^30 - 15 rows");
     const int m = A.rows;
     tm.begin("tile.convert");
     convert(p.A, A, box, ws, s, earlyA);
@@ -1080,7 +1085,7 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
     TB.valc = ws.alloc_n<double>((size_t)TB.nnz + 1);
     if (TB.numblk > 0) {
         int *cpos = ws.alloc_n<int>((size_t)TB.nnz + 1);
-        hipLaunchKernelGGL(k_col_layout, dim3(grid_for((size_t)TB.numblk * 16, 256)), dim3(256),
+        hipLaunchKernelGGL(k_col_layout, dim3(grid_for((size_t)TB.numblk, 16, MAX_GRID)), dim3(256),
                            0, s, TB.numblk, TB.tile_off, TB.mask, TB.rowptr, TB.rec, cpos);
         TSG_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_compose_perm, dim3(grid_for((size_t)TB.nnz, 256)), dim3(256), 0, s,
@@ -1230,15 +1235,18 @@ static void tile_numeric_t(TilePlan &p, const double *valB, const int64_t *d_ic,
     for (int b = 0; b < TBINS; b++) {
         const int n = p.tbin_start[b + 1] - p.tbin_start[b];
         if (n == 0) continue;
-        const int4 *units = p.tbin_units + p.tbin_start[b];
-        const dim3 grid(grid_for((size_t)n, 4 * tpw[b] * UPW));
-        if (b == 0)
-            hipLaunchKernelGGL((k_step3_out<FUSED, 4>), grid, dim3(256), 0, s, n, units, T);
-        else if (b == 1)
-            hipLaunchKernelGGL((k_step3_out<FUSED, 2>), grid, dim3(256), 0, s, n, units, T);
-        else
-            hipLaunchKernelGGL((k_step3_out<FUSED, 1>), grid, dim3(256), 0, s, n, units, T);
-        TSG_LAUNCH_CHECK();
+        const int per = 4 * tpw[b] * UPW;
+        in_launches(n, per, 256, [&](int64_t first, int count) {
+            const int4 *units = p.tbin_units + p.tbin_start[b] + first;
+            const dim3 grid(grid_for((size_t)count, per));
+            if (b == 0)
+                hipLaunchKernelGGL((k_step3_out<FUSED, 4>), grid, dim3(256), 0, s, count, units, T);
+            else if (b == 1)
+                hipLaunchKernelGGL((k_step3_out<FUSED, 2>), grid, dim3(256), 0, s, count, units, T);
+            else
+                hipLaunchKernelGGL((k_step3_out<FUSED, 1>), grid, dim3(256), 0, s, count, units, T);
+            TSG_LAUNCH_CHECK();
+        });
     }
 }
 
@@ -1284,7 +1292,7 @@ int tile_sample_step(int blkm) { return blkm > 1024 ? (blkm + 1023) / 1024 : 1; 
 
 static void tile_count_launch(const CsrIn &X, int step, unsigned long long *sums,
                               hipStream_t s) {
-    const int blkm = (X.rows + 15) / 16;
+    const int blkm = tiles_of(X.rows);
     // one block per sampled tile row: block b takes tile row b*step < blkm
     const int nrows = (blkm + step - 1) / step;
     if (nrows == 0) return;
@@ -1295,7 +1303,7 @@ static void tile_count_launch(const CsrIn &X, int step, unsigned long long *sums
 
 double tile_density(const CsrIn &X, double threshold, Arena &ws, hipStream_t s,
                     const unsigned long long *sample) {
-    const int blkm = (X.rows + 15) / 16;
+    const int blkm = tiles_of(X.rows);
     if (blkm == 0 || X.nnz == 0) return 0.0;
     unsigned long long *sums = ws.alloc_n<unsigned long long>(2);
     auto ratio = [](const unsigned long long *h) {

@@ -312,13 +312,14 @@ void csr_row_products(int m, const int *ia, const int *ja, int64_t nnz, const in
 // Row and position of every entry, 8 lanes a row.
 __global__ void k_row_pos(int m, const int *__restrict__ ia, int *__restrict__ rowidx,
                           int *__restrict__ pos) {
-    const int row = (blockIdx.x * blockDim.x + threadIdx.x) >> 3;
     const int l = threadIdx.x & 7;
-    if (row >= m) return;
-    const unsigned pe = (unsigned)ia[row + 1];
-    for (unsigned p = (unsigned)ia[row] + l; p < pe; p += 8) {
-        rowidx[p] = row;
-        pos[p] = (int)p;
+    for (int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3; row < m;
+         row += (int64_t)gridDim.x * blockDim.x >> 3) {
+        const unsigned pe = (unsigned)ia[row + 1];
+        for (unsigned p = (unsigned)ia[row] + l; p < pe; p += 8) {
+            rowidx[p] = (int)row;
+            pos[p] = (int)p;
+        }
     }
 }
 
@@ -376,7 +377,7 @@ void csr_transpose(int m, int n, const int *ia, const int *ja, const double *a, 
     int *pos_in = ws.alloc_n<int>((size_t)nnz);
     int *pos_out = ws.alloc_n<int>((size_t)nnz);
     int *keys_out = ws.alloc_n<int>((size_t)nnz);
-    hipLaunchKernelGGL(k_row_pos, dim3(grid_for((size_t)m * 8, 256)), dim3(256), 0, s, m, ia,
+    hipLaunchKernelGGL(k_row_pos, dim3(grid_for((size_t)m, 32, MAX_GRID)), dim3(256), 0, s, m, ia,
                        rowidx, pos_in);
     TSG_LAUNCH_CHECK();
     int end_bit = 1;
