@@ -240,8 +240,7 @@ __host__ __device__ __forceinline__ int64_t run_dir_block(int nblk, int shift, i
 // matrix's last (2^31 itself does not fit an int).
 constexpr int SUB_SHIFT = 10;          // 1024 columns
 __host__ __device__ __forceinline__ int sub_block_start(int sb, int k) {
-    const int64_t c = (int64_t)sb << SUB_SHIFT;
-    return c < k ? (int)c : k;
+    return sb <= (k - 1) >> SUB_SHIFT ? sb << SUB_SHIFT : k;
 }
 
 // log2 of the finest blocks of the run directory in the handle's plan, 0

@@ -611,35 +611,34 @@ __global__ void __launch_bounds__(256) k_col_layout(int numblk, const int *__res
                                                     const uint8_t *__restrict__ rowptr,
                                                     TileRec *__restrict__ rec,
                                                     int *__restrict__ cpos) {
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
     const int c = threadIdx.x & 15;
-    for (int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4; t < numblk;
-         t += (int64_t)gridDim.x * blockDim.x >> 4) {
-        const uint4 *m4 = reinterpret_cast<const uint4 *>(mask + t * 16);
-        const uint4 lo = m4[0], hi = m4[1];
-        const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        unsigned cm = 0;
+    if (t >= numblk) return;
+    const uint4 *m4 = reinterpret_cast<const uint4 *>(mask + t * 16);
+    const uint4 lo = m4[0], hi = m4[1];
+    const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    unsigned cm = 0;
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
-            cm |= ((row >> (15 - c)) & 1u) << (15 - k);
-        }
-        const int cnt = __popc(cm);
-        const int cstart = group_incl_scan<16>(cnt) - cnt;
-        const int off = tile_off[t];
-        rec[t].mask[c] = (uint16_t)cm;
-        rec[t].start[c] = (uint8_t)cstart;
-        if (c == 0) rec[t].off = off;
-        const uint4 rp = *reinterpret_cast<const uint4 *>(rowptr + t * 16);
-        int j = 0;
+    for (int k = 0; k < 16; k++) {
+        const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+        cm |= ((row >> (15 - c)) & 1u) << (15 - k);
+    }
+    const int cnt = __popc(cm);
+    const int cstart = group_incl_scan<16>(cnt) - cnt;
+    const int off = tile_off[t];
+    rec[t].mask[c] = (uint16_t)cm;
+    rec[t].start[c] = (uint8_t)cstart;
+    if (c == 0) rec[t].off = off;
+    const uint4 rp = *reinterpret_cast<const uint4 *>(rowptr + t * 16);
+    int j = 0;
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
-            if ((row >> (15 - c)) & 1u) {
-                const int rw = (int)((k < 8 ? (k < 4 ? rp.x : rp.y) : (k < 12 ? rp.z : rp.w)) >>
-                                     ((k & 3) * 8)) & 255;
-                cpos[off + rw + __popc(row >> (16 - c))] = off + cstart + j;
-                j++;
-            }
+    for (int k = 0; k < 16; k++) {
+        const unsigned row = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+        if ((row >> (15 - c)) & 1u) {
+            const int rw = (int)((k < 8 ? (k < 4 ? rp.x : rp.y) : (k < 12 ? rp.z : rp.w)) >>
+                                 ((k & 3) * 8)) & 255;
+            cpos[off + rw + __popc(row >> (16 - c))] = off + cstart + j;
+            j++;
         }
     }
 }
@@ -1085,9 +1084,12 @@ void tile_symbolic(TilePlan &p, const CsrIn &A, const CsrIn &B, bool b_is_a, int
     TB.valc = ws.alloc_n<double>((size_t)TB.nnz + 1);
     if (TB.numblk > 0) {
         int *cpos = ws.alloc_n<int>((size_t)TB.nnz + 1);
-        hipLaunchKernelGGL(k_col_layout, dim3(grid_for((size_t)TB.numblk, 16, MAX_GRID)), dim3(256),
-                           0, s, TB.numblk, TB.tile_off, TB.mask, TB.rowptr, TB.rec, cpos);
-        TSG_LAUNCH_CHECK();
+        in_launches(TB.numblk, 16, 256, [&](int64_t t0, int nt) {
+            hipLaunchKernelGGL(k_col_layout, dim3(grid_for((size_t)nt, 16)), dim3(256), 0, s, nt,
+                               TB.tile_off + t0, TB.mask + 16 * t0, TB.rowptr + 16 * t0,
+                               TB.rec + t0, cpos);
+            TSG_LAUNCH_CHECK();
+        });
         hipLaunchKernelGGL(k_compose_perm, dim3(grid_for((size_t)TB.nnz, 256)), dim3(256), 0, s,
                            TB.nnz, TB.perm, cpos, TB.permc);
         TSG_LAUNCH_CHECK();
