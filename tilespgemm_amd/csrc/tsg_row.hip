@@ -1438,7 +1438,7 @@ static BRows b_rows(const RowPlan &p, const int *b_ptr) {
 // whichever CU frees a slot first, so no CU idles behind a long tail); the
 // item kernels keep a grid-stride loop for item counts beyond the grid limit.
 static unsigned item_grid(int64_t nitems) {
-    return grid_for((size_t)nitems, ITEM_WAVES, MAX_GRID);
+    return grid_for((size_t)nitems, ITEM_WAVES, MAX_GRID * 4 / ITEM_WAVES);
 }
 
 // Raises a kernel's dynamic LDS limit once per process (later calls, e.g.
@@ -1686,8 +1686,8 @@ void row_symbolic(RowPlan &p, const CsrIn &A, const CsrIn &B, int64_t *d_ic, int
         }
         auto symbolic = p.dir.cells ? k_big_symbolic<true> : k_big_symbolic<false>;
         hipLaunchKernelGGL(symbolic,
-                           dim3(grid_for((size_t)nunits, 1, MAX_GRID)), dim3(BAND_T), 0, s, nunits,
-                           units, rowsb, k, (int)p.column_order, A.ptr, A.idx, B.idx,
+                           dim3(grid_for((size_t)nunits, 1, MAX_GRID * 256 / BAND_T)), dim3(BAND_T),
+                           0, s, nunits, units, rowsb, k, (int)p.column_order, A.ptr, A.idx, B.idx,
                            b_rows(p, B.ptr), p.span_sb0, p.sb_off, p.subcnt, front.rownnz, band_off,
                            band_base, row_cur, row_loff, d_overflow, p.subocc, p.bandwords);
         TSG_LAUNCH_CHECK();
