@@ -17,10 +17,10 @@ SOURCE = r"""
 #include "tsg_internal.h"
 #include "tsg_expand.h"
 extern "C" int at(unsigned g, unsigned pe, int parts, int part, int lane) {
-    unsigned p;
+    int p;
     const bool in = parts == 1 ? entry_at<1>(g, pe, part, lane, p)
                                : entry_at<2>(g, pe, part, lane, p);
-    return in ? (int)p : -1;
+    return in ? p : -1;
 }
 """
 LAST = 2**31 - 1

@@ -90,13 +90,15 @@ struct RowRange {
 
 // Position p of a lane's entry in the group of a row's entries that starts at
 // g (PARTS groups interleaved, the lane's the part-th); false past the row's
-// end pe.  Groups are asked for up to three ahead of a row's last, so positions
-// are unsigned: they pass 2^31 at the end of 2^31 - 1 entries.
+// end pe.  Groups are asked for up to three ahead of a row's last, so g is
+// unsigned and the lane's offset compared with the entries left: g passes 2^31
+// at the end of 2^31 - 1 entries.  (Unsigned positions, compared and indexed
+// with, cost k_big_numeric_small two registers' spills.)
 template <int PARTS>
 __host__ __device__ __forceinline__ bool entry_at(unsigned g, unsigned pe, int part, int lane,
-                                                  unsigned &p) {
-    p = g + (unsigned)(PARTS * lane + part);
-    return p < pe;
+                                                  int &p) {
+    p = (int)(g + (unsigned)(PARTS * lane + part));
+    return PARTS * lane + part < (int)(pe - g);
 }
 
 // A row's entries [pa, pe) in groups of 64, loaded ahead of their use: while
@@ -116,11 +118,11 @@ struct EntryPipe {
     int lo, hi, lo1, hi1;          // the group's ranges, and the next one's
     double a, a1;
     __device__ __forceinline__ int col(unsigned g) const {
-        unsigned p;
+        int p;
         return entry_at<PARTS>(g, pe, part, __lane_id(), p) ? ja[p] : -1;
     }
     __device__ __forceinline__ double val(unsigned g) const {
-        unsigned p;
+        int p;
         return VALUES && entry_at<PARTS>(g, pe, part, __lane_id(), p) ? aval[p] : 0.0;
     }
     __device__ __forceinline__ void load(int pa_, int pe_) {
